@@ -53,8 +53,9 @@ enum ts2_epilogue {
     /* TStoreRowTileNormalize :495-525 and TStoreRowTileNormalizeRope (src/gpt/compute/gpu_rope.cuh:25-60): cType TS2_BF16;
      * v = alpha*acc; if normalize: tileScale[n/128][m] = rms over each 128-column tile * vecScale (0 for zero tiles), v /= it;
      * if rope.ptr: rotate (even, odd) column pairs of each 128-wide head by the row's (cos, sin) table fp32 [m][128].
-     * Carried by the 256x256-tile kernel (m, n multiples of 256 and (m/256)*(n/256) >= 192, or tileConfig 1) and, for TS2_E4M3 and
-     * TS2_BF16 operands, by the 128x128-tile kernel (tileConfig 2, or implied by tileGroup: the expert-grouped expand product,
+     * Carried by the 256x256-tile kernel (m, n multiples of 256 and (m/256)*(n/256) >= 192, or tileConfig 1), by the kernel for few tiles
+     * (tileConfig bit 16, automatic up to (m/64)*(n/128) = 768) and, for TS2_E4M3 and TS2_BF16 operands, by the 128x128-tile kernel
+     * (tileConfig 2, or implied by tileGroup: the expert-grouped expand product,
      * MatmulExpand.Forward<TStoreRowTileNormalize>, src/gpt/compute/layer_moe.cu:160-162); else TS2_ERR_UNSUPPORTED and the caller
      * runs ts2_row_tile_normalize_rope on a plain product. */
     TS2_EPI_ROW_TILE_NORM = 3
@@ -106,7 +107,9 @@ typedef struct ts2_gemm_args {
      * 512 tiles of 256x128; bit 15 (32768) switches that off.  The same kernel, on exchanged operands, takes tileGroup products
      * of TS2_E4M3 operands with a 16-bit stored result (plain or ROW_TILE_NORM; also with one further product) when n % 256 = 0,
      * k >= 512 bytes, c and its stride are multiples of 16 bytes and (m/128)*(n/256) >= 512 - or when bit 12 asks for it;
-     * results are bit-identical to the 128x128 kernels'. */
+     * results are bit-identical to the 128x128 kernels'.  Results with few tiles go to a kernel whose workgroups cut the contraction
+     * between their waves (64x128 tiles; 16-byte aligned rows of C): bit 16 (65536) asks for it (TS2_ERR_UNSUPPORTED for calls it cannot
+     * run), bit 17 (131072) keeps the other kernels. */
     int32_t tileConfig;
     /* Expert-grouped products (TMoeMatMulKernelCall / TMoeDeltaMatMulKernelCall, src/gpt/compute/moe_matmul.cuh:47-215):
      * tileGroup [m/128] (device): rows of A and C are grouped by expert in 128-row tiles; tile i multiplies the B slab

@@ -18,7 +18,7 @@
 //     max-normalise), row-tile normalise + RoPE to bf16, per-k-tile scales (exact int32 per tile, fp32 across tiles); the contraction
 //     can be cut into stored slices (deterministic split-K) or expert groups (MoE), and several products can be added into one
 //     result in one launch.
-#include "gemm_epilogue.h"
+#include "gemm_slice.h"
 #include <stdlib.h>
 
 using namespace gemmk;
@@ -1063,6 +1063,37 @@ template <int TYPE> int DispatchTile(const ts2_gemm_args *a, const GemmP &p, hip
     }
     return DispatchEpi<TYPE, 2, 2>(a, p, stream);
 }
+// Where the kernel for few tiles (gemm_slice.hip) takes over: by its workgroup count, 64 x 128 of C each, one per CU.  Measured in a graph of
+// 60 launches, 128x128 / 256x256 kernels -> slice kernel, us:
+//   packed delta        i8 512x256x512 10.8 -> 5.8, 2048x512x4096 24.5 -> 15.8; e4m3 512x256x512 10.3 -> 5.7, 2048x512x4096 18.9 -> 16.1,
+//                       1024x4096x4096 (512 workgroups) 27.7 -> 32.7
+//   contraction-major   e4m3 2048x512x4096 42.0 -> 16.0, 2048x2048x8192 75.0 -> 61.3, sliced four ways (256 large tiles) 40.8 -> 77.3
+//   several products    e4m3 4 x 512x256x256 28.5 -> 8.1, 4 x 4096x512x512 37.7 -> 12.8, 4 x 8192x1024x1024 55.6 -> 69.2
+//   i8 stored           512x256x256 6.7 -> 4.9, 2048x1024x1024 10.4 -> 8.6, 4096x512x2048 13.9 -> 11.4, 3072x1536x512 (576) 11.2 -> 16.4
+//   e4m3 stored fp32    512x256x256 6.4 -> 4.9, 4096x512x512 8.2 -> 7.1, 512x256x1024 6.6 -> 7.0, 1024x1024x4096 13.8 -> 16.2; as bf16
+//                       (row-owning epilogue there) 512x256x256 4.5 -> 4.9, 4096x512x2048 9.4 -> 10.8
+//   e4m3 accumulating   512x256x256 7.8 -> 5.2, 4096x512x2048 14.3 -> 11.7, 16384x512x512 (1024) 17.5 -> 27.3
+//   bf16                4096x256x1024 13.4 -> 10.4, 4096x1024x1024 (512) 15.5 -> 21.6
+bool PreferSlice(const GemmP &p, int type, int ct, int epi)
+{
+    const long wgs = (long)(p.m / 64) * (p.n / 128) * (p.splits > 1 ? p.splits : 1) * (p.groupOffsets ? p.splitK_groups : 1);
+    if (p.kMajor) {
+        return wgs <= 512;
+    }
+    if (p.nSeg > 1) {
+        return wgs <= 640;
+    }
+    if (ct == C_BF16NORM && !p.tileGroup) {
+        return wgs <= 768; // (the alternative for this size is a product and a separate pass)
+    }
+    if (ct == C_I8PACK) {
+        return wgs <= (type == T_I8 ? 512 : 384);
+    }
+    if (type == T_I8) {
+        return wgs <= 320;
+    }
+    return wgs <= 256 && (type == T_BF16 || epi == TS2_EPI_ADD || (ct == C_F32 && p.kBytes <= 512));
+}
 } // namespace
 
 extern "C" int ts2_gemm_nt(const ts2_gemm_args *a, void *streamPtr)
@@ -1224,6 +1255,17 @@ extern "C" int ts2_gemm_nt(const ts2_gemm_args *a, void *streamPtr)
                        : a->cType == TS2_I32                     ? C_I32
                                                                  : -1;
         const int epi = a->epilogue == TS2_EPI_ADD ? TS2_EPI_ADD : TS2_EPI_STORE;
+        // the kernel for results with few tiles: bit 16 asks for it, bit 17 keeps the others (comparison)
+        const bool askSlice = a->tileConfig & 65536;
+        if (ct >= 0 && splitK <= 1 && (askSlice || (!(a->tileConfig & (3 | 8 | 16 | 128 | 2048 | 4096 | 32768 | 131072)) && PreferSlice(p, type, ct, epi)))) {
+            SliceP sp = {};
+            sp.g = p;
+            sp.ct = ct;
+            sp.epi = epi;
+            if (askSlice || SliceCanRun(sp, type, p.kMajor != 0)) {
+                return RunSlice(sp, type, p.kMajor != 0, stream);
+            }
+        }
         if (a->tileConfig & 4096) {
             // bit 12: the persistent kernel whose epilogue runs under the next tile's main loop
             if (ct < 0 || splitK > 1 || (a->tileConfig & (4 | 8 | 16))) {

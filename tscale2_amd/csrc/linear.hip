@@ -305,8 +305,11 @@ extern "C" int ts2_matmul_forward_norm_rope(int32_t mode, int32_t len, int32_t l
     g.alpha = alpha;
     g.alphaPtr = alphaPtr;
     g.splitK = 1;
-    const bool fused = lenRound % 256 == 0 && dstDim % 256 == 0 && (int64_t)(lenRound / 256) * (dstDim / 256) >= 192;
-    if (fused) {
+    // the large tile from 192 tiles on; below, the kernel for few tiles (up to 768 of its workgroups) or, for fp8, the 128x128 tile
+    const bool large = lenRound % 256 == 0 && dstDim % 256 == 0 && (int64_t)(lenRound / 256) * (dstDim / 256) >= 192;
+    const bool few = (int64_t)(lenRound / 64) * (dstDim / 128) <= 768 && Aligned16(res->ptr, res->strideBytes) &&
+                     (!ropeBuf || Aligned16(ropeBuf->ptr, ropeBuf->strideBytes));
+    if (large || few || mode == TS2_E4M3) {
         g.c = *res;
         g.cType = TS2_BF16;
         g.epilogue = TS2_EPI_ROW_TILE_NORM;
