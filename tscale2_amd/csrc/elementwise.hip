@@ -808,22 +808,37 @@ __global__ void __launch_bounds__(256) NormalizeVecsRowMax(int len, int lenRound
     }
 }
 
-// The same quantiser with one wave per row for bf16 rows of NCH * 512 elements (at most 4096): a lane holds NCH chunks of 8
-// consecutive elements (16-byte loads, 8-byte stores, each instruction of the wave covering 1 KB / 512 B of the row), the row
+// The same quantiser with one wave per row for bf16 rows of at most NCH * 512 <= 4096 elements (a multiple of 8): a lane holds NCH chunks
+// of 8 consecutive elements (16-byte loads, 8-byte stores, each instruction of the wave covering 1 KB / 512 B of the row), the row
 // maxima are wave reductions, and no workgroup barrier or LDS exchange is left.  Same arithmetic per element as NormalizeVecsRowMax.
+// blockIdx.y = source: the gradients of a layer's matrices go in one launch (rows of 384 elements, 16384 of them: 13.6 us each one by one
+// with a workgroup per row).
+struct RowQuantJobs {
+    Mat src[4], dst[4];
+    float *rowScale[4], *rowAbsMax[4];
+    uint32_t seed[4];
+};
+
 template <int NCH>
-__global__ void __launch_bounds__(256) NormalizeRowsWave(int len, int lenRound, Mat src, const float *colScale, Mat dst, float *rowScale, float *rowAbsMax,
-    uint32_t seed)
+__global__ void __launch_bounds__(256) NormalizeRowsWave(int len, int lenRound, int dim, RowQuantJobs jobs, const float *colScale)
 {
+    const Mat src = jobs.src[blockIdx.y], dst = jobs.dst[blockIdx.y];
+    float *const rowScale = jobs.rowScale[blockIdx.y], *const rowAbsMax = jobs.rowAbsMax[blockIdx.y];
+    const uint32_t seed = jobs.seed[blockIdx.y];
     const int lane = threadIdx.x & 63;
+    bool in[NCH];
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+        in[i] = (i * 64 + lane) * 8 < dim;
+    }
     const int nWaves = gridDim.x * 4;
     // the column scales of the lane's chunks stay in registers for all the rows the wave walks
     F4 cs[NCH][2];
     if (colScale) {
 #pragma unroll
         for (int i = 0; i < NCH; ++i) {
-            cs[i][0] = Load4<TF32>(colScale + (i * 64 + lane) * 8);
-            cs[i][1] = Load4<TF32>(colScale + (i * 64 + lane) * 8 + 4);
+            cs[i][0] = in[i] ? Load4<TF32>(colScale + (i * 64 + lane) * 8) : ZeroF4();
+            cs[i][1] = in[i] ? Load4<TF32>(colScale + (i * 64 + lane) * 8 + 4) : ZeroF4();
         }
     }
     for (int t = blockIdx.x * 4 + (threadIdx.x >> 6); t < lenRound; t += nWaves) {
@@ -831,7 +846,9 @@ __global__ void __launch_bounds__(256) NormalizeRowsWave(int len, int lenRound, 
         if (t >= len) {
 #pragma unroll
             for (int i = 0; i < NCH; ++i) {
-                *(uint2 *)(out + (i * 64 + lane) * 8) = make_uint2(0u, 0u);
+                if (in[i]) {
+                    *(uint2 *)(out + (i * 64 + lane) * 8) = make_uint2(0u, 0u);
+                }
             }
             if (lane == 0) {
                 rowScale[t] = 0;
@@ -841,11 +858,11 @@ __global__ void __launch_bounds__(256) NormalizeRowsWave(int len, int lenRound, 
             }
             continue;
         }
-        const uint8_t *in = src.p + (int64_t)t * src.ld;
+        const uint8_t *row = src.p + (int64_t)t * src.ld;
         uint4 raw[NCH];
 #pragma unroll
         for (int i = 0; i < NCH; ++i) {
-            raw[i] = *(const uint4 *)(in + (i * 64 + lane) * 16);
+            raw[i] = in[i] ? *(const uint4 *)(row + (i * 64 + lane) * 16) : make_uint4(0, 0, 0, 0);
         }
         F4 v[NCH][2];
         float mx = 0, plain = 0;
@@ -871,6 +888,9 @@ __global__ void __launch_bounds__(256) NormalizeRowsWave(int len, int lenRound, 
         }
 #pragma unroll
         for (int i = 0; i < NCH; ++i) {
+            if (!in[i]) {
+                continue;
+            }
             if (seed) {
                 const int col4 = (i * 64 + lane) * 2;
                 *(uint2 *)(out + (i * 64 + lane) * 8) =
@@ -890,6 +910,82 @@ __global__ void __launch_bounds__(256) NormalizeRowsWave(int len, int lenRound, 
             if (rowAbsMax) {
                 rowAbsMax[t] = plain;
             }
+        }
+    }
+}
+
+// Row-major k-tile quantiser: dst[t][x] = sat_i8(rne(src[t][x] * rowMult[t] / scale)) with one scale per kTile rows, formed from the row maxima
+// that the row quantiser left (the arithmetic and the dither of TransposeQuant, without its transpose: the delta product reads both
+// operands contraction-major).  A workgroup takes 32 rows, which lie in one k-tile; rows in [len, lenRound) are cleared.  blockIdx.y = source;
+// tileScale: [sources][lenRound / kTile].
+struct TileQuantJobs {
+    Mat src[4], dst[4];
+    const float *rowAbsMax[4];
+    uint32_t seed[4];
+};
+
+__global__ void __launch_bounds__(256) QuantTileRows(int len, int lenRound, int dim, int kTile, TileQuantJobs jobs, const float *rowMult, float *tileScale)
+{
+    __shared__ float red[4];
+    const Mat src = jobs.src[blockIdx.y], dst = jobs.dst[blockIdx.y];
+    const float *rowAbsMax = jobs.rowAbsMax[blockIdx.y];
+    const uint32_t seed = jobs.seed[blockIdx.y];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int t0 = blockIdx.x * 32, k0 = t0 / kTile * kTile;
+    float mx = 0;
+    for (int t = k0 + tid; t < k0 + kTile && t < len; t += 256) {
+        float m = rowAbsMax[t];
+        if (rowMult) {
+            m *= fabsf(rowMult[t]);
+        }
+        mx = fmaxf(mx, m);
+    }
+    mx = WaveMax(mx);
+    if (lane == 0) {
+        red[wave] = mx;
+    }
+    __syncthreads();
+    const float tm = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    const float mult = tm > 0 ? 1 / (tm / 127) : 0.f;
+    if (tid == 0 && t0 == k0) {
+        tileScale[blockIdx.y * (lenRound / kTile) + t0 / kTile] = tm > 0 ? tm / 127 : 1.f;
+    }
+    // units of 8 elements, walked by the whole workgroup: four 16-byte loads in flight per lane
+    const int perRow = dim / 8, units = 32 * perRow;
+    for (int u0 = tid; u0 < units; u0 += 1024) {
+        uint4 raw[4];
+        float rm[4];
+        int r[4], c[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int u = u0 + k * 256;
+            r[k] = u < units ? t0 + u / perRow : lenRound;
+            c[k] = (u % perRow) * 8;
+            raw[k] = r[k] < len ? *(const uint4 *)At<TBF16>(src, r[k], c[k]) : make_uint4(0, 0, 0, 0);
+            rm[k] = (rowMult && r[k] < len) ? rowMult[r[k]] : 1.f;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (r[k] >= lenRound) {
+                continue;
+            }
+            const uint32_t w[4] = {raw[k].x, raw[k].y, raw[k].z, raw[k].w};
+            uint32_t packed[2] = {0, 0};
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const uint32_t word = seed ? DitherWord(seed, r[k], c[k] / 4 + q) : 0u;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t v = w[q * 2 + (e >> 1)];
+                    float x = __uint_as_float((e & 1) ? v & 0xffff0000u : v << 16);
+                    if (rowMult) {
+                        x = x * rm[k];
+                    }
+                    const float y = seed ? __builtin_fmaf(x, mult, DitherOffset(word, e)) : x * mult;
+                    packed[q] |= (uint32_t)(CvtToI8(y) & 0xff) << (8 * e);
+                }
+            }
+            *(uint2 *)At<TI8>(dst, r[k], c[k]) = r[k] < len ? make_uint2(packed[0], packed[1]) : make_uint2(0u, 0u);
         }
     }
 }
@@ -1583,6 +1679,76 @@ extern "C" int ts2_normalize_vecs_row_max(int32_t len, int32_t lenRound, const t
     return ts2_normalize_vecs_row_max2(len, lenRound, src, srcType, colScale, dst, rowScale, nullptr, stream);
 }
 
+static int LaunchRowQuant(int count, int len, int lenRound, int dim, const RowQuantJobs &jobs, const float *colScale, void *stream)
+{
+    // with column scales a wave walks several rows (the scales stay in registers), else one row per wave
+    const int wgs = (lenRound + 3) / 4;
+    const dim3 grid(colScale && wgs > 2048 ? 2048 : wgs, count);
+#define LAUNCH_RW(N) hipLaunchKernelGGL((NormalizeRowsWave<N>), grid, dim3(256), 0, STREAM, len, lenRound, dim, jobs, colScale)
+    switch ((dim + 511) / 512) {
+    case 1: LAUNCH_RW(1); break;
+    case 2: LAUNCH_RW(2); break;
+    case 3: LAUNCH_RW(3); break;
+    case 4: LAUNCH_RW(4); break;
+    case 5: LAUNCH_RW(5); break;
+    case 6: LAUNCH_RW(6); break;
+    case 7: LAUNCH_RW(7); break;
+    default: LAUNCH_RW(8); break;
+    }
+#undef LAUNCH_RW
+    TS2_CHECK_LAUNCH();
+    return TS2_OK;
+}
+
+// The row quantiser over `count` bf16 gradients of one shape.  Rows of dst 8-byte, of src 16-byte aligned; widths up to 4096
+int Ts2QuantRowsBatch(int count, int len, int lenRound, const ts2_mat *src, const ts2_mat *dst, float *const *rowScale, float *const *rowAbsMax,
+    const uint32_t *seed, void *stream)
+{
+    if (count < 1 || count > 4 || dst[0].x % 8 || dst[0].x > 4096 || lenRound < len) {
+        return TS2_ERR_SHAPE;
+    }
+    RowQuantJobs jobs = {};
+    for (int i = 0; i < count; ++i) {
+        if (dst[i].x != dst[0].x || !MatOk(&src[i], len, dst[0].x, 2) || !MatOk(&dst[i], lenRound, dst[0].x, 1)) {
+            return TS2_ERR_SHAPE;
+        }
+        if (!Aligned16(src[i].ptr, src[i].strideBytes) || (((uintptr_t)dst[i].ptr | dst[i].strideBytes) & 7)) {
+            return TS2_ERR_ALIGN;
+        }
+        jobs.src[i] = M(src[i]);
+        jobs.dst[i] = M(dst[i]);
+        jobs.rowScale[i] = rowScale[i];
+        jobs.rowAbsMax[i] = rowAbsMax[i];
+        jobs.seed[i] = seed[i];
+    }
+    return LaunchRowQuant(count, len, lenRound, dst[0].x, jobs, nullptr, stream);
+}
+
+// The row-major k-tile quantiser over `count` bf16 gradients of one shape; tileScale [count][lenRound / kTile]
+int Ts2QuantTileRows(int count, int len, int lenRound, int kTile, const ts2_mat *src, const ts2_mat *dst, const float *const *rowAbsMax,
+    const uint32_t *seed, const float *rowMult, float *tileScale, void *stream)
+{
+    if (count < 1 || count > 4 || dst[0].x % 8 || lenRound < len || kTile <= 0 || kTile % 128 || lenRound % kTile) {
+        return TS2_ERR_SHAPE;
+    }
+    TileQuantJobs jobs = {};
+    for (int i = 0; i < count; ++i) {
+        if (dst[i].x != dst[0].x || !MatOk(&src[i], len, dst[0].x, 2) || !MatOk(&dst[i], lenRound, dst[0].x, 1)) {
+            return TS2_ERR_SHAPE;
+        }
+        if (!Aligned16(src[i].ptr, src[i].strideBytes) || (((uintptr_t)dst[i].ptr | dst[i].strideBytes) & 7)) {
+            return TS2_ERR_ALIGN;
+        }
+        jobs.src[i] = M(src[i]);
+        jobs.dst[i] = M(dst[i]);
+        jobs.rowAbsMax[i] = rowAbsMax[i];
+        jobs.seed[i] = seed[i];
+    }
+    hipLaunchKernelGGL(QuantTileRows, dim3(lenRound / 32, count), dim3(256), 0, STREAM, len, lenRound, dst[0].x, kTile, jobs, rowMult, tileScale);
+    TS2_CHECK_LAUNCH();
+    return TS2_OK;
+}
+
 extern "C" int ts2_normalize_vecs_row_max_dither(int32_t len, int32_t lenRound, const ts2_mat *src, int32_t srcType, const float *colScale,
     const ts2_mat *dst, float *rowScale, float *rowAbsMax, uint32_t ditherSeed, void *stream)
 {
@@ -1594,25 +1760,15 @@ extern "C" int ts2_normalize_vecs_row_max_dither(int32_t len, int32_t lenRound, 
         return TS2_ERR_SHAPE;
     }
     const bool reg = dim <= 4096;
-    if (srcType == TS2_BF16 && dim % 512 == 0 && dim <= 4096 && Aligned16(src->ptr, src->strideBytes) && (((uintptr_t)dst->ptr | dst->strideBytes) & 7) == 0 &&
+    if (srcType == TS2_BF16 && dim % 8 == 0 && dim <= 4096 && Aligned16(src->ptr, src->strideBytes) && (((uintptr_t)dst->ptr | dst->strideBytes) & 7) == 0 &&
         (!colScale || ((uintptr_t)colScale & 15) == 0)) {
-        // with column scales a wave walks several rows (the scales stay in registers), else one row per wave
-        const int wgs = (lenRound + 3) / 4;
-        const dim3 grid(colScale && wgs > 2048 ? 2048 : wgs);
-#define LAUNCH_RW(N) hipLaunchKernelGGL((NormalizeRowsWave<N>), grid, dim3(256), 0, STREAM, len, lenRound, M(*src), colScale, M(*dst), rowScale, rowAbsMax, ditherSeed)
-        switch (dim / 512) {
-        case 1: LAUNCH_RW(1); break;
-        case 2: LAUNCH_RW(2); break;
-        case 3: LAUNCH_RW(3); break;
-        case 4: LAUNCH_RW(4); break;
-        case 5: LAUNCH_RW(5); break;
-        case 6: LAUNCH_RW(6); break;
-        case 7: LAUNCH_RW(7); break;
-        default: LAUNCH_RW(8); break;
-        }
-#undef LAUNCH_RW
-        TS2_CHECK_LAUNCH();
-        return TS2_OK;
+        RowQuantJobs jobs = {};
+        jobs.src[0] = M(*src);
+        jobs.dst[0] = M(*dst);
+        jobs.rowScale[0] = rowScale;
+        jobs.rowAbsMax[0] = rowAbsMax;
+        jobs.seed[0] = ditherSeed;
+        return LaunchRowQuant(1, len, lenRound, dim, jobs, colScale, stream);
     }
 #define LAUNCH_RM(TS, REG) hipLaunchKernelGGL((NormalizeVecsRowMax<TS, REG>), dim3(lenRound < 4096 ? lenRound : 4096), dim3(256), 0, STREAM, len, lenRound, dim, M(*src), colScale, M(*dst), rowScale, rowAbsMax, ditherSeed)
     if (srcType == TS2_BF16) {

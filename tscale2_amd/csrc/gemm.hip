@@ -1190,12 +1190,15 @@ extern "C" int ts2_gemm_nt(const ts2_gemm_args *a, void *streamPtr)
     }
     p.nSeg = 1;
     p.rowsF16 = 0;
+    bool onlyFewTiles = false; // several products on a shape that only the kernel for few tiles takes
     if (a->extraSegments) {
         const bool bigTile = (a->m % 256) == 0 && (a->n % 256) == 0 && (a->tileConfig & 3) <= 1 && !(a->tileConfig & (4 | 8 | 16)) && !a->tileGroup;
         // the 128x128 tile (chosen with tileConfig 2, or implied by tileGroup) takes one further product
         const bool smallTile = a->extraSegments == 1 && ((a->tileConfig & 3) == 2 || a->tileGroup) && !(a->tileConfig & (4 | 8 | 16)) &&
             !a->splitSlabBytes;
-        if (a->extraSegments < 0 || a->extraSegments > 3 || !(bigTile || smallTile) || a->abType == TS2_I8 || a->rowScale || a->kTileScale ||
+        const bool fewTiles = (a->tileConfig & 65536) || (!(a->tileConfig & (3 | 8 | 16 | 128 | 2048 | 4096 | 32768 | 131072)) && !a->tileGroup &&
+            (int64_t)(a->m / 64) * (a->n / 128) <= 640 && Aligned16(a->c.ptr, a->c.strideBytes));
+        if (a->extraSegments < 0 || a->extraSegments > 3 || !(bigTile || smallTile || fewTiles) || a->abType == TS2_I8 || a->rowScale || a->kTileScale ||
             a->groupOffsets || splitK > 1 || (a->cType != TS2_F32 && a->cType != TS2_BF16) ||
             (a->epilogue != TS2_EPI_STORE && a->epilogue != TS2_EPI_ADD)) {
             return TS2_ERR_UNSUPPORTED;
@@ -1213,6 +1216,7 @@ extern "C" int ts2_gemm_nt(const ts2_gemm_args *a, void *streamPtr)
             p.segAlphaPtr[i] = a->segment[i].alphaPtr;
         }
         p.nSeg = 1 + a->extraSegments;
+        onlyFewTiles = !bigTile && !smallTile;
     }
     p.splits = 1;
     p.splitSlab = 0;
@@ -1265,6 +1269,9 @@ extern "C" int ts2_gemm_nt(const ts2_gemm_args *a, void *streamPtr)
             if (askSlice || SliceCanRun(sp, type, p.kMajor != 0)) {
                 return RunSlice(sp, type, p.kMajor != 0, stream);
             }
+        }
+        if (onlyFewTiles) {
+            return TS2_ERR_UNSUPPORTED;
         }
         if (a->tileConfig & 4096) {
             // bit 12: the persistent kernel whose epilogue runs under the next tile's main loop

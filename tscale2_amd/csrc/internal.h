@@ -19,3 +19,22 @@ int Ts2TransposeQuantRows(int len, int lenRound, const ts2_mat *src, int srcType
     int kTile, const int *rowIndex, const ts2_mat *dstT, int dstType, float *tileScale, void *stream, uint32_t ditherSeed = 0);
 // resolves, for the current device, what ts2_moe_route_static otherwise resolves on its first call there (no stream operation)
 int Ts2MoeRouteSetup();
+// the int8 row quantiser (ts2_normalize_vecs_row_max_dither) over `count` <= 4 bf16 gradients of one width <= 4096, one launch
+int Ts2QuantRowsBatch(int count, int len, int lenRound, const ts2_mat *src, const ts2_mat *dst, float *const *rowScale, float *const *rowAbsMax,
+    const uint32_t *seed, void *stream);
+// the k-tile quantiser without the transpose, over `count` <= 4 bf16 gradients of one width: dst[t][x] with one scale per kTile rows,
+// tileScale [count][lenRound / kTile]
+int Ts2QuantTileRows(int count, int len, int lenRound, int kTile, const ts2_mat *src, const ts2_mat *dst, const float *const *rowAbsMax,
+    const uint32_t *seed, const float *rowMult, float *tileScale, void *stream);
+// packed delta [gradDim][srcDim] = alpha * *alphaPtr * sum over the rows of grad^T src, both operands row-major as they lie (rows len ..
+// lenRound of both hold zeros); mode TS2_I8 (with kTileScale [gradDim / kTileScaleRows][lenRound / kTile]; kTileScaleRows 0 = one set),
+// TS2_E4M3 or TS2_BF16.  Chooses kernel and token slices by cost; partial: fp32 scratch for the slices.  TS2_ERR_UNSUPPORTED: no kernel for it
+int Ts2DeltaRows(int mode, int len, int lenRound, int srcDim, int gradDim, const ts2_mat *src, const ts2_mat *grad, const float *kTileScale, int kTile,
+    int kTileScaleRows, float alpha, const float *alphaPtr, float *partial, int64_t partialFloats, const ts2_mat *delta, const ts2_mat *tileScale,
+    void *stream);
+// int8: srcGrad (+)= sum_i alpha_i * *alphaPtr_i * rowScale_i[t] * (grad8_i W_i^T), count <= 4 products of one shape added in order
+int Ts2BackpropGroupI8(int count, int len, int lenRound, int srcDim, int gradDim, const ts2_mat *grad8, const float *const *rowScale,
+    const ts2_mat *transformT, const float *alpha, const float *const *alphaPtr, const ts2_mat *srcGrad, int srcGradType, int add, void *stream);
+// per-group deltas (TMoeDeltaMatMulKernelCall) by the kernel for few tiles: groups * gradDim rows of packed delta
+int Ts2GroupedDeltaRows(int rows, int srcDim, int gradDim, int groups, const int *groupOffsets, const ts2_mat *src, const ts2_mat *grad, float alpha,
+    const float *alphaPtr, const ts2_mat *delta, int64_t deltaSlabBytes, const ts2_mat *tileScale, int64_t tileScaleSlabBytes, void *stream);

@@ -14,6 +14,7 @@
 
 namespace
 {
+constexpr int QUANT_ROW_MAX = 4096; // widest gradient of the batched int8 row quantiser
 constexpr float VEC = 1 / 24.0f;    // STATE/Q/K/V/FFN/MOE_VEC_SCALE, src/gpt/compute/cfg_precision.h:72-77
 constexpr float DISCR = 1 / 32.0f;  // MODEL_DISCR_SCALE, src/gpt/model_params/model_dim.h:9
 constexpr float LN2F = 0.693147f;   // LOG2, model_dim.h:16
@@ -78,10 +79,9 @@ struct TLayer {
     int attId = 0;
     TMatrix w[5];
     TActs *acts = nullptr;
-    // fp8 attention layers: the packed deltas of Q, K, V and gate are row blocks of one [4Q][dim] array (and column blocks of one
-    // tile-scale array), so that one delta product over the four stacked transposed gradients fills them all
-    TMatrix qkvg;
-    bool fusedDelta = false;
+    // The packed deltas of the matrices that read the layer input (attention: Q, K, V, gate; FFN: expand, gate) are row blocks of one
+    // array (and column blocks of one tile-scale array): one delta product over their gradients, which lie side by side, fills them all
+    TMatrix stack;
 };
 
 enum { LT_ATT = 0, LT_FFN = 2, LT_MOE = 3 };
@@ -135,7 +135,6 @@ struct ts2_model {
     bool keep = false;      // FFN and attention layers own activation sets
     bool useKept = false;   // inside ModelBackprop: the backward of a layer starts from what its forward left
     int sharedOwner = -1;   // the MoE layer whose forward filled the shared set, its gathered input and the routing tables last
-    Arr g32;                                 // fp32 [R'][maxW] gradient scratch (drg / dvlg)
     Arr gf[4];                               // fast-gradient type [R'][maxW]: dwide/dq, dgate, dk, dv
     Arr g16[4];                              // bf16 [R'][maxW]: -, dVal, dK, dV
     Arr dScale;                              // fp32 [heads][R]
@@ -144,14 +143,16 @@ struct ts2_model {
     Arr normMoe, sgMoe, moeSel, dMoeSel;     // grouped 8-bit input / gradient, select logits fp32, their gradient
     float *dExpertWeight = 0;
     // final layer
-    Arr logits, gradV, gradVT, fnT, wfT;
+    Arr logits, gradV, fnT, wfT;
     Arr logits16;                            // IEEE-half logits of the backward pass (the fp32 ones serve ts2_model_forward)
     // linear backward scratch
     uint8_t *sGrad8 = 0, *sGradT = 0, *sSrcT = 0, *sWT = 0;
-    uint8_t *sGradTa = 0, *sGradTb = 0; // transposed gradients written by their producer (fp8 FFN backward)
+    int stackW = 0; // columns of the gradient scratch sGradT (and sGrad8): maxW, or the stacked gradients of a layer
+    Arr lastFast[4]; // where the layer backward that ran last left its fast-type gradients
     float *sPartial = 0;                     // fp32 slices of a delta product with few output tiles
     size_t sPartialFloats = 0;
-    float *sRowScale = 0, *sTileMax = 0, *sTileScale = 0;
+    float *sRowScale = 0, *sTileMax = 0, *sTileScale = 0; // [4][RP], [RP / 128 + 1], [4][RP / 128 + 1]
+    float *sRowAbsMax = 0;                                // [4][RP]: row maxima of the int8 gradients quantised last
     uint32_t ditherCalls = 0; // uses of the linear operator so far (seeds of the int8 dither)
     int maxW = 0, RP = 0; // RP = rows of the row-indexed scratch (max(R, lenMoe))
     int cuCount = 256;
@@ -208,6 +209,19 @@ Arr Flat(void *p, int rows, int cols, int type)
     return r;
 }
 
+// every use of an int8 quantiser draws its own noise: the call counter runs on from step to step
+uint32_t NextDither(ts2_model *M)
+{
+    if (!M->cfg.ditherSeed) {
+        return 0;
+    }
+    uint32_t h = M->cfg.ditherSeed + 0x9E3779B9u * ++M->ditherCalls;
+    h ^= h >> 15;
+    h *= 0x2C1B3C6Du;
+    h ^= h >> 12;
+    return h | 1u;
+}
+
 ts2_matmul_bwd_buffers Scratch(ts2_model *M, int rows, int srcDim, int gradDim)
 {
     ts2_matmul_bwd_buffers b = {};
@@ -218,14 +232,7 @@ ts2_matmul_bwd_buffers Scratch(ts2_model *M, int rows, int srcDim, int gradDim)
     b.tileMax = M->sTileMax;
     b.tileScale = M->sTileScale;
     b.transformT = Flat(M->sWT, srcDim, gradDim, M->mode).m;
-    if (M->cfg.ditherSeed) {
-        // every use of the operator draws its own noise: the call counter runs on from step to step
-        uint32_t h = M->cfg.ditherSeed + 0x9E3779B9u * ++M->ditherCalls;
-        h ^= h >> 15;
-        h *= 0x2C1B3C6Du;
-        h ^= h >> 12;
-        b.ditherSeed = h | 1u;
-    }
+    b.ditherSeed = NextDither(M);
     return b;
 }
 
@@ -271,11 +278,32 @@ int BackpropDXGroup(ts2_model *M, int count, TMatrix *const *W, const Arr *const
     const float *ap[4];
     const int srcDim = W[0]->srcDim, dstDim = W[0]->dstDim;
     if (M->mode != TS2_E4M3) {
-        // int8: the row-quantised gradient lives in the one shared scratch, so the products go one after the other
-        for (int i = 0; i < count; ++i) {
-            CK(BackpropDX(M, *W[i], *grad[i], alpha, useScale[i], srcGrad, add || i > 0, s));
+        if (dstDim > QUANT_ROW_MAX || count * dstDim > M->stackW) {
+            // the quantiser's one-launch form ends here: the products go one after the other through the shared scratch
+            for (int i = 0; i < count; ++i) {
+                CK(BackpropDX(M, *W[i], *grad[i], alpha, useScale[i], srcGrad, add || i > 0, s));
+            }
+            return 0;
         }
-        return 0;
+        ts2_mat g16[4], g8[4], wT[4];
+        float *rs[4], *ram[4];
+        uint32_t seed[4];
+        for (int i = 0; i < count; ++i) {
+            g16[i] = grad[i]->m;
+            g8[i] = Flat(M->sGrad8 + (size_t)i * M->R * dstDim, M->R, dstDim, TS2_I8).m;
+            rs[i] = M->sRowScale + (size_t)i * M->RP;
+            ram[i] = M->sRowAbsMax + (size_t)i * M->RP;
+            seed[i] = NextDither(M);
+            al[i] = alpha;
+            ap[i] = useScale[i] ? W[i]->scale : nullptr;
+            if (!W[i]->fastTValid) {
+                CK(ts2_transpose_quant(dstDim, dstDim, W[i]->fast.P(), M->mode, nullptr, nullptr, 0, nullptr, W[i]->fastT.P(), M->mode, nullptr, s));
+                W[i]->fastTValid = true;
+            }
+            wT[i] = W[i]->fastT.m;
+        }
+        CK(Ts2QuantRowsBatch(count, M->len, M->R, g16, g8, rs, ram, seed, s));
+        return Ts2BackpropGroupI8(count, M->len, M->R, srcDim, dstDim, g8, rs, wT, al, ap, srcGrad.P(), srcGrad.type, add, s);
     }
     for (int i = 0; i < count; ++i) {
         if (W[i]->srcDim != srcDim || W[i]->dstDim != dstDim) {
@@ -300,39 +328,6 @@ int BackpropDXGroup(ts2_model *M, int count, TMatrix *const *W, const Arr *const
     return ts2_matmul_backprop_group(M->mode, M->len, M->R, srcDim, dstDim, count, gp, bp, al, ap, srcGrad.P(), srcGrad.type, add, s);
 }
 
-// slices of the token axis for a delta product [dstDim x srcDim]: enough to give every CU a 256x256 tile, each slice a whole number of
-// k-tiles and at least 4096 tokens long
-int DeltaSplits(ts2_model *M, int srcDim, int dstDim)
-{
-    if (M->mode != TS2_E4M3) {
-        return 1;
-    }
-    if ((srcDim % 256) || (dstDim % 256)) {
-        // 128x128 tiles (the select matrix of a MoE layer: 128 x dim): two workgroups per CU, slices of at least 2048 tokens
-        int tiles = (srcDim / 128) * (dstDim / 128), splits = 1;
-        while (splits < 32 && tiles * splits < 512 && M->R % (splits * 2 * 128) == 0 && M->R / (splits * 2) >= 2048) {
-            splits *= 2;
-        }
-        return splits;
-    }
-    int tiles = (srcDim / 256) * (dstDim / 256);
-    if (tiles >= 192) {
-        return 1;
-    }
-    int splits = 1;
-    while (splits < 8 && tiles * splits < 192 && M->R % (splits * 2 * 128) == 0 && M->R / (splits * 2) >= 4096) {
-        splits *= 2;
-    }
-    return splits;
-}
-
-// fp8 operands, whole 128-row groups, both widths on the 256 grid: the delta product contracts over the rows of gradient and source as
-// they lie in memory (ts2_gemm_args.kMajor), so nobody has to leave or make a transpose of either
-bool DeltaReadsRows(ts2_model *M, int srcDim, int dstDim)
-{
-    return M->mode == TS2_E4M3 && M->fastGradType == TS2_E4M3 && M->len == M->R && (srcDim % 256) == 0 && (dstDim % 256) == 0;
-}
-
 // columns [k * cols, (k + 1) * cols) of a
 Arr ColBlock(const Arr &a, int k, int cols)
 {
@@ -342,24 +337,51 @@ Arr ColBlock(const Arr &a, int k, int cols)
     return r;
 }
 
-// delta = alpha * gradScale * gradFast^T * src8   (TMatMulBuffers::BackpropDelta)
-int BackpropDelta(ts2_model *M, TMatrix &W, const Arr &src8, const Arr &gradFast, float alpha, const float *gradScale, void *s,
-    bool sameSrcAsLastCall = false, const Arr *gradTReady = nullptr)
+// Deltas alpha * gradScale * grad_i^T * src8 (TMatMulBuffers::BackpropDelta) of `count` matrices of one shape that read the same input, as
+// row blocks of W.delta; W is the layer's stack, or the one matrix.
+// fp8: `grad` holds the gradients side by side ([R][count * width]) and the product reads both operands as they lie.
+// int8: grads[i] are bf16; their row maxima were left in slot i by the dX product that precedes this call (BackpropDXGroup with the
+// same gradients), the k-tile quantiser writes them side by side.
+int BackpropDelta(ts2_model *M, TMatrix &W, const Arr &src8, const Arr &grad, float alpha, const float *gradScale, void *s)
 {
-    ts2_matmul_bwd_buffers b = Scratch(M, M->R, W.srcDim, W.dstDim);
-    b.srcTValid = sameSrcAsLastCall; // the matrices of a layer that share their input transpose it once
-    if (gradTReady) { // the producer of the gradient left its transpose
-        b.gradT = gradTReady->m;
-        b.gradTValid = 1;
+    return Ts2DeltaRows(M->mode, M->len, M->R, W.srcDim, W.dstDim, src8.P(), grad.P(), nullptr, 0, 0, alpha, gradScale, M->sPartial,
+        (int64_t)M->sPartialFloats, W.delta.P(), W.deltaTileScale.P(), s);
+}
+
+int BackpropDeltaI8(ts2_model *M, int count, TMatrix &stack, TMatrix *const *W, const Arr &src8, const Arr *const *grads, float alpha,
+    const float *gradScale, void *s)
+{
+    const int width = W[0]->dstDim, all = count * width;
+    if (width <= QUANT_ROW_MAX && all <= M->stackW) {
+        const int nTiles = (M->R / M->kTile + 3) / 4;
+        if (nTiles == 1 || (size_t)nTiles * all * W[0]->srcDim <= M->sPartialFloats) {
+            Arr g = Flat(M->sGradT, M->R, all, TS2_I8);
+            ts2_mat g16[4], g8[4];
+            const float *ram[4];
+            uint32_t seed[4];
+            for (int i = 0; i < count; ++i) {
+                g16[i] = grads[i]->m;
+                g8[i] = ColBlock(g, i, width).m;
+                ram[i] = M->sRowAbsMax + (size_t)i * M->RP;
+                seed[i] = NextDither(M);
+            }
+            CK(Ts2QuantTileRows(count, M->len, M->R, M->kTile, g16, g8, ram, seed, nullptr, M->sTileScale, s));
+            return Ts2DeltaRows(TS2_I8, M->len, M->R, stack.srcDim, all, src8.P(), g.P(), M->sTileScale, M->kTile, width, alpha, gradScale, M->sPartial,
+                (int64_t)M->sPartialFloats, stack.delta.P(), stack.deltaTileScale.P(), s);
+        }
     }
-    // a delta with fewer large tiles than the chip has CUs runs as slices of the token axis on the large tile, packed afterwards
-    int splits = DeltaSplits(M, W.srcDim, W.dstDim);
-    if (splits > 1 && (size_t)splits * W.dstDim * W.srcDim <= M->sPartialFloats) {
-        b.partial = Flat(M->sPartial, splits * W.dstDim, W.srcDim, TS2_F32).m;
-        b.splits = splits;
+    // large results: the transposing quantiser and the large tiles, one matrix after the other
+    for (int i = 0; i < count; ++i) {
+        ts2_matmul_bwd_buffers b = Scratch(M, M->R, W[i]->srcDim, W[i]->dstDim);
+        b.srcTValid = i > 0;
+        if (width <= QUANT_ROW_MAX && all <= M->stackW) {
+            b.gradRowAbsMax = M->sRowAbsMax + (size_t)i * M->RP;
+            b.gradRowAbsMaxValid = 1;
+        }
+        CK(ts2_matmul_backprop_delta(M->mode, M->len, M->R, W[i]->srcDim, W[i]->dstDim, src8.P(), nullptr, grads[i]->P(), grads[i]->type, alpha,
+            gradScale, M->kTile, &b, W[i]->delta.P(), W[i]->deltaTileScale.P(), s));
     }
-    return ts2_matmul_backprop_delta(M->mode, M->len, M->R, W.srcDim, W.dstDim, src8.P(), nullptr, gradFast.P(), gradFast.type, alpha, gradScale,
-        M->kTile, &b, W.delta.P(), W.deltaTileScale.P(), s);
+    return 0;
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
@@ -391,31 +413,29 @@ int FfnBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
     Arr wide16 = View(A.a16[0], R, F), gate16 = View(A.a16[1], R, F), wideScale = View(A.tsc[0], F / 128, R), rg8 = View(A.rg8, R, F);
     // drg travels in bf16 (the reference uses half here): its consumer rounds to the 8-bit gradient type anyway
     Arr drg = View(M->g16[0], R, F), dwide = View(M->gf[0], R, F), dgate = View(M->gf[1], R, F);
+    const bool i8 = M->mode == TS2_I8;
+    Arr gStack = Flat(M->sGradT, R, 2 * F, M->fastGradType);
+    if (!i8) { // the two gradients side by side
+        dwide = ColBlock(gStack, 0, F);
+        dgate = ColBlock(gStack, 1, F);
+    }
+    M->lastFast[0] = dwide;
+    M->lastFast[1] = dgate;
     if (!(M->useKept && A.valid)) {
         CK(FfnComputeRG(M, L, norm8, s));
     }
-    // contract backward
-    CK(BackpropDX(M, L.w[2], M->stateGradFast, DISCR * Dot(F), true, drg, false, s));
-    // fp8: the gate/norm backward also writes the transposed gradients that the two delta products contract over
-    const bool fusedT = !DeltaReadsRows(M, D, F) && M->mode == TS2_E4M3 && M->fastGradType == TS2_E4M3 && M->sGradTa && (R % 128) == 0;
-    Arr dwideT = Flat(M->sGradTa, F, R, TS2_E4M3), dgateT = Flat(M->sGradTb, F, R, TS2_E4M3);
-    if (fusedT) {
-        CK(ts2_backprop_row_tile_normalize_lolu_t(len, R, gate16.P(), wide16.P(), VEC, wideScale.P(), drg.P(), dgate.P(), dwide.P(), dgateT.P(),
-            dwideT.P(), s));
-    } else {
-        CK(ts2_backprop_row_tile_normalize_lolu(len, R, gate16.P(), wide16.P(), VEC, wideScale.P(), drg.P(), TS2_BF16, dgate.P(), dwide.P(),
-            M->fastGradType, s));
-    }
-    {
-        TMatrix *const ws[2] = {&L.w[0], &L.w[1]};
-        const Arr *const gs[2] = {&dwide, &dgate};
-        const bool us[2] = {true, false};
-        CK(BackpropDXGroup(M, 2, ws, gs, DISCR * Dot(D), us, M->dNormState, false, s));
-    }
-    // deltas (sources are stored in 1/24 units)
-    CK(BackpropDelta(M, L.w[2], rg8, M->stateGradFast, VEC, gradScale, s));
-    CK(BackpropDelta(M, L.w[0], norm8, dwide, VEC, gradScale, s, false, fusedT ? &dwideT : nullptr));
-    return BackpropDelta(M, L.w[1], norm8, dgate, VEC, gradScale, s, true, fusedT ? &dgateT : nullptr);
+    // contract backward: dX, then the delta (its source is stored in 1/24 units)
+    TMatrix *const wc[1] = {&L.w[2]};
+    const Arr *const sg[1] = {&M->stateGradFast};
+    const bool scaled[2] = {true, false};
+    CK(BackpropDXGroup(M, 1, wc, sg, DISCR * Dot(F), scaled, drg, false, s));
+    CK(i8 ? BackpropDeltaI8(M, 1, L.w[2], wc, rg8, sg, VEC, gradScale, s) : BackpropDelta(M, L.w[2], rg8, M->stateGradFast, VEC, gradScale, s));
+    CK(ts2_backprop_row_tile_normalize_lolu(len, R, gate16.P(), wide16.P(), VEC, wideScale.P(), drg.P(), TS2_BF16, dgate.P(), dwide.P(),
+        M->fastGradType, s));
+    TMatrix *const ws[2] = {&L.w[0], &L.w[1]};
+    const Arr *const gs[2] = {&dwide, &dgate};
+    CK(BackpropDXGroup(M, 2, ws, gs, DISCR * Dot(D), scaled, M->dNormState, false, s));
+    return i8 ? BackpropDeltaI8(M, 2, L.stack, ws, norm8, gs, VEC, gradScale, s) : BackpropDelta(M, L.stack, norm8, gStack, VEC, gradScale, s);
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
@@ -467,21 +487,31 @@ int AttBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
     TActs &A = *L.acts;
     Arr q16 = View(A.a16[0], R, Q), gate16 = View(A.a16[1], R, Q), k16 = View(A.a16[2], R, Q), v16 = View(A.a16[3], R, Q);
     Arr qScale = View(A.tsc[0], H, R), vScale = View(A.tsc[1], H, R), val16 = View(A.val16, R, Q), vlg8 = View(A.rg8, R, Q);
-    Arr dvlg = View(M->g16[0], R, Q), dGate = View(M->gf[1], R, Q), dVal16 = View(M->g16[1], R, Q);
-    // one delta product for the four matrices that read the layer input, contracting over rows: their gradients are written side by side
-    // as column blocks of one [R][4Q] array (the transpose scratch, which nothing else uses then)
-    const bool stacked = L.fusedDelta && DeltaReadsRows(M, D, 4 * Q);
+    Arr dvlg = View(M->g16[0], R, Q), dVal16 = View(M->g16[1], R, Q);
+    Arr dQf = View(M->gf[0], R, Q), dGate = View(M->gf[1], R, Q), dKf = View(M->gf[2], R, Q), dVf = View(M->gf[3], R, Q);
+    const bool i8 = M->mode == TS2_I8;
+    // fp8: the gradients of the four matrices that read the layer input side by side, as column blocks of one [R][4Q] array
     Arr gStack = Flat(M->sGradT, R, 4 * Q, M->fastGradType);
-    if (stacked) {
+    if (!i8) {
+        dQf = ColBlock(gStack, 0, Q);
+        dKf = ColBlock(gStack, 1, Q);
+        dVf = ColBlock(gStack, 2, Q);
         dGate = ColBlock(gStack, 3, Q);
     }
+    M->lastFast[0] = dQf;
+    M->lastFast[1] = dGate;
+    M->lastFast[2] = dKf;
+    M->lastFast[3] = dVf;
     if (!(M->useKept && A.valid)) {
         CK(AttComputeVLG(M, L, norm8, s));
     }
     A.valid = false; // the backward reuses val16's storage for dQ
     // combiner backward
-    CK(BackpropDX(M, L.w[4], M->stateGradFast, DISCR * Dot(Q), true, dvlg, false, s));
-    CK(BackpropDelta(M, L.w[4], vlg8, M->stateGradFast, VEC, gradScale, s));
+    TMatrix *const wc[1] = {&L.w[4]};
+    const Arr *const sg[1] = {&M->stateGradFast};
+    const bool useScale[4] = {true, true, true, false};
+    CK(BackpropDXGroup(M, 1, wc, sg, DISCR * Dot(Q), useScale, dvlg, false, s));
+    CK(i8 ? BackpropDeltaI8(M, 1, L.w[4], wc, vlg8, sg, VEC, gradScale, s) : BackpropDelta(M, L.w[4], vlg8, M->stateGradFast, VEC, gradScale, s));
     // gate backward + dScale
     CK(ts2_backprop_lolu_dscale(len, R, gate16.P(), val16.P(), 1.f, dvlg.P(), TS2_BF16, dGate.P(), M->fastGradType, dVal16.P(), TS2_BF16,
         M->dScale.P(), s));
@@ -510,42 +540,13 @@ int AttBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
     ag.which = 3;
     CK(ts2_att_backward(&ag, s));
     // epilogues: norm backward against the stored rotated vector, then inverse rope (TStoreAttBack*, gpu_att_utils.cuh:280-352)
-    Arr dQf = View(M->gf[0], R, Q), dKf = View(M->gf[2], R, Q), dVf = View(M->gf[3], R, Q);
-    if (stacked) {
-        dQf = ColBlock(gStack, 0, Q);
-        dKf = ColBlock(gStack, 1, Q);
-        dVf = ColBlock(gStack, 2, Q);
-    }
     CK(ts2_backprop_row_tile_normalize_rope(len, R, dQ.P(), TS2_BF16, 1.f, q16.P(), qScale.P(), M->rope.P(), dQf.P(), M->fastGradType, s));
     CK(ts2_backprop_row_tile_normalize_rope(len, R, dK.P(), TS2_BF16, 1.f, nullptr, nullptr, M->rope.P(), dKf.P(), M->fastGradType, s));
     CK(ts2_backprop_row_tile_normalize_rope(len, R, dV.P(), TS2_BF16, 1.f, v16.P(), vScale.P(), nullptr, dVf.P(), M->fastGradType, s));
-    float a = DISCR * Dot(D);
-    {
-        TMatrix *const ws[4] = {&L.w[0], &L.w[1], &L.w[2], &L.w[3]};
-        const Arr *const gs[4] = {&dQf, &dKf, &dVf, &dGate};
-        const bool us[4] = {true, true, true, false};
-        CK(BackpropDXGroup(M, 4, ws, gs, a, us, M->dNormState, false, s));
-    }
-    if (stacked) {
-        return BackpropDelta(M, L.qkvg, norm8, gStack, VEC, gradScale, s);
-    }
-    if (L.fusedDelta) {
-        // the four transposed gradients stacked as row blocks of one [4Q][R] array, then one delta product [4Q x D]: 256 large tiles
-        // instead of four products of 64 that each need token-axis slices and a pack pass
-        Arr gT = Flat(M->sGradT, 4 * Q, R, M->mode);
-        const Arr *const gs4[4] = {&dQf, &dKf, &dVf, &dGate};
-        for (int k = 0; k < 4; ++k) {
-            Arr blk = gT;
-            blk.m.ptr = (uint8_t *)gT.m.ptr + (size_t)k * Q * gT.m.strideBytes;
-            blk.m.y = Q;
-            CK(ts2_transpose_quant(len, R, gs4[k]->P(), M->mode, nullptr, nullptr, 0, nullptr, blk.P(), M->mode, nullptr, s));
-        }
-        return BackpropDelta(M, L.qkvg, norm8, dQf, VEC, gradScale, s, false, &gT);
-    }
-    CK(BackpropDelta(M, L.w[0], norm8, dQf, VEC, gradScale, s));
-    CK(BackpropDelta(M, L.w[1], norm8, dKf, VEC, gradScale, s, true));
-    CK(BackpropDelta(M, L.w[2], norm8, dVf, VEC, gradScale, s, true));
-    return BackpropDelta(M, L.w[3], norm8, dGate, VEC, gradScale, s, true);
+    TMatrix *const ws[4] = {&L.w[0], &L.w[1], &L.w[2], &L.w[3]};
+    const Arr *const gs[4] = {&dQf, &dKf, &dVf, &dGate};
+    CK(BackpropDXGroup(M, 4, ws, gs, DISCR * Dot(D), useScale, M->dNormState, false, s));
+    return i8 ? BackpropDeltaI8(M, 4, L.stack, ws, norm8, gs, VEC, gradScale, s) : BackpropDelta(M, L.stack, norm8, gStack, VEC, gradScale, s);
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
@@ -590,26 +591,21 @@ int GroupedGemm(ts2_model *M, const Arr &a, const Arr &bSlabs, int slabRows, int
 }
 
 // per-expert delta: delta_e[gradDim][srcDim] = alpha * gradScale * sum over the expert's rows of grad^T src
-int GroupedDelta(ts2_model *M, TMatrix &W, const Arr &src8, const Arr &gradFast, float alpha, const float *gradScale, void *s,
-    bool sameSrcAsLastCall = false)
+int GroupedDelta(ts2_model *M, TMatrix &W, const Arr &src8, const Arr &gradFast, float alpha, const float *gradScale, void *s)
 {
     int E = M->cfg.expertCount, rows = M->lenMoe;
-    ts2_gemm_args g = {};
-    if (M->fastGradType == TS2_E4M3 && (W.srcDim % 256) == 0 && (W.dstDim % 256) == 0) {
-        // every row of the expert-ordered arrays is written (pad rows of an expert's group hold zeros): contract over them as they lie
-        g.a = gradFast.m;
-        g.b = src8.m;
-        g.kMajor = 1;
-        g.tileConfig = 1;
-    } else {
-        Arr gradT = Flat(M->sGradT, W.dstDim, rows, M->mode), srcT = Flat(M->sSrcT, W.srcDim, rows, M->mode);
-        CK(ts2_transpose_quant(rows, rows, gradFast.P(), M->mode, nullptr, nullptr, 0, nullptr, gradT.P(), M->mode, nullptr, s));
-        if (!sameSrcAsLastCall) { // (the expand and gate matrices share their source: one transpose)
-            CK(ts2_transpose_quant(rows, rows, src8.P(), M->mode, nullptr, nullptr, 0, nullptr, srcT.P(), M->mode, nullptr, s));
-        }
-        g.a = gradT.m;
-        g.b = srcT.m;
+    // every row of the expert-ordered arrays is written (pad rows of an expert's group hold zeros): contract over them as they lie.
+    // Few tiles, or widths off the 256 grid: the kernel for few tiles (256 x 512 per expert, 8 experts: 21.5 -> 7 us)
+    ts2_mat ts = W.deltaTileScale.m;
+    if ((W.srcDim % 256) || (W.dstDim % 256) || (int64_t)(W.dstDim / 64) * (W.srcDim / 128) * E <= 512) {
+        return Ts2GroupedDeltaRows(rows, W.srcDim, W.dstDim, E, M->moe.expertOffset, src8.P(), gradFast.P(), alpha, gradScale, W.delta.P(),
+            (int64_t)W.dstDim * W.delta.m.strideBytes, &ts, (int64_t)W.dstDim * 4, s);
     }
+    ts2_gemm_args g = {};
+    g.a = gradFast.m;
+    g.b = src8.m;
+    g.kMajor = 1;
+    g.tileConfig = 1;
     g.c = W.delta.m;
     g.c.y = W.dstDim;
     g.abType = M->mode;
@@ -702,7 +698,7 @@ int MoeBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
     // expert deltas
     CK(GroupedDelta(M, L.w[2], rg8, M->sgMoe, VEC, gradScale, s));
     CK(GroupedDelta(M, L.w[0], M->normMoe, dwide, VEC, gradScale, s));
-    return GroupedDelta(M, L.w[1], M->normMoe, dgate, VEC, gradScale, s, true);
+    return GroupedDelta(M, L.w[1], M->normMoe, dgate, VEC, gradScale, s);
 }
 } // namespace
 
@@ -710,13 +706,14 @@ int MoeBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
 // step driver
 namespace
 {
-int InitMatrix(ts2_model *M, TMatrix *W, int srcDim, int dstDim, int slabs, bool keepT = true)
+// ownDelta false: the matrix' delta is a part of its layer's stack (InitStack)
+int InitMatrix(ts2_model *M, TMatrix *W, int srcDim, int dstDim, int slabs, bool keepT = true, bool ownDelta = true)
 {
     W->srcDim = srcDim;
     W->dstDim = dstDim;
     W->slabs = slabs;
-    if (!M->Alloc(&W->fast, dstDim * slabs, srcDim, M->mode) || !M->Alloc(&W->delta, dstDim * slabs, srcDim, TS2_I8) ||
-        !M->Alloc(&W->deltaTileScale, srcDim / 128, dstDim * slabs, TS2_F32)) {
+    if (!M->Alloc(&W->fast, dstDim * slabs, srcDim, M->mode) ||
+        (ownDelta && (!M->Alloc(&W->delta, dstDim * slabs, srcDim, TS2_I8) || !M->Alloc(&W->deltaTileScale, srcDim / 128, dstDim * slabs, TS2_F32)))) {
         return TS2_ERR_LAUNCH;
     }
     // the transposed copy the dX products contract over, kept while the weights do not change (expert matrices: slab by slab)
@@ -725,6 +722,25 @@ int InitMatrix(ts2_model *M, TMatrix *W, int srcDim, int dstDim, int slabs, bool
     }
     W->scale = (float *)M->Dev(4);
     return W->scale ? 0 : TS2_ERR_LAUNCH;
+}
+
+// the first `count` matrices of a layer (equal shapes) write their deltas as row blocks of one array
+int InitStack(ts2_model *M, TLayer *L, int count, int srcDim, int dstDim)
+{
+    L->stack.srcDim = srcDim;
+    L->stack.dstDim = count * dstDim;
+    if (!M->Alloc(&L->stack.delta, count * dstDim, srcDim, TS2_I8) || !M->Alloc(&L->stack.deltaTileScale, srcDim / 128, count * dstDim, TS2_F32)) {
+        return TS2_ERR_LAUNCH;
+    }
+    for (int k = 0; k < count; ++k) {
+        L->w[k].delta = L->stack.delta;
+        L->w[k].delta.m.ptr = (uint8_t *)L->stack.delta.m.ptr + (size_t)k * dstDim * L->stack.delta.m.strideBytes;
+        L->w[k].delta.m.y = dstDim;
+        L->w[k].deltaTileScale = L->stack.deltaTileScale;
+        L->w[k].deltaTileScale.m.ptr = (uint8_t *)L->stack.deltaTileScale.m.ptr + (size_t)k * dstDim * 4;
+        L->w[k].deltaTileScale.m.x = dstDim;
+    }
+    return 0;
 }
 
 int RoundUp(int x, int m)
@@ -818,23 +834,21 @@ int FinalBackward(ts2_model *M, void *s)
     g.epilogue = TS2_EPI_STORE;
     g.splitK = 1;
     CK(ts2_gemm_nt(&g, s));
-    // delta_final[v][d] = sum_t grad[t][v] * fn[t][d]
-    ts2_gemm_args h = {};
-    if (M->len == R && (VP % 256) == 0 && (D % 256) == 0) {
-        // whole row groups: the product contracts over the rows of the gradient and of the final state as they lie
-        // (Fp16MatMul<1, 1, TStoreDelta>, gpu_final.cuh:265); the 8-bit state only changes its type
-        Arr fn16 = Flat(M->fnT.m.ptr, R, D, TS2_BF16);
-        CK(Ts2RowsToBf16(M->len, R, D, M->normState[depth].P(), M->mode, fn16.P(), s));
-        h.a = M->gradV.m;
-        h.b = fn16.m;
-        h.kMajor = 1;
-        h.tileConfig = 1;
-    } else {
-        CK(Ts2TransposeToBf16(M->len, R, VP, M->gradV.P(), TS2_BF16, M->gradVT.P(), s));
-        CK(Ts2TransposeToBf16(M->len, R, D, M->normState[depth].P(), M->mode, M->fnT.P(), s));
-        h.a = M->gradVT.m;
-        h.b = M->fnT.m;
+    // delta_final[v][d] = sum_t grad[t][v] * fn[t][d]: the product contracts over the rows of the gradient and of the final state as they
+    // lie (Fp16MatMul<1, 1, TStoreDelta>, gpu_final.cuh:265); the 8-bit state only changes its type.  Pad rows of both hold zeros
+    Arr fn16 = Flat(M->fnT.m.ptr, R, D, TS2_BF16);
+    CK(Ts2RowsToBf16(M->len, R, D, M->normState[depth].P(), M->mode, fn16.P(), s));
+    if ((VP % 256) || (D % 256) || (VP / 256) * (D / 256) < 192) {
+        CK(Ts2DeltaRows(TS2_BF16, M->len, R, D, VP, fn16.P(), M->gradV.P(), nullptr, 0, 0, VEC, nullptr, M->sPartial, (int64_t)M->sPartialFloats,
+            M->finalW.delta.P(), M->finalW.deltaTileScale.P(), s));
+        return ts2_backprop_final_normalize(M->len, R, M->normState[depth].P(), M->mode, M->stateScale[depth].P(), M->dNormState.P(),
+            M->stateGrad.P(), M->stateGradFast.P(), M->fastGradType, M->gradMaxNorm, s);
     }
+    ts2_gemm_args h = {};
+    h.a = M->gradV.m;
+    h.b = fn16.m;
+    h.kMajor = 1;
+    h.tileConfig = 1;
     h.c = M->finalW.delta.m;
     h.abType = TS2_BF16;
     h.cType = TS2_I8;
@@ -849,7 +863,7 @@ int FinalBackward(ts2_model *M, void *s)
     // their own at a fraction of the CUs.  They run as slices of the token axis instead (stored fp32 products, packed afterwards).
     const int tilesM = VP / 256, tilesN = D / 256, cus = M->cuCount;
     const int rowsPerRound = tilesN > 0 && cus % tilesN == 0 ? cus / tilesN : 0;
-    const int tailRows = h.kMajor && rowsPerRound > 0 && tilesM > rowsPerRound ? tilesM % rowsPerRound : 0;
+    const int tailRows = rowsPerRound > 0 && tilesM > rowsPerRound ? tilesM % rowsPerRound : 0;
     int tailSplits = tailRows > 0 ? cus / (tailRows * tilesN) : 0;
     tailSplits = tailSplits > 8 ? 8 : tailSplits;
     if (tailSplits >= 2 && R / tailSplits >= 2048 && (size_t)tailSplits * tailRows * 256 * D <= M->sPartialFloats) {
@@ -965,28 +979,15 @@ extern "C" ts2_model *ts2_model_create(const ts2_model_config *cfg)
         L.attId = cfg->layerAttId[d];
         if (L.type == LT_ATT) {
             for (int k = 0; k < 4; ++k) {
-                ok &= InitMatrix(M, &L.w[k], D, H * 128, 1) == 0;
+                ok &= InitMatrix(M, &L.w[k], D, H * 128, 1, true, false) == 0;
             }
             ok &= InitMatrix(M, &L.w[4], H * 128, D, 1) == 0;
-            const int Q = H * 128;
-            if (ok && M->mode == TS2_E4M3 && 4 * Q <= maxW && (Q % 256) == 0 && (D % 256) == 0) {
-                L.qkvg.srcDim = D;
-                L.qkvg.dstDim = 4 * Q;
-                ok &= M->Alloc(&L.qkvg.delta, 4 * Q, D, TS2_I8) && M->Alloc(&L.qkvg.deltaTileScale, D / 128, 4 * Q, TS2_F32);
-                for (int k = 0; k < 4 && ok; ++k) {
-                    L.w[k].delta = L.qkvg.delta;
-                    L.w[k].delta.m.ptr = (uint8_t *)L.qkvg.delta.m.ptr + (size_t)k * Q * L.qkvg.delta.m.strideBytes;
-                    L.w[k].delta.m.y = Q;
-                    L.w[k].deltaTileScale = L.qkvg.deltaTileScale;
-                    L.w[k].deltaTileScale.m.ptr = (uint8_t *)L.qkvg.deltaTileScale.m.ptr + (size_t)k * Q * 4;
-                    L.w[k].deltaTileScale.m.x = Q;
-                }
-                L.fusedDelta = ok;
-            }
+            ok = ok && InitStack(M, &L, 4, D, H * 128) == 0;
         } else if (L.type == LT_FFN) {
-            ok &= InitMatrix(M, &L.w[0], D, F, 1) == 0;
-            ok &= InitMatrix(M, &L.w[1], D, F, 1) == 0;
+            ok &= InitMatrix(M, &L.w[0], D, F, 1, true, false) == 0;
+            ok &= InitMatrix(M, &L.w[1], D, F, 1, true, false) == 0;
             ok &= InitMatrix(M, &L.w[2], F, D, 1) == 0;
+            ok = ok && InitStack(M, &L, 2, D, F) == 0;
         } else if (L.type == LT_MOE) {
             ok &= InitMatrix(M, &L.w[0], D, X, E) == 0;
             ok &= InitMatrix(M, &L.w[1], D, X, E) == 0;
@@ -1022,7 +1023,7 @@ extern "C" ts2_model *ts2_model_create(const ts2_model_config *cfg)
     M->lossSum = (float *)M->Dev(4);
     // layer scratch
     int RP = M->RP;
-    ok &= M->Alloc(&M->raw, RP, maxW, TS2_F32) && M->Alloc(&M->g32, RP, maxW, TS2_F32) && M->Alloc(&M->shared.rg8, RP, maxW, M->mode);
+    ok &= M->Alloc(&M->raw, RP, maxW, TS2_F32) && M->Alloc(&M->shared.rg8, RP, maxW, M->mode);
     for (int k = 0; k < 4; ++k) {
         ok &= M->Alloc(&M->shared.a16[k], RP, maxW, TS2_BF16) && M->Alloc(&M->g16[k], RP, maxW, TS2_BF16) &&
               M->Alloc(&M->gf[k], RP, maxW, M->fastGradType);
@@ -1069,20 +1070,22 @@ extern "C" ts2_model *ts2_model_create(const ts2_model_config *cfg)
         }
     }
     // keep the two statistics arrays on one stride
-    M->sGrad8 = (uint8_t *)M->Dev((size_t)RP * maxW);
-    M->sGradT = (uint8_t *)M->Dev((size_t)RP * maxW);
-    if (M->mode == TS2_E4M3) {
-        M->sGradTa = (uint8_t *)M->Dev((size_t)RP * maxW);
-        M->sGradTb = (uint8_t *)M->Dev((size_t)RP * maxW);
-        ok &= M->sGradTa && M->sGradTb;
+    M->stackW = maxW;
+    for (const TLayer &L : M->layers) {
+        const int w = L.type == LT_ATT ? 4 * H * 128 : L.type == LT_FFN ? 2 * F : 0;
+        M->stackW = w > M->stackW ? w : M->stackW;
     }
+    M->sGrad8 = (uint8_t *)M->Dev(M->mode == TS2_I8 ? (size_t)RP * M->stackW : 16);
+    M->sGradT = (uint8_t *)M->Dev((size_t)RP * M->stackW);
     M->sSrcT = (uint8_t *)M->Dev((size_t)RP * maxW);
     M->sWT = (uint8_t *)M->Dev((size_t)4 * maxW * maxW); // up to four transposed weights side by side (BackpropDXGroup)
     M->sPartialFloats = (size_t)8 * 2048 * 2048; // eight slices of a 2048 x 2048 delta, four of a 4096 x 2048 one
     M->sPartial = (float *)M->Dev(M->sPartialFloats * 4);
-    M->sRowScale = (float *)M->Dev((size_t)RP * 4);
+    M->sRowScale = (float *)M->Dev((size_t)4 * RP * 4);
+    M->sRowAbsMax = (float *)M->Dev((size_t)4 * RP * 4);
     M->sTileMax = (float *)M->Dev((size_t)(RP / 128 + 1) * 4);
-    M->sTileScale = (float *)M->Dev((size_t)(RP / 128 + 1) * 4);
+    M->sTileScale = (float *)M->Dev((size_t)4 * (RP / 128 + 1) * 4);
+    ok &= M->sRowScale && M->sRowAbsMax && M->sTileMax && M->sTileScale;
     if (hasMoe) {
         int total = R * cfg->moeSelected;
         M->moe.sampleExpertIds = (int *)M->Dev((size_t)total * 4);
@@ -1097,7 +1100,7 @@ extern "C" ts2_model *ts2_model_create(const ts2_model_config *cfg)
         ok &= M->Alloc(&M->normMoe, M->lenMoe, D, M->mode) && M->Alloc(&M->sgMoe, M->lenMoe, D, M->fastGradType) &&
               M->Alloc(&M->moeSel, R, SelectDim, TS2_F32) && M->Alloc(&M->dMoeSel, R, SelectDim, M->fastGradType);
     }
-    ok &= M->Alloc(&M->logits, R, VP, TS2_F32) && M->Alloc(&M->logits16, R, VP, TS2_F16) && M->Alloc(&M->gradV, R, VP, TS2_BF16) && M->Alloc(&M->gradVT, VP, R, TS2_BF16) &&
+    ok &= M->Alloc(&M->logits, R, VP, TS2_F32) && M->Alloc(&M->logits16, R, VP, TS2_F16) && M->Alloc(&M->gradV, R, VP, TS2_BF16) &&
           M->Alloc(&M->fnT, D, R, TS2_BF16) && M->Alloc(&M->wfT, D, VP, TS2_BF16);
     if (!ok || !M->sGrad8 || !M->sGradT || !M->sSrcT || !M->sWT || !M->sPartial) {
         delete M;
@@ -1344,6 +1347,9 @@ extern "C" int ts2_model_set_batch(ts2_model *M, int32_t len, const int32_t *lab
     if (stream && hipStreamSynchronize((hipStream_t)stream) != hipSuccess) {
         return TS2_ERR_LAUNCH;
     }
+    if (len < M->len && Ts2ZeroRows(M->stateGradFast.P(), M->R, M->cfg.dim * ElemSz(M->fastGradType), stream) != TS2_OK) {
+        return TS2_ERR_LAUNCH; // rows beyond the batch hold zeros: the delta products contract over whole tiles of rows
+    }
     M->len = len;
     int R = M->R;
     std::vector<int> tg(R, -1), st(R, 0), fi(R, -1);
@@ -1483,7 +1489,8 @@ extern "C" int ts2_model_array(ts2_model *M, const char *name, int32_t index, ts
         // f0..f3 fast-gradient type (dwide / dq, dgate, dk, dv), dscale fp32 [heads][lenRound]
         const char *f = name + 8;
         if ((f[0] == 'g' || f[0] == 'f') && f[1] >= '0' && f[1] <= '3' && !f[2] && index <= M->maxW) {
-            tmp = View(f[0] == 'g' ? M->g16[f[1] - '0'] : M->gf[f[1] - '0'], M->R, index);
+            const Arr &last = M->lastFast[f[1] - '0'];
+            tmp = View(f[0] == 'g' ? M->g16[f[1] - '0'] : last.m.ptr && index <= last.m.x ? last : M->gf[f[1] - '0'], M->R, index);
         } else if (!strcmp(f, "dscale")) {
             tmp = M->dScale;
         } else {

@@ -1,6 +1,7 @@
 // Linear-layer backward operator: the call sequences of TMatMulBuffers (src/gpt/compute/layer_cuda_base.cuh:153-250) expressed
 // over the kernels of this library.  Host code only; every step is enqueued on the caller's stream.
 #include "common.h"
+#include "gemm_slice.h"
 #include "internal.h"
 
 namespace
@@ -8,6 +9,59 @@ namespace
 bool Is8(int mode)
 {
     return mode == TS2_I8 || mode == TS2_E4M3;
+}
+
+int SliceType(int mode)
+{
+    return mode == TS2_I8 ? gemmk::T_I8 : mode == TS2_E4M3 ? gemmk::T_FP8 : gemmk::T_BF16;
+}
+
+// the kernel for few tiles on row-major operands: splits == 1 packs the delta, otherwise fp32 slices go to `partial` (dense slabs)
+int DeltaSlice(int mode, int len, int lenRound, int srcDim, int gradDim, const ts2_mat *src, const ts2_mat *grad, const float *kTileScale, int kTile,
+    int kTileScaleRows, float alpha, const float *alphaPtr, int splits, float *partial, const ts2_mat *delta, const ts2_mat *tileScale, void *stream)
+{
+    gemmk::SliceP sp = {};
+    gemmk::GemmP &g = sp.g;
+    g.a = (const uint8_t *)grad->ptr;
+    g.b = (const uint8_t *)src->ptr;
+    g.lda = grad->strideBytes;
+    g.ldb = src->strideBytes;
+    g.m = gradDim;
+    g.n = srcDim;
+    g.kBytes = lenRound * (mode == TS2_BF16 ? 2 : 1);
+    g.kTileScale = kTileScale;
+    g.kTileBytes = kTile;
+    g.nSeg = 1;
+    sp.kLive = len;
+    sp.kTileScaleRows = kTileScaleRows;
+    sp.epi = TS2_EPI_STORE;
+    if (grad->x < gradDim || src->x < srcDim || grad->y < len || src->y < len || delta->x < srcDim || delta->y < gradDim ||
+        tileScale->x < gradDim || tileScale->y < srcDim / TILE || (kTileScale && (grad->y < lenRound || src->y < lenRound))) {
+        return TS2_ERR_SHAPE;
+    }
+    if (splits > 1) {
+        g.c = (uint8_t *)partial;
+        g.ldc = (int64_t)srcDim * 4;
+        g.splits = splits;
+        g.splitSlab = (int64_t)gradDim * g.ldc;
+        g.alpha = 1.f;
+        sp.ct = gemmk::C_F32;
+        int rc = gemmk::RunSlice(sp, SliceType(mode), true, (hipStream_t)stream);
+        if (rc) {
+            return rc;
+        }
+        ts2_mat part = {partial, g.ldc, srcDim, splits * gradDim};
+        return ts2_pack_delta(&part, splits, g.splitSlab, gradDim, srcDim, alpha, alphaPtr, delta, tileScale, stream);
+    }
+    g.c = (uint8_t *)delta->ptr;
+    g.ldc = delta->strideBytes;
+    g.splits = 1;
+    g.alpha = alpha;
+    g.alphaPtr = alphaPtr;
+    g.tileScale = (float *)tileScale->ptr;
+    g.ldTileScale = tileScale->strideBytes / 4;
+    sp.ct = gemmk::C_I8PACK;
+    return gemmk::RunSlice(sp, SliceType(mode), true, (hipStream_t)stream);
 }
 } // namespace
 
@@ -116,7 +170,10 @@ extern "C" int ts2_matmul_backprop_group(int32_t mode, int32_t len, int32_t lenR
             return TS2_ERR_NULL;
         }
     }
-    bool one = mode == TS2_E4M3 && count > 1 && (lenRound % 256) == 0 && (srcDim % 256) == 0 && (srcGradType == TS2_F32 || srcGradType == TS2_BF16);
+    // one launch: the 256x256 tile, or the kernel for few tiles
+    bool one = mode == TS2_E4M3 && count > 1 && (srcGradType == TS2_F32 || srcGradType == TS2_BF16) &&
+               (((lenRound % 256) == 0 && (srcDim % 256) == 0) ||
+                   ((int64_t)(lenRound / 64) * (srcDim / 128) <= 640 && Aligned16(srcGrad->ptr, srcGrad->strideBytes)));
     for (int i = 1; i < count && one; ++i) {
         one = grad[i]->strideBytes == grad[0]->strideBytes && bufs[i]->transformT.strideBytes == bufs[0]->transformT.strideBytes;
     }
@@ -205,6 +262,15 @@ extern "C" int ts2_matmul_backprop_delta(int32_t mode, int32_t len, int32_t lenR
         }
         // both operands as they lie in memory, [token][feature]: the kernel's LDS reads do the transposing
         kMajor = (len == lenRound || buf->padRowsZero) && (gradDim % 256) == 0 && (srcDim % 256) == 0 && grad->y >= lenRound && src->y >= lenRound;
+        // widths off the 256 grid, or pad rows that nobody vouches for: the kernel for few tiles, which stops at row len.  Beyond 512 of
+        // its workgroups two transposes and the large tile are cheaper (measured line of the dispatcher)
+        const int cuts = buf->partial.ptr && buf->splits > 1 ? buf->splits : 1;
+        if (!kMajor && !buf->gradTValid && cuts == 1 && (int64_t)(gradDim / 64) * (srcDim / 128) <= 512) {
+            rc = DeltaSlice(TS2_E4M3, len, lenRound, srcDim, gradDim, src, grad, nullptr, 0, 0, alpha, gradScale, 1, nullptr, delta, deltaTileScale, stream);
+            if (rc != TS2_ERR_UNSUPPORTED) {
+                return rc;
+            }
+        }
         if (!kMajor && !buf->gradTValid) {
             rc = ts2_transpose_quant(len, lenRound, grad, TS2_E4M3, nullptr, nullptr, 0, nullptr, &buf->gradT, TS2_E4M3, nullptr, stream);
             if (rc) {
@@ -213,7 +279,7 @@ extern "C" int ts2_matmul_backprop_delta(int32_t mode, int32_t len, int32_t lenR
         }
     }
     const int *rowOrder = (mode == TS2_I8 && buf->sortRows) ? buf->rowOrder : nullptr;
-    if (!kMajor && (!buf->srcTValid || rowOrder)) {
+    if (!kMajor && (mode == TS2_E4M3 || !buf->srcTValid || rowOrder)) {
         rc = ts2_transpose_quant(len, lenRound, src, mode, nullptr, nullptr, 0, rowOrder, &buf->srcT, mode, nullptr, stream);
         if (rc) {
             return rc;
@@ -334,4 +400,184 @@ extern "C" int ts2_matmul_forward_norm_rope(int32_t mode, int32_t len, int32_t l
         return rc;
     }
     return ts2_row_tile_normalize_rope(len, lenRound, raw, TS2_F32, 1.f, normalize, vecScale, ropeBuf, res, tileScale, stream);
+}
+
+// ---------------------------------------------------------------------------------------------------------------------------
+// Entry points of the model driver (internal.h)
+
+// Time of a delta product in microseconds.  Both kernels walk their contraction at the rate one CU can fill its LDS from the caches, so a
+// launch is (rounds of 256 workgroups) x (start and epilogue + steps): 0.7 us per 256-byte step on 64x128 for the kernel for few tiles, 1.17 us
+// per 128-byte step on 256x256 for the ring kernel (2048 x 2048 over 8192 rows: 61 us / 75 us measured, 53 / 81 by this).  Slices add a
+// write and a read of fp32 per slice (4 TB/s from the caches) and the packing launch.
+static double DeltaCost(bool ring, int64_t tiles, int64_t rowBytes, int splits, double outElems)
+{
+    const double rounds = (double)((tiles * splits + 255) / 256);
+    const double steps = ring ? (double)((rowBytes / splits + 127) / 128) : (double)((rowBytes / splits + 255) / 256);
+    return rounds * (ring ? 6 + 1.17 * steps : 4 + 0.7 * steps) + (splits > 1 ? 3.5 + splits * outElems * 8 / 4e6 : 0);
+}
+
+int Ts2DeltaRows(int mode, int len, int lenRound, int srcDim, int gradDim, const ts2_mat *src, const ts2_mat *grad, const float *kTileScale, int kTile,
+    int kTileScaleRows, float alpha, const float *alphaPtr, float *partial, int64_t partialFloats, const ts2_mat *delta, const ts2_mat *tileScale,
+    void *stream)
+{
+    const int64_t outElems = (int64_t)gradDim * srcDim, sliceTiles = (int64_t)(gradDim / 64) * (srcDim / 128);
+    if (mode == TS2_I8) {
+        // four k-tiles per workgroup
+        const int splits = (lenRound / kTile + 3) / 4;
+        if (splits > 1 && splits * outElems > partialFloats) {
+            return TS2_ERR_UNSUPPORTED;
+        }
+        return DeltaSlice(mode, len, lenRound, srcDim, gradDim, src, grad, kTileScale, kTile, kTileScaleRows, alpha, alphaPtr, splits, partial, delta,
+            tileScale, stream);
+    }
+    const int64_t rowBytes = (int64_t)lenRound * (mode == TS2_BF16 ? 2 : 1);
+    const bool ringRuns = (gradDim % 256) == 0 && (srcDim % 256) == 0 && grad->y >= lenRound && src->y >= lenRound;
+    double best = 1e30;
+    bool ring = false;
+    int splits = 1;
+    for (int s = 1; s <= 32 && (s == 1 || s * outElems <= partialFloats); s *= 2) {
+        if (s > 1 && rowBytes / s < 512) {
+            break;
+        }
+        double c = DeltaCost(false, sliceTiles, rowBytes, s, (double)outElems);
+        if (c < best) {
+            best = c;
+            ring = false;
+            splits = s;
+        }
+        c = DeltaCost(true, sliceTiles / 8, rowBytes, s, (double)outElems);
+        if (ringRuns && c < best) {
+            best = c;
+            ring = true;
+            splits = s;
+        }
+    }
+    if (!ring) {
+        return DeltaSlice(mode, len, lenRound, srcDim, gradDim, src, grad, nullptr, 0, 0, alpha, alphaPtr, splits, partial, delta, tileScale, stream);
+    }
+    ts2_gemm_args g = {};
+    g.a = *grad;
+    g.b = *src;
+    g.abType = mode;
+    g.m = gradDim;
+    g.n = srcDim;
+    g.k = lenRound;
+    g.kMajor = 1;
+    g.tileConfig = 1;
+    g.splitK = 1;
+    if (splits > 1) {
+        g.c = {partial, (int64_t)srcDim * 4, srcDim, gradDim};
+        g.cType = TS2_F32;
+        g.alpha = 1.f;
+        g.epilogue = TS2_EPI_STORE;
+        g.splitK = splits;
+        g.splitSlabBytes = outElems * 4;
+        int rc = ts2_gemm_nt(&g, stream);
+        if (rc) {
+            return rc;
+        }
+        ts2_mat part = {partial, (int64_t)srcDim * 4, srcDim, splits * gradDim};
+        return ts2_pack_delta(&part, splits, g.splitSlabBytes, gradDim, srcDim, alpha, alphaPtr, delta, tileScale, stream);
+    }
+    g.c = *delta;
+    g.cType = TS2_I8;
+    g.alpha = alpha;
+    g.alphaPtr = alphaPtr;
+    g.epilogue = TS2_EPI_ROW_TILE_MAXNORM;
+    g.tileScale = *tileScale;
+    return ts2_gemm_nt(&g, stream);
+}
+
+int Ts2GroupedDeltaRows(int rows, int srcDim, int gradDim, int groups, const int *groupOffsets, const ts2_mat *src, const ts2_mat *grad, float alpha,
+    const float *alphaPtr, const ts2_mat *delta, int64_t deltaSlabBytes, const ts2_mat *tileScale, int64_t tileScaleSlabBytes, void *stream)
+{
+    gemmk::SliceP sp = {};
+    gemmk::GemmP &g = sp.g;
+    g.a = (const uint8_t *)grad->ptr;
+    g.b = (const uint8_t *)src->ptr;
+    g.c = (uint8_t *)delta->ptr;
+    g.lda = grad->strideBytes;
+    g.ldb = src->strideBytes;
+    g.ldc = delta->strideBytes;
+    g.m = gradDim;
+    g.n = srcDim;
+    g.kBytes = rows;
+    g.alpha = alpha;
+    g.alphaPtr = alphaPtr;
+    g.tileScale = (float *)tileScale->ptr;
+    g.ldTileScale = tileScale->strideBytes / 4;
+    g.nSeg = 1;
+    g.splits = 1;
+    g.groupOffsets = groupOffsets;
+    g.splitK_groups = groups;
+    g.cSlab = deltaSlabBytes;
+    g.tileScaleSlab = tileScaleSlabBytes / 4;
+    sp.ct = gemmk::C_I8PACK;
+    sp.epi = TS2_EPI_STORE;
+    return gemmk::RunSlice(sp, gemmk::T_FP8, true, (hipStream_t)stream);
+}
+
+int Ts2BackpropGroupI8(int count, int len, int lenRound, int srcDim, int gradDim, const ts2_mat *grad8, const float *const *rowScale,
+    const ts2_mat *transformT, const float *alpha, const float *const *alphaPtr, const ts2_mat *srcGrad, int srcGradType, int add, void *stream)
+{
+    if (count < 1 || count > 4) {
+        return TS2_ERR_SHAPE;
+    }
+    bool one = count > 1 && (srcGradType == TS2_F32 || srcGradType == TS2_BF16) && (int64_t)(lenRound / 64) * (srcDim / 128) <= 640;
+    for (int i = 1; i < count && one; ++i) {
+        one = grad8[i].strideBytes == grad8[0].strideBytes && transformT[i].strideBytes == transformT[0].strideBytes;
+    }
+    if (one) {
+        gemmk::SliceP sp = {};
+        gemmk::GemmP &g = sp.g;
+        g.a = (const uint8_t *)grad8[0].ptr;
+        g.b = (const uint8_t *)transformT[0].ptr;
+        g.c = (uint8_t *)srcGrad->ptr;
+        g.lda = grad8[0].strideBytes;
+        g.ldb = transformT[0].strideBytes;
+        g.ldc = srcGrad->strideBytes;
+        g.m = lenRound;
+        g.n = srcDim;
+        g.kBytes = gradDim;
+        g.mLive = len;
+        g.rowScale = rowScale[0];
+        g.alpha = alpha[0];
+        g.alphaPtr = alphaPtr[0];
+        g.splits = 1;
+        g.nSeg = count;
+        for (int i = 1; i < count; ++i) {
+            g.segA[i - 1] = (const uint8_t *)grad8[i].ptr;
+            g.segB[i - 1] = (const uint8_t *)transformT[i].ptr;
+            g.segAlpha[i - 1] = alpha[i];
+            g.segAlphaPtr[i - 1] = alphaPtr[i];
+            sp.segRowScale[i - 1] = rowScale[i];
+        }
+        sp.ct = srcGradType == TS2_F32 ? gemmk::C_F32 : gemmk::C_BF16;
+        sp.epi = add ? TS2_EPI_ADD : TS2_EPI_STORE;
+        if (gemmk::SliceCanRun(sp, gemmk::T_I8, false)) {
+            return gemmk::RunSlice(sp, gemmk::T_I8, false, (hipStream_t)stream);
+        }
+    }
+    for (int i = 0; i < count; ++i) {
+        ts2_gemm_args g = {};
+        g.a = grad8[i];
+        g.b = transformT[i];
+        g.c = *srcGrad;
+        g.abType = TS2_I8;
+        g.cType = srcGradType;
+        g.m = lenRound;
+        g.n = srcDim;
+        g.k = gradDim;
+        g.mLive = len;
+        g.rowScale = rowScale[i];
+        g.alpha = alpha[i];
+        g.alphaPtr = alphaPtr[i];
+        g.epilogue = (add || i > 0) ? TS2_EPI_ADD : TS2_EPI_STORE;
+        g.splitK = 1;
+        int rc = ts2_gemm_nt(&g, stream);
+        if (rc) {
+            return rc;
+        }
+    }
+    return TS2_OK;
 }
