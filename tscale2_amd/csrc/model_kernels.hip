@@ -26,7 +26,8 @@ __global__ void __launch_bounds__(256) EmbedForward(int len, int dim, const int 
     }
 }
 
-// deltaLabel[label] += +-grad[t]  (src/gpt/compute/cpu_transformer.cpp:182-197); fp32 atomics, delta cleared by the caller
+// deltaLabel[label] += +-grad[t]  (src/gpt/compute/cpu_transformer.cpp:182-197); fp32 atomics, delta cleared by the caller.  The memory is
+// the model's own device memory, where the hardware's fp32 add applies: plain atomicAdd compiles to a compare-and-swap loop
 __global__ void __launch_bounds__(256) EmbedBackward(int len, int dim, const int *labelPtr, const uint32_t *labels, const float *grad, int64_t ldGrad,
     float *delta, int64_t ldDelta)
 {
@@ -36,7 +37,7 @@ __global__ void __launch_bounds__(256) EmbedBackward(int len, int dim, const int
         float w = (label & 0x80000000u) ? -1.f : 1.f;
         label &= 0x7fffffffu;
         for (int col = threadIdx.x; col < dim; col += 256) {
-            atomicAdd(delta + (int64_t)label * ldDelta / 4 + col, grad[(int64_t)t * ldGrad / 4 + col] * w);
+            unsafeAtomicAdd(delta + (int64_t)label * ldDelta / 4 + col, grad[(int64_t)t * ldGrad / 4 + col] * w);
         }
     }
 }
@@ -331,6 +332,7 @@ __global__ void __launch_bounds__(1024) FinalSoftmaxGradHalfRow(int rows, int vo
             biasTop = fmaxf(fmaxf(fmaxf(biasTop, fmaxf(b0.x, b0.y)), fmaxf(b0.z, b0.w)), fmaxf(fmaxf(b1.x, b1.y), fmaxf(b1.z, b1.w)));
         }
     }
+    float loss = 0; // of the thread that met the rows' labels: one atomic per workgroup, not one per row (13 ns each on one address)
     for (; t < rows; t += gridDim.x) {
 #pragma unroll
         for (int i = 0; i < ROW_ROUNDS; ++i) {
@@ -419,14 +421,134 @@ __global__ void __launch_bounds__(1024) FinalSoftmaxGradHalfRow(int rows, int vo
                     for (int e = 0; e < 8; ++e) {
                         g[e] = e == tg - k ? gt : g[e];
                     }
-                    if (lossSum) {
-                        atomicAdd(lossSum, logf(pr));
-                    }
+                    loss += logf(pr);
                 }
                 *(uint4 *)(grow + k) = make_uint4(PackBf16x2(g[0], g[1]), PackBf16x2(g[2], g[3]), PackBf16x2(g[4], g[5]), PackBf16x2(g[6], g[7]));
             }
         }
         __syncthreads(); // the reduction slots are free again
+    }
+    if (lossSum) {
+        loss = WaveSum(loss);
+        if ((tid & 63) == 0) {
+            redS[tid >> 6] = loss;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            float total = 0;
+            for (int w = 0; w < 16; ++w) {
+                total += redS[w];
+            }
+            if (total != 0) {
+                unsafeAtomicAdd(lossSum, total);
+            }
+        }
+    }
+}
+
+// Vocabularies below 2048: one wave per row, the row in its registers (NCH chunks of 512 halves), waves walk rows with the grid's stride,
+// the next row's loads in flight.  Per logit one exponential in fp32, the arithmetic of the two-pass kernel.  A workgroup adds its
+// rows' loss once: the per-row atomic on one address alone took 13 ns a row (16384 x 1024 logits: 213 us, now 24; 65536 x 128: 834 us).
+template <int NCH>
+__global__ void __launch_bounds__(256) FinalSoftmaxGradHalfWave(int rows, int vocab, const _Float16 *logits, int64_t ldLogits, const float *bias,
+    const int *target, float gradMult, bf16_t *grad, int64_t ldGrad, float *lossSum)
+{
+    typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+    __shared__ float red[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int stride = gridDim.x * 4;
+    float bv[NCH][8];
+    bool in[NCH];
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+        const int k = (i * 64 + lane) * 8;
+        in[i] = k < vocab;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            bv[i][e] = in[i] ? bias[k + e] : 0.f;
+        }
+    }
+    v8h nxt[NCH];
+    int tgNext = -1;
+    auto prefetch = [&](int t) {
+        const _Float16 *row = (const _Float16 *)((const uint8_t *)logits + (int64_t)t * ldLogits);
+        tgNext = target[t];
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) {
+            nxt[i] = in[i] ? *(const v8h *)(row + (i * 64 + lane) * 8) : (v8h)(_Float16)-60000.f;
+        }
+    };
+    int t = blockIdx.x * 4 + wave;
+    if (t < rows) {
+        prefetch(t);
+    }
+    float loss = 0;
+    for (; t < rows; t += stride) {
+        v8h cur[NCH];
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) {
+            cur[i] = nxt[i];
+        }
+        const int tg = tgNext;
+        if (t + stride < rows) {
+            prefetch(t + stride);
+        }
+        bf16_t *grow = (bf16_t *)((uint8_t *)grad + (int64_t)t * ldGrad);
+        if (tg < 0) { // (uniform over the wave) no label: zero gradient
+#pragma unroll
+            for (int i = 0; i < NCH; ++i) {
+                if (in[i]) {
+                    *(uint4 *)(grow + (i * 64 + lane) * 8) = make_uint4(0, 0, 0, 0);
+                }
+            }
+            continue;
+        }
+        float m = 0;
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                m = fmaxf(m, (float)cur[i][e]);
+            }
+        }
+        m = WaveMax(m);
+        float p[NCH][8], sum = 0;
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                p[i][e] = in[i] ? exp2f((float)cur[i][e] + bv[i][e] - m) : 0.f;
+                sum += p[i][e];
+            }
+        }
+        const float scale = 1 / WaveSum(sum);
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) {
+            const int k = (i * 64 + lane) * 8;
+            float g[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float pr = p[i][e] * scale;
+                g[e] = ((k + e == tg ? 1.f : 0.f) - pr) * gradMult;
+                if (k + e == tg) {
+                    loss += logf(pr);
+                }
+            }
+            if (in[i]) {
+                *(uint4 *)(grow + k) = make_uint4(PackBf16x2(g[0], g[1]), PackBf16x2(g[2], g[3]), PackBf16x2(g[4], g[5]), PackBf16x2(g[6], g[7]));
+            }
+        }
+    }
+    loss = WaveSum(loss);
+    if (lane == 0) {
+        red[wave] = loss;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && lossSum) {
+        const float total = (red[0] + red[1]) + (red[2] + red[3]);
+        if (total != 0) {
+            unsafeAtomicAdd(lossSum, total);
+        }
     }
 }
 } // namespace
@@ -467,7 +589,20 @@ int Ts2FinalSoftmaxGradHalf(int rows, int vocab, const ts2_mat *logits, const fl
         ((uintptr_t)bias & 15)) {
         return TS2_ERR_ALIGN;
     }
-    if (vocab >= 2048 && vocab <= ROW_ROUNDS * 8192) {
+    if (vocab <= 2048) {
+        // eight workgroups of four waves per CU at most: each walks several rows and adds one loss
+        const int wgs = (rows + 3) / 4 < 2048 ? (rows + 3) / 4 : 2048;
+#define LAUNCH_SW(N)                                                                                                                       \
+    hipLaunchKernelGGL((FinalSoftmaxGradHalfWave<N>), dim3(wgs), dim3(256), 0, STREAM, rows, vocab, (const _Float16 *)logits->ptr,          \
+        logits->strideBytes, bias, target, gradMult, (bf16_t *)grad->ptr, grad->strideBytes, lossSum)
+        switch ((vocab + 511) / 512) {
+        case 1: LAUNCH_SW(1); break;
+        case 2: LAUNCH_SW(2); break;
+        case 3: LAUNCH_SW(3); break;
+        default: LAUNCH_SW(4); break;
+        }
+#undef LAUNCH_SW
+    } else if (vocab <= ROW_ROUNDS * 8192) {
         const int wgs = rows < 512 ? rows : 512; // one workgroup of 16 waves per CU is resident (registers); two per CU in the queue
         hipLaunchKernelGGL(FinalSoftmaxGradHalfRow, dim3(wgs), dim3(1024), 0, STREAM, rows, vocab, (const _Float16 *)logits->ptr,
             logits->strideBytes, bias, target, gradMult, (bf16_t *)grad->ptr, grad->strideBytes, lossSum);
