@@ -10,6 +10,13 @@ struct SliceP {
     int kLive;                   // K-major operands: contraction rows that count (0 = all); later rows read as zeros
     const float *segRowScale[3]; // i8: row scales of the further products
     int kTileScaleRows;          // kTileScale: > 0 = every so many rows of C have a set of scales of their own (sets one after the other)
+    // > 1: blockIdx.z picks one of several products of one shape that share A and are stored separately (C_BF16NORM; of p, b, c, tileScale,
+    // alphaPtr, normalize and rope's use are each product's own)
+    int jobs, jobNormalize, jobRope; // the latter two: bit per product
+    const uint8_t *jobB[4];
+    uint8_t *jobC[4];
+    float *jobTileScale[4];
+    const float *jobAlphaPtr[4];
 };
 bool SliceCanRun(const SliceP &sp, int type, bool tn);
 int RunSlice(const SliceP &sp, int type, bool tn, hipStream_t stream);

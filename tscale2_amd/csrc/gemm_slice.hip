@@ -60,6 +60,18 @@ template <int TYPE, bool TN, bool KT = false> __global__ void __launch_bounds__(
     int kBeg = 0, kUnits = p.kBytes / BKB;
     uint8_t *cBase = p.c;
     float *tileScale = p.tileScale;
+    const uint8_t *bBase = p.b;
+    const float *alphaPtr = p.alphaPtr;
+    bool normalize = p.normalize, rotate = p.rope != nullptr;
+    if (sp.jobs > 1) {
+        const int j = blockIdx.z;
+        bBase = sp.jobB[j];
+        cBase = sp.jobC[j];
+        tileScale = sp.jobTileScale[j];
+        alphaPtr = sp.jobAlphaPtr[j];
+        normalize = (sp.jobNormalize >> j) & 1;
+        rotate = (sp.jobRope >> j) & 1;
+    }
     int64_t bSlab = 0;
     if (p.tileGroup) {
         const int g = p.tileGroup[rowBase / TILE];
@@ -319,11 +331,11 @@ template <int TYPE, bool TN, bool KT = false> __global__ void __launch_bounds__(
     // ---- products
     auto factorOf = [&](int seg) -> float {
         float f = seg == 0 ? p.alpha : seg == 1 ? p.segAlpha[0] : seg == 2 ? p.segAlpha[1] : p.segAlpha[2];
-        const float *q = seg == 0 ? p.alphaPtr : seg == 1 ? p.segAlphaPtr[0] : seg == 2 ? p.segAlphaPtr[1] : p.segAlphaPtr[2];
+        const float *q = seg == 0 ? alphaPtr : seg == 1 ? p.segAlphaPtr[0] : seg == 2 ? p.segAlphaPtr[1] : p.segAlphaPtr[2];
         return q ? f * *q : f;
     };
     auto aOf = [&](int seg) { return seg == 0 ? p.a : seg == 1 ? p.segA[0] : seg == 2 ? p.segA[1] : p.segA[2]; };
-    auto bOf = [&](int seg) { return (seg == 0 ? p.b : seg == 1 ? p.segB[0] : seg == 2 ? p.segB[1] : p.segB[2]) + bSlab; };
+    auto bOf = [&](int seg) { return (seg == 0 ? bBase : seg == 1 ? p.segB[0] : seg == 2 ? p.segB[1] : p.segB[2]) + bSlab; };
     // partial tiles of the four wave pairs -> LDS, sums of the thread's 16 columns back.  16-byte chunks of a 512-byte row are swizzled
     // by the row like the stages.
     float val[16]; // KT: the scaled sum over the k-tiles; otherwise set from the sum
@@ -538,7 +550,7 @@ template <int TYPE, bool TN, bool KT = false> __global__ void __launch_bounds__(
         out[e] = live ? out[e] + val[e] * sumScale : 0.f;
     }
     if (ct == C_BF16NORM) {
-        if (p.normalize) {
+        if (normalize) {
             // the association of the stand-alone pass (sums of four columns, then a butterfly over the 32 of them), so that the stored rows
             // do not depend on whether this epilogue or that pass normalised them
             float q[4];
@@ -567,7 +579,7 @@ template <int TYPE, bool TN, bool KT = false> __global__ void __launch_bounds__(
                 tileScale[(int64_t)tn * p.ldTileScale + row] = discr;
             }
         }
-        if (p.rope && live) {
+        if (rotate && live) {
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 const float4 cs = *(const float4 *)(p.rope + (int64_t)row * p.ldRope + chunkOf(c) * 4);
@@ -625,6 +637,17 @@ bool SliceCanRun(const SliceP &sp, int type, bool tn)
     if (sp.ct == C_I8PACK && p.nSeg > 1) {
         return false;
     }
+    if (sp.jobs > 1) {
+        if (sp.jobs > 4 || sp.ct != C_BF16NORM || sp.epi != TS2_EPI_STORE || tn || p.splits > 1 || p.groupOffsets || p.tileGroup || p.nSeg > 1 ||
+            p.kTileScale || (sp.jobRope && !p.rope)) {
+            return false;
+        }
+        for (int i = 0; i < sp.jobs; ++i) {
+            if (((uintptr_t)sp.jobB[i] | (uintptr_t)sp.jobC[i]) & 15 || (((sp.jobNormalize >> i) & 1) && !sp.jobTileScale[i])) {
+                return false;
+            }
+        }
+    }
     if (p.kTileScale) {
         // four k-tiles per workgroup; the sets of scales change between workgroups only
         const int tiles = p.kTileBytes > 0 ? p.kBytes / p.kTileBytes : 0;
@@ -646,7 +669,8 @@ int RunSlice(const SliceP &in, int type, bool tn, hipStream_t stream)
     SliceP sp = in;
     sp.g.tilesM = sp.g.m / SBM;
     sp.g.tilesN = sp.g.n / SBN;
-    const dim3 grid(sp.g.tilesM * sp.g.tilesN, sp.g.groupOffsets ? sp.g.splitK_groups : sp.g.splits > 1 ? sp.g.splits : 1);
+    const dim3 grid(sp.g.tilesM * sp.g.tilesN, sp.g.groupOffsets ? sp.g.splitK_groups : sp.g.splits > 1 ? sp.g.splits : 1,
+        sp.jobs > 1 ? sp.jobs : 1);
     if (type == T_I8 && sp.g.kTileScale) {
         if (tn) {
             hipLaunchKernelGGL((GemmSlice<T_I8, true, true>), grid, dim3(512), 0, stream, sp);

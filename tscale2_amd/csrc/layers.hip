@@ -393,9 +393,17 @@ int FfnComputeRG(ts2_model *M, TLayer &L, const Arr &norm8, void *s)
     Arr wideRaw = View(M->raw, R, F), wide16 = View(A.a16[0], R, F), gate16 = View(A.a16[1], R, F), wideScale = View(A.tsc[0], F / 128, R);
     Arr rg8 = View(A.rg8, R, F);
     // wide = MulForward(n, We) in true units, then per-tile normalisation to 1/24 units + tile scale
-    CK(ForwardNormRope(M, L.w[0], norm8, VEC * DISCR * Dot(D), true, true, VEC, nullptr, wide16, &wideScale, s));
     // gate uses the matrix without its scale (GetDataNoScale)
-    CK(Forward(M, L.w[1], norm8, VEC * DISCR * Dot(D), false, gate16, false, s));
+    const ts2_mat *const w[2] = {&L.w[0].fast.m, &L.w[1].fast.m}, *const scales[2] = {&wideScale.m, nullptr};
+    const ts2_mat res[2] = {wide16.m, gate16.m};
+    const float *const factors[2] = {L.w[0].scale, nullptr};
+    const int rc = Ts2ForwardGroup(M->mode, 2, len, R, D, F, norm8.P(), w, VEC * DISCR * Dot(D), factors, 1, VEC, 0, nullptr, res, scales, s);
+    if (rc == TS2_ERR_UNSUPPORTED) {
+        CK(ForwardNormRope(M, L.w[0], norm8, VEC * DISCR * Dot(D), true, true, VEC, nullptr, wide16, &wideScale, s));
+        CK(Forward(M, L.w[1], norm8, VEC * DISCR * Dot(D), false, gate16, false, s));
+    } else {
+        CK(rc);
+    }
     return ts2_matrix_lolu(len, R, gate16.P(), wide16.P(), 1.f, rg8.P(), M->mode, s);
 }
 
@@ -452,10 +460,18 @@ int AttComputeVLG(ts2_model *M, TLayer &L, const Arr &norm8, void *s)
     Arr raw = View(M->raw, R, Q), q16 = View(A.a16[0], R, Q), gate16 = View(A.a16[1], R, Q), k16 = View(A.a16[2], R, Q), v16 = View(A.a16[3], R, Q);
     Arr qScale = View(A.tsc[0], H, R), vScale = View(A.tsc[1], H, R), val16 = View(A.val16, R, Q), vlg8 = View(A.rg8, R, Q);
     float a = VEC * DISCR * Dot(D);
-    CK(ForwardNormRope(M, L.w[0], norm8, a, true, true, 1.f, &M->rope, q16, &qScale, s));
-    CK(ForwardNormRope(M, L.w[1], norm8, a, true, false, 1.f, &M->rope, k16, nullptr, s));
-    CK(ForwardNormRope(M, L.w[2], norm8, a, true, true, 1.f, nullptr, v16, &vScale, s));
-    CK(Forward(M, L.w[3], norm8, a, false, gate16, false, s));
+    const ts2_mat *const w[4] = {&L.w[0].fast.m, &L.w[1].fast.m, &L.w[2].fast.m, &L.w[3].fast.m};
+    const ts2_mat *const scales[4] = {&qScale.m, nullptr, &vScale.m, nullptr}, res[4] = {q16.m, k16.m, v16.m, gate16.m};
+    const float *const factors[4] = {L.w[0].scale, L.w[1].scale, L.w[2].scale, nullptr};
+    const int rc = Ts2ForwardGroup(M->mode, 4, len, R, D, Q, norm8.P(), w, a, factors, 1 | 4, 1.f, 1 | 2, M->rope.P(), res, scales, s);
+    if (rc == TS2_ERR_UNSUPPORTED) {
+        CK(ForwardNormRope(M, L.w[0], norm8, a, true, true, 1.f, &M->rope, q16, &qScale, s));
+        CK(ForwardNormRope(M, L.w[1], norm8, a, true, false, 1.f, &M->rope, k16, nullptr, s));
+        CK(ForwardNormRope(M, L.w[2], norm8, a, true, true, 1.f, nullptr, v16, &vScale, s));
+        CK(Forward(M, L.w[3], norm8, a, false, gate16, false, s));
+    } else {
+        CK(rc);
+    }
     ts2_att_args at = {};
     at.len = len;
     at.lenRound = R;
@@ -1383,7 +1399,7 @@ extern "C" int ts2_model_forward(ts2_model *M, void *stream)
     CK(ModelForward(M, stream));
     CK(FinalLogits(M, M->logits, stream));
     // probabilities in place of the logits; the gradient buffer is scratch here
-    return Ts2FinalSoftmaxGrad(M->R, M->cfg.vocab, M->logits.P(), M->bias, M->target, 1.f, M->gradV.P(), nullptr, 1, stream);
+    return Ts2FinalSoftmaxGrad(M->len, M->cfg.vocab, M->logits.P(), M->bias, M->target, 1.f, M->gradV.P(), nullptr, 1, stream);
 }
 
 extern "C" int ts2_model_backprop(ts2_model *M, void *stream)

@@ -387,7 +387,16 @@ extern "C" int ts2_matmul_forward_norm_rope(int32_t mode, int32_t len, int32_t l
         if (normalize) {
             g.tileScale = *tileScale;
         }
-        return ts2_gemm_nt(&g, stream);
+        const int rc = ts2_gemm_nt(&g, stream);
+        // rows off 16 bytes and the like: a product and the stand-alone pass take them
+        if (large || !raw || (rc != TS2_ERR_UNSUPPORTED && rc != TS2_ERR_ALIGN)) {
+            return rc;
+        }
+        g.epilogue = TS2_EPI_STORE;
+        g.normalize = 0;
+        g.vecScale = 0;
+        g.rope = {};
+        g.tileScale = {};
     }
     if (!raw) {
         return TS2_ERR_NULL;
@@ -580,4 +589,60 @@ int Ts2BackpropGroupI8(int count, int len, int lenRound, int srcDim, int gradDim
         }
     }
     return TS2_OK;
+}
+
+// While one product alone fits the chip (256 workgroups, one per CU), a launch is a chain of latencies and four of them cost four.  Whole passes,
+// separate -> one launch: 512-token int8 step 1133 -> 1016 us, 777-token prompt 1007 -> 853 (softmax of the live rows included), 3885-token
+// 8-expert step 1632 -> 1538.  Beyond, the large-tile kernels are as good one by one
+int Ts2ForwardGroup(int mode, int count, int len, int lenRound, int srcDim, int dstDim, const ts2_mat *src, const ts2_mat *const *w, float alpha,
+    const float *const *alphaPtr, int normalizeBits, float vecScale, int rotateBits, const ts2_mat *rope, const ts2_mat *res,
+    const ts2_mat *const *tileScale, void *stream)
+{
+    const int64_t wgs = (int64_t)(lenRound / 64) * (dstDim / 128);
+    if (count < 2 || count > 4 || !Is8(mode) || wgs > 256 || lenRound % 128 || dstDim % 128 || srcDim % 128 || src->x < srcDim || src->y < lenRound) {
+        return TS2_ERR_UNSUPPORTED;
+    }
+    gemmk::SliceP sp = {};
+    gemmk::GemmP &g = sp.g;
+    g.a = (const uint8_t *)src->ptr;
+    g.b = (const uint8_t *)w[0]->ptr;
+    g.c = (uint8_t *)res[0].ptr;
+    g.lda = src->strideBytes;
+    g.ldb = w[0]->strideBytes;
+    g.ldc = res[0].strideBytes;
+    g.m = lenRound;
+    g.n = dstDim;
+    g.kBytes = srcDim;
+    g.mLive = len;
+    g.alpha = alpha;
+    g.alphaPtr = alphaPtr[0];
+    g.vecScale = vecScale;
+    g.splits = 1;
+    g.nSeg = 1;
+    if (rotateBits) {
+        g.rope = (const float *)rope->ptr;
+        g.ldRope = rope->strideBytes / 4;
+    }
+    sp.ct = gemmk::C_BF16NORM;
+    sp.epi = TS2_EPI_STORE;
+    sp.jobs = count;
+    sp.jobNormalize = normalizeBits;
+    sp.jobRope = rotateBits;
+    for (int i = 0; i < count; ++i) {
+        if (w[i]->strideBytes != g.ldb || res[i].strideBytes != g.ldc || w[i]->x < srcDim || w[i]->y < dstDim || res[i].x < dstDim || res[i].y < lenRound) {
+            return TS2_ERR_UNSUPPORTED;
+        }
+        sp.jobB[i] = (const uint8_t *)w[i]->ptr;
+        sp.jobC[i] = (uint8_t *)res[i].ptr;
+        sp.jobAlphaPtr[i] = alphaPtr[i];
+        if ((normalizeBits >> i) & 1) {
+            const int64_t ld = tileScale[i]->strideBytes / 4;
+            if (tileScale[i]->x < lenRound || tileScale[i]->y < dstDim / TILE || (g.ldTileScale && g.ldTileScale != ld)) {
+                return TS2_ERR_UNSUPPORTED;
+            }
+            g.ldTileScale = ld;
+            sp.jobTileScale[i] = (float *)tileScale[i]->ptr;
+        }
+    }
+    return gemmk::RunSlice(sp, SliceType(mode), false, (hipStream_t)stream);
 }
