@@ -106,13 +106,31 @@ __global__ void __launch_bounds__(256) LayerNormalizeStateVecs(int len, int lenR
     StoreScales(normScale, tile, t0, lenRound, h, discr);
 }
 
+// the maximum over a workgroup of NT threads to *p
+template <int NT> __device__ __forceinline__ void PublishBlockMax(float v, float *red, float *p)
+{
+    v = WaveMax(v);
+    if ((threadIdx.x & 63) == 0) {
+        red[threadIdx.x >> 6] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && p) {
+        float m = red[0];
+#pragma unroll
+        for (int w = 1; w < NT / 64; ++w) {
+            m = fmaxf(m, red[w]);
+        }
+        AtomicMaxPos(p, m);
+    }
+}
+
 // Every workgroup walks many units and issues ONE atomic max at the end: one atomic per unit (the reference's scheme,
 // gpu_layer_norm.cuh:111-114) serialises half a million updates of a single address at this problem size.
-template <class TNorm, class TFast, bool FINAL>
-__global__ void __launch_bounds__(256) BackpropLayerNormalize(int len, int rows, int tiles, Mat normState, Mat stateScale, Mat dNormState,
+template <class TNorm, class TFast, bool FINAL, int NT>
+__global__ void __launch_bounds__(NT) BackpropLayerNormalize(int len, int rows, int tiles, Mat normState, Mat stateScale, Mat dNormState,
     const float *combinerScale, const float *gradScale, const float *gradMult, Mat stateGrad, Mat stateGradFast, float *nextMaxNorm)
 {
-    __shared__ float red[8];
+    __shared__ float red[NT / 64];
     const int h = threadIdx.x & 31;
     const long units = (long)((rows + U - 1) / U) * tiles;
     float s = 1;
@@ -126,7 +144,7 @@ __global__ void __launch_bounds__(256) BackpropLayerNormalize(int len, int rows,
     }
     const float gm = (!FINAL && gradMult) ? *gradMult : 1.f;
     float gmax = 0;
-    for (long u = ((long)blockIdx.x * 256 + threadIdx.x) >> 5; u < units; u += (long)gridDim.x * 8) {
+    for (long u = ((long)blockIdx.x * NT + threadIdx.x) >> 5; u < units; u += (long)gridDim.x * (NT / 32)) {
         long rb = u / tiles;
         int tile = (int)(u - rb * tiles);
         int t0 = (int)rb * U;
@@ -161,26 +179,18 @@ __global__ void __launch_bounds__(256) BackpropLayerNormalize(int len, int rows,
             Store4<TFast>(At<TFast>(stateGradFast, t, col), g * gm);
         }
     }
-    gmax = Half32Max(gmax);
-    if (h == 0) {
-        red[threadIdx.x >> 5] = gmax;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0 && nextMaxNorm) {
-        float m = fmaxf(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])), fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7])));
-        AtomicMaxPos(nextMaxNorm, m);
-    }
+    PublishBlockMax<NT>(gmax, red, nextMaxNorm);
 }
 
 // e4m3 norm state and e4m3 fast gradient with eight elements per lane (a tile = 16 lanes, 16-byte accesses to the fp32 arrays): the
 // form the fp8 model runs.  Same arithmetic per element as BackpropLayerNormalize; Row16Sum is defined with the 8-wide LoLU kernel.
 __device__ __forceinline__ float Row16SumFwd(float v);
 
-template <bool FINAL>
-__global__ void __launch_bounds__(256) BackpropLayerNormalize8(int len, int rows, int tiles, Mat normState, Mat stateScale, Mat dNormState,
+template <bool FINAL, int NT>
+__global__ void __launch_bounds__(NT) BackpropLayerNormalize8(int len, int rows, int tiles, Mat normState, Mat stateScale, Mat dNormState,
     const float *combinerScale, const float *gradScale, const float *gradMult, Mat stateGrad, Mat stateGradFast, float *nextMaxNorm)
 {
-    __shared__ float red[4];
+    __shared__ float red[NT / 64];
     const int l16 = threadIdx.x & 15;
     const long units = (long)rows * tiles;
     float s = 1;
@@ -195,8 +205,8 @@ __global__ void __launch_bounds__(256) BackpropLayerNormalize8(int len, int rows
     const float gm = (!FINAL && gradMult) ? *gradMult : 1.f;
     float gmax = 0;
     // every lane of a wave takes part in every iteration (the reductions are cross-lane): the loop bound is wave-uniform
-    const long unitFirst = ((long)blockIdx.x * 256 + (threadIdx.x & ~63)) >> 4;
-    for (long ub = unitFirst; ub < units; ub += (long)gridDim.x * 16) {
+    const long unitFirst = ((long)blockIdx.x * NT + (threadIdx.x & ~63)) >> 4;
+    for (long ub = unitFirst; ub < units; ub += (long)gridDim.x * (NT / 16)) {
         const long u = ub + ((threadIdx.x & 63) >> 4);
         const bool any = u < units;
         const int t = any ? (int)(u / tiles) : 0;
@@ -253,14 +263,7 @@ __global__ void __launch_bounds__(256) BackpropLayerNormalize8(int len, int rows
         uint32_t hi = CvtPkE4m3(out[4] * gm, out[5] * gm) | (CvtPkE4m3(out[6] * gm, out[7] * gm) << 16);
         *(uint2 *)At<TE4M3>(stateGradFast, t, col) = make_uint2(lo, hi);
     }
-    gmax = WaveMax(gmax);
-    if ((threadIdx.x & 63) == 0) {
-        red[threadIdx.x >> 6] = gmax;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0 && nextMaxNorm) {
-        AtomicMaxPos(nextMaxNorm, fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
-    }
+    PublishBlockMax<NT>(gmax, red, nextMaxNorm);
 }
 
 __device__ __forceinline__ float ComputeGradMult(float gradMaxNorm)
@@ -831,7 +834,8 @@ struct RowQuantJobs {
     uint32_t seed[4];
 };
 
-template <int NCH>
+// FULL: rows of exactly NCH * 512 elements.
+template <int NCH, bool FULL>
 __global__ void __launch_bounds__(256) NormalizeRowsWave(int len, int lenRound, int dim, RowQuantJobs jobs, const float *colScale)
 {
     const Mat src = jobs.src[blockIdx.y], dst = jobs.dst[blockIdx.y];
@@ -841,7 +845,7 @@ __global__ void __launch_bounds__(256) NormalizeRowsWave(int len, int lenRound, 
     bool in[NCH];
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
-        in[i] = (i * 64 + lane) * 8 < dim;
+        in[i] = FULL || (i * 64 + lane) * 8 < dim;
     }
     const int nWaves = gridDim.x * 4;
     // the column scales of the lane's chunks stay in registers for all the rows the wave walks
@@ -1470,35 +1474,57 @@ static int BackpropNormImpl(bool final, int len, int rows, const ts2_mat *normSt
         return TS2_ERR_UNSUPPORTED;
     }
     int tiles = dim / TILE;
-    long nUnits = (long)rows * tiles;
-    dim3 bnGrid((unsigned)((nUnits + 7) / 8 < 2048 ? (nUnits + 7) / 8 : 2048));
+    // The workgroups that start together all find the maximum still low and queue at its address, 10 ns each: 1024 threads each once there
+    // are more than 256 workgroups of 256, two per CU (4096 x 512, e4m3: 20 -> 11.6 us).  Many times as much work outweighs the queue, and
+    // small workgroups share the memory better (65536 x 1024, this pass and the final one: 305 us, 350 with large ones)
+    const long units4 = (long)((rows + U - 1) / U) * tiles, units1 = (long)rows * tiles;
+    auto grid = [](long units, int perBlock, int most) { const long n = (units + perBlock - 1) / perBlock; return dim3((unsigned)(n < most ? n : most)); };
     if (normType == TS2_E4M3 && fastType == TS2_E4M3 && (((uintptr_t)normState->ptr | normState->strideBytes | (uintptr_t)stateGradFast->ptr |
                                                          stateGradFast->strideBytes) & 7) == 0 &&
         Aligned16(dNormState->ptr, dNormState->strideBytes) && Aligned16(stateGrad->ptr, stateGrad->strideBytes)) {
-        dim3 grid8((unsigned)((nUnits + 15) / 16 < 8192 ? (nUnits + 15) / 16 : 8192));
+#define LAUNCH_BN8(FINAL, NT)                                                                                                              \
+    hipLaunchKernelGGL((BackpropLayerNormalize8<FINAL, NT>), grid(units1, NT / 16, NT == 256 ? 8192 : 512), dim3(NT), 0, STREAM, len, rows, tiles, M(*normState), \
+        M(*stateScale), M(*dNormState), combinerScale, gradScale, gradMult, M(*stateGrad), M(*stateGradFast), nextMaxNorm)
+        const bool many = units1 > 4096 && units1 <= 131072;
         if (final) {
-            hipLaunchKernelGGL((BackpropLayerNormalize8<true>), grid8, dim3(256), 0, STREAM, len, rows, tiles, M(*normState), M(*stateScale),
-                M(*dNormState), combinerScale, gradScale, gradMult, M(*stateGrad), M(*stateGradFast), nextMaxNorm);
+            if (many) {
+                LAUNCH_BN8(true, 1024);
+            } else {
+                LAUNCH_BN8(true, 256);
+            }
         } else {
-            hipLaunchKernelGGL((BackpropLayerNormalize8<false>), grid8, dim3(256), 0, STREAM, len, rows, tiles, M(*normState), M(*stateScale),
-                M(*dNormState), combinerScale, gradScale, gradMult, M(*stateGrad), M(*stateGradFast), nextMaxNorm);
+            if (many) {
+                LAUNCH_BN8(false, 1024);
+            } else {
+                LAUNCH_BN8(false, 256);
+            }
         }
+#undef LAUNCH_BN8
         TS2_CHECK_LAUNCH();
         return TS2_OK;
     }
+#define LAUNCH_BN_AS(TN, TFA, FINAL, NT)                                                                                                   \
+    hipLaunchKernelGGL((BackpropLayerNormalize<TN, TFA, FINAL, NT>), grid(units4, NT / 32, NT == 256 ? 2048 : 512), dim3(NT), 0, STREAM, len, rows, tiles,    \
+        M(*normState), M(*stateScale), M(*dNormState), combinerScale, gradScale, gradMult, M(*stateGrad), M(*stateGradFast), nextMaxNorm)
 #define LAUNCH_BN(TN, TFA)                                                                                                                 \
-    if (final)                                                                                                                             \
-        hipLaunchKernelGGL((BackpropLayerNormalize<TN, TFA, true>), bnGrid, dim3(256), 0, STREAM, len, rows, tiles,         \
-            M(*normState), M(*stateScale), M(*dNormState), combinerScale, gradScale, gradMult, M(*stateGrad), M(*stateGradFast), nextMaxNorm); \
-    else                                                                                                                                   \
-        hipLaunchKernelGGL((BackpropLayerNormalize<TN, TFA, false>), bnGrid, dim3(256), 0, STREAM, len, rows, tiles,        \
-            M(*normState), M(*stateScale), M(*dNormState), combinerScale, gradScale, gradMult, M(*stateGrad), M(*stateGradFast), nextMaxNorm)
+    if (units4 <= 2048 || units4 > 32768) {                                                                                                               \
+        if (final) {                                                                                                                       \
+            LAUNCH_BN_AS(TN, TFA, true, 256);                                                                                              \
+        } else {                                                                                                                           \
+            LAUNCH_BN_AS(TN, TFA, false, 256);                                                                                             \
+        }                                                                                                                                  \
+    } else if (final) {                                                                                                                    \
+        LAUNCH_BN_AS(TN, TFA, true, 1024);                                                                                                 \
+    } else {                                                                                                                               \
+        LAUNCH_BN_AS(TN, TFA, false, 1024);                                                                                                \
+    }
     if (fastType == TS2_BF16) {
         TS2_DISPATCH_TYPE(normType, TN, LAUNCH_BN(TN, TBF16));
     } else {
         TS2_DISPATCH_TYPE(normType, TN, LAUNCH_BN(TN, TE4M3));
     }
 #undef LAUNCH_BN
+#undef LAUNCH_BN_AS
     TS2_CHECK_LAUNCH();
     return TS2_OK;
 }
@@ -1702,7 +1728,12 @@ static int LaunchRowQuant(int count, int len, int lenRound, int dim, const RowQu
     // with column scales a wave walks several rows (the scales stay in registers), else one row per wave
     const int wgs = (lenRound + 3) / 4;
     const dim3 grid(colScale && wgs > 2048 ? 2048 : wgs, count);
-#define LAUNCH_RW(N) hipLaunchKernelGGL((NormalizeRowsWave<N>), grid, dim3(256), 0, STREAM, len, lenRound, dim, jobs, colScale)
+#define LAUNCH_RW(N)                                                                                                                       \
+    if (dim == N * 512) {                                                                                                                  \
+        hipLaunchKernelGGL((NormalizeRowsWave<N, true>), grid, dim3(256), 0, STREAM, len, lenRound, dim, jobs, colScale);                  \
+    } else {                                                                                                                               \
+        hipLaunchKernelGGL((NormalizeRowsWave<N, false>), grid, dim3(256), 0, STREAM, len, lenRound, dim, jobs, colScale);                 \
+    }
     switch ((dim + 511) / 512) {
     case 1: LAUNCH_RW(1); break;
     case 2: LAUNCH_RW(2); break;
