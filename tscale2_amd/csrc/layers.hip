@@ -1265,12 +1265,20 @@ extern "C" int ts2_model_apply_deltas(ts2_model *M, const ts2_add_gradient_param
     if (hipMemcpyAsync(M->optParams, paramsHost, sizeof(ts2_add_gradient_params), hipMemcpyHostToDevice, (hipStream_t)stream) != hipSuccess) {
         return TS2_ERR_LAUNCH;
     }
+    std::vector<const ts2_opt_matrix *> batch; // matrices whose updates share launches
+    std::vector<const ts2_mat *> deltas, scales;
     auto apply = [&](TMatrix &W, bool packed) -> int {
         if (!W.hasOpt) {
             return 0;
         }
         W.fastTValid = false;
         const ts2_opt_matrix &o = W.opt;
+        if (packed && Ts2OptBatchable(&o)) {
+            batch.push_back(&o);
+            deltas.push_back(W.delta.P());
+            scales.push_back(W.deltaTileScale.P());
+            return 0;
+        }
         if (packed) {
             return ts2_opt_add_delta(&o, W.delta.P(), W.deltaTileScale.P(), TS2_BM_GRAD_APPLY, M->optParams, stream);
         }
@@ -1289,7 +1297,7 @@ extern "C" int ts2_model_apply_deltas(ts2_model *M, const ts2_add_gradient_param
             }
         }
     }
-    return 0;
+    return Ts2OptApplyBatch((int)batch.size(), batch.data(), deltas.data(), scales.data(), M->optParams, stream);
 }
 
 // host copy of a matrix's master weights [rows][cols] (synchronises the device)

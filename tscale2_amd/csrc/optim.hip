@@ -10,6 +10,7 @@
 // array - its row sums are taken from the bytes (1 B/element read) and AddGradient reads the bytes again - 23 B/element of traffic where
 // the unpack / row-sum / add / convert sequence moves 34.
 #include "vec.h"
+#include "internal.h"
 
 namespace
 {
@@ -181,9 +182,8 @@ __global__ void __launch_bounds__(256) AddGradient(int xSize, int ySize, DeltaSr
 
 // first half of ConvertMatrixKernel (agpu_cuda.cuh:65-101): sko = rms of the whole matrix from the row sums, mult = 32 / sko (0 for a zero
 // matrix).  The reference recomputes this in every workgroup of the conversion; here one small launch leaves both scalars on the device.
-__global__ void __launch_bounds__(1024) MatrixSko(int totalXSize, int totalYSize, const float *sum2arr, float *resDiscrScale, float *convertMult)
+__device__ __forceinline__ void MatrixSkoBlock(int totalXSize, int totalYSize, const float *sum2arr, float *resDiscrScale, float *convertMult, float *red)
 {
-    __shared__ float red[16];
     float sum2 = 0;
     for (int k = threadIdx.x; k < totalYSize; k += 1024) {
         sum2 += sum2arr[k];
@@ -203,6 +203,12 @@ __global__ void __launch_bounds__(1024) MatrixSko(int totalXSize, int totalYSize
         convertMult[0] = sko == 0 ? 0.f : 1 / discrScale;
         resDiscrScale[0] = sko;
     }
+}
+
+__global__ void __launch_bounds__(1024) MatrixSko(int totalXSize, int totalYSize, const float *sum2arr, float *resDiscrScale, float *convertMult)
+{
+    __shared__ float red[16];
+    MatrixSkoBlock(totalXSize, totalYSize, sum2arr, resDiscrScale, convertMult, red);
 }
 
 // second half: fast = cvt(weights * mult), rows ySize .. yBufSize cleared
@@ -226,6 +232,143 @@ __global__ void __launch_bounds__(256) ConvertMatrix(int xSize, int ySize, int y
             for (int x = threadIdx.x * 4; x < xSize; x += 1024) {
                 Store4<TDst>(drow + (int64_t)x * TDst::SIZE, ZeroF4());
             }
+        }
+    }
+}
+
+// ---- "one delta, apply now" with a dispersion estimate per row, over up to OPT_JOBS matrices in three launches: rows, matrix scale,
+// conversion.  Small matrices are bound by launches (a 512 x 512 one took five of 2 to 4 us each), large ones by the second read of the
+// delta and by the two single-workgroup launches.
+constexpr int OPT_JOBS = 16; // jobs travel as kernel arguments
+constexpr int OPT_ROW_MAX = 4096;
+
+struct OptJob {
+    Mat delta, tileScale, avgGrad, weights, fast;
+    float *gradRowSum2, *weightsRowSum2, *rowScale, *rowDisp, *sumWeight, *matrixScale, *convertMult;
+    const float *sparsity;
+    int xSize, ySize, yBufSize, fastType;
+};
+
+struct OptJobs {
+    OptJob j[OPT_JOBS];
+};
+
+// RowSum2, UpdateGlobalRowDisp (one row per estimate) and AddGradient of a row by one team - a wave, or the workgroup - that keeps the
+// packed row in registers between its sum and its use (NCH chunks of four elements per thread), all operands of the row in flight at
+// once.  sumWeight is only read here; OptScale, which follows, moves it on.  8192 x 2048, with the row sums and estimates it
+// replaces: 50.5 + 8.4 + 5.9 us in three launches -> 53.5 (a wave per row, eight chunks in two goes: 57.8)
+template <int NCH, bool WG> __global__ void __launch_bounds__(256) OptRows(OptJobs jobs, const ts2_add_gradient_params *pParams)
+{
+    constexpr int STEP = WG ? 1024 : 256, TEAMS = WG ? 1 : 4;
+    __shared__ float red[4];
+    const OptJob &o = jobs.j[blockIdx.y];
+    const int lane = WG ? threadIdx.x : threadIdx.x & 63;
+    const ts2_add_gradient_params params = *pParams;
+    const float rowDispNorm = 1 / (o.sumWeight[0] * params.dispDecay + 1);
+    const float stepMult = params.stepMult * sqrtf(o.sparsity[0]);
+    const float shrinkMult = 1 - stepMult * params.l2Reg;
+    const float betaMult = 1 - params.beta1;
+    for (int y = blockIdx.x * TEAMS + (WG ? 0 : threadIdx.x >> 6); y < o.ySize; y += gridDim.x * TEAMS) {
+        const uint8_t *drow = o.delta.p + (int64_t)y * o.delta.ld;
+        float *ag = (float *)(o.avgGrad.p + (int64_t)y * o.avgGrad.ld);
+        float *wr = (float *)(o.weights.p + (int64_t)y * o.weights.ld);
+        int raw[NCH];
+        float ts[NCH];
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+            const int x = c * STEP + lane * 4;
+            const bool in = x < o.xSize;
+            raw[c] = in ? *(const int *)(drow + x) : 0;
+            ts[c] = in ? *(const float *)(o.tileScale.p + (int64_t)(x >> 7) * o.tileScale.ld + (int64_t)y * 4) : 0.f;
+        }
+        const float oldDisp = o.rowDisp[y];
+        F4 a[NCH], w[NCH];
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+            const int x = c * STEP + lane * 4;
+            a[c] = x < o.xSize ? Load4<TF32>(ag + x) : ZeroF4();
+            w[c] = x < o.xSize ? Load4<TF32>(wr + x) : ZeroF4();
+        }
+        float s = 0;
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+            const F4 d = Load4<TI8>(&raw[c]) * ts[c];
+            s += HSum(d * d);
+        }
+        s = WG ? BlockSum256(s, red) : WaveSum(s);
+        const float disp = (oldDisp * params.dispDecay) + (s / o.xSize);
+        const float deltaScale = CalcRowScale(disp * rowDispNorm);
+        if (lane == 0) {
+            o.gradRowSum2[y] = s;
+            o.rowDisp[y] = disp;
+            o.rowScale[y] = deltaScale;
+        }
+        float sum2 = 0;
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+            const int x = c * STEP + lane * 4;
+            if (x < o.xSize) {
+                const F4 dl = Load4<TI8>(&raw[c]) * ts[c] * deltaScale;
+                const F4 newAG = a[c] * params.beta1 + dl * betaMult;
+                const F4 totalDelta = newAG * params.weight1 + dl * params.weight0;
+                const F4 val = w[c] * shrinkMult + totalDelta * stepMult;
+                sum2 += HSum(val * val);
+                Store4<TF32>(ag + x, newAG);
+                Store4<TF32>(wr + x, val);
+            }
+        }
+        sum2 = WG ? BlockSum256(sum2, red) : WaveSum(sum2);
+        if (lane == 0) {
+            o.weightsRowSum2[y] = sum2;
+        }
+    }
+}
+
+// MatrixSko per job, and the weight of the dispersion estimates that OptRows used
+__global__ void __launch_bounds__(1024) OptScale(OptJobs jobs, const ts2_add_gradient_params *pParams)
+{
+    __shared__ float red[16];
+    const OptJob &o = jobs.j[blockIdx.x];
+    MatrixSkoBlock(o.xSize, o.ySize, o.weightsRowSum2, o.matrixScale, o.convertMult, red);
+    if (threadIdx.x == 0) {
+        o.sumWeight[0] = o.sumWeight[0] * pParams->dispDecay + 1;
+    }
+}
+
+template <class TDst> __device__ __forceinline__ void ConvertRow(const OptJob &o, int y, int lane, float mult)
+{
+    uint8_t *drow = o.fast.p + (int64_t)y * o.fast.ld;
+    const float *srow = (const float *)(o.weights.p + (int64_t)y * o.weights.ld);
+    const bool live = y < o.ySize;
+    for (int x0 = lane * 4; x0 < o.xSize; x0 += 1024) {
+        F4 v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int x = x0 + k * 256;
+            v[k] = live && x < o.xSize ? Load4<TF32>(srow + x) : ZeroF4();
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int x = x0 + k * 256;
+            if (x < o.xSize) {
+                Store4<TDst>(drow + (int64_t)x * TDst::SIZE, live ? v[k] * mult : ZeroF4());
+            }
+        }
+    }
+}
+
+// ConvertMatrix per job, a wave per row
+__global__ void __launch_bounds__(256) OptConvert(OptJobs jobs)
+{
+    const OptJob &o = jobs.j[blockIdx.y];
+    const float mult = o.convertMult[0];
+    for (int y = blockIdx.x * 4 + (threadIdx.x >> 6); y < o.yBufSize; y += gridDim.x * 4) {
+        if (o.fastType == TS2_I8) {
+            ConvertRow<TI8>(o, y, threadIdx.x & 63, mult);
+        } else if (o.fastType == TS2_E4M3) {
+            ConvertRow<TE4M3>(o, y, threadIdx.x & 63, mult);
+        } else {
+            ConvertRow<TBF16>(o, y, threadIdx.x & 63, mult);
         }
     }
 }
@@ -385,6 +528,63 @@ extern "C" int ts2_opt_convert(const ts2_opt_matrix *m, void *stream)
         m->convertMult, stream);
 }
 
+bool Ts2OptBatchable(const ts2_opt_matrix *m)
+{
+    return m->rowDispSize == m->ySize && m->xSize <= OPT_ROW_MAX;
+}
+
+int Ts2OptApplyBatch(int count, const ts2_opt_matrix *const *mats, const ts2_mat *const *delta, const ts2_mat *const *tileScale,
+    const ts2_add_gradient_params *params, void *stream)
+{
+    for (int first = 0; first < count; first += OPT_JOBS) {
+        OptJobs jobs = {};
+        const int n = count - first < OPT_JOBS ? count - first : OPT_JOBS;
+        int maxX = 0, maxRows = 0, maxBuf = 0;
+        for (int i = 0; i < n; ++i) {
+            const ts2_opt_matrix *m = mats[first + i];
+            const ts2_mat *d = delta[first + i], *ts = tileScale[first + i];
+            if (m->xSize <= 0 || m->ySize <= 0 || m->xSize % 128 || !Ts2OptBatchable(m) || !PackedOk(d, ts, m->xSize, m->ySize)) {
+                return TS2_ERR_SHAPE;
+            }
+            if (!params || !m->gradRowSum2 || !m->sumWeight || !m->rowDisp || !m->rowScale || !m->sparsity || !m->weightsRowSum2) {
+                return TS2_ERR_NULL;
+            }
+            if (!F32Ok(&m->avgGrad, m->xSize, m->ySize) || !F32Ok(&m->weights, m->xSize, m->ySize)) {
+                return TS2_ERR_SHAPE;
+            }
+            if (!m->fast.ptr || !m->matrixScale || !m->convertMult) {
+                return TS2_ERR_NULL;
+            }
+            if (m->yBufSize < m->ySize || m->fast.x < m->xSize || m->fast.y < m->yBufSize || (((uintptr_t)m->fast.ptr | m->fast.strideBytes) & 3)) {
+                return TS2_ERR_SHAPE;
+            }
+            if (m->fastType != TS2_I8 && m->fastType != TS2_E4M3 && m->fastType != TS2_BF16) {
+                return TS2_ERR_UNSUPPORTED;
+            }
+            jobs.j[i] = {M(*d), M(*ts), M(m->avgGrad), M(m->weights), M(m->fast), m->gradRowSum2, m->weightsRowSum2, m->rowScale, m->rowDisp,
+                m->sumWeight, m->matrixScale, m->convertMult, m->sparsity, m->xSize, m->ySize, m->yBufSize, m->fastType};
+            maxX = maxX > m->xSize ? maxX : m->xSize;
+            maxRows = maxRows > m->ySize ? maxRows : m->ySize;
+            maxBuf = maxBuf > m->yBufSize ? maxBuf : m->yBufSize;
+        }
+        if (maxX <= 512) {
+            hipLaunchKernelGGL((OptRows<2, false>), dim3(RowGrid((maxRows + 3) / 4), n), dim3(256), 0, STREAM, jobs, params);
+        } else if (maxX <= 1024) {
+            hipLaunchKernelGGL((OptRows<4, false>), dim3(RowGrid((maxRows + 3) / 4), n), dim3(256), 0, STREAM, jobs, params);
+        } else if (maxX <= 2048) {
+            hipLaunchKernelGGL((OptRows<2, true>), dim3(RowGrid(maxRows), n), dim3(256), 0, STREAM, jobs, params);
+        } else {
+            hipLaunchKernelGGL((OptRows<4, true>), dim3(RowGrid(maxRows), n), dim3(256), 0, STREAM, jobs, params);
+        }
+        TS2_CHECK_LAUNCH();
+        hipLaunchKernelGGL(OptScale, dim3(n), dim3(1024), 0, STREAM, jobs, params);
+        TS2_CHECK_LAUNCH();
+        hipLaunchKernelGGL(OptConvert, dim3(RowGrid((maxBuf + 3) / 4), n), dim3(256), 0, STREAM, jobs);
+        TS2_CHECK_LAUNCH();
+    }
+    return TS2_OK;
+}
+
 // TAgpuCudaModelMatrix::AddDelta(packed, bm) + ApplyGradientImpl (agpu_cuda.cuh:484-590) on one device
 extern "C" int ts2_opt_add_delta(const ts2_opt_matrix *m, const ts2_mat *delta, const ts2_mat *tileScale, int32_t backpropMode,
     const ts2_add_gradient_params *params, void *stream)
@@ -394,6 +594,9 @@ extern "C" int ts2_opt_add_delta(const ts2_opt_matrix *m, const ts2_mat *delta, 
     }
     const bool add = backpropMode & TS2_BM_GRAD_ADD, apply = backpropMode & TS2_BM_GRAD_APPLY;
     int rc;
+    if (!add && apply && Ts2OptBatchable(m)) {
+        return Ts2OptApplyBatch(1, &m, &delta, &tileScale, params, stream);
+    }
     if (!add && apply) {
         // one delta, applied now: the fp32 gradient array is never written
         rc = ts2_packed_delta_row_sum2(m->xSize, m->ySize, delta, tileScale, m->gradRowSum2, stream);
