@@ -33,7 +33,8 @@ namespace
 // that the operand reads of one stage do not alias the in-flight loads into the other and does not serialise them.
 
 // SEG: two products into the same accumulators (C = alpha0 A0 B0^T + alpha1 A1 B1^T with the same k), the second operand pair and its
-// factors in segA[0], segB[0], segAlpha[0], segAlphaPtr[0]; with tileGroup both B operands take the tile's slab.
+// factors in segA[0], segB[0], segAlpha[0], segAlphaPtr[0]; with tileGroup both B operands take the tile's slab.  i8 (with KT: the second
+// accumulator set): p.nSeg products, each with row scales of its own, added in fp32 in their order.
 template <int TYPE, int WTM, int WTN, int CT, int EPI, bool KT, int WM = 2, int WN = 2, bool SEG = false>
 __global__ void __launch_bounds__(64 * WM * WN, (WM * WN) / 4) GemmNTDirect(GemmP p)
 {
@@ -42,8 +43,9 @@ __global__ void __launch_bounds__(64 * WM * WN, (WM * WN) / 4) GemmNTDirect(Gemm
     constexpr int BM = 32 * WTM * WM;
     constexpr int BN = 32 * WTN * WN;
     // plain 16-bit results of the 128x128 e4m3 tile leave through the row-owning epilogue (a lane owns a row: operands swapped)
-    constexpr bool SWAPC = TYPE == T_FP8 && WTM == 2 && WTN == 2 && WM == 2 && WN == 2 && !KT &&
-                           (CT == C_BF16NORM || ((CT == C_BF16 || CT == C_F16) && EPI == TS2_EPI_STORE));
+    constexpr bool SWAPC = WTM == 2 && WTN == 2 && WM == 2 && WN == 2 && !KT &&
+                           ((TYPE == T_FP8 && (CT == C_BF16NORM || ((CT == C_BF16 || CT == C_F16) && EPI == TS2_EPI_STORE))) ||
+                               (TYPE == T_I8 && CT == C_BF16 && EPI == TS2_EPI_STORE));
     __shared__ __attribute__((aligned(1024))) uint8_t sA0[BM * BKB];
     __shared__ __attribute__((aligned(1024))) uint8_t sB0[BN * BKB];
     __shared__ __attribute__((aligned(1024))) uint8_t sA1[BM * BKB];
@@ -173,7 +175,7 @@ __global__ void __launch_bounds__(64 * WM * WN, (WM * WN) / 4) GemmNTDirect(Gemm
             mfma(SWAPC ? fb[SET][j] : fa[SET][i], SWAPC ? fa[SET][i] : fb[SET][j], acc[i][j]);                                             \
     } while (0)
 #define WAIT_VM0() __builtin_amdgcn_s_waitcnt(0x0F70) /* vmcnt(0): the direct loads have landed in LDS */
-    const int tileSteps = KT ? p.kTileBytes / BKB : 0;
+    const int tileSteps = KT && !SEG ? p.kTileBytes / BKB : 0;
     // one K step computing from stage (CA, CB) while the next tile streams into (NA, NB)
 #define STEP(CA, CB, NA, NB, S)                                                                                                            \
     do {                                                                                                                                   \
@@ -201,7 +203,7 @@ __global__ void __launch_bounds__(64 * WM * WN, (WM * WN) / 4) GemmNTDirect(Gemm
         }                                                                                                                                  \
         __builtin_amdgcn_sched_barrier(0);                                                                                                 \
         MFMA_ROWS(1, WTM / 2, WTM);                                                                                                        \
-        if (KT) {                                                                                                                          \
+        if (KT && !SEG) {                                                                                                                  \
             if ((kBeg + (S) + 1) % tileSteps == 0 || (S) + 1 == kSteps) {                                                                  \
                 float sc = p.kTileScale[(kBeg + (S)) / tileSteps];                                                                         \
                 _Pragma("unroll") for (int i = 0; i < (KT ? WTM : 1); ++i) _Pragma("unroll") for (int j = 0; j < (KT ? WTN : 1); ++j)      \
@@ -215,10 +217,10 @@ __global__ void __launch_bounds__(64 * WM * WN, (WM * WN) / 4) GemmNTDirect(Gemm
     } while (0)
 
     float segUnits = 0; // SEG: the one factor the epilogue applies
-    for (int seg = 0; seg < (SEG ? 2 : 1); ++seg) {
-    if (SEG && seg == 1) {
-        gaTile = p.segA[0] + aTileOff;
-        gbTile = p.segB[0] + bTileOff;
+    for (int seg = 0; seg < (SEG ? (TYPE == T_I8 ? p.nSeg : 2) : 1); ++seg) {
+    if (SEG && seg >= 1) {
+        gaTile = (seg == 1 ? p.segA[0] : seg == 2 ? p.segA[1] : p.segA[2]) + aTileOff;
+        gbTile = (seg == 1 ? p.segB[0] : seg == 2 ? p.segB[1] : p.segB[2]) + bTileOff;
     }
     if (kSteps > 0) {
         DIRECT_LOAD(sA0, sB0, 0);
@@ -236,6 +238,31 @@ __global__ void __launch_bounds__(64 * WM * WN, (WM * WN) / 4) GemmNTDirect(Gemm
     }
     if (s < kSteps) {
         STEP(sA0, sB0, sA1, sB1, s);
+    }
+    if constexpr (SEG && TYPE == T_I8) {
+        float f = seg == 0 ? p.alpha : seg == 1 ? p.segAlpha[0] : seg == 2 ? p.segAlpha[1] : p.segAlpha[2];
+        const float *fp = seg == 0 ? p.alphaPtr : seg == 1 ? p.segAlphaPtr[0] : seg == 2 ? p.segAlphaPtr[1] : p.segAlphaPtr[2];
+        const float *rs = seg == 0 ? p.rowScale : seg == 1 ? p.segRowScale[0] : seg == 2 ? p.segRowScale[1] : p.segRowScale[2];
+        if (fp) {
+            f *= *fp;
+        }
+#pragma unroll
+        for (int i = 0; i < WTM; ++i) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 r4 = *(const float4 *)(rs + rowBase + wm * (32 * WTM) + i * 32 + q * 8 + half * 4);
+                const float r[4] = {f * r4.x, f * r4.y, f * r4.z, f * r4.w};
+#pragma unroll
+                for (int j = 0; j < WTN; ++j) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        facc[i][j][q * 4 + e] = facc[i][j][q * 4 + e] + (float)acc[i][j][q * 4 + e] * r[e];
+                        acc[i][j][q * 4 + e] = 0;
+                    }
+                }
+            }
+        }
+        __syncthreads(); // every wave has read its last operands of this product before the stages are refilled
     }
     if constexpr (SEG && TYPE != T_I8) {
         if (seg == 0) {
@@ -271,9 +298,12 @@ __global__ void __launch_bounds__(64 * WM * WN, (WM * WN) / 4) GemmNTDirect(Gemm
         }
     }
     } // products
-    if constexpr (SEG && TYPE != T_I8) {
-        p.alpha = segUnits;
+    if constexpr (SEG) {
+        p.alpha = TYPE == T_I8 ? 1.f : segUnits;
         p.alphaPtr = nullptr;
+    }
+    if constexpr (SEG && TYPE == T_I8) {
+        p.rowScale = nullptr;
     }
 #undef STEP
 #undef LOAD_FRAGS
@@ -1095,6 +1125,26 @@ bool PreferSlice(const GemmP &p, int type, int ct, int epi)
     return wgs <= 256 && (type == T_BF16 || epi == TS2_EPI_ADD || (ct == C_F32 && p.kBytes <= 512));
 }
 } // namespace
+
+int gemmk::RunSumI8(const GemmP &p, hipStream_t stream)
+{
+    if (p.nSeg < 2 || p.nSeg > 4 || (p.m % 128) || (p.n % 128) || (p.kBytes % BKB) || p.splits > 1 ||
+        (((uintptr_t)p.a | (uintptr_t)p.lda | (uintptr_t)p.b | (uintptr_t)p.ldb | (uintptr_t)p.rowScale) & 15) ||
+        (((uintptr_t)p.c | (uintptr_t)p.ldc) & 3) || !p.rowScale || 128 * p.lda >= ((int64_t)1 << 31) || 128 * p.ldb >= ((int64_t)1 << 31)) {
+        return TS2_ERR_UNSUPPORTED;
+    }
+    for (int i = 0; i + 1 < p.nSeg; ++i) {
+        if (!p.segRowScale[i] || (((uintptr_t)p.segA[i] | (uintptr_t)p.segB[i] | (uintptr_t)p.segRowScale[i]) & 15)) {
+            return TS2_ERR_UNSUPPORTED;
+        }
+    }
+    GemmP q = p;
+    q.tilesM = p.m / 128;
+    q.tilesN = p.n / 128;
+    hipLaunchKernelGGL((GemmNTDirect<T_I8, 2, 2, C_F32, TS2_EPI_STORE, true, 2, 2, true>), dim3(q.tilesM * q.tilesN), dim3(256), 0, stream, q);
+    TS2_CHECK_LAUNCH();
+    return TS2_OK;
+}
 
 extern "C" int ts2_gemm_nt(const ts2_gemm_args *a, void *streamPtr)
 {

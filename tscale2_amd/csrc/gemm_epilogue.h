@@ -49,6 +49,7 @@ struct GemmP {
     const uint8_t *segA[3], *segB[3];
     float segAlpha[3];
     const float *segAlphaPtr[3];
+    const float *segRowScale[3]; // i8: row scales of the further products
     int rowsF16; // persistent kernel, row-owning epilogue: the 16-bit rows are IEEE half instead of bf16
 };
 

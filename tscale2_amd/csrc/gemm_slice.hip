@@ -457,7 +457,7 @@ template <int TYPE, bool TN, bool KT = false> __global__ void __launch_bounds__(
         for (int seg = 0; seg < p.nSeg; ++seg) {
             zeroAcc();
             float f = factorOf(seg);
-            const float *rsp = seg == 0 ? p.rowScale : seg == 1 ? sp.segRowScale[0] : seg == 2 ? sp.segRowScale[1] : sp.segRowScale[2];
+            const float *rsp = seg == 0 ? p.rowScale : seg == 1 ? p.segRowScale[0] : seg == 2 ? p.segRowScale[1] : p.segRowScale[2];
             if (rsp) {
                 f *= rsp[row];
             }

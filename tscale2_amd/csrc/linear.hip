@@ -177,7 +177,7 @@ extern "C" int ts2_matmul_backprop_group(int32_t mode, int32_t len, int32_t lenR
     for (int i = 1; i < count && one; ++i) {
         one = grad[i]->strideBytes == grad[0]->strideBytes && bufs[i]->transformT.strideBytes == bufs[0]->transformT.strideBytes;
     }
-    if (!one) {
+    auto oneByOne = [&]() -> int {
         for (int i = 0; i < count; ++i) {
             int rc = ts2_matmul_backprop(mode, len, lenRound, srcDim, gradDim, grad[i], bufs[i], alpha[i], alphaPtr ? alphaPtr[i] : nullptr, srcGrad,
                 srcGradType, add || i > 0, stream);
@@ -186,6 +186,9 @@ extern "C" int ts2_matmul_backprop_group(int32_t mode, int32_t len, int32_t lenR
             }
         }
         return TS2_OK;
+    };
+    if (!one) {
+        return oneByOne();
     }
     ts2_gemm_args g = {};
     g.a = *grad[0];
@@ -208,7 +211,9 @@ extern "C" int ts2_matmul_backprop_group(int32_t mode, int32_t len, int32_t lenR
         g.segment[i - 1].alpha = alpha[i];
         g.segment[i - 1].alphaPtr = alphaPtr ? alphaPtr[i] : nullptr;
     }
-    return ts2_gemm_nt(&g, stream);
+    const int rc = ts2_gemm_nt(&g, stream);
+    // (strides beyond what the kernel for few tiles addresses: one product after the other)
+    return rc == TS2_ERR_UNSUPPORTED && ((lenRound % 256) || (srcDim % 256)) ? oneByOne() : rc;
 }
 
 extern "C" int ts2_matmul_backprop_delta(int32_t mode, int32_t len, int32_t lenRound, int32_t srcDim, int32_t gradDim, const ts2_mat *src,
@@ -532,7 +537,11 @@ int Ts2BackpropGroupI8(int count, int len, int lenRound, int srcDim, int gradDim
     if (count < 1 || count > 4) {
         return TS2_ERR_SHAPE;
     }
-    bool one = count > 1 && (srcGradType == TS2_F32 || srcGradType == TS2_BF16) && (int64_t)(lenRound / 64) * (srcDim / 128) <= 640;
+    // one launch: the kernel for few tiles, or up to the size where 256x256 tiles fill the chip the 128x128 one (16384 x 512 x 512, four
+    // products: 75 us in four launches, 47 in one; two products 36 -> 25)
+    const bool few = (int64_t)(lenRound / 64) * (srcDim / 128) <= 640;
+    const bool sum = srcGradType == TS2_F32 && !add && (int64_t)lenRound * srcDim < (int64_t)192 * 65536;
+    bool one = count > 1 && (srcGradType == TS2_F32 || srcGradType == TS2_BF16) && (few || sum);
     for (int i = 1; i < count && one; ++i) {
         one = grad8[i].strideBytes == grad8[0].strideBytes && transformT[i].strideBytes == transformT[0].strideBytes;
     }
@@ -559,12 +568,16 @@ int Ts2BackpropGroupI8(int count, int len, int lenRound, int srcDim, int gradDim
             g.segB[i - 1] = (const uint8_t *)transformT[i].ptr;
             g.segAlpha[i - 1] = alpha[i];
             g.segAlphaPtr[i - 1] = alphaPtr[i];
-            sp.segRowScale[i - 1] = rowScale[i];
+            g.segRowScale[i - 1] = rowScale[i];
         }
         sp.ct = srcGradType == TS2_F32 ? gemmk::C_F32 : gemmk::C_BF16;
         sp.epi = add ? TS2_EPI_ADD : TS2_EPI_STORE;
-        if (gemmk::SliceCanRun(sp, gemmk::T_I8, false)) {
+        if (few && gemmk::SliceCanRun(sp, gemmk::T_I8, false)) {
             return gemmk::RunSlice(sp, gemmk::T_I8, false, (hipStream_t)stream);
+        }
+        const int rc = sum ? gemmk::RunSumI8(g, (hipStream_t)stream) : TS2_ERR_UNSUPPORTED;
+        if (rc != TS2_ERR_UNSUPPORTED) {
+            return rc;
         }
     }
     for (int i = 0; i < count; ++i) {
