@@ -932,8 +932,9 @@ __global__ void __launch_bounds__(256) NormalizeRowsWave(int len, int lenRound, 
 
 // Row-major k-tile quantiser: dst[t][x] = sat_i8(rne(src[t][x] * rowMult[t] / scale)) with one scale per kTile rows, formed from the row maxima
 // that the row quantiser left (the arithmetic and the dither of TransposeQuant, without its transpose: the delta product reads both
-// operands contraction-major).  A workgroup takes 32 rows, which lie in one k-tile; rows in [len, lenRound) are cleared.  blockIdx.y = source;
-// tileScale: [sources][lenRound / kTile].
+// operands contraction-major).  A workgroup takes QT_ROWS rows, which lie in one k-tile; rows in [len, lenRound) are cleared.  blockIdx.y =
+// source; tileScale: [sources][lenRound / kTile].  Rows per workgroup 32 -> 8: 512 x 1024, two gradients 13.1 -> 5.3 us; 16384 x 512 9.6 -> 7.9
+constexpr int QT_ROWS = 8;
 struct TileQuantJobs {
     Mat src[4], dst[4];
     const float *rowAbsMax[4];
@@ -947,7 +948,7 @@ __global__ void __launch_bounds__(256) QuantTileRows(int len, int lenRound, int 
     const float *rowAbsMax = jobs.rowAbsMax[blockIdx.y];
     const uint32_t seed = jobs.seed[blockIdx.y];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int t0 = blockIdx.x * 32, k0 = t0 / kTile * kTile;
+    const int t0 = blockIdx.x * QT_ROWS, k0 = t0 / kTile * kTile;
     float mx = 0;
     for (int t = k0 + tid; t < k0 + kTile && t < len; t += 256) {
         float m = rowAbsMax[t];
@@ -967,7 +968,7 @@ __global__ void __launch_bounds__(256) QuantTileRows(int len, int lenRound, int 
         tileScale[blockIdx.y * (lenRound / kTile) + t0 / kTile] = tm > 0 ? tm / 127 : 1.f;
     }
     // units of 8 elements, walked by the whole workgroup: four 16-byte loads in flight per lane
-    const int perRow = dim / 8, units = 32 * perRow;
+    const int perRow = dim / 8, units = QT_ROWS * perRow;
     for (int u0 = tid; u0 < units; u0 += 1024) {
         uint4 raw[4];
         float rm[4];
@@ -1206,6 +1207,42 @@ __global__ void __launch_bounds__(256) TransposeQuant(int len, int lenRound, Mat
 }
 
 
+// dst_i = src_i^T for up to TRANSPOSE_JOBS byte matrices in one launch (dimensions multiples of 128; a workgroup per 128x128 tile):
+// after an update every matrix of a model is transposed again (28 of a 512-wide model: 123 -> 8.7 us)
+constexpr int TRANSPOSE_JOBS = 32;
+struct TransposeJobs {
+    Mat src[TRANSPOSE_JOBS], dst[TRANSPOSE_JOBS];
+    int tilesX[TRANSPOSE_JOBS], first[TRANSPOSE_JOBS + 1]; // column tiles of src; tiles before the job
+};
+
+__global__ void __launch_bounds__(256) TransposeBytes(int count, TransposeJobs jobs)
+{
+    constexpr int PITCH = 132;
+    __shared__ __attribute__((aligned(16))) uint8_t buf[128 * PITCH];
+    int j = 0;
+    while (j + 1 < count && (int)blockIdx.x >= jobs.first[j + 1]) {
+        ++j;
+    }
+    const int tile = blockIdx.x - jobs.first[j], xBlock = tile % jobs.tilesX[j] * 128, tBlock = tile / jobs.tilesX[j] * 128;
+    const Mat src = jobs.src[j];
+    const int tid = threadIdx.x, lr = tid >> 3, lc = tid & 7;
+    v4i raw[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        raw[k] = *(const v4i *)(src.p + (int64_t)(tBlock + k * 32 + lr) * src.ld + xBlock + lc * 16);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        uint32_t *d = (uint32_t *)(buf + (k * 32 + lr) * PITCH + lc * 16);
+        d[0] = (uint32_t)raw[k][0];
+        d[1] = (uint32_t)raw[k][1];
+        d[2] = (uint32_t)raw[k][2];
+        d[3] = (uint32_t)raw[k][3];
+    }
+    __syncthreads();
+    TransposeOut128<PITCH>(buf, jobs.dst[j], xBlock, tBlock, tid);
+}
+
 // rope pairs are (cos, sin) interleaved: lane holds two pairs
 __device__ __forceinline__ F4 ApplyRope4(F4 v, F4 rope, float dir)
 {
@@ -1256,10 +1293,16 @@ __global__ void __launch_bounds__(256) RowTileNormalizeRope(int len, int lenRoun
     }
 }
 
+// blockIdx.y = job: the gradients of Q, K and V go in one launch (4096 x 512, e4m3: 3 x 4.4 -> 7.7 us; 16384 x 384, bf16: 3 x 9.8 -> 24.3)
+struct NormRopeJobs {
+    Mat grad[4], srcNorm[4], srcTileScale[4], rope[4], dst[4];
+};
+
 template <class TGrad, class TDst>
-__global__ void __launch_bounds__(256) BackpropRowTileNormalizeRope(int len, int lenRound, int tiles, Mat grad, float gradMult, Mat srcNorm,
-    Mat srcTileScale, Mat rope, Mat dst)
+__global__ void __launch_bounds__(256) BackpropRowTileNormalizeRope(int len, int lenRound, int tiles, float gradMult, NormRopeJobs jobs)
 {
+    const Mat grad = jobs.grad[blockIdx.y], srcNorm = jobs.srcNorm[blockIdx.y], srcTileScale = jobs.srcTileScale[blockIdx.y],
+              rope = jobs.rope[blockIdx.y], dst = jobs.dst[blockIdx.y];
     int t0, tile, h;
     if (!Unit(lenRound, tiles, &t0, &tile, &h)) {
         return;
@@ -1297,9 +1340,10 @@ __global__ void __launch_bounds__(256) BackpropRowTileNormalizeRope(int len, int
 
 // bf16 gradient -> e4m3 with eight elements per lane (a tile = 16 lanes, the tile sums are four DPP steps, the rotated pairs sit in
 // one lane): the form the model's attention backward uses.  Same arithmetic per element as BackpropRowTileNormalizeRope.
-__global__ void __launch_bounds__(256) BackpropRowTileNormalizeRope8(int len, int lenRound, int tiles, Mat grad, float gradMult, Mat srcNorm,
-    Mat srcTileScale, Mat rope, Mat dst)
+__global__ void __launch_bounds__(256) BackpropRowTileNormalizeRope8(int len, int lenRound, int tiles, float gradMult, NormRopeJobs jobs)
 {
+    const Mat grad = jobs.grad[blockIdx.y], srcNorm = jobs.srcNorm[blockIdx.y], srcTileScale = jobs.srcTileScale[blockIdx.y],
+              rope = jobs.rope[blockIdx.y], dst = jobs.dst[blockIdx.y];
     constexpr int UU = 2;
     const int l16 = threadIdx.x & 15;
     const long unit0 = ((long)blockIdx.x * 256 + threadIdx.x) >> 4;
@@ -1793,7 +1837,7 @@ int Ts2QuantTileRows(int count, int len, int lenRound, int kTile, const ts2_mat 
         jobs.rowAbsMax[i] = rowAbsMax[i];
         jobs.seed[i] = seed[i];
     }
-    hipLaunchKernelGGL(QuantTileRows, dim3(lenRound / 32, count), dim3(256), 0, STREAM, len, lenRound, dst[0].x, kTile, jobs, rowMult, tileScale);
+    hipLaunchKernelGGL(QuantTileRows, dim3(lenRound / QT_ROWS, count), dim3(256), 0, STREAM, len, lenRound, dst[0].x, kTile, jobs, rowMult, tileScale);
     TS2_CHECK_LAUNCH();
     return TS2_OK;
 }
@@ -1924,6 +1968,31 @@ int Ts2TransposeQuantRows(int len, int lenRound, const ts2_mat *src, int srcType
     return TS2_OK;
 }
 
+int Ts2TransposeBytesBatch(int count, const ts2_mat *const *src, const ts2_mat *const *dst, int const *rows, const int *cols, void *stream)
+{
+    for (int i = 0; i < count; ++i) {
+        if (rows[i] <= 0 || cols[i] <= 0 || rows[i] % 128 || cols[i] % 128 || src[i]->x < cols[i] || src[i]->y < rows[i] || dst[i]->x < rows[i] || dst[i]->y < cols[i]) {
+            return TS2_ERR_SHAPE;
+        }
+        if (!Aligned16(src[i]->ptr, src[i]->strideBytes) || !Aligned16(dst[i]->ptr, dst[i]->strideBytes)) {
+            return TS2_ERR_ALIGN;
+        }
+    }
+    for (int done = 0; done < count; done += TRANSPOSE_JOBS) {
+        TransposeJobs jobs = {};
+        const int n = count - done < TRANSPOSE_JOBS ? count - done : TRANSPOSE_JOBS;
+        for (int i = 0; i < n; ++i) {
+            jobs.src[i] = M(*src[done + i]);
+            jobs.dst[i] = M(*dst[done + i]);
+            jobs.tilesX[i] = cols[done + i] / 128;
+            jobs.first[i + 1] = jobs.first[i] + jobs.tilesX[i] * (rows[done + i] / 128);
+        }
+        hipLaunchKernelGGL(TransposeBytes, dim3(jobs.first[n]), dim3(256), 0, STREAM, n, jobs);
+        TS2_CHECK_LAUNCH();
+    }
+    return TS2_OK;
+}
+
 extern "C" int ts2_row_tile_normalize_rope(int32_t len, int32_t lenRound, const ts2_mat *src, int32_t srcType, float srcMult, int32_t normalize,
     float vecScale, const ts2_mat *ropeBuf, const ts2_mat *dst, const ts2_mat *tileScale, void *stream)
 {
@@ -1954,32 +2023,54 @@ extern "C" int ts2_row_tile_normalize_rope(int32_t len, int32_t lenRound, const 
 extern "C" int ts2_backprop_row_tile_normalize_rope(int32_t len, int32_t lenRound, const ts2_mat *grad, int32_t gradType, float gradMult,
     const ts2_mat *srcNorm, const ts2_mat *srcTileScale, const ts2_mat *ropeBuf, const ts2_mat *dst, int32_t dstType, void *stream)
 {
-    if (!grad || !dst || (srcNorm && !srcTileScale)) {
-        return TS2_ERR_NULL;
-    }
-    int dim = dst->x;
-    if (dim % TILE || !MatOk(grad, len, dim, ElemSize(gradType)) || !MatOk(dst, lenRound, dim, ElemSize(dstType)) ||
-        (srcNorm && (!MatOk(srcNorm, len, dim, 2) || !MatOk(srcTileScale, dim / TILE, len, 4))) || (ropeBuf && !MatOk(ropeBuf, len, TILE, 4))) {
+    return Ts2BackpropNormRopeGroup(1, len, lenRound, &grad, gradType, gradMult, &srcNorm, &srcTileScale, &ropeBuf, &dst, dstType, stream);
+}
+
+// the same for up to four gradients of one width, each with or without normalisation and rotation
+int Ts2BackpropNormRopeGroup(int count, int len, int lenRound, const ts2_mat *const *grad, int gradType, float gradMult, const ts2_mat *const *srcNorm,
+    const ts2_mat *const *srcTileScale, const ts2_mat *const *ropeBuf, const ts2_mat *const *dst, int dstType, void *stream)
+{
+    if (count < 1 || count > 4) {
         return TS2_ERR_SHAPE;
     }
-    int tiles = dim / TILE;
-    Mat rope = ropeBuf ? M(*ropeBuf) : Mat{nullptr, 0};
-    Mat sn = srcNorm ? M(*srcNorm) : Mat{nullptr, 0};
-    Mat st = srcNorm ? M(*srcTileScale) : Mat{nullptr, 0};
+    NormRopeJobs jobs = {};
+    bool wide = gradType == TS2_BF16 && dstType == TS2_E4M3; // eight elements per lane
+    for (int i = 0; i < count; ++i) {
+        if (!grad[i] || !dst[i] || (srcNorm[i] && !srcTileScale[i])) {
+            return TS2_ERR_NULL;
+        }
+        const int dim = dst[i]->x;
+        if (dim % TILE || dim != dst[0]->x || !MatOk(grad[i], len, dim, ElemSize(gradType)) || !MatOk(dst[i], lenRound, dim, ElemSize(dstType)) ||
+            (srcNorm[i] && (!MatOk(srcNorm[i], len, dim, 2) || !MatOk(srcTileScale[i], dim / TILE, len, 4))) ||
+            (ropeBuf[i] && !MatOk(ropeBuf[i], len, TILE, 4))) {
+            return TS2_ERR_SHAPE;
+        }
+        jobs.grad[i] = M(*grad[i]);
+        jobs.dst[i] = M(*dst[i]);
+        if (srcNorm[i]) {
+            jobs.srcNorm[i] = M(*srcNorm[i]);
+            jobs.srcTileScale[i] = M(*srcTileScale[i]);
+        }
+        if (ropeBuf[i]) {
+            jobs.rope[i] = M(*ropeBuf[i]);
+        }
+        wide = wide && Aligned16(grad[i]->ptr, grad[i]->strideBytes) && (!srcNorm[i] || Aligned16(srcNorm[i]->ptr, srcNorm[i]->strideBytes)) &&
+               (!ropeBuf[i] || Aligned16(ropeBuf[i]->ptr, ropeBuf[i]->strideBytes)) && (((uintptr_t)dst[i]->ptr | dst[i]->strideBytes) & 7) == 0;
+    }
+    const int tiles = dst[0]->x / TILE;
     if (gradType != TS2_F32 && gradType != TS2_BF16) {
         return TS2_ERR_UNSUPPORTED;
     }
-    if (gradType == TS2_BF16 && dstType == TS2_E4M3 && Aligned16(grad->ptr, grad->strideBytes) && (!srcNorm || Aligned16(srcNorm->ptr, srcNorm->strideBytes)) &&
-        (!ropeBuf || Aligned16(ropeBuf->ptr, ropeBuf->strideBytes)) && (((uintptr_t)dst->ptr | dst->strideBytes) & 7) == 0) {
+    if (wide) {
         const long lanes = ((long)lenRound * tiles * 16 + 1) / 2;
-        hipLaunchKernelGGL(BackpropRowTileNormalizeRope8, dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, STREAM, len, lenRound, tiles, M(*grad),
-            gradMult, sn, st, rope, M(*dst));
+        hipLaunchKernelGGL(BackpropRowTileNormalizeRope8, dim3((unsigned)((lanes + 255) / 256), count), dim3(256), 0, STREAM, len, lenRound, tiles,
+            gradMult, jobs);
         TS2_CHECK_LAUNCH();
         return TS2_OK;
     }
 #define LAUNCH_BR(TG, TD)                                                                                                                  \
-    hipLaunchKernelGGL((BackpropRowTileNormalizeRope<TG, TD>), GridFor(lenRound, tiles), dim3(256), 0, STREAM, len, lenRound, tiles, M(*grad), \
-        gradMult, sn, st, rope, M(*dst))
+    hipLaunchKernelGGL((BackpropRowTileNormalizeRope<TG, TD>), dim3(GridFor(lenRound, tiles).x, count), dim3(256), 0, STREAM, len, lenRound, tiles, \
+        gradMult, jobs)
     if (gradType == TS2_F32) {
         TS2_DISPATCH_TYPE(dstType, TD, LAUNCH_BR(TF32, TD));
     } else {

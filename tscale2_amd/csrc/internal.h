@@ -46,6 +46,11 @@ int Ts2ForwardGroup(int mode, int count, int len, int lenRound, int srcDim, int 
 bool Ts2OptBatchable(const ts2_opt_matrix *m);
 int Ts2OptApplyBatch(int count, const ts2_opt_matrix *const *mats, const ts2_mat *const *delta, const ts2_mat *const *tileScale,
     const ts2_add_gradient_params *params, void *stream);
+// ts2_backprop_row_tile_normalize_rope of up to four gradients of one width in one launch
+int Ts2BackpropNormRopeGroup(int count, int len, int lenRound, const ts2_mat *const *grad, int gradType, float gradMult, const ts2_mat *const *srcNorm,
+    const ts2_mat *const *srcTileScale, const ts2_mat *const *ropeBuf, const ts2_mat *const *dst, int dstType, void *stream);
+// dst_i [cols][rows] = src_i [rows][cols]^T for byte matrices whose dimensions are multiples of 128, 32 to a launch
+int Ts2TransposeBytesBatch(int count, const ts2_mat *const *src, const ts2_mat *const *dst, const int *rows, const int *cols, void *stream);
 // per-group deltas (TMoeDeltaMatMulKernelCall) by the kernel for few tiles: groups * gradDim rows of packed delta
 int Ts2GroupedDeltaRows(int rows, int srcDim, int gradDim, int groups, const int *groupOffsets, const ts2_mat *src, const ts2_mat *grad, float alpha,
     const float *alphaPtr, const ts2_mat *delta, int64_t deltaSlabBytes, const ts2_mat *tileScale, int64_t tileScaleSlabBytes, void *stream);

@@ -556,9 +556,10 @@ int AttBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
     ag.which = 3;
     CK(ts2_att_backward(&ag, s));
     // epilogues: norm backward against the stored rotated vector, then inverse rope (TStoreAttBack*, gpu_att_utils.cuh:280-352)
-    CK(ts2_backprop_row_tile_normalize_rope(len, R, dQ.P(), TS2_BF16, 1.f, q16.P(), qScale.P(), M->rope.P(), dQf.P(), M->fastGradType, s));
-    CK(ts2_backprop_row_tile_normalize_rope(len, R, dK.P(), TS2_BF16, 1.f, nullptr, nullptr, M->rope.P(), dKf.P(), M->fastGradType, s));
-    CK(ts2_backprop_row_tile_normalize_rope(len, R, dV.P(), TS2_BF16, 1.f, v16.P(), vScale.P(), nullptr, dVf.P(), M->fastGradType, s));
+    const ts2_mat *const nrGrad[3] = {dQ.P(), dK.P(), dV.P()}, *const nrNorm[3] = {q16.P(), nullptr, v16.P()};
+    const ts2_mat *const nrScale[3] = {qScale.P(), nullptr, vScale.P()}, *const nrRope[3] = {M->rope.P(), M->rope.P(), nullptr};
+    const ts2_mat *const nrDst[3] = {dQf.P(), dKf.P(), dVf.P()};
+    CK(Ts2BackpropNormRopeGroup(3, len, R, nrGrad, TS2_BF16, 1.f, nrNorm, nrScale, nrRope, nrDst, M->fastGradType, s));
     TMatrix *const ws[4] = {&L.w[0], &L.w[1], &L.w[2], &L.w[3]};
     const Arr *const gs[4] = {&dQf, &dKf, &dVf, &dGate};
     CK(BackpropDXGroup(M, 4, ws, gs, DISCR * Dot(D), useScale, M->dNormState, false, s));
@@ -914,6 +915,31 @@ int FinalBackward(ts2_model *M, void *s)
 }
 
 // CreateBackpropGraph, src/gpt/compute/gpu_transformer.cu:326-471 (one device, one micro batch)
+// the transposes of the attention and feed-forward matrices that changed since they were made
+int TransposeWeights(ts2_model *M, void *s)
+{
+    std::vector<const ts2_mat *> src, dst;
+    std::vector<int> rows, cols;
+    std::vector<TMatrix *> made;
+    for (TLayer &L : M->layers) {
+        for (int k = 0; k < 5 && L.type != LT_MOE; ++k) {
+            TMatrix &W = L.w[k];
+            if (W.fastT.m.ptr && !W.fastTValid) {
+                src.push_back(W.fast.P());
+                dst.push_back(W.fastT.P());
+                rows.push_back(W.dstDim);
+                cols.push_back(W.srcDim);
+                made.push_back(&W);
+            }
+        }
+    }
+    CK(Ts2TransposeBytesBatch((int)made.size(), src.data(), dst.data(), rows.data(), cols.data(), s));
+    for (TMatrix *W : made) {
+        W->fastTValid = true;
+    }
+    return 0;
+}
+
 int ModelBackprop(ts2_model *M, void *s)
 {
     int D = M->cfg.dim, depth = (int)M->layers.size();
@@ -921,6 +947,7 @@ int ModelBackprop(ts2_model *M, void *s)
     CK(Ts2ZeroRows(Flat(M->gradMaxNorm, 1, depth + 2, TS2_F32).P(), 1, (depth + 2) * 4, s));
     CK(Ts2FillFloats(M->gradMult, 1, 1.f, s)); // the multiplier the final normalisation applies to the fast gradient
     CK(FinalBackward(M, s));
+    CK(TransposeWeights(M, s));
     M->useKept = M->keep;
     struct TReset {
         ts2_model *M;

@@ -537,8 +537,8 @@ int Ts2BackpropGroupI8(int count, int len, int lenRound, int srcDim, int gradDim
     if (count < 1 || count > 4) {
         return TS2_ERR_SHAPE;
     }
-    // one launch: the kernel for few tiles, or up to the size where 256x256 tiles fill the chip the 128x128 one (16384 x 512 x 512, four
-    // products: 75 us in four launches, 47 in one; two products 36 -> 25)
+    // one launch: the kernel for few tiles, or up to the size where 256x256 tiles fill the chip the 128x128 one (16384 x 512 x 512 inside the
+    // e512 step: a sum of four and a sum of two products 111 us together as six launches, 72 as two)
     const bool few = (int64_t)(lenRound / 64) * (srcDim / 128) <= 640;
     const bool sum = srcGradType == TS2_F32 && !add && (int64_t)lenRound * srcDim < (int64_t)192 * 65536;
     bool one = count > 1 && (srcGradType == TS2_F32 || srcGradType == TS2_BF16) && (few || sum);
