@@ -914,32 +914,40 @@ int FinalBackward(ts2_model *M, void *s)
         M->stateGradFast.P(), M->fastGradType, M->gradMaxNorm, s);
 }
 
-// CreateBackpropGraph, src/gpt/compute/gpu_transformer.cu:326-471 (one device, one micro batch)
 // the transposes of the attention and feed-forward matrices that changed since they were made
 int TransposeWeights(ts2_model *M, void *s)
 {
-    std::vector<const ts2_mat *> src, dst;
-    std::vector<int> rows, cols;
-    std::vector<TMatrix *> made;
+    constexpr int BATCH = 32;
+    const ts2_mat *src[BATCH], *dst[BATCH];
+    TMatrix *made[BATCH];
+    int rows[BATCH], cols[BATCH], n = 0;
+    auto flush = [&]() -> int {
+        CK(Ts2TransposeBytesBatch(n, src, dst, rows, cols, s));
+        for (int i = 0; i < n; ++i) {
+            made[i]->fastTValid = true;
+        }
+        n = 0;
+        return 0;
+    };
     for (TLayer &L : M->layers) {
         for (int k = 0; k < 5 && L.type != LT_MOE; ++k) {
             TMatrix &W = L.w[k];
             if (W.fastT.m.ptr && !W.fastTValid) {
-                src.push_back(W.fast.P());
-                dst.push_back(W.fastT.P());
-                rows.push_back(W.dstDim);
-                cols.push_back(W.srcDim);
-                made.push_back(&W);
+                src[n] = W.fast.P();
+                dst[n] = W.fastT.P();
+                rows[n] = W.dstDim;
+                cols[n] = W.srcDim;
+                made[n] = &W;
+                if (++n == BATCH) {
+                    CK(flush());
+                }
             }
         }
     }
-    CK(Ts2TransposeBytesBatch((int)made.size(), src.data(), dst.data(), rows.data(), cols.data(), s));
-    for (TMatrix *W : made) {
-        W->fastTValid = true;
-    }
-    return 0;
+    return flush();
 }
 
+// CreateBackpropGraph, src/gpt/compute/gpu_transformer.cu:326-471 (one device, one micro batch)
 int ModelBackprop(ts2_model *M, void *s)
 {
     int D = M->cfg.dim, depth = (int)M->layers.size();
@@ -1292,8 +1300,15 @@ extern "C" int ts2_model_apply_deltas(ts2_model *M, const ts2_add_gradient_param
     if (hipMemcpyAsync(M->optParams, paramsHost, sizeof(ts2_add_gradient_params), hipMemcpyHostToDevice, (hipStream_t)stream) != hipSuccess) {
         return TS2_ERR_LAUNCH;
     }
-    std::vector<const ts2_opt_matrix *> batch; // matrices whose updates share launches
-    std::vector<const ts2_mat *> deltas, scales;
+    constexpr int BATCH = 16;
+    const ts2_opt_matrix *batch[BATCH]; // matrices whose updates share launches
+    const ts2_mat *deltas[BATCH], *scales[BATCH];
+    int pending = 0;
+    auto flush = [&]() -> int {
+        const int n = pending;
+        pending = 0;
+        return Ts2OptApplyBatch(n, batch, deltas, scales, M->optParams, stream);
+    };
     auto apply = [&](TMatrix &W, bool packed) -> int {
         if (!W.hasOpt) {
             return 0;
@@ -1301,10 +1316,10 @@ extern "C" int ts2_model_apply_deltas(ts2_model *M, const ts2_add_gradient_param
         W.fastTValid = false;
         const ts2_opt_matrix &o = W.opt;
         if (packed && Ts2OptBatchable(&o)) {
-            batch.push_back(&o);
-            deltas.push_back(W.delta.P());
-            scales.push_back(W.deltaTileScale.P());
-            return 0;
+            batch[pending] = &o;
+            deltas[pending] = W.delta.P();
+            scales[pending] = W.deltaTileScale.P();
+            return ++pending == BATCH ? flush() : 0;
         }
         if (packed) {
             return ts2_opt_add_delta(&o, W.delta.P(), W.deltaTileScale.P(), TS2_BM_GRAD_APPLY, M->optParams, stream);
@@ -1324,7 +1339,7 @@ extern "C" int ts2_model_apply_deltas(ts2_model *M, const ts2_add_gradient_param
             }
         }
     }
-    return Ts2OptApplyBatch((int)batch.size(), batch.data(), deltas.data(), scales.data(), M->optParams, stream);
+    return flush();
 }
 
 // host copy of a matrix's master weights [rows][cols] (synchronises the device)
