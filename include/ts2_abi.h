@@ -293,8 +293,9 @@ typedef struct ts2_matmul_bwd_buffers {
      * scanning the gradient again when gradRowAbsMaxValid != 0: the caller sets that when both calls get the same gradient tensor. */
     float *gradRowAbsMax;
     int32_t gradRowAbsMaxValid;
-    /* != 0: srcT already holds the transpose of the `src` given to BackpropDelta (an earlier BackpropDelta call with the same buffers
-     * and the same source tensor left it there, as for the matrices of one layer that share their input); the transpose is skipped. */
+    /* != 0 (I8): srcT already holds the transpose of the `src` given to BackpropDelta (an earlier BackpropDelta call with the same buffers
+     * and the same source tensor left it there, as for the matrices of one layer that share their input); the transpose is skipped.
+     * E4M3 does not read the flag: its calls for few tiles read the source as it lies and leave no transpose. */
     int32_t srcTValid;
     /* != 0 (E4M3): gradT already holds the transpose of the `grad` given to BackpropDelta (its producer wrote it, e.g.
      * ts2_backprop_row_tile_normalize_lolu_t); the transpose is skipped. */

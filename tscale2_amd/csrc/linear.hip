@@ -36,8 +36,9 @@ int DeltaSlice(int mode, int len, int lenRound, int srcDim, int gradDim, const t
     sp.kTileScaleRows = kTileScaleRows;
     sp.epi = TS2_EPI_STORE;
     if (grad->x < gradDim || src->x < srcDim || grad->y < len || src->y < len || delta->x < srcDim || delta->y < gradDim ||
-        tileScale->x < gradDim || tileScale->y < srcDim / TILE || (kTileScale && (grad->y < lenRound || src->y < lenRound))) {
-        return TS2_ERR_SHAPE;
+        tileScale->x < gradDim || tileScale->y < srcDim / TILE || !grad->ptr || !src->ptr || !delta->ptr || !tileScale->ptr ||
+        (kTileScale && (grad->y < lenRound || src->y < lenRound))) {
+        return TS2_ERR_UNSUPPORTED; // (the general path, where there is one, names what is wrong)
     }
     if (splits > 1) {
         g.c = (uint8_t *)partial;
