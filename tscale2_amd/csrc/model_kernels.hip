@@ -446,8 +446,9 @@ __global__ void __launch_bounds__(1024) FinalSoftmaxGradHalfRow(int rows, int vo
     }
 }
 
-// Vocabularies below 2048: one wave per row, the row in its registers (NCH chunks of 512 halves), waves walk rows with the grid's stride,
-// the next row's loads in flight.  Per logit one exponential in fp32, the arithmetic of the two-pass kernel.  A workgroup adds its
+// Vocabularies up to 2048: one wave per row, the row in its registers (NCH chunks of 512 halves), waves walk rows with the grid's stride,
+// the next row's loads in flight.  Per logit one exponential in fp32, the arithmetic of the two-pass kernel but for the reference, which
+// counts the bias.  A workgroup adds its
 // rows' loss once: the per-row atomic on one address alone took 13 ns a row (16384 x 1024 logits: 213 us, now 24; 65536 x 128: 834 us).
 template <int NCH>
 __global__ void __launch_bounds__(256) FinalSoftmaxGradHalfWave(int rows, int vocab, const _Float16 *logits, int64_t ldLogits, const float *bias,
@@ -508,7 +509,7 @@ __global__ void __launch_bounds__(256) FinalSoftmaxGradHalfWave(int rows, int vo
         for (int i = 0; i < NCH; ++i) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                m = fmaxf(m, (float)cur[i][e]);
+                m = fmaxf(m, (float)cur[i][e] + bv[i][e]); // (with its bias: no bias overflows the exponential)
             }
         }
         m = WaveMax(m);
