@@ -826,7 +826,7 @@ __global__ void __launch_bounds__(256) NormalizeVecsRowMax(int len, int lenRound
 // The same quantiser with one wave per row for bf16 rows of at most NCH * 512 <= 4096 elements (a multiple of 8): a lane holds NCH chunks
 // of 8 consecutive elements (16-byte loads, 8-byte stores, each instruction of the wave covering 1 KB / 512 B of the row), the row
 // maxima are wave reductions, and no workgroup barrier or LDS exchange is left.  Same arithmetic per element as NormalizeVecsRowMax.
-// blockIdx.y = source: the gradients of a layer's matrices go in one launch (rows of 384 elements, 16384 of them: 13.6 us each one by one
+// Batch: blockIdx.y = source, the gradients of a layer's matrices go in one launch (rows of 384 elements, 16384 of them: 13.6 us each one by one
 // with a workgroup per row).
 struct RowQuantJobs {
     Mat src[4], dst[4];
@@ -836,11 +836,9 @@ struct RowQuantJobs {
 
 // FULL: rows of exactly NCH * 512 elements.
 template <int NCH, bool FULL>
-__global__ void __launch_bounds__(256) NormalizeRowsWave(int len, int lenRound, int dim, RowQuantJobs jobs, const float *colScale)
+__device__ __forceinline__ void NormalizeRowsWaveOf(int len, int lenRound, int dim, const Mat &src, const float *colScale, const Mat &dst,
+    float *rowScale, float *rowAbsMax, uint32_t seed)
 {
-    const Mat src = jobs.src[blockIdx.y], dst = jobs.dst[blockIdx.y];
-    float *const rowScale = jobs.rowScale[blockIdx.y], *const rowAbsMax = jobs.rowAbsMax[blockIdx.y];
-    const uint32_t seed = jobs.seed[blockIdx.y];
     const int lane = threadIdx.x & 63;
     bool in[NCH];
 #pragma unroll
@@ -928,6 +926,21 @@ __global__ void __launch_bounds__(256) NormalizeRowsWave(int len, int lenRound, 
             }
         }
     }
+}
+
+template <int NCH, bool FULL>
+__global__ void __launch_bounds__(256) NormalizeRowsWaveBatch(int len, int lenRound, int dim, RowQuantJobs jobs)
+{
+    const int j = blockIdx.y;
+    NormalizeRowsWaveOf<NCH, FULL>(len, lenRound, dim, jobs.src[j], nullptr, jobs.dst[j], jobs.rowScale[j], jobs.rowAbsMax[j], jobs.seed[j]);
+}
+
+// one source: its description lies in scalar registers from the start (16384 x 4096: 36.5 us, 37.6 through the job table)
+template <int NCH, bool FULL>
+__global__ void __launch_bounds__(256) NormalizeRowsWave(int len, int lenRound, int dim, Mat src, const float *colScale, Mat dst, float *rowScale,
+    float *rowAbsMax, uint32_t seed)
+{
+    NormalizeRowsWaveOf<NCH, FULL>(len, lenRound, FULL ? NCH * 512 : dim, src, colScale, dst, rowScale, rowAbsMax, seed);
 }
 
 // Row-major k-tile quantiser: dst[t][x] = sat_i8(rne(src[t][x] * rowMult[t] / scale)) with one scale per kTile rows, formed from the row maxima
@@ -1767,16 +1780,21 @@ extern "C" int ts2_normalize_vecs_row_max(int32_t len, int32_t lenRound, const t
     return ts2_normalize_vecs_row_max2(len, lenRound, src, srcType, colScale, dst, rowScale, nullptr, stream);
 }
 
+// (column scales: one source only)
 static int LaunchRowQuant(int count, int len, int lenRound, int dim, const RowQuantJobs &jobs, const float *colScale, void *stream)
 {
     // with column scales a wave walks several rows (the scales stay in registers), else one row per wave
     const int wgs = (lenRound + 3) / 4;
     const dim3 grid(colScale && wgs > 2048 ? 2048 : wgs, count);
 #define LAUNCH_RW(N)                                                                                                                       \
-    if (dim == N * 512) {                                                                                                                  \
-        hipLaunchKernelGGL((NormalizeRowsWave<N, true>), grid, dim3(256), 0, STREAM, len, lenRound, dim, jobs, colScale);                  \
+    if (count == 1 && dim == N * 512) {                                                                                                    \
+        hipLaunchKernelGGL((NormalizeRowsWave<N, true>), grid, dim3(256), 0, STREAM, len, lenRound, dim, jobs.src[0], colScale, jobs.dst[0], jobs.rowScale[0], jobs.rowAbsMax[0], jobs.seed[0]); \
+    } else if (count == 1) {                                                                                                               \
+        hipLaunchKernelGGL((NormalizeRowsWave<N, false>), grid, dim3(256), 0, STREAM, len, lenRound, dim, jobs.src[0], colScale, jobs.dst[0], jobs.rowScale[0], jobs.rowAbsMax[0], jobs.seed[0]); \
+    } else if (dim == N * 512) {                                                                                                           \
+        hipLaunchKernelGGL((NormalizeRowsWaveBatch<N, true>), grid, dim3(256), 0, STREAM, len, lenRound, dim, jobs);                       \
     } else {                                                                                                                               \
-        hipLaunchKernelGGL((NormalizeRowsWave<N, false>), grid, dim3(256), 0, STREAM, len, lenRound, dim, jobs, colScale);                 \
+        hipLaunchKernelGGL((NormalizeRowsWaveBatch<N, false>), grid, dim3(256), 0, STREAM, len, lenRound, dim, jobs);                      \
     }
     switch ((dim + 511) / 512) {
     case 1: LAUNCH_RW(1); break;
