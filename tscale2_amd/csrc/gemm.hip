@@ -1100,6 +1100,7 @@ template <int TYPE> int DispatchTile(const ts2_gemm_args *a, const GemmP &p, hip
 //   contraction-major   e4m3 2048x512x4096 42.0 -> 16.0, 2048x2048x8192 75.0 -> 61.3, sliced four ways (256 large tiles) 40.8 -> 77.3
 //   several products    e4m3 4 x 512x256x256 28.5 -> 8.1, 4 x 4096x512x512 37.7 -> 12.8, 4 x 8192x1024x1024 55.6 -> 69.2
 //   i8 stored           512x256x256 6.7 -> 4.9, 2048x1024x1024 10.4 -> 8.6, 4096x512x2048 13.9 -> 11.4, 3072x1536x512 (576) 11.2 -> 16.4
+//                       one per CU and no more: 2048x1024x8192 (256) 47.4 -> 27.6, but 2816x768x2048 (264) 13.9 -> 19.7, x8192 47.9 -> 50.8
 //   e4m3 stored fp32    512x256x256 6.4 -> 4.9, 4096x512x512 8.2 -> 7.1, 512x256x1024 6.6 -> 7.0, 1024x1024x4096 13.8 -> 16.2; as bf16
 //                       (row-owning epilogue there) 512x256x256 4.5 -> 4.9, 4096x512x2048 9.4 -> 10.8
 //   e4m3 accumulating   512x256x256 7.8 -> 5.2, 4096x512x2048 14.3 -> 11.7, 16384x512x512 (1024) 17.5 -> 27.3
@@ -1120,7 +1121,7 @@ bool PreferSlice(const GemmP &p, int type, int ct, int epi)
         return wgs <= (type == T_I8 ? 512 : 384);
     }
     if (type == T_I8) {
-        return wgs <= 320;
+        return wgs <= 256;
     }
     return wgs <= 256 && (type == T_BF16 || epi == TS2_EPI_ADD || (ct == C_F32 && p.kBytes <= 512));
 }
