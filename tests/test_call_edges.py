@@ -1,0 +1,43 @@
+"""Calls that the operators refuse before anything is launched.  The arrays are host memory: nothing here may reach a kernel, so the file
+does not run where a GPU is present."""
+import ctypes as C
+
+import pytest
+
+torch = pytest.importorskip("torch")
+from tscale2_amd import lib as L  # noqa: E402
+
+pytestmark = pytest.mark.skipif(torch.cuda.device_count() > 0, reason="refusals only: no launch may see these host arrays")
+SHAPE, UNSUPPORTED = -1, -3
+
+
+def u8(rows, cols):
+    return torch.zeros((rows, cols), dtype=torch.uint8)
+
+
+def buffers(rows, src, grad, t_cols=None):
+    b = L.BwdBuffers()
+    keep = {"gradT": u8(grad, t_cols or rows), "srcT": u8(src, t_cols or rows), "transformT": u8(src, grad)}
+    for k, v in keep.items():
+        setattr(b, k, L.mat(v))
+    return b, keep
+
+
+def delta(n, rows, src, grad, buf):
+    x, dy, d, s = u8(512, src), u8(512, grad), torch.zeros((grad, src), dtype=torch.int8), torch.zeros((src // 128, grad))
+    m = [L.mat(t) for t in (x, dy, d, s)]
+    return L.load().dll.ts2_matmul_backprop_delta(L.E4M3, n, rows, src, grad, C.byref(m[0]), None, C.byref(m[1]), L.E4M3, C.c_float(1), None, 512,
+                                                  C.byref(buf), C.byref(m[2]), C.byref(m[3]), None)
+
+
+@pytest.mark.parametrize("n,rows,grad", [(180, 192, 384), (300, 256, 384), (64, 64, 384), (256, 256, 192)])
+def test_packed_delta_refuses_sizes_off_the_tile_grid_and_more_rows_than_there_are(n, rows, grad):
+    b, _keep = buffers(rows, 256, grad, 512)
+    assert delta(n, rows, 256, grad, b) == SHAPE
+
+
+def test_the_kernel_for_few_tiles_refuses_a_contraction_that_ends_inside_its_unit():
+    """bit 11 admits contractions of 64 bytes, bit 16 asks for the kernel whose unit is 128"""
+    g = L.GemmArgs(a=L.mat(u8(128, 192)), b=L.mat(u8(128, 192)), c=L.mat(torch.zeros((128, 128))), abType=L.E4M3, cType=L.F32, m=128, n=128, k=192, alpha=1,
+                   splitK=1, tileConfig=65536 | 2048)
+    assert L.load().dll.ts2_gemm_nt(C.byref(g), None) == UNSUPPORTED

@@ -1315,6 +1315,7 @@ extern "C" int ts2_gemm_nt(const ts2_gemm_args *a, void *streamPtr)
         if (ct >= 0 && splitK <= 1 && (askSlice || (!(a->tileConfig & (3 | 8 | 16 | 128 | 2048 | 4096 | 32768 | 131072)) && PreferSlice(p, type, ct, epi)))) {
             SliceP sp = {};
             sp.g = p;
+            sp.kLive = a->k;
             sp.ct = ct;
             sp.epi = epi;
             if (askSlice || SliceCanRun(sp, type, p.kMajor != 0)) {

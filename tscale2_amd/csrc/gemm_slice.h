@@ -7,7 +7,7 @@ namespace gemmk
 struct SliceP {
     GemmP g;
     int ct, epi;                 // C_*, TS2_EPI_STORE / TS2_EPI_ADD
-    int kLive;                   // K-major operands: contraction rows that count (0 = all); later rows read as zeros
+    int kLive;                   // K-major operands: contraction rows that count (none if 0); later rows read as zeros
     int kTileScaleRows;          // kTileScale: > 0 = every so many rows of C have a set of scales of their own (sets one after the other)
     // > 1: blockIdx.z picks one of several products of one shape that share A and are stored separately (C_BF16NORM; of p, b, c, tileScale,
     // alphaPtr, normalize and rope's use are each product's own)

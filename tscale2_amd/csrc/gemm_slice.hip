@@ -186,7 +186,7 @@ template <int TYPE, bool TN, bool KT = false> __global__ void __launch_bounds__(
     }
 #define SLICE_LOAD(M0VAL, VOFF, RSRC)                                                                                                      \
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(M0VAL), "v"(VOFF), "s"(RSRC) : "memory")
-    const int kLive = TN ? (sp.kLive > 0 ? sp.kLive : p.kBytes / ESZ) : 0;
+    const int kLive = sp.kLive;
     auto loadStep = [&](const uint8_t *a, const uint8_t *b, int step, int stage) {
         const unsigned st = ldsBase + stage * STAGE;
         v4i ra, rb;
@@ -618,7 +618,11 @@ namespace gemmk
 bool SliceCanRun(const SliceP &sp, int type, bool tn)
 {
     const GemmP &p = sp.g;
-    if ((p.m % SBM) || (p.n % SBN) || (p.splits > 1 && p.groupOffsets) || p.splitK > 1) {
+    // (a contraction of whole 128-byte units: what is left over would not be multiplied)
+    if (p.m <= 0 || p.n <= 0 || p.kBytes <= 0 || (p.m % SBM) || (p.n % SBN) || (p.kBytes % BKB) || (p.splits > 1 && p.groupOffsets) || p.splitK > 1) {
+        return false;
+    }
+    if (tn && (int64_t)sp.kLive * (type == T_BF16 ? 2 : 1) > p.kBytes) {
         return false;
     }
     if (type == T_I8 ? (sp.ct == C_F16 && sp.epi != TS2_EPI_STORE) : sp.ct == C_I32) {

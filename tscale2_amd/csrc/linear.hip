@@ -35,7 +35,7 @@ int DeltaSlice(int mode, int len, int lenRound, int srcDim, int gradDim, const t
     sp.kLive = len;
     sp.kTileScaleRows = kTileScaleRows;
     sp.epi = TS2_EPI_STORE;
-    if (grad->x < gradDim || src->x < srcDim || grad->y < len || src->y < len || delta->x < srcDim || delta->y < gradDim ||
+    if (len < 0 || len > lenRound || (gradDim % TILE) || grad->x < gradDim || src->x < srcDim || grad->y < len || src->y < len || delta->x < srcDim || delta->y < gradDim ||
         tileScale->x < gradDim || tileScale->y < srcDim / TILE || !grad->ptr || !src->ptr || !delta->ptr || !tileScale->ptr ||
         (kTileScale && (grad->y < lenRound || src->y < lenRound))) {
         return TS2_ERR_UNSUPPORTED; // (the general path, where there is one, names what is wrong)
@@ -517,6 +517,7 @@ int Ts2GroupedDeltaRows(int rows, int srcDim, int gradDim, int groups, const int
     g.m = gradDim;
     g.n = srcDim;
     g.kBytes = rows;
+    sp.kLive = rows;
     g.alpha = alpha;
     g.alphaPtr = alphaPtr;
     g.tileScale = (float *)tileScale->ptr;
