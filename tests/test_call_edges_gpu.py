@@ -29,3 +29,23 @@ def test_packed_delta_of_an_empty_batch_is_zero():
         b.backprop_delta(n, x, None, dy, L.E4M3)
         torch.cuda.synchronize()
         assert bool(b.delta.any()) == (n > 0) and bool(b.delta_tile_scale.any()) == (n > 0)
+
+
+@pytest.mark.parametrize("k,splits", [(2048, 4), (2048, 2), (3072, 2), (4608, 3)])
+def test_stored_slices_with_k_tile_scales_hold_their_own_part_of_the_contraction(k, splits):
+    """int8 with one scale per 512 contraction elements, the contraction cut into stored slices: slab i is the sum over slice i (whole
+    k-tiles, ceil(tiles / splits) of them).  int32 sums are exact; per k-tile one fp32 product and one fp32 addition are left."""
+    print("case k-tile scales and slices", k, splits, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(k + splits)
+    m, n, kt = 256, 256, 512
+    a, b = [torch.randint(-127, 128, (d, k), device="cuda", generator=gen, dtype=torch.int8) for d in (m, n)]
+    scale = torch.rand(k // kt, device="cuda", generator=gen) + 0.5
+    c = torch.full((splits * m, n), 9.0, device="cuda")
+    L.load().gemm_nt(a, b, c, L.I8, L.F32, k_tile_scale=scale, k_tile=kt, split_k=splits, split_slab_bytes=m * n * 4, m=m, n=n)
+    per = -(-(k // kt) // splits) * kt
+    for i in range(splits):
+        want, mag = torch.zeros((m, n), device="cuda", dtype=torch.float64), 0
+        for t in range(i * per, min((i + 1) * per, k), kt):
+            p = (a[:, t:t + kt].double() @ b[:, t:t + kt].double().t()) * scale[t // kt].double()
+            want, mag = want + p, mag + p.abs()
+        assert bool(((c[i * m:(i + 1) * m].double() - want).abs() <= (per // kt + 2) * 2.0 ** -24 * mag).all()), i

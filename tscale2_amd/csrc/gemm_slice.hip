@@ -12,8 +12,9 @@
 //
 // K-major operands (TN: A [k][m], B [k][n]) are read by the transposing LDS reads as in the ring kernel; contraction rows at and beyond
 // kLive read as zeros (the descriptor of a step ends there), so ragged batches need no transposed or cleared copies.
-// KT (i8): one scale per kTile contraction elements.  A workgroup takes up to four k-tiles, wave pair kg the whole of the kg-th (a step is
-// 64 elements of each), so every pair holds one tile's exact int32 sum at the end and the reduction adds them scaled, in tile order.
+// KT (i8): one scale per kTile contraction elements.  A workgroup takes the k-tiles of its slice, up to four, wave pair kg the whole of the
+// kg-th (a step is 64 elements of each), so every pair holds one tile's exact int32 sum at the end and the reduction adds them scaled, in
+// tile order.
 // Several products into one result: fp8 / bf16 keep one set of accumulators, brought to the next product's factor at each seam; i8
 // products carry row scales of their own and are added one after the other in fp32, in the order of separate accumulating launches.
 #include "gemm_slice.h"
@@ -98,9 +99,9 @@ template <int TYPE, bool TN, bool KT = false> __global__ void __launch_bounds__(
     const bool oddTail = !TN && !KT && (kUnits & 1); // NT: the last step holds 128 bytes of K only
     int kt0 = 0, ktCount = 0;                        // KT: first k-tile of the workgroup, number of its k-tiles
     if constexpr (KT) {
-        const int all = p.kBytes / p.kTileBytes;
-        kt0 = p.splits > 1 ? (int)blockIdx.y * 4 : 0;
-        ktCount = min(4, max(all - kt0, 0));
+        const int all = p.kBytes / p.kTileBytes, per = p.splits > 1 ? (all + p.splits - 1) / p.splits : all;
+        kt0 = blockIdx.y * per;
+        ktCount = min(per, max(all - kt0, 0));
         nSteps = ktCount > 0 ? p.kTileBytes / 64 : 0;
     }
 
@@ -653,10 +654,12 @@ bool SliceCanRun(const SliceP &sp, int type, bool tn)
         }
     }
     if (p.kTileScale) {
-        // four k-tiles per workgroup; the sets of scales change between workgroups only
-        const int tiles = p.kTileBytes > 0 ? p.kBytes / p.kTileBytes : 0;
-        if (type != T_I8 || p.groupOffsets || p.nSeg > 1 || sp.ct == C_I32 || tiles < 1 || (p.splits > 1 ? p.splits * 4 < tiles : tiles > 4) ||
-            (sp.kTileScaleRows % SBM)) {
+        // whole k-tiles of whole steps, up to four per workgroup; the sets of scales change between workgroups only
+        if (p.kTileBytes <= 0 || (p.kTileBytes % 64) || (p.kBytes % p.kTileBytes)) {
+            return false;
+        }
+        const int tiles = p.kBytes / p.kTileBytes, slices = p.splits > 1 ? p.splits : 1;
+        if (type != T_I8 || p.groupOffsets || p.nSeg > 1 || sp.ct == C_I32 || (tiles + slices - 1) / slices > 4 || (sp.kTileScaleRows % SBM)) {
             return false;
         }
     }

@@ -437,7 +437,7 @@ int Ts2DeltaRows(int mode, int len, int lenRound, int srcDim, int gradDim, const
 {
     const int64_t outElems = (int64_t)gradDim * srcDim, sliceTiles = (int64_t)(gradDim / 64) * (srcDim / 128);
     if (mode == TS2_I8) {
-        // four k-tiles per workgroup
+        // up to four k-tiles per workgroup
         const int splits = (lenRound / kTile + 3) / 4;
         if (splits > 1 && splits * outElems > partialFloats) {
             return TS2_ERR_UNSUPPORTED;
