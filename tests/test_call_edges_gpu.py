@@ -49,3 +49,16 @@ def test_stored_slices_with_k_tile_scales_hold_their_own_part_of_the_contraction
             p = (a[:, t:t + kt].double() @ b[:, t:t + kt].double().t()) * scale[t // kt].double()
             want, mag = want + p, mag + p.abs()
         assert bool(((c[i * m:(i + 1) * m].double() - want).abs() <= (per // kt + 2) * 2.0 ** -24 * mag).all()), i
+
+
+@pytest.mark.parametrize("mode", [L.E4M3, L.I8])
+def test_normalised_forward_of_an_empty_batch_is_zero(mode):
+    print("case normalised forward of an empty batch", mode, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    rows, src, dst = 256, 256, 384
+    x, w = [e4m3(randn(gen, r, src) * 8) if mode == L.E4M3 else (randn(gen, r, src) * 30).to(torch.int8) for r in (rows, dst)]
+    res = torch.full((rows, dst), 7, dtype=torch.int16, device="cuda")
+    scale, raw = torch.full((dst // 128, rows), 7.0, device="cuda"), torch.empty((rows, dst), device="cuda")
+    L.call("ts2_matmul_forward_norm_rope", mode, 0, rows, src, dst, x, w, 0.01, None, 1, 1 / 24, None, res, scale, raw)
+    torch.cuda.synchronize()
+    assert not bool(res.any()) and not bool(scale.any())

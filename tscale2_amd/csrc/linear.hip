@@ -381,7 +381,8 @@ extern "C" int ts2_matmul_forward_norm_rope(int32_t mode, int32_t len, int32_t l
     const bool large = lenRound % 256 == 0 && dstDim % 256 == 0 && (int64_t)(lenRound / 256) * (dstDim / 256) >= 192;
     const bool few = (int64_t)(lenRound / 64) * (dstDim / 128) <= 768 && Aligned16(res->ptr, res->strideBytes) &&
                      (!ropeBuf || Aligned16(ropeBuf->ptr, ropeBuf->strideBytes));
-    if (large || few || mode == TS2_E4M3) {
+    // (an empty batch: the product's live length of 0 would mean all rows, the stand-alone pass clears them)
+    if (large || (len > 0 && (few || mode == TS2_E4M3))) {
         g.c = *res;
         g.cType = TS2_BF16;
         g.epilogue = TS2_EPI_ROW_TILE_NORM;
