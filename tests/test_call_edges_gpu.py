@@ -62,3 +62,28 @@ def test_normalised_forward_of_an_empty_batch_is_zero(mode):
     L.call("ts2_matmul_forward_norm_rope", mode, 0, rows, src, dst, x, w, 0.01, None, 1, 1 / 24, None, res, scale, raw)
     torch.cuda.synchronize()
     assert not bool(res.any()) and not bool(scale.any())
+
+
+def two_launches(mode, n, rows, src, dst, x, w, normalize, vec, rope, res, scale, raw):
+    L.call("ts2_matmul_forward", mode, n, rows, src, dst, x, w, 1.0, None, raw, L.F32, 0)
+    L.call("ts2_row_tile_normalize_rope", n, rows, raw, L.F32, 1.0, normalize, vec, rope, res, scale)
+
+
+@pytest.mark.parametrize("rows,dst", [(256, 256), (4096, 1664)])
+@pytest.mark.parametrize("offset,pitch", [(1, 128), (0, 129)])
+def test_rotation_tables_off_the_eight_byte_grid(rows, dst, offset, pitch):
+    """a table at any fp32 address and stride is taken by the product and the stand-alone pass where the fused store cannot read it"""
+    print("case rotation table alignment", rows, dst, offset, pitch, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    src, n = 128, rows - 5
+    x, w = [torch.randint(-1, 2, (r, src), device="cuda", generator=gen).float() for r in (rows, dst)]
+    x8, w8 = e4m3(x), e4m3(w)
+    flat = randn(gen, rows * pitch + offset)
+    rope = flat[offset:].view(rows, pitch)[:, :128]
+    new = lambda: (torch.zeros((rows, dst), dtype=torch.int16, device="cuda"), torch.zeros((dst // 128, rows), device="cuda"))  # noqa: E731
+    raw = torch.empty((rows, dst), device="cuda")
+    (got, gs), (want, ws) = new(), new()
+    two_launches(L.E4M3, n, rows, src, dst, x8, w8, 1, 1 / 24, rope, want, ws, raw)
+    L.call("ts2_matmul_forward_norm_rope", L.E4M3, n, rows, src, dst, x8, w8, 1.0, None, 1, 1 / 24, rope, got, gs, raw)
+    torch.cuda.synchronize()
+    assert torch.equal(gs, ws) and torch.equal(got, want)

@@ -381,8 +381,10 @@ extern "C" int ts2_matmul_forward_norm_rope(int32_t mode, int32_t len, int32_t l
     const bool large = lenRound % 256 == 0 && dstDim % 256 == 0 && (int64_t)(lenRound / 256) * (dstDim / 256) >= 192;
     const bool few = (int64_t)(lenRound / 64) * (dstDim / 128) <= 768 && Aligned16(res->ptr, res->strideBytes) &&
                      (!ropeBuf || Aligned16(ropeBuf->ptr, ropeBuf->strideBytes));
+    // the 128x128 tile reads the rotation table in pairs; the stand-alone pass takes it at any fp32 address and stride
+    const bool small = mode == TS2_E4M3 && (!ropeBuf || (((uintptr_t)ropeBuf->ptr | ropeBuf->strideBytes) & 7) == 0);
     // (an empty batch: the product's live length of 0 would mean all rows, the stand-alone pass clears them)
-    if (large || (len > 0 && (few || mode == TS2_E4M3))) {
+    if (large || (len > 0 && (few || small))) {
         g.c = *res;
         g.cType = TS2_BF16;
         g.epilogue = TS2_EPI_ROW_TILE_NORM;
