@@ -1,0 +1,40 @@
+"""What the step driver's accessors show at the edges: rows beyond the batch, gradient scratch by layer type, wide k-tiles."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+from model_harness import E4M3, I8, Harness  # noqa: E402
+from tscale2_amd import lib as L  # noqa: E402
+
+
+def test_gradient_scratch_of_a_mixture_of_experts_layer_is_its_own():
+    """"scratch.f0" / "scratch.f1" after the backward of a mixture-of-experts layer are its gradients of the expand and gate products, not
+    those of the attention layer before it: expert 0's rows come first (one tile of 128), and its packed deltas are sums of products with
+    exactly those rows, so they lie in the rows' span up to the packing (1/254 of a row-tile's largest value per element)."""
+    print("case gradient scratch of an expert layer", flush=True)
+    h = Harness(E4M3, dim=256, heads=2, ffn_tiles=2, depth=3, vocab=256, frag_count=2, frag_len=30, wide_window=64, experts=8, selected=2, xp=128,
+                seed=11, std=0.05)
+    att, moe = list(h.lt).index(0), list(h.lt).index(3)
+    m = h.device_model()
+    try:
+        m.backprop()
+        torch.cuda.synchronize()
+        G = m.array("stateGrad").clone()
+        for layer in (att, moe):
+            m.array("stateGrad").copy_(G)
+            m.array("gradMaxNorm")[0, 0] = G.abs().max()
+            m.layer_forward(layer)
+            m.layer_backward(layer)
+        torch.cuda.synchronize()
+        for i in (0, 1):
+            rows = m.array(f"scratch.f{i}", 128)[:128].contiguous().view(torch.float8_e4m3fn).double().cpu()
+            d = torch.from_numpy(m.get_delta(moe, i, 8 * 128, h.dim)[:128]).double()
+            assert 2 <= int(rows.any(1).sum()) <= 64 and bool(d.any())
+            _, s, basis = torch.linalg.svd(rows, full_matrices=False)
+            basis = basis[s > 1e-6 * s.max()]
+            left = d - basis.t() @ (basis @ d)
+            print("matrix", i, "rows", len(basis), "outside the span", float(left.norm() / d.norm()))
+            assert float(left.norm()) <= 0.03 * float(d.norm())
+    finally:
+        m.close()

@@ -414,6 +414,15 @@ int FfnForward(ts2_model *M, TLayer &L, const Arr &norm8, void *s)
     return Forward(M, L.w[2], View(L.acts->rg8, M->R, F), VEC * DISCR * Dot(F), true, M->state, true, s);
 }
 
+// where a layer's backward leaves its fast-type gradients (null: the layer has none in that slot)
+void SetLastFast(ts2_model *M, const Arr *f0, const Arr *f1, const Arr *f2, const Arr *f3)
+{
+    const Arr *const f[4] = {f0, f1, f2, f3};
+    for (int k = 0; k < 4; ++k) {
+        M->lastFast[k] = f[k] ? *f[k] : Arr();
+    }
+}
+
 int FfnBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScale, void *s)
 {
     int D = M->cfg.dim, F = M->cfg.ffnDim, len = M->len, R = M->R;
@@ -427,8 +436,7 @@ int FfnBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
         dwide = ColBlock(gStack, 0, F);
         dgate = ColBlock(gStack, 1, F);
     }
-    M->lastFast[0] = dwide;
-    M->lastFast[1] = dgate;
+    SetLastFast(M, &dwide, &dgate, nullptr, nullptr);
     if (!(M->useKept && A.valid)) {
         CK(FfnComputeRG(M, L, norm8, s));
     }
@@ -514,10 +522,7 @@ int AttBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
         dVf = ColBlock(gStack, 2, Q);
         dGate = ColBlock(gStack, 3, Q);
     }
-    M->lastFast[0] = dQf;
-    M->lastFast[1] = dGate;
-    M->lastFast[2] = dKf;
-    M->lastFast[3] = dVf;
+    SetLastFast(M, &dQf, &dGate, &dKf, &dVf);
     if (!(M->useKept && A.valid)) {
         CK(AttComputeVLG(M, L, norm8, s));
     }
@@ -695,6 +700,7 @@ int MoeBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
     Arr drg = View(M->g16[0], RM, X); // 16 bits like the reference's DRG and StateGradFull (layer_moe.cu:35,46)
     CK(GroupedGemm(M, M->sgMoe, wcT, X, X, D, drg, DISCR * Dot(E * X), L.w[2].scale, false, s));
     Arr dwide = View(M->gf[0], RM, X), dgate = View(M->gf[1], RM, X);
+    SetLastFast(M, &dwide, &dgate, nullptr, nullptr);
     CK(ts2_backprop_row_tile_normalize_lolu_moe(RM, M->moe.xpSampleWeight, gate16.P(), wide16.P(), VEC, wideScale.P(), drg.P(), TS2_BF16, 1.f,
         dgate.P(), dwide.P(), M->fastGradType, M->dExpertWeight, s));
     // dExpertWeight was computed against rg in 1/24 units of nothing: vals*valsScale is the true normalised wide, so it is in true
