@@ -38,3 +38,21 @@ def test_gradient_scratch_of_a_mixture_of_experts_layer_is_its_own():
             assert float(left.norm()) <= 0.03 * float(d.norm())
     finally:
         m.close()
+
+
+@pytest.mark.parametrize("mode", [I8, E4M3])
+def test_predictions_beyond_the_batch_are_probabilities_too(mode):
+    """the view has every row of the last row group: rows beyond the batch have logits zero, so they hold the soft-max of the bias"""
+    print("case predictions beyond the batch", mode, flush=True)
+    h = Harness(mode, dim=256, heads=2, ffn_tiles=2, depth=1, vocab=384, frag_count=1, frag_len=100, wide_window=64, seed=12, bias_std=1.0)
+    m = h.device_model()
+    try:
+        m.forward()
+        torch.cuda.synchronize()
+        p = m.array("prediction")[:, :h.vocab].double().cpu().numpy()
+    finally:
+        m.close()
+    assert p.shape[0] > h.n
+    assert np.abs(p.sum(1) - 1).max() <= 1e-5
+    want = np.exp2(h.bias.astype(np.float64))
+    assert np.abs(p[h.n:] - want / want.sum()).max() <= 1e-6
