@@ -135,8 +135,8 @@ typedef struct ts2_gemm_args {
      * and one pass over C instead of one read-modify-write of C per product: the gradient of a layer input that feeds several
      * matrices (Backprop of Q, K, V and gate in src/gpt/compute/layer_att.cu:236-260 adds four products into the same array).
      * 256x256-tile kernel (m, n multiples of 256), or one further product on the 128x128 tile (tileConfig 2, or with tileGroup: the
-     * expert-grouped dX of wide and gate, src/gpt/compute/layer_moe.cu:236-250, where every B_i takes the tile's slab); TS2_E4M3 or
-     * TS2_BF16 operands, fp32 or bf16 C, TS2_EPI_STORE or TS2_EPI_ADD, no rowScale, kTileScale, groupOffsets or splitK; the fp32 sums
+     * expert-grouped dX of wide and gate, src/gpt/compute/layer_moe.cu:236-250, where every B_i takes the tile's slab), or, asked for by
+     * bit 16 of tileConfig, the kernel for few tiles at any m, n, k it takes; TS2_E4M3 or TS2_BF16 operands, fp32 or bf16 C, TS2_EPI_STORE or TS2_EPI_ADD, no rowScale, kTileScale, groupOffsets or splitK; the fp32 sums
      * of the products are rescaled in registers between products. */
     int32_t extraSegments;
     struct {
@@ -342,8 +342,9 @@ int ts2_matmul_backprop(int32_t mode, int32_t len, int32_t lenRound, int32_t src
 /* Backprop() of `count` (2..4) matrices that share their input (Q, K, V and gate of an attention layer,
  * src/gpt/compute/layer_att.cu:236-260; wide and gate of an FFN layer, layer_ffn.cu): srcGrad (+)= sum_i alpha[i] * (*alphaPtr[i]) *
  * grad[i] * W_i, where the reference adds one product after the other into the same array.  Every bufs[i] must have been prepared by
- * ts2_matmul_backprop_multi for its matrix; all matrices are [gradDim][srcDim].  TS2_E4M3 with srcDim and lenRound multiples of 256
- * runs as one launch (one pass over srcGrad); otherwise the products are launched one after the other as the reference does. */
+ * ts2_matmul_backprop_multi for its matrix; all matrices are [gradDim][srcDim].  TS2_E4M3 with srcDim and lenRound multiples of 256,
+ * or with at most 640 tiles of 64 x 128, runs as one launch: one pass over srcGrad, the sum of all products rounded once to its type.
+ * Otherwise the products are launched one after the other as the reference does, with a rounding after each. */
 int ts2_matmul_backprop_group(int32_t mode, int32_t len, int32_t lenRound, int32_t srcDim, int32_t gradDim, int32_t count,
     const ts2_mat *const *grad, const ts2_matmul_bwd_buffers *const *bufs, const float *alpha, const float *const *alphaPtr,
     const ts2_mat *srcGrad, int32_t srcGradType, int32_t add, void *stream);

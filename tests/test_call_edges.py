@@ -41,3 +41,14 @@ def test_the_kernel_for_few_tiles_refuses_a_contraction_that_ends_inside_its_uni
     g = L.GemmArgs(a=L.mat(u8(128, 192)), b=L.mat(u8(128, 192)), c=L.mat(torch.zeros((128, 128))), abType=L.E4M3, cType=L.F32, m=128, n=128, k=192, alpha=1,
                    splitK=1, tileConfig=65536 | 2048)
     assert L.load().dll.ts2_gemm_nt(C.byref(g), None) == UNSUPPORTED
+
+
+@pytest.mark.parametrize("m,n,config", [(384, 256, 0), (256, 384, 0), (384, 384, 0), (384, 384, 2)])
+def test_several_products_off_the_256_grid_only_where_the_call_asks_for_the_kernel(m, n, config):
+    """two further products: the 256x256 kernel's call; other sizes run with bit 16 of tileConfig and are refused without it"""
+    a, b, c = u8(m, 128), u8(n, 128), torch.zeros((m, n))
+    g = L.GemmArgs(a=L.mat(a), b=L.mat(b), c=L.mat(c), abType=L.E4M3, cType=L.F32, m=m, n=n, k=128, alpha=1, splitK=1, tileConfig=config,
+                   extraSegments=2)
+    for i in range(2):
+        g.segment[i].a, g.segment[i].b, g.segment[i].alpha = a.data_ptr(), b.data_ptr(), 1
+    assert L.load().dll.ts2_gemm_nt(C.byref(g), None) == UNSUPPORTED

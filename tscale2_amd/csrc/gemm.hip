@@ -1241,14 +1241,12 @@ extern "C" int ts2_gemm_nt(const ts2_gemm_args *a, void *streamPtr)
     }
     p.nSeg = 1;
     p.rowsF16 = 0;
-    bool onlyFewTiles = false; // several products on a shape that only the kernel for few tiles takes
     if (a->extraSegments) {
         const bool bigTile = (a->m % 256) == 0 && (a->n % 256) == 0 && (a->tileConfig & 3) <= 1 && !(a->tileConfig & (4 | 8 | 16)) && !a->tileGroup;
         // the 128x128 tile (chosen with tileConfig 2, or implied by tileGroup) takes one further product
         const bool smallTile = a->extraSegments == 1 && ((a->tileConfig & 3) == 2 || a->tileGroup) && !(a->tileConfig & (4 | 8 | 16)) &&
             !a->splitSlabBytes;
-        const bool fewTiles = (a->tileConfig & 65536) || (!(a->tileConfig & (3 | 8 | 16 | 128 | 2048 | 4096 | 32768 | 131072)) && !a->tileGroup &&
-            (int64_t)(a->m / 64) * (a->n / 128) <= 640 && Aligned16(a->c.ptr, a->c.strideBytes));
+        const bool fewTiles = (a->tileConfig & 65536) != 0; // (asked for: sizes off the 256 grid too)
         if (a->extraSegments < 0 || a->extraSegments > 3 || !(bigTile || smallTile || fewTiles) || a->abType == TS2_I8 || a->rowScale || a->kTileScale ||
             a->groupOffsets || splitK > 1 || (a->cType != TS2_F32 && a->cType != TS2_BF16) ||
             (a->epilogue != TS2_EPI_STORE && a->epilogue != TS2_EPI_ADD)) {
@@ -1267,7 +1265,6 @@ extern "C" int ts2_gemm_nt(const ts2_gemm_args *a, void *streamPtr)
             p.segAlphaPtr[i] = a->segment[i].alphaPtr;
         }
         p.nSeg = 1 + a->extraSegments;
-        onlyFewTiles = !bigTile && !smallTile;
     }
     p.splits = 1;
     p.splitSlab = 0;
@@ -1321,9 +1318,6 @@ extern "C" int ts2_gemm_nt(const ts2_gemm_args *a, void *streamPtr)
             if (askSlice || SliceCanRun(sp, type, p.kMajor != 0)) {
                 return RunSlice(sp, type, p.kMajor != 0, stream);
             }
-        }
-        if (onlyFewTiles) {
-            return TS2_ERR_UNSUPPORTED;
         }
         if (a->tileConfig & 4096) {
             // bit 12: the persistent kernel whose epilogue runs under the next tile's main loop

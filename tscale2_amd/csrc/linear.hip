@@ -171,10 +171,10 @@ extern "C" int ts2_matmul_backprop_group(int32_t mode, int32_t len, int32_t lenR
             return TS2_ERR_NULL;
         }
     }
-    // one launch: the 256x256 tile, or the kernel for few tiles
+    // one launch: the 256x256 tile (or what the dispatcher puts in its place), off its grid the kernel for few tiles
+    const bool grid256 = (lenRound % 256) == 0 && (srcDim % 256) == 0;
     bool one = mode == TS2_E4M3 && count > 1 && (srcGradType == TS2_F32 || srcGradType == TS2_BF16) &&
-               (((lenRound % 256) == 0 && (srcDim % 256) == 0) ||
-                   ((int64_t)(lenRound / 64) * (srcDim / 128) <= 640 && Aligned16(srcGrad->ptr, srcGrad->strideBytes)));
+               (grid256 || (int64_t)(lenRound / 64) * (srcDim / 128) <= 640);
     for (int i = 1; i < count && one; ++i) {
         one = grad[i]->strideBytes == grad[0]->strideBytes && bufs[i]->transformT.strideBytes == bufs[0]->transformT.strideBytes;
     }
@@ -212,9 +212,10 @@ extern "C" int ts2_matmul_backprop_group(int32_t mode, int32_t len, int32_t lenR
         g.segment[i - 1].alpha = alpha[i];
         g.segment[i - 1].alphaPtr = alphaPtr ? alphaPtr[i] : nullptr;
     }
+    g.tileConfig = grid256 ? 0 : 65536;
     const int rc = ts2_gemm_nt(&g, stream);
-    // (strides beyond what the kernel for few tiles addresses: one product after the other)
-    return rc == TS2_ERR_UNSUPPORTED && ((lenRound % 256) || (srcDim % 256)) ? oneByOne() : rc;
+    // (rows of the result off 16 bytes, strides beyond what the kernel for few tiles addresses: one product after the other)
+    return rc == TS2_ERR_UNSUPPORTED && !grid256 ? oneByOne() : rc;
 }
 
 extern "C" int ts2_matmul_backprop_delta(int32_t mode, int32_t len, int32_t lenRound, int32_t srcDim, int32_t gradDim, const ts2_mat *src,
