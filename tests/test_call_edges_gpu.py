@@ -87,3 +87,28 @@ def test_rotation_tables_off_the_eight_byte_grid(rows, dst, offset, pitch):
     L.call("ts2_matmul_forward_norm_rope", L.E4M3, n, rows, src, dst, x8, w8, 1.0, None, 1, 1 / 24, rope, got, gs, raw)
     torch.cuda.synchronize()
     assert torch.equal(gs, ws) and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("mode", [L.E4M3, L.I8])
+@pytest.mark.parametrize("rows,src,dst", [(256, 384, 256), (1024, 128, 1152), (4096, 256, 1664), (8192, 256, 1024), (16384, 1024, 1152)])
+def test_normalised_store_rounds_like_the_stand_alone_pass(mode, rows, src, dst):
+    """below the large tile's range: sums of squares of small whole numbers are exact in any order, so what is left is one division, one
+    square root, one product and one reciprocal in fp32 - the fused store has to give the very bits of product + pass"""
+    print("case normalised store", mode, rows, src, dst, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(rows + dst)
+    n = rows - 3
+    x, w = [torch.randint(-1, 2, (r, src), device="cuda", generator=gen) for r in (rows, dst)]
+    x8, w8 = [e4m3(t.float()) if mode == L.E4M3 else t.to(torch.int8) for t in (x, w)]
+    new = lambda: (torch.zeros((rows, dst), dtype=torch.int16, device="cuda"), torch.zeros((dst // 128, rows), device="cuda"))  # noqa: E731
+    raw = torch.empty((rows, dst), device="cuda")
+    for table in (None, randn(gen, rows, 128), randn(gen, rows, 130)[:, :128]):  # (rows on 16 bytes, rows on 8)
+        (got, gs), (want, ws) = new(), new()
+        two_launches(mode, n, rows, src, dst, x8, w8, 1, 1 / 24, table, want, ws, raw)
+        L.call("ts2_matmul_forward_norm_rope", mode, n, rows, src, dst, x8, w8, 1.0, None, 1, 1 / 24, table, got, gs, raw)
+        torch.cuda.synchronize()
+        assert torch.equal(gs, ws)
+        if table is None:
+            assert torch.equal(got, want)
+        else:  # (the rotation may contract its products differently: one step of bf16)
+            a, b = got.view(torch.bfloat16).double(), want.view(torch.bfloat16).double()
+            assert bool(((a - b).abs() <= 2.0 ** -7 * b.abs() + 2.0 ** -20 * b.abs().max()).all())

@@ -606,8 +606,15 @@ __device__ __forceinline__ void NormRowValues(const GemmP &p, TAcc (&accRow)[WT]
         }
         float discr = 0;
         if (sum2 > 0) {
-            discr = __builtin_amdgcn_sqrtf(sum2 * (1.f / TILE)) * p.vecScale;
-            const float inv = __builtin_amdgcn_rcpf(discr);
+            float inv;
+            if (WT == 2 && !p.tileGroup) {
+                // the 128x128 tile stands in for the stand-alone pass, whose square root and division are correctly rounded
+                discr = sqrtf(sum2 / TILE) * p.vecScale;
+                inv = 1 / discr;
+            } else {
+                discr = __builtin_amdgcn_sqrtf(sum2 * (1.f / TILE)) * p.vecScale;
+                inv = __builtin_amdgcn_rcpf(discr);
+            }
 #pragma unroll
             for (int j = 0; j < WT; ++j) {
 #pragma unroll

@@ -382,7 +382,8 @@ extern "C" int ts2_matmul_forward_norm_rope(int32_t mode, int32_t len, int32_t l
     const bool large = lenRound % 256 == 0 && dstDim % 256 == 0 && (int64_t)(lenRound / 256) * (dstDim / 256) >= 192;
     const bool few = (int64_t)(lenRound / 64) * (dstDim / 128) <= 768 && Aligned16(res->ptr, res->strideBytes) &&
                      (!ropeBuf || Aligned16(ropeBuf->ptr, ropeBuf->strideBytes));
-    // the 128x128 tile reads the rotation table in pairs; the stand-alone pass takes it at any fp32 address and stride
+    // the 128x128 tile, whose normalising store rounds like the stand-alone pass (the large ones use the hardware's square root and
+    // reciprocal), reads the rotation table in pairs; the pass takes it at any fp32 address and stride
     const bool small = mode == TS2_E4M3 && (!ropeBuf || (((uintptr_t)ropeBuf->ptr | ropeBuf->strideBytes) & 7) == 0);
     // (an empty batch: the product's live length of 0 would mean all rows, the stand-alone pass clears them)
     if (large || (len > 0 && (few || small))) {
@@ -397,12 +398,14 @@ extern "C" int ts2_matmul_forward_norm_rope(int32_t mode, int32_t len, int32_t l
         if (normalize) {
             g.tileScale = *tileScale;
         }
+        g.tileConfig = large || few ? 0 : 2;
         const int rc = ts2_gemm_nt(&g, stream);
         // rows off 16 bytes and the like: a product and the stand-alone pass take them
         if (large || !raw || (rc != TS2_ERR_UNSUPPORTED && rc != TS2_ERR_ALIGN)) {
             return rc;
         }
         g.epilogue = TS2_EPI_STORE;
+        g.tileConfig = 0;
         g.normalize = 0;
         g.vecScale = 0;
         g.rope = {};
