@@ -52,3 +52,25 @@ def test_several_products_off_the_256_grid_only_where_the_call_asks_for_the_kern
     for i in range(2):
         g.segment[i].a, g.segment[i].b, g.segment[i].alpha = a.data_ptr(), b.data_ptr(), 1
     assert L.load().dll.ts2_gemm_nt(C.byref(g), None) == UNSUPPORTED
+
+
+@pytest.mark.parametrize("rows,src", [(384, 384), (512, 512)])
+@pytest.mark.parametrize("wrong", ["rows of a gradient", "columns of a gradient", "rows of a transposed matrix", "columns of a transposed matrix"])
+def test_grouped_input_gradient_checks_every_product(rows, src, wrong):
+    """the second product's operands count as much as the first's, at sizes that run as one launch"""
+    grad = 256
+    bufs, keep = zip(*[buffers(rows, src, grad) for _ in range(2)])
+    grads = [L.mat(u8(rows, grad)) for _ in range(2)]
+    if wrong == "rows of a gradient":
+        grads[1].y = rows - 128
+    elif wrong == "columns of a gradient":
+        grads[1].x = grad - 128
+    elif wrong == "rows of a transposed matrix":
+        bufs[1].transformT.y = src - 128
+    else:
+        bufs[1].transformT.x = grad - 128
+    out = torch.zeros((rows, src))
+    c = L.mat(out)
+    gp, bp = (C.POINTER(L.Mat) * 2)(*[C.pointer(g) for g in grads]), (C.POINTER(L.BwdBuffers) * 2)(*[C.pointer(b) for b in bufs])
+    alpha = (C.c_float * 2)(1, 1)
+    assert L.load().dll.ts2_matmul_backprop_group(L.E4M3, rows, rows, src, grad, 2, gp, bp, alpha, None, C.byref(c), L.F32, 0, None) == SHAPE

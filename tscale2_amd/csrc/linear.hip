@@ -171,6 +171,14 @@ extern "C" int ts2_matmul_backprop_group(int32_t mode, int32_t len, int32_t lenR
             return TS2_ERR_NULL;
         }
     }
+    if (mode == TS2_E4M3) { // (one launch checks the first product's operands only)
+        for (int i = 0; i < count; ++i) {
+            const ts2_mat &t = bufs[i]->transformT;
+            if (grad[i]->x < gradDim || grad[i]->y < lenRound || t.x < gradDim || t.y < srcDim) {
+                return TS2_ERR_SHAPE;
+            }
+        }
+    }
     // one launch: the 256x256 tile (or what the dispatcher puts in its place), off its grid the kernel for few tiles
     const bool grid256 = (lenRound % 256) == 0 && (srcDim % 256) == 0;
     bool one = mode == TS2_E4M3 && count > 1 && (srcGradType == TS2_F32 || srcGradType == TS2_BF16) &&
