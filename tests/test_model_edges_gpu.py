@@ -56,3 +56,22 @@ def test_predictions_beyond_the_batch_are_probabilities_too(mode):
     assert np.abs(p.sum(1) - 1).max() <= 1e-5
     want = np.exp2(h.bias.astype(np.float64))
     assert np.abs(p[h.n:] - want / want.sum()).max() <= 1e-6
+
+
+def test_k_tiles_too_wide_for_the_row_major_delta_product():
+    """int8, one k-tile of 32768 rows over two gradients of 4096 columns side by side: the product that reads them as they lie cannot
+    address a k-tile's rows, so the step takes the transposing sequence.  The batch fills a part of one k-tile either way: the same
+    scales, the same exact integer sums, so the same deltas as with k-tiles of 16384."""
+    print("case wide k-tiles", flush=True)
+    h = Harness(I8, dim=128, heads=1, ffn_tiles=32, depth=1, vocab=128, frag_count=2, frag_len=150, wide_window=64, seed=13)
+    out = []
+    for k_tile in (16384, 32768):
+        m = h.device_model(k_tile=k_tile)
+        try:
+            m.backprop()
+            torch.cuda.synchronize()
+            out.append([m.get_delta(d, i, *q.fast.shape) for d in range(h.depth) for i, q in enumerate(h.layers[d])])
+        finally:
+            m.close()
+    for a, b in zip(*out):
+        assert np.isfinite(a).all() and a.any() and np.array_equal(a, b)

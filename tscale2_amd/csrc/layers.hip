@@ -366,11 +366,15 @@ int BackpropDeltaI8(ts2_model *M, int count, TMatrix &stack, TMatrix *const *W, 
                 seed[i] = NextDither(M);
             }
             CK(Ts2QuantTileRows(count, M->len, M->R, M->kTile, g16, g8, ram, seed, nullptr, M->sTileScale, s));
-            return Ts2DeltaRows(TS2_I8, M->len, M->R, stack.srcDim, all, src8.P(), g.P(), M->sTileScale, M->kTile, width, alpha, gradScale, M->sPartial,
-                (int64_t)M->sPartialFloats, stack.delta.P(), stack.deltaTileScale.P(), s);
+            const int rc = Ts2DeltaRows(TS2_I8, M->len, M->R, stack.srcDim, all, src8.P(), g.P(), M->sTileScale, M->kTile, width, alpha, gradScale,
+                M->sPartial, (int64_t)M->sPartialFloats, stack.delta.P(), stack.deltaTileScale.P(), s);
+            if (rc != TS2_ERR_UNSUPPORTED) {
+                return rc;
+            }
         }
     }
-    // large results: the transposing quantiser and the large tiles, one matrix after the other
+    // large results, and k-tiles whose rows one workgroup cannot address: the transposing quantiser and the large tiles, one matrix after
+    // the other
     for (int i = 0; i < count; ++i) {
         ts2_matmul_bwd_buffers b = Scratch(M, M->R, W[i]->srcDim, W[i]->dstDim);
         b.srcTValid = i > 0;
