@@ -74,3 +74,11 @@ def test_grouped_input_gradient_checks_every_product(rows, src, wrong):
     gp, bp = (C.POINTER(L.Mat) * 2)(*[C.pointer(g) for g in grads]), (C.POINTER(L.BwdBuffers) * 2)(*[C.pointer(b) for b in bufs])
     alpha = (C.c_float * 2)(1, 1)
     assert L.load().dll.ts2_matmul_backprop_group(L.E4M3, rows, rows, src, grad, 2, gp, bp, alpha, None, C.byref(c), L.F32, 0, None) == SHAPE
+
+
+@pytest.mark.parametrize("columns", [0, 128])
+def test_packed_delta_wants_its_transposing_scratch_whichever_kernel_runs(columns):
+    """e4m3 pad rows that nobody vouches for: the caller provides gradT (and srcT), also where the product reads the operands as they lie"""
+    b, keep = buffers(256, 256, 384)
+    b.gradT = L.mat(keep["gradT"][:, :columns]) if columns else L.Mat(None, 0, 0, 0)
+    assert delta(200, 256, 256, 384, b) == SHAPE

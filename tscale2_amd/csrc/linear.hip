@@ -280,7 +280,10 @@ extern "C" int ts2_matmul_backprop_delta(int32_t mode, int32_t len, int32_t lenR
         // widths off the 256 grid, or pad rows that nobody vouches for: the kernel for few tiles, which stops at row len.  Beyond 512 of
         // its workgroups two transposes and the large tile are cheaper (measured line of the dispatcher)
         const int cuts = buf->partial.ptr && buf->splits > 1 ? buf->splits : 1;
-        if (!kMajor && !buf->gradTValid && cuts == 1 && (int64_t)(gradDim / 64) * (srcDim / 128) <= 512) {
+        // (the scratch of the transposing sequence is part of the call, whichever kernel runs)
+        const bool scratch = buf->gradT.ptr && buf->gradT.x >= lenRound && buf->gradT.y >= gradDim && buf->srcT.ptr && buf->srcT.x >= lenRound &&
+                             buf->srcT.y >= srcDim;
+        if (!kMajor && !buf->gradTValid && cuts == 1 && scratch && (int64_t)(gradDim / 64) * (srcDim / 128) <= 512) {
             rc = DeltaSlice(TS2_E4M3, len, lenRound, srcDim, gradDim, src, grad, nullptr, 0, 0, alpha, gradScale, 1, nullptr, delta, deltaTileScale, stream);
             if (rc != TS2_ERR_UNSUPPORTED) {
                 return rc;
