@@ -8,7 +8,7 @@ torch = pytest.importorskip("torch")
 from tscale2_amd import lib as L  # noqa: E402
 
 pytestmark = pytest.mark.skipif(torch.cuda.device_count() > 0, reason="refusals only: no launch may see these host arrays")
-SHAPE, UNSUPPORTED = -1, -3
+SHAPE, UNSUPPORTED, NULL = -1, -3, -4
 
 
 def u8(rows, cols):
@@ -82,3 +82,14 @@ def test_packed_delta_wants_its_transposing_scratch_whichever_kernel_runs(column
     b, keep = buffers(256, 256, 384)
     b.gradT = L.mat(keep["gradT"][:, :columns]) if columns else L.Mat(None, 0, 0, 0)
     assert delta(200, 256, 256, 384, b) == SHAPE
+
+
+@pytest.mark.parametrize("mode", [L.E4M3, L.I8])
+@pytest.mark.parametrize("rows,columns,code", [(0, 0, NULL), (128, 384, SHAPE), (256, 256, SHAPE)])
+def test_normalised_forward_wants_its_scratch_below_the_large_tile(mode, rows, columns, code):
+    """the fp32 scratch of product + pass belongs to the call, also where a fused store makes no use of it"""
+    x, w, res, scale = u8(256, 128), u8(384, 128), torch.zeros((256, 384), dtype=torch.int16), torch.zeros((3, 256))
+    raw = torch.zeros((rows, columns)) if rows else None
+    m = [L.mat(t) for t in (x, w, res, scale, raw)]
+    assert L.load().dll.ts2_matmul_forward_norm_rope(mode, 200, 256, 128, 384, C.byref(m[0]), C.byref(m[1]), C.c_float(1), None, 1, C.c_float(1), None,
+                                                     C.byref(m[2]), C.byref(m[3]), C.byref(m[4]) if rows else None, None) == code

@@ -396,8 +396,10 @@ extern "C" int ts2_matmul_forward_norm_rope(int32_t mode, int32_t len, int32_t l
     // the 128x128 tile, whose normalising store rounds like the stand-alone pass (the large ones use the hardware's square root and
     // reciprocal), reads the rotation table in pairs; the pass takes it at any fp32 address and stride
     const bool small = mode == TS2_E4M3 && (!ropeBuf || (((uintptr_t)ropeBuf->ptr | ropeBuf->strideBytes) & 7) == 0);
-    // (an empty batch: the product's live length of 0 would mean all rows, the stand-alone pass clears them)
-    if (large || (len > 0 && (few || small))) {
+    // (the scratch of the two-launch sequence is part of the call, whichever kernel runs; an empty batch: the product's live length of 0
+    // would mean all rows, the stand-alone pass clears them)
+    const bool scratch = raw && raw->ptr && raw->x >= dstDim && raw->y >= lenRound;
+    if (large || (len > 0 && scratch && (few || small))) {
         g.c = *res;
         g.cType = TS2_BF16;
         g.epilogue = TS2_EPI_ROW_TILE_NORM;
@@ -412,7 +414,7 @@ extern "C" int ts2_matmul_forward_norm_rope(int32_t mode, int32_t len, int32_t l
         g.tileConfig = large || few ? 0 : 2;
         const int rc = ts2_gemm_nt(&g, stream);
         // rows off 16 bytes and the like: a product and the stand-alone pass take them
-        if (large || !raw || (rc != TS2_ERR_UNSUPPORTED && rc != TS2_ERR_ALIGN)) {
+        if (large || (rc != TS2_ERR_UNSUPPORTED && rc != TS2_ERR_ALIGN)) {
             return rc;
         }
         g.epilogue = TS2_EPI_STORE;
