@@ -343,8 +343,9 @@ int ts2_matmul_backprop(int32_t mode, int32_t len, int32_t lenRound, int32_t src
  * src/gpt/compute/layer_att.cu:236-260; wide and gate of an FFN layer, layer_ffn.cu): srcGrad (+)= sum_i alpha[i] * (*alphaPtr[i]) *
  * grad[i] * W_i, where the reference adds one product after the other into the same array.  Every bufs[i] must have been prepared by
  * ts2_matmul_backprop_multi for its matrix; all matrices are [gradDim][srcDim].  TS2_E4M3 with srcDim and lenRound multiples of 256,
- * or with at most 640 tiles of 64 x 128, runs as one launch: one pass over srcGrad, the sum of all products rounded once to its type.
- * Otherwise the products are launched one after the other as the reference does, with a rounding after each. */
+ * or with few tiles of 64 x 128 (256; 512 for gradDim <= 2048; 640 for gradDim <= 1024, or 2048 with more than two products), runs as one
+ * launch: one pass over srcGrad, the sum of all products rounded once to its type.  Otherwise the products are launched one after the
+ * other as the reference does, with a rounding after each. */
 int ts2_matmul_backprop_group(int32_t mode, int32_t len, int32_t lenRound, int32_t srcDim, int32_t gradDim, int32_t count,
     const ts2_mat *const *grad, const ts2_matmul_bwd_buffers *const *bufs, const float *alpha, const float *const *alphaPtr,
     const ts2_mat *srcGrad, int32_t srcGradType, int32_t add, void *stream);

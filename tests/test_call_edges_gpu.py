@@ -90,7 +90,7 @@ def test_rotation_tables_off_the_eight_byte_grid(rows, dst, offset, pitch):
 
 
 @pytest.mark.parametrize("mode", [L.E4M3, L.I8])
-@pytest.mark.parametrize("rows,src,dst", [(256, 384, 256), (1024, 128, 1152), (4096, 256, 1664), (8192, 256, 1024), (16384, 1024, 1152)])
+@pytest.mark.parametrize("rows,src,dst", [(256, 384, 256), (1024, 128, 1152), (2048, 2048, 1536), (4096, 256, 1664), (8192, 256, 1024), (16384, 1024, 1152)])
 def test_normalised_store_rounds_like_the_stand_alone_pass(mode, rows, src, dst):
     """below the large tile's range: sums of squares of small whole numbers are exact in any order, so what is left is one division, one
     square root, one product and one reciprocal in fp32 - the fused store has to give the very bits of product + pass"""

@@ -1093,18 +1093,22 @@ template <int TYPE> int DispatchTile(const ts2_gemm_args *a, const GemmP &p, hip
     }
     return DispatchEpi<TYPE, 2, 2>(a, p, stream);
 }
-// Where the kernel for few tiles (gemm_slice.hip) takes over: by its workgroup count, 64 x 128 of C each, one per CU.  Measured in a graph of
-// 60 launches, 128x128 / 256x256 kernels -> slice kernel, us:
-//   packed delta        i8 512x256x512 10.8 -> 5.8, 2048x512x4096 24.5 -> 15.8; e4m3 512x256x512 10.3 -> 5.7, 2048x512x4096 18.9 -> 16.1,
-//                       1024x4096x4096 (512 workgroups) 27.7 -> 32.7
-//   contraction-major   e4m3 2048x512x4096 42.0 -> 16.0, 2048x2048x8192 75.0 -> 61.3, sliced four ways (256 large tiles) 40.8 -> 77.3
-//   several products    e4m3 4 x 512x256x256 28.5 -> 8.1, 4 x 4096x512x512 37.7 -> 12.8, 4 x 8192x1024x1024 55.6 -> 69.2
-//   i8 stored           512x256x256 6.7 -> 4.9, 2048x1024x1024 10.4 -> 8.6, 4096x512x2048 13.9 -> 11.4, 3072x1536x512 (576) 11.2 -> 16.4
-//                       one per CU and no more: 2048x1024x8192 (256) 47.4 -> 27.6, but 2816x768x2048 (264) 13.9 -> 19.7, x8192 47.9 -> 50.8
-//   e4m3 stored fp32    512x256x256 6.4 -> 4.9, 4096x512x512 8.2 -> 7.1, 512x256x1024 6.6 -> 7.0, 1024x1024x4096 13.8 -> 16.2; as bf16
-//                       (row-owning epilogue there) 512x256x256 4.5 -> 4.9, 4096x512x2048 9.4 -> 10.8
-//   e4m3 accumulating   512x256x256 7.8 -> 5.2, 4096x512x2048 14.3 -> 11.7, 16384x512x512 (1024) 17.5 -> 27.3
-//   bf16                4096x256x1024 13.4 -> 10.4, 4096x1024x1024 (512) 15.5 -> 21.6
+// Where the kernel for few tiles (gemm_slice.hip) takes over: by its workgroup count, 64 x 128 of C each, one per CU of the 256.  Up to one
+// round it wins everywhere; a second or third round pays only where the other kernels start slowly or need further launches.  Measured in a
+// graph of 40 launches, other kernels -> this one, us; K in bytes:
+//   one round          packed delta i8 512x256x512 10.8 -> 5.8, e4m3 4096x512x8192 40.1 -> 27.9; i8 stored 2048x1024x8192 47.4 -> 27.6;
+//                      e4m3 stored fp32 512x256x512 6.4 -> 4.9 but x1024 6.6 -> 7.0; as bf16 (row-owning epilogue there) 4.5 -> 4.9;
+//                      e4m3 accumulating 4096x512x2048 14.3 -> 11.7; bf16 4096x256x2048 13.4 -> 10.4
+//   contraction-major  two rounds: e4m3 3072x1024x1024 (384 workgroups) 18.4 -> 13.3, 2048x2048x8192 (512) 75.4 -> 58.1, bf16 2048x2048x8192
+//                      88.4 -> 54.5; three: e4m3 2560x2048x2048 (640) 27.9 -> 29.3, x8192 77.5 -> 86.8
+//   several products   e4m3, two, 256x256 tile -> this: 4096x1024x1024 (512) 28.1 -> 21.2, 2048x2048x8192 (512) 140 -> 98.8, 2560x2048x512
+//                      (640) 23.2 -> 22.4, x2048 45.6 -> 45.8, x8192 141 -> 146; four 83.6 -> 80.7 and 274 -> 281; 3584x2048x1024 (896) 29.7 -> 38.4
+//   normalised rows    i8 as product + pass -> this: 2048x2048x4096 (512) 35.8 -> 33.2, 3072x2048x1024 (768) 24.7 -> 21.9, x2048 29.2 -> 30.0.
+//                      Up to 768 here, where the alternative is to refuse; ts2_matmul_forward_norm_rope has the finer lines
+//   packed             K 512: e4m3 4096x1024 (512) 11.3 -> 10.8, 2560x2048 (640) 14.2 -> 15.6; K 1024 (512): i8 13.6 -> 13.5, e4m3 12.5 ->
+//                      13.4; K 2048 (512): i8 17.9 -> 18.5, e4m3 15.5 -> 18.6, bf16 17.6 -> 18.5.  With k-tile scales a wave pair multiplies
+//                      alone: 4096x512x512 (256) 11.5 -> 11.0, x2048 18.7 -> 12.7, 5120x512x512 (320) 11.5 -> 18.9, x2048 18.7 -> 22.0
+//   i8 stored          2816x768x2048 (264) 13.9 -> 19.7; e4m3 accumulating 16384x512x512 (1024) 17.5 -> 27.3; bf16 4096x1024x2048 (512) 15.5 -> 21.6
 bool PreferSlice(const GemmP &p, int type, int ct, int epi)
 {
     const long wgs = (long)(p.m / 64) * (p.n / 128) * (p.splits > 1 ? p.splits : 1) * (p.groupOffsets ? p.splitK_groups : 1);
@@ -1112,13 +1116,13 @@ bool PreferSlice(const GemmP &p, int type, int ct, int epi)
         return wgs <= 512;
     }
     if (p.nSeg > 1) {
-        return wgs <= 640;
+        return wgs <= (p.kBytes <= 2048 ? 640 : 512);
     }
     if (ct == C_BF16NORM && !p.tileGroup) {
-        return wgs <= 768; // (the alternative for this size is a product and a separate pass)
+        return wgs <= 768;
     }
     if (ct == C_I8PACK) {
-        return wgs <= (type == T_I8 ? 512 : 384);
+        return wgs <= 256 || (wgs <= 512 && p.kBytes <= 512 && !p.kTileScale);
     }
     if (type == T_I8) {
         return wgs <= 256;

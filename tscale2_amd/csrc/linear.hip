@@ -179,10 +179,13 @@ extern "C" int ts2_matmul_backprop_group(int32_t mode, int32_t len, int32_t lenR
             }
         }
     }
-    // one launch: the 256x256 tile (or what the dispatcher puts in its place), off its grid the kernel for few tiles
+    // one launch: the 256x256 tile (or what the dispatcher puts in its place), off its grid the kernel for few tiles while it beats one product
+    // after the other: one round of its workgroups always; two products of K = 2048 as two rounds 35.0 -> 31.8 us, as three 42.6 -> 45.8, of
+    // K = 1024 as three 32.2 -> 29.5; four of K = 2048 as three 93.1 -> 80.7, of K = 4096 135 -> 147; two of K = 4096 as two 46.0 -> 52.8
     const bool grid256 = (lenRound % 256) == 0 && (srcDim % 256) == 0;
-    bool one = mode == TS2_E4M3 && count > 1 && (srcGradType == TS2_F32 || srcGradType == TS2_BF16) &&
-               (grid256 || (int64_t)(lenRound / 64) * (srcDim / 128) <= 640);
+    const int64_t wgs = (int64_t)(lenRound / 64) * (srcDim / 128);
+    const bool few = wgs <= 256 || (wgs <= 512 && gradDim <= 2048) || (wgs <= 640 && gradDim <= (count > 2 ? 2048 : 1024));
+    bool one = mode == TS2_E4M3 && count > 1 && (srcGradType == TS2_F32 || srcGradType == TS2_BF16) && (grid256 || few);
     for (int i = 1; i < count && one; ++i) {
         one = grad[i]->strideBytes == grad[0]->strideBytes && bufs[i]->transformT.strideBytes == bufs[0]->transformT.strideBytes;
     }
@@ -277,13 +280,14 @@ extern "C" int ts2_matmul_backprop_delta(int32_t mode, int32_t len, int32_t lenR
         }
         // both operands as they lie in memory, [token][feature]: the kernel's LDS reads do the transposing
         kMajor = (len == lenRound || buf->padRowsZero) && (gradDim % 256) == 0 && (srcDim % 256) == 0 && grad->y >= lenRound && src->y >= lenRound;
-        // widths off the 256 grid, or pad rows that nobody vouches for: the kernel for few tiles, which stops at row len.  Beyond 512 of
-        // its workgroups two transposes and the large tile are cheaper (measured line of the dispatcher)
+        // widths off the 256 grid, or pad rows that nobody vouches for: the kernel for few tiles, which stops at row len, in place of two
+        // transposes and a product.  One round of its workgroups always; two up to 4096 rows (5120x512 over 2048 31.2 -> 20.0 us, 4096 38.1 ->
+        // 35.6, 8192 57.9 -> 63.1; 2048x2048 over 4096 39.9 -> 32.0, 8192 57.3 -> 58.1)
         const int cuts = buf->partial.ptr && buf->splits > 1 ? buf->splits : 1;
         // (the scratch of the transposing sequence is part of the call, whichever kernel runs)
         const bool scratch = buf->gradT.ptr && buf->gradT.x >= lenRound && buf->gradT.y >= gradDim && buf->srcT.ptr && buf->srcT.x >= lenRound &&
                              buf->srcT.y >= srcDim;
-        if (!kMajor && !buf->gradTValid && cuts == 1 && scratch && (int64_t)(gradDim / 64) * (srcDim / 128) <= 512) {
+        if (!kMajor && !buf->gradTValid && cuts == 1 && scratch && (int64_t)(gradDim / 64) * (srcDim / 128) <= (lenRound <= 4096 ? 512 : 256)) {
             rc = DeltaSlice(TS2_E4M3, len, lenRound, srcDim, gradDim, src, grad, nullptr, 0, 0, alpha, gradScale, 1, nullptr, delta, deltaTileScale, stream);
             if (rc != TS2_ERR_UNSUPPORTED) {
                 return rc;
@@ -389,10 +393,13 @@ extern "C" int ts2_matmul_forward_norm_rope(int32_t mode, int32_t len, int32_t l
     g.alpha = alpha;
     g.alphaPtr = alphaPtr;
     g.splitK = 1;
-    // the large tile from 192 tiles on; below, the kernel for few tiles (up to 768 of its workgroups) or, for fp8, the 128x128 tile
+    // the large tile from 192 tiles on; below, the kernel for few tiles or, for fp8 beyond one round of its workgroups, the 128x128 tile
+    // (4096x1024, K = 512 .. 4096: 12.5, 15.0, 20.7, 32.3 -> 9.6, 9.7, 13.0, 23.9 us).  int8 and bf16: as product + pass -> for few tiles 512
+    // workgroups at any K (K = 512 bytes 21.8 -> 12.7, 4096 35.8 -> 33.2), 768 up to K = 1024 bytes (24.7 -> 21.9; K = 2048 29.2 -> 30.0)
     const bool large = lenRound % 256 == 0 && dstDim % 256 == 0 && (int64_t)(lenRound / 256) * (dstDim / 256) >= 192;
-    const bool few = (int64_t)(lenRound / 64) * (dstDim / 128) <= 768 && Aligned16(res->ptr, res->strideBytes) &&
-                     (!ropeBuf || Aligned16(ropeBuf->ptr, ropeBuf->strideBytes));
+    const int64_t wgs = (int64_t)(lenRound / 64) * (dstDim / 128);
+    const bool few = wgs <= (mode == TS2_E4M3 ? 256 : (int64_t)srcDim * (mode == TS2_BF16 ? 2 : 1) <= 1024 ? 768 : 512) &&
+                     Aligned16(res->ptr, res->strideBytes) && (!ropeBuf || Aligned16(ropeBuf->ptr, ropeBuf->strideBytes));
     // the 128x128 tile, whose normalising store rounds like the stand-alone pass (the large ones use the hardware's square root and
     // reciprocal), reads the rotation table in pairs; the pass takes it at any fp32 address and stride
     const bool small = mode == TS2_E4M3 && (!ropeBuf || (((uintptr_t)ropeBuf->ptr | ropeBuf->strideBytes) & 7) == 0);
