@@ -1,5 +1,5 @@
 """The kernel for products with few output tiles (ts2_gemm_args.tileConfig bit 16) against fp64 products of the same 8-bit / bf16 values:
-every operand type and layout, contractions of one, an odd and an even number of its half steps and more than its pipeline holds, every
+every operand type and layout (int8 with k-tile scales and int8 sums: test_grouped_products_gpu.py), contractions of one, an odd and an even number of its half steps and more than its pipeline holds, every
 result type.  Bounds: i8 sums are exact (one rounding to fp32 is left); fp32 sums of bf16 products in any order stay within K * 2^-24 of
 sum |a b|; the e4m3 instruction adds its 64 products with fewer bits than an fp32 sum has (1.5e-5 rms of the result on every kernel
 here), and its products are held to 2e-4 of the largest result like in the tests of the other kernels; a bf16 result adds half a unit in

@@ -1,5 +1,7 @@
 """The step driver over batches of several lengths: what a batch leaves in the model's arrays must not reach the next one, and the products
 chosen for a long batch must give what those chosen for a short one give."""
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 
@@ -46,7 +48,8 @@ def results(m, h, n):
 @pytest.mark.parametrize("mode,dim,experts", [(I8, 256, 0), (E4M3, 256, 0), (E4M3, 384, 0), (E4M3, 256, 8)])
 @pytest.mark.parametrize("n", [1, 129, 777])
 def test_a_short_batch_after_a_long_one_equals_the_same_batch_alone(mode, dim, experts, n):
-    """the delta products read gradients and states up to the end of the last row group: what a longer batch left there must be gone"""
+    """rows beyond the batch, of what a longer batch left in the model's arrays: int8 delta products read them up to the end of the last row
+    group, at these sizes e4m3 ones stop at the last live row (the large tile does not: next test)"""
     print("case short batch after a long one", mode, dim, experts, n, flush=True)
     h = Harness(mode, dim=dim, heads=2, ffn_tiles=4, depth=2, vocab=256, frag_count=2, frag_len=64, wide_window=64, seed=3, experts=experts)
     r = np.random.default_rng(5)
@@ -65,6 +68,67 @@ def test_a_short_batch_after_a_long_one_equals_the_same_batch_alone(mode, dim, e
             m.close()
     for a, b in zip(*out):
         assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
+class Weights:
+    """e4m3 weights drawn on the device: models whose oracle copy would take minutes"""
+
+    def __init__(self, dim, heads, ffn, vocab, seed):
+        self.mode, self.dim, self.heads, self.ffn, self.vocab, self.label_count = E4M3, dim, heads, ffn, vocab, vocab + 1
+        self.experts = 0
+        self.lt, self.la, self.ls, self.att_width = L.model_schedule(1, 0, 64)
+        self.depth = len(self.lt)
+        gen = torch.Generator(device="cuda").manual_seed(seed)
+
+        def matrix(rows, cols):
+            return SimpleNamespace(fast=(torch.randn((rows, cols), device="cuda", generator=gen) * 32).to(torch.float8_e4m3fn).view(torch.uint8).cpu().numpy(),
+                                   scale=0.02)
+        self.layers = [[matrix(r, c) for r, c in L.layer_shapes(int(t), dim, heads, ffn)] for t in self.lt]
+        self.embed, self.final = matrix(self.label_count, dim), matrix(vocab, dim)
+        self.bias = np.zeros(vocab, np.float32)
+
+
+def reads_rows_beyond(m, layer, n, shape):
+    """whether the delta of a layer's first matrix changes when its source holds NaN beyond the batch: the 256x256 tile contracts over the
+    whole row group (its gradients are zero there, NaN times zero is not), the kernel for few tiles stops at the last live row"""
+    grad = torch.randn(tuple(m.array("stateGrad").shape), device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    m.layer_forward(layer)
+    out = []
+    for poison in (False, True):
+        m.array("stateGrad").copy_(grad)
+        m.array("gradMaxNorm")[0, 0] = grad.abs().max()
+        if poison:
+            m.array("normState", layer)[n:].fill_(0x7f)
+        m.layer_backward(layer)
+        out.append(m.get_delta(layer, 0, *shape))
+    return not np.array_equal(*out)
+
+
+@pytest.mark.parametrize("dim,heads,ffn,rows,n", [(1024, 8, 2048, 16384, 12001), (2048, 16, 4096, 4096, 2777)])
+def test_a_short_batch_after_a_long_one_where_the_large_tile_reads_whole_row_groups(dim, heads, ffn, rows, n):
+    """e4m3 widths on the 256 grid and results large enough for the 256x256 tile, in stored slices that are packed (dim 1024) and whole (dim
+    2048): its delta products read the rows beyond the batch, so what a longer batch left there must be gone"""
+    print("case large tile after a long batch", dim, rows, n, flush=True)
+    h = Weights(dim, heads, ffn, 512, 21)
+    r = np.random.default_rng(22)
+    long, short = r.integers(0, h.vocab, rows), r.integers(0, h.vocab, n)
+    out, beyond = [], []
+    for first in (long, None):
+        m = load(h, rows)
+        try:
+            if first is not None:
+                batch(m, h, first, 512)
+                m.backprop()
+            k = batch(m, h, short, 512)
+            m.backprop()
+            out.append(results(m, h, k))
+            if first is None:
+                beyond = [reads_rows_beyond(m, d, n, h.layers[d][0].fast.shape) for d in range(h.depth)]
+        finally:
+            m.close()
+    for a, b in zip(*out):
+        assert np.isfinite(a).all() and a.any() and np.array_equal(a, b)
+    assert all(beyond), beyond  # (else these sizes no longer test what they are here for)
 
 
 @pytest.mark.parametrize("mode,dim", [(I8, 384), (E4M3, 384)])
