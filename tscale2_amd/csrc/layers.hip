@@ -135,7 +135,9 @@ struct ts2_model {
     bool keep = false;      // FFN and attention layers own activation sets
     bool useKept = false;   // inside ModelBackprop: the backward of a layer starts from what its forward left
     int sharedOwner = -1;   // the MoE layer whose forward filled the shared set, its gathered input and the routing tables last
-    Arr gf[4];                               // fast-gradient type [R'][maxW]: dwide/dq, dgate, dk, dv
+    // fast-gradient type [R'][maxW]: dwide/dq, dgate, dk, dv of int8 layers, dwide and dgate of MoE layers.  fp8 layers write theirs side by
+    // side into sGradT, which the slots that no layer writes name
+    Arr gf[4];
     Arr g16[4];                              // bf16 [R'][maxW]: -, dVal, dK, dV
     Arr dScale;                              // fp32 [heads][R]
     // MoE
@@ -1086,8 +1088,10 @@ extern "C" ts2_model *ts2_model_create(const ts2_model_config *cfg)
     int RP = M->RP;
     ok &= M->Alloc(&M->raw, RP, maxW, TS2_F32) && M->Alloc(&M->shared.rg8, RP, maxW, M->mode);
     for (int k = 0; k < 4; ++k) {
-        ok &= M->Alloc(&M->shared.a16[k], RP, maxW, TS2_BF16) && M->Alloc(&M->g16[k], RP, maxW, TS2_BF16) &&
-              M->Alloc(&M->gf[k], RP, maxW, M->fastGradType);
+        ok &= M->Alloc(&M->shared.a16[k], RP, maxW, TS2_BF16) && M->Alloc(&M->g16[k], RP, maxW, TS2_BF16);
+        if (M->mode == TS2_I8 || (hasMoe && k < 2)) {
+            ok &= M->Alloc(&M->gf[k], RP, maxW, M->fastGradType);
+        }
     }
     for (int k = 0; k < 2; ++k) {
         ok &= M->Alloc(&M->shared.tsc[k], maxW / 128, RP, TS2_F32);
@@ -1138,7 +1142,12 @@ extern "C" ts2_model *ts2_model_create(const ts2_model_config *cfg)
     }
     M->sGrad8 = (uint8_t *)M->Dev(M->mode == TS2_I8 ? (size_t)RP * M->stackW : 16);
     M->sGradT = (uint8_t *)M->Dev((size_t)RP * M->stackW);
-    M->sSrcT = (uint8_t *)M->Dev((size_t)RP * maxW);
+    for (int k = 0; k < 4; ++k) {
+        if (!M->gf[k].m.ptr) {
+            M->gf[k] = Flat(M->sGradT, RP, maxW, M->fastGradType);
+        }
+    }
+    M->sSrcT = (uint8_t *)M->Dev(M->mode == TS2_I8 ? (size_t)RP * maxW : 16);
     M->sWT = (uint8_t *)M->Dev((size_t)4 * maxW * maxW); // up to four transposed weights side by side (BackpropDXGroup)
     M->sPartialFloats = (size_t)8 * 2048 * 2048; // eight slices of a 2048 x 2048 delta, four of a 4096 x 2048 one
     M->sPartial = (float *)M->Dev(M->sPartialFloats * 4);
