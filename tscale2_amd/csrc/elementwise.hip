@@ -54,13 +54,12 @@ inline dim3 GridFor(int rows, int tiles)
 }
 
 // non-negative float max through the integer ordering, like the reference's atomicMax((int*)p, __float_as_int(x))
-// A read-modify-write of one address costs 10 ns whoever issues it (one per workgroup: 41 of 58 us on 16384 x 512); a maximum that is not
-// above the value already there changes nothing, and almost all of them are not.
+// Nothing waits for it.  (Looking first whether the value there is lower already saves most of the updates, 10 ns each on one address, but the
+// answer takes microseconds while the address is contended and holds the workgroup's place that long: maxima of the k-tiles of 16384 x 4096
+// 76.3 us with the look, 30.5 without, normalisation backward of 16384 x 1024 e4m3 48.3 / 44.2, of 32768 x 2048 185.4 / 177.8.)
 __device__ __forceinline__ void AtomicMaxPos(float *p, float v)
 {
-    if (__float_as_int(v) > __hip_atomic_load((int *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-        atomicMax((int *)p, __float_as_int(v));
-    }
+    atomicMax((int *)p, __float_as_int(v));
 }
 
 // lanes 0..U-1 of the group store the U per-row scalars of one tile column (16 contiguous bytes)
