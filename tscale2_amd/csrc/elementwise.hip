@@ -1305,16 +1305,17 @@ __global__ void __launch_bounds__(256) RowTileNormalizeRope(int len, int lenRoun
     }
 }
 
-// blockIdx.y = job: the gradients of Q, K and V go in one launch (4096 x 512, e4m3: 3 x 4.4 -> 7.7 us; 16384 x 384, bf16: 3 x 9.8 -> 24.3)
-struct NormRopeJobs {
-    Mat grad[4], srcNorm[4], srcTileScale[4], rope[4], dst[4];
+// blockIdx.y = job: the gradients of Q, K and V go in one launch (4096 x 512, e4m3: 3 x 4.4 -> 7.7 us; 16384 x 384, bf16: 3 x 9.8 -> 24.3).
+// N = 1: one gradient, its description in scalar registers from the start (16384 x 512, bf16: 15.1 us, 15.4 through the table)
+template <int N> struct NormRopeJobs {
+    Mat grad[N], srcNorm[N], srcTileScale[N], rope[N], dst[N];
 };
 
-template <class TGrad, class TDst>
-__global__ void __launch_bounds__(256) BackpropRowTileNormalizeRope(int len, int lenRound, int tiles, float gradMult, NormRopeJobs jobs)
+template <class TGrad, class TDst, int N>
+__global__ void __launch_bounds__(256) BackpropRowTileNormalizeRope(int len, int lenRound, int tiles, float gradMult, NormRopeJobs<N> jobs)
 {
-    const Mat grad = jobs.grad[blockIdx.y], srcNorm = jobs.srcNorm[blockIdx.y], srcTileScale = jobs.srcTileScale[blockIdx.y],
-              rope = jobs.rope[blockIdx.y], dst = jobs.dst[blockIdx.y];
+    const int j = N == 1 ? 0 : blockIdx.y;
+    const Mat grad = jobs.grad[j], srcNorm = jobs.srcNorm[j], srcTileScale = jobs.srcTileScale[j], rope = jobs.rope[j], dst = jobs.dst[j];
     int t0, tile, h;
     if (!Unit(lenRound, tiles, &t0, &tile, &h)) {
         return;
@@ -1352,10 +1353,11 @@ __global__ void __launch_bounds__(256) BackpropRowTileNormalizeRope(int len, int
 
 // bf16 gradient -> e4m3 with eight elements per lane (a tile = 16 lanes, the tile sums are four DPP steps, the rotated pairs sit in
 // one lane): the form the model's attention backward uses.  Same arithmetic per element as BackpropRowTileNormalizeRope.
-__global__ void __launch_bounds__(256) BackpropRowTileNormalizeRope8(int len, int lenRound, int tiles, float gradMult, NormRopeJobs jobs)
+template <int N>
+__global__ void __launch_bounds__(256) BackpropRowTileNormalizeRope8(int len, int lenRound, int tiles, float gradMult, NormRopeJobs<N> jobs)
 {
-    const Mat grad = jobs.grad[blockIdx.y], srcNorm = jobs.srcNorm[blockIdx.y], srcTileScale = jobs.srcTileScale[blockIdx.y],
-              rope = jobs.rope[blockIdx.y], dst = jobs.dst[blockIdx.y];
+    const int j = N == 1 ? 0 : blockIdx.y;
+    const Mat grad = jobs.grad[j], srcNorm = jobs.srcNorm[j], srcTileScale = jobs.srcTileScale[j], rope = jobs.rope[j], dst = jobs.dst[j];
     constexpr int UU = 2;
     const int l16 = threadIdx.x & 15;
     const long unit0 = ((long)blockIdx.x * 256 + threadIdx.x) >> 4;
@@ -2052,7 +2054,7 @@ int Ts2BackpropNormRopeGroup(int count, int len, int lenRound, const ts2_mat *co
     if (count < 1 || count > 4) {
         return TS2_ERR_SHAPE;
     }
-    NormRopeJobs jobs = {};
+    NormRopeJobs<4> jobs = {};
     bool wide = gradType == TS2_BF16 && dstType == TS2_E4M3; // eight elements per lane
     for (int i = 0; i < count; ++i) {
         if (!grad[i] || !dst[i] || (srcNorm[i] && !srcTileScale[i])) {
@@ -2080,16 +2082,24 @@ int Ts2BackpropNormRopeGroup(int count, int len, int lenRound, const ts2_mat *co
     if (gradType != TS2_F32 && gradType != TS2_BF16) {
         return TS2_ERR_UNSUPPORTED;
     }
+    const NormRopeJobs<1> one = {{jobs.grad[0]}, {jobs.srcNorm[0]}, {jobs.srcTileScale[0]}, {jobs.rope[0]}, {jobs.dst[0]}};
     if (wide) {
         const long lanes = ((long)lenRound * tiles * 16 + 1) / 2;
-        hipLaunchKernelGGL(BackpropRowTileNormalizeRope8, dim3((unsigned)((lanes + 255) / 256), count), dim3(256), 0, STREAM, len, lenRound, tiles,
-            gradMult, jobs);
+        const dim3 grid((unsigned)((lanes + 255) / 256), count);
+        if (count == 1) {
+            hipLaunchKernelGGL(BackpropRowTileNormalizeRope8<1>, grid, dim3(256), 0, STREAM, len, lenRound, tiles, gradMult, one);
+        } else {
+            hipLaunchKernelGGL(BackpropRowTileNormalizeRope8<4>, grid, dim3(256), 0, STREAM, len, lenRound, tiles, gradMult, jobs);
+        }
         TS2_CHECK_LAUNCH();
         return TS2_OK;
     }
+    const dim3 grid(GridFor(lenRound, tiles).x, count);
 #define LAUNCH_BR(TG, TD)                                                                                                                  \
-    hipLaunchKernelGGL((BackpropRowTileNormalizeRope<TG, TD>), dim3(GridFor(lenRound, tiles).x, count), dim3(256), 0, STREAM, len, lenRound, tiles, \
-        gradMult, jobs)
+    if (count == 1)                                                                                                                        \
+        hipLaunchKernelGGL((BackpropRowTileNormalizeRope<TG, TD, 1>), grid, dim3(256), 0, STREAM, len, lenRound, tiles, gradMult, one);     \
+    else                                                                                                                                   \
+        hipLaunchKernelGGL((BackpropRowTileNormalizeRope<TG, TD, 4>), grid, dim3(256), 0, STREAM, len, lenRound, tiles, gradMult, jobs)
     if (gradType == TS2_F32) {
         TS2_DISPATCH_TYPE(dstType, TD, LAUNCH_BR(TF32, TD));
     } else {
