@@ -1108,6 +1108,9 @@ template <int TYPE> int DispatchTile(const ts2_gemm_args *a, const GemmP &p, hip
 //   packed             K 512: e4m3 4096x1024 (512) 11.3 -> 10.8, 2560x2048 (640) 14.2 -> 15.6; K 1024 (512): i8 13.6 -> 13.5, e4m3 12.5 ->
 //                      13.4; K 2048 (512): i8 17.9 -> 18.5, e4m3 15.5 -> 18.6, bf16 17.6 -> 18.5.  With k-tile scales a wave pair multiplies
 //                      alone: 4096x512x512 (256) 11.5 -> 11.0, x2048 18.7 -> 12.7, 5120x512x512 (320) 11.5 -> 18.9, x2048 18.7 -> 22.0
+//   short contraction  i8 1024x1024, as bf16 x128 4.7 -> 5.6, x512 5.5 -> 5.6; raw int32 x256 4.7 -> 5.6, x512 5.6 -> 6.3 (fp32 and accumulating
+//                      ones win at every K: this kernel's stores are whole rows); one or two k-tiles with scales leave wave pairs idle:
+//                      fp32 2048x1024, k-tiles of 512, one 9.1 -> 11.4, two 11.5 -> 11.9, three 13.6 -> 12.4, four 15.9 -> 13.5
 //   i8 stored          2816x768x2048 (264) 13.9 -> 19.7; e4m3 accumulating 16384x512x512 (1024) 17.5 -> 27.3; bf16 4096x1024x2048 (512) 15.5 -> 21.6
 bool PreferSlice(const GemmP &p, int type, int ct, int epi)
 {
@@ -1125,7 +1128,9 @@ bool PreferSlice(const GemmP &p, int type, int ct, int epi)
         return wgs <= 256 || (wgs <= 512 && p.kBytes <= 512 && !p.kTileScale);
     }
     if (type == T_I8) {
-        return wgs <= 256;
+        const int slice = p.splits > 1 ? (p.kBytes + p.splits - 1) / p.splits : p.kBytes;
+        return wgs <= 256 && (!p.kTileScale || slice > 2 * p.kTileBytes) &&
+               (ct == C_F32 || epi == TS2_EPI_ADD || p.kBytes > (ct == C_F16 ? 128 : ct == C_BF16 ? 512 : 1536));
     }
     return wgs <= 256 && (type == T_BF16 || epi == TS2_EPI_ADD || (ct == C_F32 && p.kBytes <= 512));
 }
