@@ -1533,10 +1533,11 @@ static int BackpropNormImpl(bool final, int len, int rows, const ts2_mat *normSt
     }
     int tiles = dim / TILE;
     // One update of the maximum per workgroup, 10 ns each on its one address: 1024 threads each, two workgroups per CU, once there are more than
-    // 256 workgroups of 256 and until many times as much work outweighs the queue and small workgroups share the memory better.  This pass and
-    // the final one, workgroups of 256 -> of 1024, us: e4m3 4096 x 512 15.7, 15.7 -> 7.5, 7.1; 16384 x 1024 103, 101 -> 44.2, 33.4; 16384 x 2048
-    // 117, 107 -> 92.4, 68.8; int8 4096 x 1024 51.4, 50.8 -> 13.2, 11.2; 16384 x 2048 104, 92.2 -> 102, 79.7.  65536 x 1024 e4m3, both together,
-    // 305 -> 350.  The widest int8 passes, 2048 -> 4096 workgroups, 32768 x 2048: 197, 169 -> 202, 154
+    // 100 (e4m3) or 256 workgroups of 256 and until many times as much work outweighs the queue and small workgroups share the memory better.
+    // This pass and the final one, workgroups of 256 -> of 1024, us: e4m3 200 x 1024 3.5, 3.3 -> 3.6, 3.3; 500 x 512 3.8, 3.5 -> 3.6, 3.3;
+    // 1024 x 512 5.4, 5.3 -> 4.1, 3.7; 4096 x 512 15.7, 15.7 -> 7.5, 7.1; 16384 x 1024 103, 101 -> 44.2, 33.4; 16384 x 2048 117, 107 -> 92.4,
+    // 68.8; 65536 x 1024, both together, 305 -> 350; int8 1024 x 512 5.7, 5.4 -> 6.2, 5.8; 4096 x 1024 51.4, 50.8 -> 13.2, 11.2; 16384 x 2048
+    // 104, 92.2 -> 102, 79.7.  The widest int8 passes, 2048 -> 4096 workgroups, 32768 x 2048: 197, 169 -> 202, 154
     const long units4 = (long)((rows + U - 1) / U) * tiles, units1 = (long)rows * tiles;
     auto grid = [](long units, int perBlock, int most) { const long n = (units + perBlock - 1) / perBlock; return dim3((unsigned)(n < most ? n : most)); };
     if (normType == TS2_E4M3 && fastType == TS2_E4M3 && (((uintptr_t)normState->ptr | normState->strideBytes | (uintptr_t)stateGradFast->ptr |
@@ -1545,7 +1546,7 @@ static int BackpropNormImpl(bool final, int len, int rows, const ts2_mat *normSt
 #define LAUNCH_BN8(FINAL, NT)                                                                                                              \
     hipLaunchKernelGGL((BackpropLayerNormalize8<FINAL, NT>), grid(units1, NT / 16, NT == 256 ? 8192 : 512), dim3(NT), 0, STREAM, len, rows, tiles, M(*normState), \
         M(*stateScale), M(*dNormState), combinerScale, gradScale, gradMult, M(*stateGrad), M(*stateGradFast), nextMaxNorm)
-        const bool many = units1 > 4096 && units1 <= 262144;
+        const bool many = units1 > 1600 && units1 <= 262144;
         if (final) {
             if (many) {
                 LAUNCH_BN8(true, 1024);
