@@ -395,10 +395,11 @@ extern "C" int ts2_matmul_forward_norm_rope(int32_t mode, int32_t len, int32_t l
     g.splitK = 1;
     // the large tile from 192 tiles on; below, the kernel for few tiles or, for fp8 beyond one round of its workgroups, the 128x128 tile
     // (4096x1024, K = 512 .. 4096: 12.5, 15.0, 20.7, 32.3 -> 9.6, 9.7, 13.0, 23.9 us).  int8 and bf16: as product + pass -> for few tiles 512
-    // workgroups at any K (K = 512 bytes 21.8 -> 12.7, 4096 35.8 -> 33.2), 768 up to K = 1024 bytes (24.7 -> 21.9; K = 2048 29.2 -> 30.0)
+    // workgroups at any K (K = 512 bytes 21.8 -> 12.7, 4096 35.8 -> 33.2), 768 up to K = 1536 bytes (K = 1024 24.7 -> 21.9;
+    // K = 2048 29.2 -> 30.0; an int8 attention and feed-forward pair of 1536 x 3072 over 2000 tokens, whole step 835 -> 826)
     const bool large = lenRound % 256 == 0 && dstDim % 256 == 0 && (int64_t)(lenRound / 256) * (dstDim / 256) >= 192;
     const int64_t wgs = (int64_t)(lenRound / 64) * (dstDim / 128);
-    const bool few = wgs <= (mode == TS2_E4M3 ? 256 : (int64_t)srcDim * (mode == TS2_BF16 ? 2 : 1) <= 1024 ? 768 : 512) &&
+    const bool few = wgs <= (mode == TS2_E4M3 ? 256 : (int64_t)srcDim * (mode == TS2_BF16 ? 2 : 1) <= 1536 ? 768 : 512) &&
                      Aligned16(res->ptr, res->strideBytes) && (!ropeBuf || Aligned16(ropeBuf->ptr, ropeBuf->strideBytes));
     // the 128x128 tile, whose normalising store rounds like the stand-alone pass (the large ones use the hardware's square root and
     // reciprocal), reads the rotation table in pairs; the pass takes it at any fp32 address and stride
