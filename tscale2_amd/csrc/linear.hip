@@ -635,7 +635,7 @@ int Ts2BackpropGroupI8(int count, int len, int lenRound, int srcDim, int gradDim
 }
 
 // While one product alone fits the chip (256 workgroups, one per CU), a launch is a chain of latencies and four of them cost four.  Whole passes,
-// separate -> one launch: 512-token int8 step 1133 -> 1016 us, 777-token prompt 1007 -> 853 (softmax of the live rows included), 3885-token
+// separate -> one launch: 512-token int8 step 1133 -> 1016 us, 777-token prompt 1007 -> 874, 3885-token
 // 8-expert step 1632 -> 1538.  Beyond, the large-tile kernels are as good one by one
 int Ts2ForwardGroup(int mode, int count, int len, int lenRound, int srcDim, int dstDim, const ts2_mat *src, const ts2_mat *const *w, float alpha,
     const float *const *alphaPtr, int normalizeBits, float vecScale, int rotateBits, const ts2_mat *rope, const ts2_mat *res,
