@@ -199,7 +199,8 @@ int ts2_backprop_row_tile_normalize_lolu(int32_t len, int32_t lenRound, const ts
 /* The same for TS2_BF16 gradients and TS2_E4M3 results, leaving also the transposed copies gradGateT, gradValsT [dim][lenRound] that
  * the delta products of the two matrices contract over (the reference's producers can save a transposed copy the same way: saveTransposed
  * of ComputeRG, src/gpt/compute/layer_moe.cu:117, and the transposing MoeGroupSamples, moe_kernels.cuh:89-143).  BackpropDelta is then
- * called with gradT pointing at the copy and gradTValid set.  lenRound must be a multiple of 128. */
+ * called with gradT pointing at the copy and gradTValid set (the step driver's deltas read the gradients as they lie and need no copy).
+ * lenRound must be a multiple of 128. */
 int ts2_backprop_row_tile_normalize_lolu_t(int32_t len, int32_t lenRound, const ts2_mat *gate, const ts2_mat *vals, float valsScale,
     const ts2_mat *valsSrcTileScale, const ts2_mat *grad, const ts2_mat *gradGate, const ts2_mat *gradVals, const ts2_mat *gradGateT,
     const ts2_mat *gradValsT, void *stream);

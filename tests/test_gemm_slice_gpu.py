@@ -1,6 +1,6 @@
 """The kernel for products with few output tiles (ts2_gemm_args.tileConfig bit 16) against fp64 products of the same 8-bit / bf16 values:
-every operand type and layout (int8 with k-tile scales and int8 sums: test_grouped_products_gpu.py), contractions of one, an odd and an even number of its half steps and more than its pipeline holds, every
-result type.  Bounds: i8 sums are exact (one rounding to fp32 is left); fp32 sums of bf16 products in any order stay within K * 2^-24 of
+every operand type and layout (int8 with k-tile scales and int8 sums: test_grouped_products_gpu.py), contractions of one, an odd and an
+even number of its half steps and more than its pipeline holds, every result type.  Bounds: i8 sums are exact (one rounding to fp32 is left); fp32 sums of bf16 products in any order stay within K * 2^-24 of
 sum |a b|; the e4m3 instruction adds its 64 products with fewer bits than an fp32 sum has (1.5e-5 rms of the result on every kernel
 here), and its products are held to 2e-4 of the largest result like in the tests of the other kernels; a bf16 result adds half a unit in
 the last place (2^-9), a packed one half of its row's step (max / 254)."""
@@ -138,3 +138,33 @@ def test_normalised_rows_and_several_products(t):
     w = want * 0.5 + want2 * 0.25
     tol = bound(t, 2 * k, mag * 0.5 + mag2 * 0.25, w)
     assert bool(((c.double() - w).abs() <= tol + 2.0 ** -22 * w.abs()).all())
+
+
+@pytest.mark.parametrize("k", [128, 512, 640, 1536, 1664, 2048])
+@pytest.mark.parametrize("ct,dt", [(L.F32, torch.float32), (L.BF16, torch.bfloat16), (L.F16, torch.float16), (L.I32, torch.int32)])
+def test_int8_stored_results_have_the_same_bits_from_every_kernel(k, ct, dt):
+    """both sides of the contractions where the dispatcher changes kernels: int32 sums are exact, what is left is their conversion to fp32, one
+    product with alpha * rowScale and one rounding; also rows that start on the 4-byte grid only, which the kernel for few tiles declines"""
+    print("case int8 stored, every kernel", k, ct, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    m, n, live = 384, 256, 333
+    a, b, want, _ = product(L.I8, m, n, k, False, gen)
+    rs = torch.rand(m, device="cuda", generator=gen) + 0.5
+    raw = ct == L.I32
+    if raw:
+        want = want.to(torch.int32)
+    else:
+        want = (want.float() * (rs * 2.0 ** -10)[:, None]).to(dt)  # (inside the range of a half)
+        want[live:] = 0
+    for config in (0, SLICE, 2 * SLICE):
+        for pad in (0, 4 // torch.empty(0, dtype=dt).element_size()):
+            if pad and config == SLICE:
+                continue
+            wide = torch.full((m, n + pad), 7, dtype=dt, device="cuda")
+            c = wide[:, :n]
+            out = c.view(torch.int16) if ct == L.BF16 else c
+            if raw:
+                L.load().gemm_nt(a, b, out, L.I8, ct, tile_config=config)
+            else:
+                L.load().gemm_nt(a, b, out, L.I8, ct, row_scale=rs, alpha=2.0 ** -10, m_live=live, tile_config=config)
+            assert torch.equal(c, want) and bool((wide[:, n:] == 7).all()), (config, pad)
