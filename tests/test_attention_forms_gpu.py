@@ -1,0 +1,144 @@
+"""The forms of the attention kernels, which a rule on the number of workgroups (and on the key range of a workgroup) chooses between:
+a pipelined forward for long key ranges and a plain one for narrow windows; the backward as one launch with two waves (or pairs of waves)
+per row block where there are few workgroups, as two launches where there are many.  The repetition of two heads of data fills a launch of any size, and the oracle computes those two only.
+Inputs are bf16-representable; the device rounds probabilities and score gradients to bf16 before a product, hence the same tolerance as in
+test_attention_gpu.py: max |err| <= 1e-2 * max |ref| per tensor."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+from oracle_lib import Oracle  # noqa: E402
+from test_attention_gpu import bf16_round, ragged_spans, spans_to_ranges  # noqa: E402
+
+SCALE = float(np.float32(np.sqrt(np.float32(1.0 / 128))) * np.float32(0.5 / 0.693147))
+
+
+@pytest.fixture(scope="module")
+def L():
+    from tscale2_amd import lib
+    lib.load()
+    return lib
+
+
+@pytest.fixture(scope="module")
+def orc():
+    return Oracle()
+
+
+def device_pass(L, n, heads, arrays, start, finish, slope, scale=SCALE, dscale=None):
+    """val, sumWeightLog and, with dscale, dq, dk, dv (each [n_round, heads * 128], statistics [heads, n_round])"""
+    n_round, i16 = start.size, torch.int16
+
+    def padded(a):
+        t = torch.zeros((n_round, a.shape[1]), dtype=torch.bfloat16, device="cuda")
+        t[:n] = torch.from_numpy(a).cuda().bfloat16()
+        return t
+    q, k, v, dval = [padded(a) for a in arrays]
+    ts, tf = torch.from_numpy(start).cuda(), torch.from_numpy(finish).cuda()
+    out = [torch.full((n_round, heads * 128), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(4)]
+    swl = torch.full((heads, n_round), -5.0, device="cuda")
+    L.att_forward(n, heads, q.view(i16), k.view(i16), v.view(i16), ts, tf, scale, slope, out[0].view(i16), swl)
+    if dscale is not None:
+        ds = torch.zeros((heads, n_round), device="cuda")
+        ds[:, :n] = torch.from_numpy(dscale).cuda()
+        lo = torch.zeros(n_round // 128, dtype=torch.int32, device="cuda")
+        hi = torch.zeros_like(lo)
+        L.call("ts2_att_build_rev", n, n_round, ts, tf, lo, hi)
+        L.att_backward(n, heads, q.view(i16), k.view(i16), v.view(i16), dval.view(i16), ts, tf, lo, hi, scale, slope, swl, ds,
+                       *[t.view(i16) for t in out[1:]], L.BF16)
+    torch.cuda.synchronize()
+    return out, swl
+
+
+def inputs(n, heads, seed, q_mul=1.0):
+    r = np.random.default_rng(seed)
+    a = [bf16_round(r.standard_normal((n, heads * 128)).astype(np.float32)) for _ in range(4)]
+    a[0] = bf16_round(a[0] * np.float32(q_mul))
+    return a
+
+
+# documents, window, heads of the launch, slope.  1100 tokens are nine 128-row blocks: with 2 heads the backward is one launch of 54 workgroups,
+# with 10 and 16 it is two.  Windows of 40 keep a workgroup's keys within five tiles, whole documents go beyond; 64 and 65 tokens end a document
+# on a tile and one past it
+CASES = [
+    ([300, 1, 299, 500], 40, 2, 0.0), ([300, 1, 299, 500], 40, 16, 0.0), ([300, 1, 299, 500], 40, 16, 0.25),
+    ([1100], 4096, 10, 0.0), ([1100], 4096, 16, 0.0), ([1100], 4096, 16, 0.01), ([1100], 4096, 2, 0.01),
+    ([64, 65, 63, 128, 129, 651], 300, 16, 0.0), ([64, 65, 63, 128, 129, 651], 300, 2, 0.125), ([64, 65, 63, 128, 129, 651], 4096, 10, 0.125),
+    ([31, 33, 1, 5], 4096, 1, 0.0), ([1], 4096, 1, 0.0),
+]
+
+
+@pytest.mark.parametrize("docs,window,heads,slope", CASES)
+def test_forms_against_the_oracle(L, orc, docs, window, heads, slope):
+    print("case att forms", docs, window, heads, slope, flush=True)
+    sp, spans = ragged_spans(docs, window)
+    n, base = sp.size - 1, min(heads, 2)
+    n_round = (n + 127) // 128 * 128
+    start, finish = spans_to_ranges(sp, spans, n, n_round)
+    a = inputs(n, base, seed=n + heads)
+    ref = orc.attention(base, 128, 128, slope, sp, spans, *a)
+    rep = heads // base
+    out, swl = device_pass(L, n, heads, [np.tile(x, (1, rep)) for x in a], start, finish, slope, dscale=np.tile(ref["dscale"], (rep, 1)))
+    want_l = ref["max_dp"] + np.log2(ref["sum_weight"])
+    np.testing.assert_allclose(swl.cpu().numpy()[:, :n], np.tile(want_l, (rep, 1)), rtol=1e-4, atol=1e-4)
+    for name, t in zip(("val", "dq", "dk", "dv"), out):
+        g = t.float().cpu().numpy()
+        assert np.all(g[n:] == 0), name
+        for h in range(rep):
+            got = g[:n, h * base * 128:(h + 1) * base * 128]
+            assert np.abs(got - ref[name]).max() <= 1e-2 * max(np.abs(ref[name]).max(), 1e-30), (name, h)
+
+
+@pytest.mark.parametrize("heads", [2, 16])
+def test_logits_far_beyond_the_reference(L, orc, heads):
+    """logits of +-40: the reference of the running weights has to move, in the middle of a sequence too; peaked weights"""
+    print("case att large logits", heads, flush=True)
+    sp, spans = ragged_spans([1100], 4096)
+    n, n_round = 1100, 1152
+    start, finish = spans_to_ranges(sp, spans, n, n_round)
+    a = inputs(n, 2, seed=5, q_mul=14.0)
+    ref = orc.attention(2, 128, 128, 0.0, sp, spans, *a)
+    assert ref["max_dp"].max() > 24
+    rep = heads // 2
+    out, swl = device_pass(L, n, heads, [np.tile(x, (1, rep)) for x in a], start, finish, 0.0, dscale=np.tile(ref["dscale"], (rep, 1)))
+    np.testing.assert_allclose(swl.cpu().numpy()[:, :n], np.tile(ref["max_dp"] + np.log2(ref["sum_weight"]), (rep, 1)), rtol=1e-4, atol=1e-4)
+    for name, t in zip(("val", "dq", "dk", "dv"), out):
+        got = t.float().cpu().numpy()[:n, :256]
+        assert np.abs(got - ref[name]).max() <= 1e-2 * np.abs(ref[name]).max(), name
+
+
+@pytest.mark.parametrize("heads,window", [(2, 4096), (16, 4096), (16, 40)])
+def test_negative_scale(L, heads, window):
+    """a negative scale with negated queries is the same computation, dQ with the other sign.  The matrix instruction need not round a
+    negated sum to the negated value, so fp32 sums may differ by their own error, 1100 * 2^-24 of the largest term (far below 2^-14 of the
+    largest result), and what is stored by one bf16 step (at most 2^-7 of the value)"""
+    print("case att negative scale", heads, window, flush=True)
+    sp, spans = ragged_spans([700, 400], window)
+    n, n_round = 1100, 1152
+    start, finish = spans_to_ranges(sp, spans, n, n_round)
+    a = inputs(n, heads, seed=6)
+    ds = np.random.default_rng(7).standard_normal((heads, n)).astype(np.float32) * 0.1
+    x, lx = device_pass(L, n, heads, a, start, finish, 0.0, dscale=ds)
+    y, ly = device_pass(L, n, heads, [-a[0]] + a[1:], start, finish, 0.0, scale=-SCALE, dscale=ds)
+    assert ((lx - ly).abs() <= 2.0 ** -14 * lx.abs().max()).all()
+    for name, s, t in zip(("val", "dq", "dk", "dv"), x, y):
+        s, t = s.float(), -t.float() if name == "dq" else t.float()
+        assert ((s - t).abs() <= 2.0 ** -7 * s.abs() + 2.0 ** -14 * s.abs().max()).all(), name
+
+
+@pytest.mark.parametrize("heads", [2, 16])
+def test_zero_scale_and_masked_rows(L, heads):
+    """scale 0: every key that is seen weighs the same as the sink, whatever lies under the mask"""
+    print("case att zero scale", heads, flush=True)
+    sp, spans = ragged_spans([37, 400, 663], 333)
+    n, n_round = 1100, 1152
+    start, finish = spans_to_ranges(sp, spans, n, n_round)
+    a = inputs(n, heads, seed=8)
+    out, swl = device_pass(L, n, heads, a, start, finish, 0.0, scale=0.0)
+    count = np.where(finish[:n] >= start[:n], finish[:n] - start[:n] + 1, 0)
+    np.testing.assert_allclose(swl.cpu().numpy()[0, :n], np.log2(1 + count), rtol=1e-5, atol=1e-5)
+    v = np.concatenate([np.zeros((1, heads * 128)), np.cumsum(a[2].astype(np.float64), 0)])
+    want = (v[np.maximum(finish[:n], -1) + 1] - v[np.where(count > 0, start[:n], finish[:n] + 1)]) / (1 + count)[:, None]
+    got = out[0].float().cpu().numpy()[:n]
+    assert np.abs(got - want).max() <= 2.0 ** -8 * np.abs(want).max() + 1e-3

@@ -32,6 +32,8 @@
 //     copies of the code in one loop body (an operand fetch names its LDS array, so it never waits for the loads in flight into the
 //     other array); values needed once per tile (lane offsets of the loads, the statistics pass) are recomputed from a lane index
 //     obtained on the spot instead of living across the loop.
+//   * the forward works a tile ahead of itself (the first product of the next tile between the exponentials of this one), in an order of issue
+//     that the source fixes slot by slot.
 //   * workgroup ids are remapped so that an XCD works on consecutive blocks of one head, whose streamed rows overlap in its L2.
 //   * spans are one inclusive key range per query (every causal window / document-start pattern of
 //     src/gpt/att/sliding_window.cpp:111-118,226-240); masking is one unsigned compare per element, blocks outside a wave's range are
@@ -48,6 +50,7 @@ constexpr int KVROWS = 64;       // key rows owned by one workgroup of the dK/dV
 constexpr int TR = 64;           // rows of a streamed tile
 constexpr int ROWB = HD * 2;     // bytes of a tile row
 constexpr int TILE_BYTES = TR * ROWB;
+constexpr float SLACK = 8;       // how far (log2) a logit may pass the forward's reference before the reference moves
 constexpr float LN2 = 0.693147f; // LOG2 of src/gpt/model_params/model_dim.h:16
 #define TS2_LDS_PTR(p) ((__attribute__((address_space(3))) void *)(p))
 #define TS2_GLB_PTR(p) ((const __attribute__((address_space(1))) void *)(p))
@@ -82,6 +85,14 @@ __device__ __forceinline__ v8bf PackB(const float *x, int s)
         r[w] = (int)PackBf16x2(x[8 * s + 2 * w], x[8 * s + 2 * w + 1]);
     }
     return __builtin_bit_cast(v8bf, r);
+}
+
+// acc + the two bf16 values of a word, in fp32
+__device__ __forceinline__ float AddBf16x2(float acc, int word)
+{
+    typedef __bf16 v2bf_t __attribute__((ext_vector_type(2)));
+    const v2bf_t one = {(__bf16)1.f, (__bf16)1.f};
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2bf_t, word), one, acc, false);
 }
 
 // row index inside a 32x32 MFMA result block held in register e by a lane of the given half
@@ -305,24 +316,94 @@ __device__ __forceinline__ void MapAttBlock(int *blk, int *head)
     *blk = id - *head * nbx;
 }
 
-// forward: grid (lenRound/128, heads); a wave owns 32 query rows
-template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP p)
+// Tile loads as inline asm: the compiler does not see them, so it adds no waits of its own to the operand fetches, and the kernel's waits
+// at its barriers are the only ones.  The descriptor of a tile ends with its last row.
+__device__ __forceinline__ v4i TileRsrc(const uint8_t *g, int bytes)
 {
-    __shared__ __attribute__((aligned(1024))) uint8_t kT0[TILE_BYTES], kT1[TILE_BYTES], vT0[TILE_BYTES], vT1[TILE_BYTES];
-    __shared__ int red[8];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, half = lane >> 5;
-    int blk, head;
-    MapAttBlock(&blk, &head);
-    // later query blocks of a causal sequence see more keys: they start first so that the short ones fill the tail of the launch
-    const int myRow = (gridDim.x - 1 - blk) * BROWS + wave * WROWS + l32;
-    const int64_t hoff = (int64_t)head * HD * 2;
-    const int start = p.spanStart[myRow], finish = p.spanFinish[myRow];
-    int kLo, kHi;
-    BlockKeyRange(start, finish, tid, &kLo, &kHi, red);
-    kLo = __builtin_amdgcn_readfirstlane(kLo);
-    kHi = __builtin_amdgcn_readfirstlane(kHi);
-    const int tFirst = kHi >= kLo ? (kLo / TR) * TR : 1;
-    const uint8_t *gk = p.k + hoff, *gv = p.v + hoff;
+    const uint64_t u = (uint64_t)(uintptr_t)g; // (a user address: bits 48 and up are zero)
+    return v4i{__builtin_amdgcn_readfirstlane((int)(uint32_t)u), __builtin_amdgcn_readfirstlane((int)(u >> 32)), bytes, 0x00020000};
+}
+
+// The waves w = 0 .. WPG - 1 (WPG = 2 or 4) fetch a tile of ROWS rows together, one row group (4 rows, 1 KB) per load: groups with the same
+// number modulo 4, which share one swizzle per lane (two of them where two waves fetch a tile).  What a lane adds is held in registers, what
+// a row group adds in scalar ones; a request is a handful of scalar instructions.
+template <int WPG, int ROWS> struct TTileLoader {
+    static constexpr int SWZ = WPG == 2 ? 2 : 1, PER = ROWS / 4 / WPG / SWZ; // swizzles of a wave, loads with each
+    int laneOff[SWZ];
+    int ld, dst; // bytes of a row; LDS offset of the wave's first row group
+    __device__ __forceinline__ TTileLoader(int64_t ld64, int w, int lane) : ld((int)ld64), dst(w * 1024)
+    {
+        const int lrow = lane >> 4;
+#pragma unroll
+        for (int c = 0; c < SWZ; ++c) {
+            const int u = w + 2 * c;
+            laneOff[c] = (lrow + 4 * u) * ld + (((lane & 15) ^ ((lrow << 2) | (u & 3))) << 4);
+            asm volatile("" : "+v"(laneOff[c]));
+        }
+    }
+    __device__ __forceinline__ void Request(unsigned ldsTile, const uint8_t *g) const
+    {
+        const v4i rsrc = TileRsrc(g, ROWS * ld);
+        const unsigned m0 = ldsTile + dst;
+#pragma unroll
+        for (int c = 0; c < SWZ; ++c) {
+#pragma unroll
+            for (int i = 0; i < PER; ++i) {
+                const int u = WPG * SWZ * i;
+                asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(m0), "v"(laneOff[c]), "s"(rsrc),
+                             "s"(4 * u * ld), "n"(u * 1024 + c * 2048)
+                             : "memory", "scc");
+            }
+        }
+    }
+};
+
+// every operand fetch as one address register and a constant offset (TFragLane adds two of its terms at each use: 24 additions per tile)
+struct TFragAddr {
+    int row[8], trLo[4], trHi[4];
+};
+
+__device__ __forceinline__ TFragAddr MakeFragAddr(int lane, int base)
+{
+    const TFragLane f = MakeFragLane(lane);
+    TFragAddr r;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        r.row[j] = f.row[j] + base;
+        r.row[j + 4] = f.row[j] + f.rowHi + base;
+        r.trLo[j] = f.trLo[j] + base;
+        r.trHi[j] = f.trLo[j] + f.trHi + base;
+        asm volatile("" : "+v"(r.row[j]), "+v"(r.row[j + 4]), "+v"(r.trLo[j]), "+v"(r.trHi[j]));
+    }
+    return r;
+}
+
+// A operand, contraction over d (see FragRow above)
+__device__ __forceinline__ v8bf FragRow(const uint8_t *tile, int ds, const TFragAddr &f)
+{
+    TLdsBytes b = (TLdsBytes)TS2_LDS_PTR(tile);
+    return __builtin_bit_cast(v8bf, *(const __attribute__((address_space(3))) v4i *)(b + f.row[ds]));
+}
+
+// A operand, contraction over tile rows (see FragTr above)
+__device__ __forceinline__ v8bf FragTr(const uint8_t *tile, int ks, int db, const TFragAddr &f)
+{
+    typedef __attribute__((address_space(3))) v4s16 *TTrPtr;
+    TLdsBytes b = (TLdsBytes)TS2_LDS_PTR(tile) + 16 * ks * ROWB;
+    const v4s16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TTrPtr)(b + f.trLo[db]));
+    const v4s16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TTrPtr)(b + f.trHi[db]));
+    typedef short v8s16 __attribute__((ext_vector_type(8)));
+    v8s16 r = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    return __builtin_bit_cast(v8bf, r);
+}
+
+// A workgroup whose keys fit a few tiles (narrow windows): one 32-key block after the other, skipped where the wave sees none of it, with the
+// exact running maximum.  The pipelined form below needs a barrier more and works on 64 keys at a time: 22.5 against 25 us for 16800 tokens,
+// 4 heads, 64-token windows over documents of unequal length.
+template <bool ALIBI>
+__device__ __forceinline__ void ForwardFewTiles(const AttP &p, uint8_t *kT0, uint8_t *kT1, uint8_t *vT0, uint8_t *vT1, const uint8_t *gk, const uint8_t *gv,
+    int tFirst, int kHi, int wave, int myRow, int l32, int half, int lane, int64_t hoff, int start, int finish, v16f (&oacc)[4], float &m, float &sum)
+{
     if (tFirst <= kHi) {
         LoadTileDirect(kT0, gk + (int64_t)tFirst * p.ldk, p.ldk, wave);
         LoadTileDirect(vT0, gv + (int64_t)tFirst * p.ldv, p.ldv, wave);
@@ -333,7 +414,6 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
     const TFragLane fl = MakeFragLane(lane);
     float zero = 0; // opaque, as in AttGradQ
     asm volatile("" : "+v"(zero));
-    v16f oacc[4];
 #pragma unroll
     for (int db = 0; db < 4; ++db) {
 #pragma unroll
@@ -341,7 +421,8 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
             oacc[db][e] = zero;
         }
     }
-    float m = 0, sum = 1; // the sink: a zero vector with weight 2^-m
+    m = 0;
+    sum = 1; // the sink: a zero vector with weight 2^-m
     auto tile = [&](const uint8_t *kt, const uint8_t *vt, int t0) __attribute__((always_inline)) {
 #pragma unroll
         for (int kb = 0; kb < TR / 32; ++kb) {
@@ -473,7 +554,337 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
         tile(kT1, vT1, t0);
         t0 += TR;
     }
-    StoreOwnRows<false>(p.out0 + (int64_t)(myRow - l32) * p.ldo0, p.ldo0, head * HD, oacc, 1 / sum, l32, half);
+}
+
+// forward: grid (lenRound / 128, heads); a wave owns 32 query rows.
+//
+// Bounded by issue: per 32 x 32 block 16 MFMAs (512 cycles) stand against 78 vector instructions, 24 LDS reads and their waits, and a wave
+// issues one instruction in five cycles.  So the kernel saves instructions: the exponential's argument is one fused multiply-add of the raw
+// product, the maximum of a tile is only compared with the reference it uses (weights are floats: a reference that lags by up to SLACK
+// powers of two loses no digit, and the accumulators are rescaled hardly ever; with the exact maximum of 32 rows, every second block; a row is
+// divided by the sum of its weights as they were rounded for the product, so that a single dominating weight leaves its row of V exact), masks
+// are a pass of their own over the tiles that need one.  And it overlaps: S of tile i + 1 is formed between the exponentials of tile i, its
+// maximum between the products with V, operands are requested six products ahead.  16 x 2048 tokens causal, 16 heads: 407 -> 356 us; without
+// the tile loads about 300, without the exponentials 338: what is left is the two together with the latency of the tiles.  One sequence of
+// 2048 tokens, one head 54 -> 40 (a second wave per block, sharing its tiles, was tried: 36, but windows of 64 tokens 9.2 -> 10).
+template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP p)
+{
+    constexpr int QB = 4;  // query blocks of the workgroup; as many waves stream its tiles
+    constexpr int FEW = 5; // key tiles up to which ForwardFewTiles is the faster one
+    // K and V of the even tiles, of the odd ones
+    __shared__ __attribute__((aligned(1024))) uint8_t kT0[TILE_BYTES], kT1[TILE_BYTES], vT0[TILE_BYTES], vT1[TILE_BYTES];
+    __shared__ int red[8];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, half = lane >> 5;
+    int blk, head;
+    MapAttBlock(&blk, &head);
+    // later query blocks of a causal sequence see more keys: they start first so that the short ones fill the tail of the launch
+    const int row0 = (gridDim.x - 1 - blk) * BROWS, myRow = row0 + wave * WROWS + l32;
+    const int64_t hoff = (int64_t)head * HD * 2;
+    const int start = p.spanStart[myRow], finish = p.spanFinish[myRow];
+    int kLo, kHi;
+    BlockKeyRange(start, finish, tid, &kLo, &kHi, red);
+    kLo = __builtin_amdgcn_readfirstlane(kLo);
+    kHi = __builtin_amdgcn_readfirstlane(kHi);
+    const int tile0 = kHi >= kLo ? kLo / TR : 0, nTiles = kHi >= kLo ? kHi / TR - tile0 + 1 : 0;
+    const uint8_t *gk = p.k + hoff, *gv = p.v + hoff;
+    v16f oacc[4];
+    if (__builtin_expect(nTiles <= FEW, 1)) { // (straight on in the code: short launches wait for their instructions too)
+        float m, sum;
+        ForwardFewTiles<ALIBI>(p, kT0, kT1, vT0, vT1, gk, gv, nTiles ? tile0 * TR : 1, nTiles ? kHi : 0, wave, myRow, l32, half, lane, hoff, start, finish, oacc, m, sum);
+        StoreOwnRows<false>(p.out0 + (int64_t)(myRow - l32) * p.ldo0, p.ldo0, head * HD, oacc, 1 / sum, l32, half);
+        if (half == 0) {
+            p.sumWeightLog[(int64_t)head * p.ldStat + myRow] = m + log2f(sum);
+        }
+        return;
+    }
+    const TRowSpan sp = MakeRowSpan(start, finish);
+    float zero = 0; // opaque, as in AttGradQ
+    asm volatile("" : "+v"(zero));
+#pragma unroll
+    for (int db = 0; db < 4; ++db) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            oacc[db][e] = zero;
+        }
+    }
+    v8bf qf[8];
+    LoadOwnFrags(qf, p.q + (int64_t)(myRow - l32) * p.ldq + hoff, p.ldq, l32, half);
+    // the exponential's argument is one fused multiply-add of the raw product: a negative scale goes into the sign of the queries, so
+    // that the largest product is the largest logit
+    const float sc = fabsf(p.attDotScale);
+    if (p.attDotScale < 0) {
+#pragma unroll
+        for (int ds = 0; ds < 8; ++ds) {
+            qf[ds] = __builtin_bit_cast(v8bf, __builtin_bit_cast(v4i, qf[ds]) ^ (int)0x80008000);
+        }
+    }
+    const unsigned ldsK0 = (unsigned)(uintptr_t)TS2_LDS_PTR(kT0), ldsK1 = (unsigned)(uintptr_t)TS2_LDS_PTR(kT1);
+    const unsigned ldsV0 = (unsigned)(uintptr_t)TS2_LDS_PTR(vT0), ldsV1 = (unsigned)(uintptr_t)TS2_LDS_PTR(vT1);
+    const TTileLoader<QB, TR> loadK(p.ldk, wave, lane), loadV(p.ldv, wave, lane);
+    auto tileKey = [&](int i) { return (tile0 + i) * TR; }; // first key of tile i
+    auto requestK = [&](int i, int buf) {
+        if (i < nTiles) {
+            loadK.Request(buf ? ldsK1 : ldsK0, gk + (int64_t)tileKey(i) * p.ldk);
+        }
+    };
+    auto requestV = [&](int i, int buf) {
+        if (i < nTiles) {
+            loadV.Request(buf ? ldsV1 : ldsV0, gv + (int64_t)tileKey(i) * p.ldv);
+        }
+    };
+#pragma unroll
+    for (int ds = 0; ds < 8; ++ds) {
+        // waited for here, together with the spans, and not by the compiler's count (which knows no tile loads) inside the loop
+        asm volatile("" : "+v"(qf[ds]));
+    }
+    requestK(0, 0);
+    requestV(0, 0);
+    requestK(1, 1);
+    const TFragAddr fl = MakeFragAddr(lane, 0);
+    v16f s0, s1;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        s0[e] = zero;
+        s1[e] = zero;
+    }
+    v4i pb[4] = {};
+    // the sink: a zero vector with weight 2^-m.  `sum` is the half's own part (the two halves of a row see different keys)
+    float m = 0, sum = half == 0 ? 1.f : 0.f, norm = sum, scT = sc; // norm: the sum of the weights as the products take them, rounded
+    auto seenAt = [&](int i) {
+        const int t = tileKey(i);
+        return i < nTiles && !(t > sp.waveMaxFinish || t + TR - 1 < sp.waveMinStart);
+    };
+    constexpr int AHEAD = 6; // operands requested ahead of their product: an LDS read takes the time of about four products
+    // The pieces below are written in the order they are issued: SCHED_FENCE ends a slot of one product, the operand fetch of the product
+    // AHEAD slots on and an eighth of the arithmetic that goes with it.
+#define SCHED_FENCE() __builtin_amdgcn_sched_barrier(0)
+    // weights of two keys of a block: 2^(logit - m), rounded into word j of the operand, and their sum
+    float wa = 0, wb = 0, wr = 0;
+    auto weights2 = [&](const v16f &s, v4i *pq, int j) __attribute__((always_inline)) {
+        float x0 = s[2 * j], x1 = s[2 * j + 1];
+        asm volatile("" : "+v"(x0), "+v"(x1)); // (arithmetic alone is not held by a fence: it stays between these two)
+        const float w0 = __builtin_amdgcn_exp2f(fmaf(x0, scT, -m)), w1 = __builtin_amdgcn_exp2f(fmaf(x1, scT, -m));
+        wa += w0;
+        wb += w1;
+        int word = (int)PackBf16x2(w0, w1);
+        wr = AddBf16x2(wr, word);
+        asm volatile("" : "+v"(wa), "+v"(wb), "+v"(wr), "+v"(word));
+        pq[j >> 2][j & 3] = word;
+    };
+    // O^T += V^T P^T of a block of 32 keys (rows from vt on); the caller has requested the first AHEAD operands; `arith` is called in every
+    // slot, `next` when the slot has no operand of its own to request
+    auto product2 = [&](const uint8_t *vt, v8bf (&ft)[AHEAD + 1], const v4i *pq, auto arith, auto next) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const v8bf a = ft[i % (AHEAD + 1)];
+            if (i + AHEAD < 8) {
+                ft[(i + AHEAD) % (AHEAD + 1)] = FragTr(vt, (i + AHEAD) >> 2, (i + AHEAD) & 3, fl);
+            } else {
+                next(i + AHEAD - 8);
+            }
+            oacc[i & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(v8bf, pq[i >> 2]), oacc[i & 3], 0, 0, 0);
+            arith(i);
+            SCHED_FENCE();
+        }
+    };
+    // S^T = K Q^T of the tile's 64 keys
+    auto product1 = [&](const uint8_t *kt, auto arith, auto next) __attribute__((always_inline)) {
+        v16f x[2];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            x[0][e] = 0;
+            x[1][e] = 0;
+        }
+        v8bf fk[AHEAD + 1];
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j) {
+            fk[j] = FragRow(kt, j, fl);
+        }
+        SCHED_FENCE();
+        arith(0);
+        arith(1);
+        SCHED_FENCE();
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const v8bf a = fk[j % (AHEAD + 1)];
+            if (j + AHEAD < 16) {
+                fk[(j + AHEAD) % (AHEAD + 1)] = FragRow(kt + ((j + AHEAD) >> 3) * (32 * ROWB), (j + AHEAD) & 7, fl);
+            } else {
+                next(j + AHEAD - 16);
+            }
+            x[j >> 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[j & 7], x[j >> 3], 0, 0, 0);
+            if (j < 14) {
+                arith(j + 2);
+            }
+            SCHED_FENCE();
+        }
+        s0 = x[0];
+        s1 = x[1];
+    };
+    // a tile that some row of the wave sees in part (every tile if there is a slope): logits in place of the products, -inf where masked
+    auto maskTile = [&](int t0) __attribute__((always_inline)) {
+        const bool full = t0 >= sp.waveMaxStart && t0 + TR - 1 <= sp.waveMinFinish;
+        int trips = __builtin_amdgcn_readfirstlane((int)(ALIBI || !full));
+        scT = trips ? 1.f : sc;
+        asm volatile("" : "+s"(trips));
+#pragma unroll 1
+        for (int r = 0; __builtin_expect(r < trips, 0); ++r) {
+            // (opaque: what follows from these two would otherwise be computed ahead of the loop, in every round)
+            int rel0 = t0 + half * 4 - sp.start;
+            float kc = ALIBI ? p.slope * (float)(t0 + half * 4 - myRow) : 0.f;
+            asm volatile("" : "+v"(rel0), "+v"(kc));
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const float x0 = ALIBI ? fmaf(s0[e], sc, fmaf(p.slope, (float)BlkRow(e, 0), kc)) : s0[e] * sc;
+                const float x1 = ALIBI ? fmaf(s1[e], sc, fmaf(p.slope, (float)(BlkRow(e, 0) + 32), kc)) : s1[e] * sc;
+                s0[e] = (unsigned)(rel0 + BlkRow(e, 0)) <= sp.len ? x0 : -INFINITY;
+                s1[e] = (unsigned)(rel0 + 32 + BlkRow(e, 0)) <= sp.len ? x1 : -INFINITY;
+            }
+        }
+    };
+    auto tileMax = [&]() __attribute__((always_inline)) {
+        float a = fmaxf(s0[0], s0[1]), b = fmaxf(s1[0], s1[1]);
+#pragma unroll
+        for (int e = 2; e < 16; e += 2) {
+            a = fmaxf(fmaxf(a, s0[e]), s0[e + 1]);
+            b = fmaxf(fmaxf(b, s1[e]), s1[e + 1]);
+        }
+        return fmaxf(a, b);
+    };
+    // moves the reference when a logit of some row has passed it by more than SLACK; returns whether it did
+    auto moveReference = [&](float mx, float &alpha) __attribute__((always_inline)) {
+        int trips = __builtin_amdgcn_readfirstlane((int)(__any(mx * scT > m + SLACK) != 0));
+        asm volatile("" : "+s"(trips));
+#pragma unroll 1
+        for (int r = 0; __builtin_expect(r < trips, 0); ++r) {
+            float lo, hi;
+            LaneSwap32(mx, &lo, &hi);
+            const float to = fmaxf(m, ceilf(fmaxf(lo, hi) * scT)); // (whole: the weights' bits and the factor below do not depend on it)
+            alpha = __builtin_amdgcn_exp2f(m - to);
+            m = to;
+        }
+        return trips;
+    };
+    bool seenPrev = false;
+    // round i: S of tile i, O += P V of tile i - 1.  K of tile i lies in buffer PAR = i % 2, V of tile i - 1 in the other one
+    auto round = [&](auto parTag, int i) __attribute__((always_inline)) {
+        constexpr int PAR = decltype(parTag)::value;
+        const uint8_t *kt = PAR ? kT1 : kT0, *vt = PAR ? vT0 : vT1;
+        if (i == 0) {
+            // K of the first tile has landed (loads complete in order; V and the second K may still be under way)
+            if (nTiles > 1) {
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * 16 / QB) : "memory");
+            } else {
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(16 / QB) : "memory");
+            }
+            __syncthreads();
+        } else {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // K of tile i and V of tile i - 1 have landed
+            __syncthreads();                                   // ... for every wave, and every wave is done with the other buffers
+            requestK(i + 1, PAR ^ 1);
+            requestV(i, PAR);
+        }
+        const int t0 = tileKey(i);
+        const bool seen = seenAt(i);
+        int hot = __builtin_amdgcn_readfirstlane((int)(seen && seenPrev)), first = __builtin_amdgcn_readfirstlane((int)(seen && !seenPrev)),
+            last = __builtin_amdgcn_readfirstlane((int)(!seen && seenPrev));
+        asm volatile("" : "+s"(hot), "+s"(first), "+s"(last));
+#pragma unroll 1
+        for (int r = 0; __builtin_expect(r < hot, 1); ++r) {
+            v8bf ft[AHEAD + 1], fu[AHEAD + 1];
+            wa = wb = wr = 0;
+            const v16f old = s1;
+            product1(
+                kt,
+                [&](int j) __attribute__((always_inline)) {
+                    if (j < 8) {
+                        weights2(old, pb + 2, j);
+                    }
+                },
+                [&](int i) __attribute__((always_inline)) { ft[i] = FragTr(vt, i >> 2, i & 3, fl); });
+            sum += wa + wb;
+            norm += wr;
+            maskTile(t0);
+            float ma = -INFINITY, mb = -INFINITY;
+            product2(
+                vt, ft, pb,
+                [&](int i) __attribute__((always_inline)) {
+                    const v16f &x = i < 4 ? s0 : s1;
+                    const int e = (i & 3) * 4;
+                    ma = fmaxf(fmaxf(ma, x[e]), x[e + 1]);
+                    mb = fmaxf(fmaxf(mb, x[e + 2]), x[e + 3]);
+                    asm volatile("" : "+v"(ma), "+v"(mb));
+                },
+                [&](int i) __attribute__((always_inline)) { fu[i] = FragTr(vt + 32 * ROWB, i >> 2, i & 3, fl); });
+            float alpha = 1;
+            int moved = moveReference(fmaxf(ma, mb), alpha);
+            wa = wb = wr = 0;
+            product2(vt + 32 * ROWB, fu, pb + 2, [&](int i) __attribute__((always_inline)) { weights2(s0, pb, i); }, [](int) {});
+            asm volatile("" : "+s"(moved));
+#pragma unroll 1
+            for (int q = 0; __builtin_expect(q < moved, 0); ++q) {
+                sum *= alpha;
+                norm *= alpha;
+#pragma unroll
+                for (int db = 0; db < 4; ++db) {
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        oacc[db][e] *= alpha;
+                    }
+                }
+            }
+            sum += wa + wb;
+            norm += wr;
+        }
+#pragma unroll 1
+        for (int r = 0; __builtin_expect(r < first, 0); ++r) { // the wave's first tile: nothing accumulated yet but the sink
+            product1(kt, [](int) {}, [](int) {});
+            maskTile(t0);
+            float alpha = 1;
+            moveReference(tileMax(), alpha);
+            wa = wb = wr = 0;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                weights2(s0, pb, j);
+            }
+            sum = sum * alpha + (wa + wb);
+            norm = norm * alpha + wr;
+        }
+#pragma unroll 1
+        for (int r = 0; __builtin_expect(r < last, 0); ++r) { // one round after its last tile
+            v8bf ft[AHEAD + 1], fu[AHEAD + 1];
+            wa = wb = wr = 0;
+#pragma unroll
+            for (int i = 0; i < AHEAD; ++i) {
+                ft[i] = FragTr(vt, i >> 2, i & 3, fl);
+            }
+            product2(
+                vt, ft, pb, [&](int i) __attribute__((always_inline)) { weights2(s1, pb + 2, i); },
+                [&](int i) __attribute__((always_inline)) { fu[i] = FragTr(vt + 32 * ROWB, i >> 2, i & 3, fl); });
+            sum += wa + wb;
+            norm += wr;
+            product2(vt + 32 * ROWB, fu, pb + 2, [](int) {}, [](int) {});
+        }
+        seenPrev = seen;
+    };
+    for (int i = 0;;) {
+        round(std::integral_constant<int, 0>{}, i);
+        if (++i > nTiles) {
+            break;
+        }
+        round(std::integral_constant<int, 1>{}, i);
+        if (++i > nTiles) {
+            break;
+        }
+    }
+    {
+        float lo, hi;
+        LaneSwap32(sum, &lo, &hi);
+        sum = lo + hi;
+        LaneSwap32(norm, &lo, &hi);
+        norm = lo + hi;
+    }
+    StoreOwnRows<false>(p.out0 + (int64_t)(myRow - l32) * p.ldo0, p.ldo0, head * HD, oacc, 1 / norm, l32, half);
     if (half == 0) {
         p.sumWeightLog[(int64_t)head * p.ldStat + myRow] = m + log2f(sum);
     }
