@@ -32,8 +32,11 @@
 //     copies of the code in one loop body (an operand fetch names its LDS array, so it never waits for the loads in flight into the
 //     other array); values needed once per tile (lane offsets of the loads, the statistics pass) are recomputed from a lane index
 //     obtained on the spot instead of living across the loop.
-//   * the forward works a tile ahead of itself (the first product of the next tile between the exponentials of this one), in an order of issue
-//     that the source fixes slot by slot.
+//   * few workgroups (short batches, few heads): the chip idles and a workgroup's time is a chain of blocks.  In the backward two waves then
+//     share a row block and take every other tile each, their partial results meet in LDS, and dQ runs beside dK/dV in one launch
+//     (OneLaunch below).
+//   * the forward and those kernels work a block or a tile ahead of themselves (the first products of the next one between the exponentials
+//     of this one), in an order of issue that the source fixes slot by slot.
 //   * workgroup ids are remapped so that an XCD works on consecutive blocks of one head, whose streamed rows overlap in its L2.
 //   * spans are one inclusive key range per query (every causal window / document-start pattern of
 //     src/gpt/att/sliding_window.cpp:111-118,226-240); masking is one unsigned compare per element, blocks outside a wave's range are
@@ -66,6 +69,8 @@ struct AttP {
     int64_t ldStat;
     uint8_t *out0, *out1; // forward: valLookup; dQ kernel: dQ; dK/dV kernel: dK, dV
     int64_t ldo0, ldo1;
+    uint8_t *out2; // dQ where dK and dV are out0 and out1 of the same launch
+    int64_t ldo2;
     int lenRound;
     // score gradients handed from the dK/dV kernel to the dQ kernel (optional): per query row the number of its 32-query block's first
     // block of dS (dsBase[lenRound] = blocks per head), the blocks themselves (2 KB each), and how many of them the array holds
@@ -395,6 +400,23 @@ __device__ __forceinline__ v8bf FragTr(const uint8_t *tile, int ks, int db, cons
     typedef short v8s16 __attribute__((ext_vector_type(8)));
     v8s16 r = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     return __builtin_bit_cast(v8bf, r);
+}
+
+// first and last key that any of the ROWS query rows from row0 on sees; every wave finds it by itself (no LDS, no barrier)
+template <int ROWS>
+__device__ __forceinline__ void WaveKeyRange(const int *spanStart, const int *spanFinish, int row0, int lane, int *lo, int *hi)
+{
+    int s = 0x7fffffff, f = -1;
+#pragma unroll
+    for (int i = 0; i < ROWS / 64; ++i) {
+        const int a = spanStart[row0 + i * 64 + lane], b = spanFinish[row0 + i * 64 + lane];
+        if (b >= a) {
+            s = min(s, a);
+            f = max(f, b);
+        }
+    }
+    *lo = __builtin_amdgcn_readfirstlane(WaveMinInt(s));
+    *hi = __builtin_amdgcn_readfirstlane(WaveMaxInt(f));
 }
 
 // A workgroup whose keys fit a few tiles (narrow windows): one 32-key block after the other, skipped where the wave sees none of it, with the
@@ -1518,6 +1540,679 @@ template <bool F32, bool ALIBI, bool DS> __global__ void __launch_bounds__(256, 
     }
 }
 
+// adds the accumulators of the second group of waves to those of the first, through LDS: [wave of the group][register / 4][lane][4]
+template <int QB, int N> __device__ __forceinline__ void AddGroups(uint8_t *lds, v16f (&acc)[N], int grp, int qb, int lane)
+{
+    __syncthreads();
+    v4f *box = (v4f *)(lds + qb * (N * 16 * 64 * 4)) + lane;
+    if (grp == 1) {
+#pragma unroll
+        for (int k = 0; k < 4 * N; ++k) {
+            const int a = k >> 2, g = k & 3;
+            box[k * 64] = v4f{acc[a][4 * g], acc[a][4 * g + 1], acc[a][4 * g + 2], acc[a][4 * g + 3]};
+        }
+    }
+    __syncthreads();
+    if (grp == 0) {
+#pragma unroll
+        for (int k = 0; k < 4 * N; ++k) {
+            const int a = k >> 2, g = k & 3;
+            const v4f o = box[k * 64];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                acc[a][4 * g + j] += o[j];
+            }
+        }
+    }
+}
+
+// ---- backward of few rows --------------------------------------------------------------------------------------------------------------
+// Both halves of AttGradSmall walk blocks of 32 x 32 (a wave's own 32 rows against a streamed tile of 32 rows) one block ahead of themselves: while the
+// matrix cores form the first two products of block i + 1, the wave turns those of block i into score gradients, and while they multiply
+// with these, it forms the weights of block i + 1.
+constexpr int BT = 32;                    // rows of a streamed tile
+constexpr int BT_BYTES = BT * ROWB;       // 8 KB
+constexpr int BSTAGE = 2 * BT_BYTES;      // two tiles: what the first products read by rows
+constexpr int BSTAGES = 4;                // stages in LDS: block i, i + 1, and two under way
+constexpr int BAHEAD = 6;                 // operands requested ahead of their product
+constexpr int BSTAT_SLOTS = 8;            // dK/dV: statistics of a tile, requested one tile further ahead than its rows
+constexpr int BSTAT_BYTES = 4 * BT * 4;   // L, dScale, span start, span finish of 32 queries
+
+typedef v8bf TOperands[BAHEAD + 1];
+
+// eight MFMAs against a row-major tile (contraction over d): x += tile * own^T.  The caller has requested the first BAHEAD operands; `arith`
+// is called in every slot, `next` in the slots that have no operand of their own left to request (argument 0 .. BAHEAD - 1)
+template <class TArith, class TNext>
+__device__ __forceinline__ void RowProduct(v16f &x, const uint8_t *tile, TOperands &f, const v8bf (&own)[8], const TFragAddr &fl, TArith arith, TNext next)
+{
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const v8bf a = f[j % (BAHEAD + 1)];
+        if (j + BAHEAD < 8) {
+            f[(j + BAHEAD) % (BAHEAD + 1)] = FragRow(tile, j + BAHEAD, fl);
+        } else {
+            next(j + BAHEAD - 8);
+        }
+        x = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, own[j], x, 0, 0, 0);
+        arith(j);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// eight MFMAs against the transpose of a row-major tile (contraction over its rows): acc += tile^T * p
+template <class TArith, class TNext>
+__device__ __forceinline__ void TransposedProduct(v16f (&acc)[4], const uint8_t *tile, TOperands &f, const v4i (&p)[2], const TFragAddr &fl, TArith arith,
+    TNext next)
+{
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const v8bf a = f[j % (BAHEAD + 1)];
+        if (j + BAHEAD < 8) {
+            f[(j + BAHEAD) % (BAHEAD + 1)] = FragTr(tile, (j + BAHEAD) >> 2, (j + BAHEAD) & 3, fl);
+        } else {
+            next(j + BAHEAD - 8);
+        }
+        acc[j & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(v8bf, p[j >> 2]), acc[j & 3], 0, 0, 0);
+        arith(j);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// (arithmetic is not held by a scheduling fence: it stays between two of these)
+__device__ __forceinline__ void Pin(float &a, float &b)
+{
+    asm volatile("" : "+v"(a), "+v"(b));
+}
+
+// dQ of 128 queries of one head by eight waves: a wave owns 32 query rows, two waves share them and take every other key tile each
+template <bool F32, bool ALIBI> __device__ __forceinline__ void GradQSplit(const AttP &p, uint8_t *lds, int blk, int nBlk, int head)
+{
+    constexpr int KS = 2, QB = 4, ROWS = QB * WROWS, LOADS = 2 * (BT / 4) / QB; // wave-level loads per tile
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, half = lane >> 5;
+    const int grp = wave / QB, qb = wave % QB;
+    const int row0 = (nBlk - 1 - blk) * ROWS, myRow = row0 + qb * WROWS + l32; // long blocks of a causal sequence first
+    const int64_t hoff = (int64_t)head * HD * 2;
+    int kLo, kHi;
+    WaveKeyRange<ROWS>(p.spanStart, p.spanFinish, row0, lane, &kLo, &kHi);
+    const TRowSpan sp = MakeRowSpan(p.spanStart[myRow], p.spanFinish[myRow]);
+    v8bf qf[8], of[8];
+    LoadOwnFrags(qf, p.q + (int64_t)(myRow - l32) * p.ldq + hoff, p.ldq, l32, half);
+    LoadOwnFrags(of, p.dO + (int64_t)(myRow - l32) * p.lddo + hoff, p.lddo, l32, half);
+    const float gmul = p.attDotScale * LN2;
+    float negL = -p.sumWeightLog[(int64_t)head * p.ldStat + myRow], negDScale = -p.dScale[(int64_t)head * p.ldStat + myRow] * gmul;
+    const int tile0 = kHi >= kLo ? kLo / BT : 0, nTiles = kHi >= kLo ? kHi / BT - tile0 + 1 : 0;
+    const int nIter = (nTiles + KS - 1) / KS, nMine = (nTiles - grp + KS - 1) / KS;
+    const uint8_t *gk = p.k + hoff, *gv = p.v + hoff;
+    const unsigned ldsGrp = (unsigned)(uintptr_t)TS2_LDS_PTR(lds) + grp * (BSTAGES * BSTAGE);
+    const TTileLoader<QB, BT> loadK(p.ldk, qb, lane), loadV(p.ldv, qb, lane);
+    auto tileKey = [&](int i) { return (tile0 + i * KS + grp) * BT; };
+    auto request = [&](int i, int stage) __attribute__((always_inline)) {
+        if (i < nMine) {
+            loadK.Request(ldsGrp + stage * BSTAGE, gk + (int64_t)tileKey(i) * p.ldk);
+            loadV.Request(ldsGrp + stage * BSTAGE + BT_BYTES, gv + (int64_t)tileKey(i) * p.ldv);
+        }
+    };
+    request(0, 0);
+    request(1, 1);
+    request(2, 2);
+    const TFragAddr fl = MakeFragAddr(lane, grp * (BSTAGES * BSTAGE));
+#pragma unroll
+    for (int ds = 0; ds < 8; ++ds) {
+        asm volatile("" : "+v"(qf[ds]), "+v"(of[ds])); // waited for here (see AttForward)
+    }
+    Pin(negL, negDScale);
+    float zero = 0; // cleared from a register the optimiser cannot see through (see AttForward)
+    asm volatile("" : "+v"(zero));
+    v16f acc[4], x, dp;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        acc[0][e] = acc[1][e] = acc[2][e] = acc[3][e] = zero;
+        x[e] = dp[e] = zero;
+    }
+    float w[16]; // weights of the block in hand
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        w[e] = zero;
+    }
+    const float sc = p.attDotScale;
+    float scT = sc;
+    auto seenAt = [&](int i) {
+        const int t = tileKey(i);
+        return i < nMine && !(t > sp.waveMaxFinish || t + BT - 1 < sp.waveMinStart);
+    };
+    bool seenPrev = false;
+    // step i: dQ += K^T dS of block i, first products and weights of block i + 1
+    auto step = [&](auto stageTag, int i) __attribute__((always_inline)) {
+        constexpr int NXT = decltype(stageTag)::value, CUR = (NXT + BSTAGES - 1) % BSTAGES; // stages of tiles i + 1 and i
+        const uint8_t *kn = lds + NXT * BSTAGE, *vn = kn + BT_BYTES, *kc = lds + CUR * BSTAGE;
+        if (i + 2 < nMine && i >= 0) {
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory"); // all but tile i + 2
+        } else {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+        __syncthreads(); // tile i + 1 has landed for every wave, and every wave is done with tile i - 1
+        if (i >= 0) {
+            request(i + 3, (NXT + 2) % BSTAGES);
+        }
+        const int t0 = tileKey(i + 1);
+        const bool seen = seenAt(i + 1);
+        int hot = __builtin_amdgcn_readfirstlane((int)(seen && seenPrev)), first = __builtin_amdgcn_readfirstlane((int)(seen && !seenPrev)),
+            last = __builtin_amdgcn_readfirstlane((int)(!seen && seenPrev));
+        asm volatile("" : "+s"(hot), "+s"(first), "+s"(last));
+        seenPrev = seen;
+        v4i ps[2];
+        // dS of two keys: w (dP - dScale) attDotScale ln2, by the operations of AttGradQ (the same bits)
+        auto gradient2 = [&](int j) __attribute__((always_inline)) {
+            float a = dp[2 * j], b = dp[2 * j + 1];
+            Pin(a, b);
+            a = w[2 * j] * fmaf(a, gmul, negDScale);
+            b = w[2 * j + 1] * fmaf(b, gmul, negDScale);
+            int word = (int)PackBf16x2(a, b);
+            asm volatile("" : "+v"(word));
+            ps[j >> 2][j & 3] = word;
+        };
+        // (a slope's position term joins the logit here; masked keys are -inf already)
+        float kq = 0;
+        auto weights2 = [&](int j) __attribute__((always_inline)) {
+            float a = x[2 * j], b = x[2 * j + 1];
+            Pin(a, b);
+            a = fmaf(a, scT, ALIBI ? fmaf(p.slope, (float)BlkRow(2 * j, 0), kq) : negL);
+            b = fmaf(b, scT, ALIBI ? fmaf(p.slope, (float)BlkRow(2 * j + 1, 0), kq) : negL);
+            a = __builtin_amdgcn_exp2f(a);
+            b = __builtin_amdgcn_exp2f(b);
+            Pin(a, b);
+            w[2 * j] = a;
+            w[2 * j + 1] = b;
+        };
+        auto mask = [&]() __attribute__((always_inline)) {
+            int trips = __builtin_amdgcn_readfirstlane((int)!(t0 >= sp.waveMaxStart && t0 + BT - 1 <= sp.waveMinFinish));
+            scT = trips ? 1.f : sc;
+            asm volatile("" : "+s"(trips));
+#pragma unroll 1
+            for (int r = 0; __builtin_expect(r < trips, 0); ++r) {
+                int rel0 = t0 + half * 4 - sp.start;
+                asm volatile("" : "+v"(rel0));
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    x[e] = (unsigned)(rel0 + BlkRow(e, 0)) <= sp.len ? x[e] * sc : -INFINITY;
+                }
+            }
+            if (ALIBI) {
+                kq = p.slope * (float)(t0 + half * 4 - myRow) + negL;
+            }
+        };
+        auto none = [](int) {};
+#pragma unroll 1
+        for (int r = 0; __builtin_expect(r < hot, 1); ++r) {
+            TOperands fa, fb, fc;
+            v16f xn, dn;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                xn[e] = 0;
+                dn[e] = 0;
+            }
+#pragma unroll
+            for (int j = 0; j < BAHEAD; ++j) {
+                fa[j] = FragRow(kn, j, fl);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            gradient2(0);
+            gradient2(1);
+            __builtin_amdgcn_sched_barrier(0);
+            RowProduct(
+                xn, kn, fa, qf, fl, [&](int j) __attribute__((always_inline)) { if (j < 6) { gradient2(j + 2); } },
+                [&](int k) __attribute__((always_inline)) { fb[k] = FragRow(vn, k, fl); });
+            x = xn;
+            mask();
+            RowProduct(
+                dn, vn, fb, of, fl, [&](int j) __attribute__((always_inline)) { if (j >= 2) { weights2(j - 2); } },
+                [&](int k) __attribute__((always_inline)) { fc[k] = FragTr(kc, k >> 2, k & 3, fl); });
+            TransposedProduct(
+                acc, kc, fc, ps, fl, [&](int j) __attribute__((always_inline)) { if (j < 2) { weights2(j + 6); } }, none);
+            dp = dn;
+        }
+#pragma unroll 1
+        for (int r = 0; __builtin_expect(r < first, 0); ++r) { // the wave's first block
+            TOperands fa, fb;
+            v16f xn, dn;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                xn[e] = 0;
+                dn[e] = 0;
+            }
+#pragma unroll
+            for (int j = 0; j < BAHEAD; ++j) {
+                fa[j] = FragRow(kn, j, fl);
+            }
+            RowProduct(xn, kn, fa, qf, fl, none, [&](int k) __attribute__((always_inline)) { fb[k] = FragRow(vn, k, fl); });
+            x = xn;
+            mask();
+            RowProduct(dn, vn, fb, of, fl, [&](int j) __attribute__((always_inline)) { weights2(j); }, none);
+            dp = dn;
+        }
+#pragma unroll 1
+        for (int r = 0; __builtin_expect(r < last, 0); ++r) { // after its last block
+            TOperands fc;
+#pragma unroll
+            for (int k = 0; k < BAHEAD; ++k) {
+                fc[k] = FragTr(kc, k >> 2, k & 3, fl);
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                gradient2(j);
+            }
+            TransposedProduct(acc, kc, fc, ps, fl, none, none);
+        }
+    };
+    if (nIter > 0) {
+        for (int i = -1;;) {
+            step(std::integral_constant<int, 0>{}, i);
+            if (++i >= nIter) {
+                break;
+            }
+            step(std::integral_constant<int, 1>{}, i);
+            if (++i >= nIter) {
+                break;
+            }
+            step(std::integral_constant<int, 2>{}, i);
+            if (++i >= nIter) {
+                break;
+            }
+            step(std::integral_constant<int, 3>{}, i);
+            if (++i >= nIter) {
+                break;
+            }
+        }
+    }
+    AddGroups<QB>(lds, acc, grp, qb, lane);
+    if (grp) {
+        return;
+    }
+    StoreOwnRows<F32>(p.out2 + (int64_t)(myRow - l32) * p.ldo2, p.ldo2, head * HD, acc, 1.f, l32, half);
+}
+
+// dK and dV of 64 keys of one head by eight waves.  Both accumulators of a key block in one wave would leave room for one wave per SIMD, and a lone
+// wave waits out every latency; so two waves share a key block: the dV wave forms S = Q K^T and the weights P and accumulates
+// dV^T += dO^T P; the dK wave forms dP = dO V^T, takes P from the dV wave through LDS (fp32, the very values), forms dS and accumulates
+// dK^T += Q^T dS: four products, two per wave.  The hand-over needs no signals of its own: the dV wave writes the weights of block i + 1
+// while the dK wave works on block i, and the barrier that every step has for its tiles lies between writing and reading (two slots per
+// key block, used in turn).  Two pairs share a key block and take every other query tile each.
+constexpr int KV_STAGES = 3;                                              // tiles i, i + 1 and the one under way
+constexpr int KV_STAT = KV_STAGES * BSTAGE;                               // statistics of BSTAT_SLOTS tiles
+constexpr int KV_GROUP = KV_STAT + BSTAT_SLOTS * BSTAT_BYTES;             // LDS of a group of waves that share their tiles
+constexpr int KV_P = 2 * KV_GROUP, KV_P_SLOT = 4096;                      // [pair of waves][slot][quarter][lane][4 values]
+constexpr int KV_LDS = KV_P + 4 * 2 * KV_P_SLOT;
+
+template <bool F32, bool ALIBI, bool DS, int ROLE> __device__ __forceinline__ void GradKVSplit(const AttP &p, uint8_t *lds, int blk, int head)
+{
+    constexpr int KS = 2, NST = KV_STAGES, KB = 4 / KS, GW = 2 * KB; // key blocks of the workgroup; waves that share a group's tiles
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, half = lane >> 5;
+    const int pair = wave & 3, grp = pair / KB, kb = pair % KB, loader = ROLE * KB + kb;
+    const int key0 = (blk * KB + kb) * WROWS, myRow = key0 + l32; // first key of the wave, my key
+    const int64_t hoff = (int64_t)head * HD * 2;
+    const int qLo = p.revLo[key0 / BROWS], qHi = p.revHi[key0 / BROWS];
+    v8bf own[8]; // the wave's keys as B operands: K for S, V for dP
+    if constexpr (ROLE) {
+        LoadOwnFrags(own, p.v + (int64_t)key0 * p.ldv + hoff, p.ldv, l32, half);
+    } else {
+        LoadOwnFrags(own, p.k + (int64_t)key0 * p.ldk + hoff, p.ldk, l32, half);
+    }
+    const int tile0 = __builtin_amdgcn_readfirstlane(qHi >= qLo ? qLo / BT : 0);
+    const int nTiles = __builtin_amdgcn_readfirstlane(qHi >= qLo ? qHi / BT - tile0 + 1 : 0);
+    const int nIter = (nTiles + KS - 1) / KS, nMine = (nTiles - grp + KS - 1) / KS;
+    const unsigned ldsGrp = (unsigned)(uintptr_t)TS2_LDS_PTR(lds) + grp * KV_GROUP;
+    const int query0 = (tile0 + grp) * BT; // first query of the group's first tile
+    const TTileLoader<GW, BT> loadQ(p.ldq, loader, lane), loadO(p.lddo, loader, lane);
+    const uint8_t *gq = p.q + hoff + (int64_t)query0 * p.ldq, *go = p.dO + hoff + (int64_t)query0 * p.lddo; // next tile to request
+    const int64_t stepQ = (int64_t)(KS * BT) * p.ldq, stepO = (int64_t)(KS * BT) * p.lddo;
+    auto requestRows = [&](int i, int stage) __attribute__((always_inline)) {
+        if (i < nMine) {
+            loadQ.Request(ldsGrp + stage * BSTAGE, gq);
+            loadO.Request(ldsGrp + stage * BSTAGE + BT_BYTES, go);
+            gq += stepQ;
+            go += stepO;
+        }
+    };
+    // statistics of a tile: even loaders fetch L (lanes 0..31) and dScale (32..63), odd ones span starts and finishes
+    const uint8_t *statLane = ((loader & 1) ? (const uint8_t *)((half ? p.spanFinish : p.spanStart) + l32)
+                                            : (const uint8_t *)((half ? p.dScale : p.sumWeightLog) + (int64_t)head * p.ldStat + l32)) + (int64_t)query0 * 4;
+    const unsigned statDst = ldsGrp + KV_STAT + (loader & 1) * (BSTAT_BYTES / 2);
+    auto requestStats = [&](int i) __attribute__((always_inline)) {
+        if (i < nMine) {
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(statDst + (i & (BSTAT_SLOTS - 1)) * BSTAT_BYTES), "v"(statLane)
+                         : "memory");
+            statLane += KS * BT * 4;
+        }
+    };
+    requestStats(0);
+    requestStats(1);
+#pragma unroll
+    for (int i = 0; i < NST - 1; ++i) {
+        if (i > 0) {
+            requestStats(i + 1);
+        }
+        requestRows(i, i);
+    }
+    const TFragAddr fl = MakeFragAddr(lane, grp * KV_GROUP);
+    const float sc = p.attDotScale, gmul = sc * LN2;
+#pragma unroll
+    for (int ds = 0; ds < 8; ++ds) {
+        asm volatile("" : "+v"(own[ds])); // waited for here (see AttForward)
+    }
+    float zero = 0; // cleared from a register the optimiser cannot see through (see AttForward)
+    asm volatile("" : "+v"(zero));
+    v16f acc[4], x[2]; // x: S (dV wave, [0] only), dP of the blocks in hand and ahead (dK wave, by turns)
+    float w[16];       // weights of the block in hand
+    v4i b[2] = {};     // second operand of the second product: weights or score gradients, rounded
+    v4f st[4];         // L of the block ahead (dV wave), dScale of the block in hand (dK wave): queries of registers 4 g .. + 3
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            acc[a][e] = zero;
+        }
+        x[0][e] = x[1][e] = w[e] = zero;
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        st[g] = v4f{zero, zero, zero, zero};
+    }
+    float scT = sc;
+    typedef __attribute__((address_space(3))) uint8_t *TLds;
+    const TLds ldsB = (TLds)TS2_LDS_PTR(lds), statB = ldsB + grp * KV_GROUP + KV_STAT;
+    // statistic `which` (0 L, 1 dScale, 2 start, 3 finish) of tile i for the queries of this half's registers
+    auto stats = [&](int i, int which, v4f (&s)[4]) __attribute__((always_inline)) {
+        const TLds a = statB + (i & (BSTAT_SLOTS - 1)) * BSTAT_BYTES + half * 16;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            s[g] = *(const __attribute__((address_space(3))) v4f *)(a + which * (BT * 4) + g * 32);
+        }
+    };
+    const TLds pMine = ldsB + KV_P + pair * (2 * KV_P_SLOT) + lane * 16;
+    // does some query of the tile see some key of the wave, and does every query see all of them: read early in a step, asked at its end
+    int lookS = 0, lookF = 0;
+    bool seenNext = false, fullNext = false;
+    auto lookRead = [&](int i) __attribute__((always_inline)) {
+        const TLds a = statB + (i & (BSTAT_SLOTS - 1)) * BSTAT_BYTES + l32 * 4;
+        lookS = *(const __attribute__((address_space(3))) int *)(a + 2 * BT * 4);
+        lookF = *(const __attribute__((address_space(3))) int *)(a + 3 * BT * 4);
+    };
+    auto look = [&](int i) __attribute__((always_inline)) {
+        seenNext = i < nMine && __any(lookF >= lookS && lookF >= key0 && lookS <= key0 + WROWS - 1);
+        fullNext = __all(lookS <= key0 && lookF >= key0 + WROWS - 1);
+    };
+    bool seenPrev = false;
+    // step i: second product of block i, first product (and weights) of block i + 1
+    auto step = [&](auto stageTag, int i) __attribute__((always_inline)) {
+        constexpr int NXT = decltype(stageTag)::value % NST, CUR = (NXT + NST - 1) % NST; // stages of tiles i + 1 and i
+        constexpr int SLOT = decltype(stageTag)::value & 1;                                // hand-over slot of block i + 1
+        const uint8_t *rows = lds + NXT * BSTAGE + ROLE * BT_BYTES;         // what the first product reads by rows: Q for S, dO for dP
+        const uint8_t *cols = lds + CUR * BSTAGE + (1 - ROLE) * BT_BYTES;   // whose transpose the second product takes: dO for dV, Q for dK
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads(); // rows of tile i + 1 and statistics of tile i + 2 have landed for every wave, every wave is done with tile i - 1
+        if (i >= 0) {
+            requestStats(i + NST);
+            requestRows(i + NST - 1, (NXT + NST - 2) % NST);
+        } else {
+            lookRead(0);
+            look(0);
+        }
+        lookRead(i + 2);
+        const bool seen = seenNext, full = fullNext;
+        int hot = __builtin_amdgcn_readfirstlane((int)(seen && seenPrev)), first = __builtin_amdgcn_readfirstlane((int)(seen && !seenPrev)),
+            last = __builtin_amdgcn_readfirstlane((int)(!seen && seenPrev));
+        asm volatile("" : "+s"(hot), "+s"(first), "+s"(last));
+        seenPrev = seen;
+        auto none = [](int) {};
+        auto rows6 = [&](TOperands &f) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < BAHEAD; ++j) {
+                f[j] = FragRow(rows, j, fl);
+            }
+        };
+        auto cols6 = [&](TOperands &f) __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < BAHEAD; ++k) {
+                f[k] = FragTr(cols, k >> 2, k & 3, fl);
+            }
+        };
+        if constexpr (ROLE == 0) {
+            float kq = 0;
+            auto weights2 = [&](int j) __attribute__((always_inline)) {
+                float u = x[0][2 * j], v = x[0][2 * j + 1], lu = st[j >> 1][(j & 1) * 2], lv = st[j >> 1][(j & 1) * 2 + 1];
+                Pin(u, v);
+                if (ALIBI) {
+                    lu = lu + fmaf(p.slope, (float)BlkRow(2 * j, 0), kq);
+                    lv = lv + fmaf(p.slope, (float)BlkRow(2 * j + 1, 0), kq);
+                }
+                u = __builtin_amdgcn_exp2f(fmaf(u, scT, -lu));
+                v = __builtin_amdgcn_exp2f(fmaf(v, scT, -lv));
+                Pin(u, v);
+                w[2 * j] = u;
+                w[2 * j + 1] = v;
+                if (j & 1) { // four more for the dK wave
+                    const int g = j >> 1;
+                    *(__attribute__((address_space(3))) v4f *)(pMine + SLOT * KV_P_SLOT + g * 1024) = v4f{w[4 * g], w[4 * g + 1], w[4 * g + 2], w[4 * g + 3]};
+                }
+            };
+            auto round2 = [&](int j) __attribute__((always_inline)) {
+                int word = (int)PackBf16x2(w[2 * j], w[2 * j + 1]);
+                asm volatile("" : "+v"(word));
+                b[j >> 2][j & 3] = word;
+            };
+            // a block that is seen in part: logits in place of the products, -inf where masked
+            auto mask = [&]() __attribute__((always_inline)) {
+                int trips = __builtin_amdgcn_readfirstlane((int)!full);
+                scT = trips ? 1.f : sc;
+                asm volatile("" : "+s"(trips));
+#pragma unroll 1
+                for (int r = 0; __builtin_expect(r < trips, 0); ++r) {
+                    v4f s4[4], f4[4];
+                    stats(i + 1, 2, s4);
+                    stats(i + 1, 3, f4);
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        const int s = __float_as_int(s4[e >> 2][e & 3]), f = __float_as_int(f4[e >> 2][e & 3]);
+                        x[0][e] = myRow >= s && myRow <= f ? x[0][e] * sc : -INFINITY;
+                    }
+                }
+                if (ALIBI) {
+                    kq = p.slope * (float)(query0 + (i + 1) * (KS * BT) + half * 4 - myRow);
+                }
+            };
+#pragma unroll 1
+            for (int r = 0; __builtin_expect(r < hot, 1); ++r) {
+                TOperands fa, fc;
+                v16f n;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    n[e] = 0;
+                }
+                rows6(fa);
+                stats(i + 1, 0, st);
+                __builtin_amdgcn_sched_barrier(0);
+                RowProduct(n, rows, fa, own, fl, [&](int j) __attribute__((always_inline)) { round2(j); },
+                    [&](int k) __attribute__((always_inline)) { fc[k] = FragTr(cols, k >> 2, k & 3, fl); });
+                x[0] = n;
+                mask();
+                TransposedProduct(acc, cols, fc, b, fl, [&](int j) __attribute__((always_inline)) { if (j) { weights2(j - 1); } }, none);
+                weights2(7);
+            }
+#pragma unroll 1
+            for (int r = 0; __builtin_expect(r < first, 0); ++r) { // the wave's first block
+                TOperands fa;
+                v16f n;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    n[e] = 0;
+                }
+                rows6(fa);
+                stats(i + 1, 0, st);
+                RowProduct(n, rows, fa, own, fl, none, none);
+                x[0] = n;
+                mask();
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    weights2(j);
+                }
+            }
+#pragma unroll 1
+            for (int r = 0; __builtin_expect(r < last, 0); ++r) { // after its last block
+                TOperands fc;
+                cols6(fc);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    round2(j);
+                }
+                TransposedProduct(acc, cols, fc, b, fl, none, none);
+            }
+        } else {
+            v16f &cur = x[SLOT ^ 1], &nxt = x[SLOT];
+            v4f pw[4];
+            auto take = [&]() __attribute__((always_inline)) {
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    pw[g] = *(const __attribute__((address_space(3))) v4f *)(pMine + (SLOT ^ 1) * KV_P_SLOT + g * 1024);
+                }
+            };
+            // dS of two queries: P (dP - dScale) attDotScale ln2, by the operations of AttGradKV (the same bits)
+            auto gradient2 = [&](int j) __attribute__((always_inline)) {
+                float u = cur[2 * j], v = cur[2 * j + 1];
+                Pin(u, v);
+                u = fmaf(u, gmul, -st[j >> 1][(j & 1) * 2] * gmul) * pw[j >> 1][(j & 1) * 2];
+                v = fmaf(v, gmul, -st[j >> 1][(j & 1) * 2 + 1] * gmul) * pw[j >> 1][(j & 1) * 2 + 1];
+                int word = (int)PackBf16x2(u, v);
+                asm volatile("" : "+v"(word));
+                b[j >> 2][j & 3] = word;
+            };
+            // The block of dS goes to the dQ kernel, transposed on the way.  Here a lane is a key and its registers walk over the queries; the
+            // dQ kernel's lanes are queries.  The operand pair the wave is about to multiply with, taken as the A operand of two more MFMAs
+            // against the matching slices of the identity, comes back as dS^T with lane = query, registers = keys in the order of the other
+            // kernel's operand fetches (exact: every sum has one term, and the values are bf16 already).  Block number first(query block) +
+            // (this key block - first key block the query block sees); a lane's two operands of 16 bytes sit at lane * 16 and
+            // 1024 + lane * 16: a wave writes, and the dQ kernel's wave reads, 1 KB contiguous per instruction.
+            auto giveDs = [&]() __attribute__((always_inline)) {
+                if constexpr (DS) {
+                    const int s = *(const __attribute__((address_space(3))) int *)(statB + (i & (BSTAT_SLOTS - 1)) * BSTAT_BYTES + 2 * BT * 4 + l32 * 4);
+                    const int f = *(const __attribute__((address_space(3))) int *)(statB + (i & (BSTAT_SLOTS - 1)) * BSTAT_BYTES + 3 * BT * 4 + l32 * 4);
+                    const int startMin = __builtin_amdgcn_readfirstlane(WaveMinInt(f >= s ? s : 0x7fffffff));
+                    const int64_t id = (int64_t)head * p.dsBase[p.lenRound] + p.dsBase[query0 + i * (KS * BT)] + ((key0 >> 5) - (startMin >> 5));
+                    v16f tr;
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        tr[e] = 0;
+                    }
+#pragma unroll
+                    for (int sl = 0; sl < 2; ++sl) {
+                        v4i r;
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            // slot j of operand sl in a lane of half h stands for query 16 sl + (j >> 2) * 8 + 4 h + (j & 3)
+                            const int qa = 16 * sl + ((2 * q) >> 2) * 8 + 4 * half + ((2 * q) & 3), qb2 = qa + 1;
+                            r[q] = (qa == l32 ? 0x3f80 : 0) | (qb2 == l32 ? 0x3f800000 : 0);
+                        }
+                        tr = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, b[sl]), __builtin_bit_cast(v8bf, r), tr, 0, 0, 0);
+                    }
+                    float tv[16];
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        tv[e] = tr[e];
+                    }
+                    if (id >= 0 && id < p.dsCap) {
+                        uint8_t *dst16 = p.ds + id * DS_BLOCK_BYTES + lane * 16;
+                        *(v8bf *)dst16 = PackB(tv, 0);
+                        *(v8bf *)(dst16 + 1024) = PackB(tv, 1);
+                    }
+                }
+            };
+#pragma unroll 1
+            for (int r = 0; __builtin_expect(r < hot, 1); ++r) {
+                TOperands fa, fc;
+                v16f n;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    n[e] = 0;
+                }
+                rows6(fa);
+                take();
+                __builtin_amdgcn_sched_barrier(0);
+                RowProduct(n, rows, fa, own, fl, [&](int j) __attribute__((always_inline)) { gradient2(j); },
+                    [&](int k) __attribute__((always_inline)) { fc[k] = FragTr(cols, k >> 2, k & 3, fl); });
+                nxt = n;
+                giveDs();
+                TransposedProduct(acc, cols, fc, b, fl, [&](int j) __attribute__((always_inline)) { if (j == 4) { stats(i + 1, 1, st); } }, none);
+            }
+#pragma unroll 1
+            for (int r = 0; __builtin_expect(r < first, 0); ++r) { // the wave's first block
+                TOperands fa;
+                v16f n;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    n[e] = 0;
+                }
+                rows6(fa);
+                stats(i + 1, 1, st);
+                RowProduct(n, rows, fa, own, fl, none, none);
+                nxt = n;
+            }
+#pragma unroll 1
+            for (int r = 0; __builtin_expect(r < last, 0); ++r) { // after its last block
+                TOperands fc;
+                take();
+                cols6(fc);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    gradient2(j);
+                }
+                giveDs();
+                TransposedProduct(acc, cols, fc, b, fl, none, none);
+            }
+        }
+        look(i + 2);
+    };
+    if (nIter > 0) {
+        // (the stage and the hand-over slot of a step are constants: six steps bring both back)
+#define KV_STEP(S)                                                                                                                         \
+    step(std::integral_constant<int, S>{}, i);                                                                                             \
+    if (++i >= nIter) {                                                                                                                    \
+        break;                                                                                                                             \
+    }
+        for (int i = -1;;) {
+            KV_STEP(0)
+            KV_STEP(1)
+            KV_STEP(2)
+            KV_STEP(3)
+            KV_STEP(4)
+            KV_STEP(5)
+        }
+#undef KV_STEP
+    }
+    AddGroups<GW>(lds, acc, grp, loader, lane);
+    if (grp) {
+        return;
+    }
+    uint8_t *out = ROLE ? p.out0 : p.out1;
+    const int64_t ldo = ROLE ? p.ldo0 : p.ldo1;
+    StoreOwnRows<F32>(out + (int64_t)key0 * ldo, ldo, head * HD, acc, 1.f, l32, half);
+}
+
+// The backward of a launch that cannot fill the chip: dK/dV workgroups (64 keys) and dQ workgroups (128 queries) side by side in one grid
+template <bool F32, bool ALIBI, bool DS> __global__ void __launch_bounds__(512, 2) AttGradSmall(AttP p, int nKv, int nQ, int heads)
+{
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[KV_LDS > 2 * BSTAGES * BSTAGE ? KV_LDS : 2 * BSTAGES * BSTAGE];
+    int id = blockIdx.x;
+    if (id < nKv * heads) {
+        if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 8)) { // waves 4..7, one beside each dV wave on its SIMD
+            GradKVSplit<F32, ALIBI, DS, 1>(p, lds, id % nKv, id / nKv);
+        } else {
+            GradKVSplit<F32, ALIBI, DS, 0>(p, lds, id % nKv, id / nKv);
+        }
+    } else {
+        id -= nKv * heads;
+        GradQSplit<F32, ALIBI>(p, lds, id % nQ, nQ, id / nQ);
+    }
+}
+
 // dQ from the score gradients the dK/dV kernel left behind: dQ^T += K^T dS^T, one product per block, no statistics, no exponentials.
 // grid (lenRound/128, heads); a wave owns 32 query rows (as in AttGradQ) and streams the key tiles its rows reach through LDS.  Its blocks
 // of dS arrive transposed and in operand order (see giveDs), one after the other in memory: 32 bytes per lane and block straight into
@@ -1681,6 +2376,14 @@ bool ActOk(const ts2_mat *m, int rows, int cols)
     return m && m->ptr && m->y >= rows && m->x >= cols && Aligned16(m->ptr, m->strideBytes) && m->strideBytes > 0 && m->strideBytes < (1 << 24);
 }
 
+// The backward as one launch (AttGradSmall) while all of its workgroups are on the chip at once: dK/dV workgroups of 64 keys and dQ
+// workgroups of 128 queries, one to a CU.  2048 tokens, one head 118 -> 45 us; 512-token documents x 4, 4 heads (192 workgroups) 38.0 -> 20.0,
+// with 64-token windows 19.5 -> 13.7; beyond 256 workgroups (that with 6 heads, 288) 39.4 against 34.0 but 20.8 against 23.6 in narrow windows.
+bool OneLaunch(int lenRound, int heads)
+{
+    return (int64_t)(lenRound / KVROWS + lenRound / BROWS) * heads <= 256;
+}
+
 } // namespace
 
 extern "C" int ts2_att_build_rev(int32_t len, int32_t lenRound, const int32_t *spanStart, const int32_t *spanFinish, int32_t *revLo, int32_t *revHi,
@@ -1814,26 +2517,46 @@ extern "C" int ts2_att_backward(const ts2_att_grad_args *a, void *stream)
         p.ds = (uint8_t *)a->dsScratch;
         p.dsCap = a->dsCapacityBlocks;
     }
-    if ((a->which & 1) && !viaDs) {
-        p.out0 = (uint8_t *)a->dQ.ptr;
-        p.ldo0 = a->dQ.strideBytes;
-        auto kernel = f32 ? (alibi ? AttGradQ<true, true> : AttGradQ<true, false>) : (alibi ? AttGradQ<false, true> : AttGradQ<false, false>);
-        hipLaunchKernelGGL(kernel, dim3(a->lenRound / BROWS, a->heads), dim3(256), 0, (hipStream_t)stream, p);
-        TS2_CHECK_LAUNCH();
-    }
-    if (a->which & 2) {
+    if (OneLaunch(a->lenRound, a->heads)) {
         p.out0 = (uint8_t *)a->dK.ptr;
         p.ldo0 = a->dK.strideBytes;
         p.out1 = (uint8_t *)a->dV.ptr;
         p.ldo1 = a->dV.strideBytes;
-        auto kernel = f32 ? (alibi ? AttGradKV<true, true, false> : AttGradKV<true, false, false>)
-                          : (alibi ? AttGradKV<false, true, false> : AttGradKV<false, false, false>);
-        if (viaDs) {
-            kernel = f32 ? (alibi ? AttGradKV<true, true, true> : AttGradKV<true, false, true>)
-                         : (alibi ? AttGradKV<false, true, true> : AttGradKV<false, false, true>);
+        p.out2 = (uint8_t *)a->dQ.ptr;
+        p.ldo2 = a->dQ.strideBytes;
+        const int nKv = (a->which & 2) ? a->lenRound / 64 : 0, nQ = (a->which & 1) && !viaDs ? a->lenRound / BROWS : 0;
+        if (nKv + nQ > 0) {
+            auto kernel = f32 ? (alibi ? AttGradSmall<true, true, false> : AttGradSmall<true, false, false>)
+                              : (alibi ? AttGradSmall<false, true, false> : AttGradSmall<false, false, false>);
+            if (viaDs) {
+                kernel = f32 ? (alibi ? AttGradSmall<true, true, true> : AttGradSmall<true, false, true>)
+                             : (alibi ? AttGradSmall<false, true, true> : AttGradSmall<false, false, true>);
+            }
+            hipLaunchKernelGGL(kernel, dim3((nKv + nQ) * a->heads), dim3(512), 0, (hipStream_t)stream, p, nKv, nQ, a->heads);
+            TS2_CHECK_LAUNCH();
         }
-        hipLaunchKernelGGL(kernel, dim3(a->lenRound / KVROWS, a->heads), dim3(256), 0, (hipStream_t)stream, p);
-        TS2_CHECK_LAUNCH();
+    } else {
+        if ((a->which & 1) && !viaDs) {
+            p.out0 = (uint8_t *)a->dQ.ptr;
+            p.ldo0 = a->dQ.strideBytes;
+            auto kernel = f32 ? (alibi ? AttGradQ<true, true> : AttGradQ<true, false>) : (alibi ? AttGradQ<false, true> : AttGradQ<false, false>);
+            hipLaunchKernelGGL(kernel, dim3(a->lenRound / BROWS, a->heads), dim3(256), 0, (hipStream_t)stream, p);
+            TS2_CHECK_LAUNCH();
+        }
+        if (a->which & 2) {
+            p.out0 = (uint8_t *)a->dK.ptr;
+            p.ldo0 = a->dK.strideBytes;
+            p.out1 = (uint8_t *)a->dV.ptr;
+            p.ldo1 = a->dV.strideBytes;
+            auto kernel = f32 ? (alibi ? AttGradKV<true, true, false> : AttGradKV<true, false, false>)
+                              : (alibi ? AttGradKV<false, true, false> : AttGradKV<false, false, false>);
+            if (viaDs) {
+                kernel = f32 ? (alibi ? AttGradKV<true, true, true> : AttGradKV<true, false, true>)
+                             : (alibi ? AttGradKV<false, true, true> : AttGradKV<false, false, true>);
+            }
+            hipLaunchKernelGGL(kernel, dim3(a->lenRound / KVROWS, a->heads), dim3(256), 0, (hipStream_t)stream, p);
+            TS2_CHECK_LAUNCH();
+        }
     }
     if (viaDs) {
         p.out0 = (uint8_t *)a->dQ.ptr;
