@@ -1433,47 +1433,66 @@ __global__ void __launch_bounds__(256) BackpropRowTileNormalizeRope8(int len, in
 }
 
 // sum of `splits` fp32 partial products (slabs of [rows][cols]) -> packed delta: per row and 128-column tile scale = maxabs/127,
-// bytes = sat_i8(rne(v/scale)), TileScale[tile][row] = scale: the arithmetic of the GEMM's ROW_TILE_MAXNORM epilogue applied to the sum
+// bytes = sat_i8(rne(v/scale)), TileScale[tile][row] = scale: the arithmetic of the GEMM's ROW_TILE_MAXNORM epilogue applied to the sum.
+//
+// Bounded by latency: one slice after the other is one trip to memory each.  So RU rows times SU slices are requested together, eight loads
+// per lane (the sum keeps the order of the slices, and its bits).  A small matrix of many slices gets one row per group of lanes and all of
+// eight slices at once, which also gives four times the groups: 512 x 512 of 8 slices 5.8 -> 2.8 us (10.8 -> 4 inside a step, from HBM),
+// 1024 x 512 of 32 32.9 -> 12.0, 1024 x 1024 of 8 7.2 -> 4.0, 256 x 256 of one 3.1 -> 2.9; 8192 x 2048 of 2 28.5 -> 23.8.
+template <int RU, int SU>
 __global__ void __launch_bounds__(256) PackDelta(int rows, int tiles, int splits, const uint8_t *partial, int64_t ldPartial, int64_t slab, float alpha,
     const float *alphaPtr, Mat delta, Mat tileScale)
 {
-    int t0, tile, h;
-    if (!Unit(rows, tiles, &t0, &tile, &h)) {
+    const long u = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 5;
+    const int h = threadIdx.x & 31, tile = (int)(u % tiles), t0 = (int)(u / tiles) * RU;
+    if (t0 >= rows) {
         return;
     }
     float scale = alpha;
     if (alphaPtr) {
         scale *= *alphaPtr;
     }
-    int col = tile * TILE + h * 4;
-    F4 v[U];
-    float discr[U];
+    const int col = tile * TILE + h * 4;
+    const uint8_t *src = partial + (int64_t)t0 * ldPartial + (int64_t)col * 4;
+    F4 v[RU];
 #pragma unroll
-    for (int k = 0; k < U; ++k) {
+    for (int k = 0; k < RU; ++k) {
         v[k] = ZeroF4();
     }
-    for (int sIdx = 0; sIdx < splits; ++sIdx) {
+    for (int s0 = 0; s0 < splits; s0 += SU) {
+        F4 x[SU][RU];
 #pragma unroll
-        for (int k = 0; k < U; ++k) {
-            if (t0 + k < rows) {
-                v[k] = v[k] + Load4<TF32>(partial + sIdx * slab + (int64_t)(t0 + k) * ldPartial + (int64_t)col * 4);
+        for (int j = 0; j < SU; ++j) {
+#pragma unroll
+            for (int k = 0; k < RU; ++k) {
+                x[j][k] = s0 + j < splits && t0 + k < rows ? Load4<TF32>(src + (int64_t)(s0 + j) * slab + k * ldPartial) : ZeroF4();
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < SU; ++j) {
+            if (s0 + j < splits) {
+#pragma unroll
+                for (int k = 0; k < RU; ++k) {
+                    v[k] = v[k] + x[j][k];
+                }
             }
         }
     }
 #pragma unroll
-    for (int k = 0; k < U; ++k) {
-        float mx = Half32Max(HMaxAbs(v[k])) * fabsf(scale);
-        discr[k] = 0;
-        float mult = 0;
+    for (int k = 0; k < RU; ++k) {
+        const float mx = Half32Max(HMaxAbs(v[k])) * fabsf(scale);
+        float discr = 0, mult = 0;
         if (mx > 0) {
-            discr[k] = mx / 127;
-            mult = 1 / discr[k];
+            discr = mx / 127;
+            mult = 1 / discr;
         }
         if (t0 + k < rows) {
             Store4<TI8>(At<TI8>(delta, t0 + k, col), v[k] * scale * mult);
+            if (h == 0) {
+                ScaleAt(tileScale, tile, t0 + k) = discr;
+            }
         }
     }
-    StoreScales(tileScale, tile, t0, rows, h, discr);
 }
 
 bool MatOk(const ts2_mat *m, int rows, int cols, int elemSize)
@@ -2122,8 +2141,13 @@ extern "C" int ts2_pack_delta(const ts2_mat *partial, int32_t splits, int64_t sl
         return TS2_ERR_SHAPE;
     }
     int tiles = cols / TILE;
-    hipLaunchKernelGGL(PackDelta, GridFor(rows, tiles), dim3(256), 0, STREAM, rows, tiles, splits, (const uint8_t *)partial->ptr, partial->strideBytes,
-        slabBytes, alpha, alphaPtr, M(*delta), M(*deltaTileScale));
+    // one row per group of lanes up to 16384 groups (eight waves on each SIMD of the chip; 1024 x 1024 of 8 slices takes 4.0 us so), and for
+    // more than two slices (of two, both forms have all in flight)
+    const bool small = splits > 2 && (int64_t)rows * tiles <= 16384;
+    const long units = (long)(small ? rows : (rows + 3) / 4) * tiles;
+    auto kernel = small ? PackDelta<1, 8> : PackDelta<4, 2>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((units * 32 + 255) / 256)), dim3(256), 0, STREAM, rows, tiles, splits, (const uint8_t *)partial->ptr,
+        partial->strideBytes, slabBytes, alpha, alphaPtr, M(*delta), M(*deltaTileScale));
     TS2_CHECK_LAUNCH();
     return TS2_OK;
 }
