@@ -1468,7 +1468,7 @@ extern "C" int ts2_model_forward(ts2_model *M, void *stream)
     CK(ModelForward(M, stream));
     CK(FinalLogits(M, M->logits, stream));
     // probabilities in place of the logits, in every row that "prediction" shows; the gradient buffer is scratch here
-    return Ts2FinalSoftmaxGrad(M->R, M->cfg.vocab, M->logits.P(), M->bias, M->target, 1.f, M->gradV.P(), nullptr, 1, stream);
+    return Ts2FinalProbabilities(M->R, M->cfg.vocab, M->logits.P(), M->bias, M->target, 1.f, M->gradV.P(), stream);
 }
 
 extern "C" int ts2_model_backprop(ts2_model *M, void *stream)

@@ -43,11 +43,97 @@ __global__ void __launch_bounds__(256) EmbedBackward(int len, int dim, const int
 }
 
 // SoftMax base 2 with running max starting at 0 and the (onehot - p) gradient (src/gpt/compute/cpu_transformer.cpp:12-37,146-159).
-// One workgroup per row; logits fp32 [row][vocab] are overwritten by probabilities when keepProb, grad is bf16.  Two passes over the
-// row with 16-byte accesses: the first finds the maximum and the sum together (the sum is rescaled whenever a lane's maximum grows),
-// the second, served by the caches, writes the gradient.  vocab is a multiple of 4.
-__global__ void __launch_bounds__(256) FinalSoftmaxGrad(int vocab, float *logits, int64_t ldLogits, const float *bias, const int *target,
-    float gradMult, bf16_t *grad, int64_t ldGrad, float *lossSum, int keepProb)
+// logits fp32 [row][vocab] are overwritten by probabilities, grad is bf16, zero in rows without a target; vocab is a multiple of 4.
+//
+// Bounded by HBM: a row is read once and held in registers, NCH chunks of four per lane, by W waves (one wave and no barrier for small
+// vocabularies, up to sixteen for large ones); one exponential and six other instructions per logit.  Against two passes by a workgroup of
+// four waves: 4096 x 1024 14.3 -> 9.2 us, x 8192 67 -> 54, x 16384 169 -> 113 (671 MB: 108 at the rate of a copy), 777 x 50304 133 -> 107
+// (three rounds of one workgroup per CU; twice the registers per lane and two workgroups to a CU spilled: 145).
+template <int W, int NCH>
+__global__ void __launch_bounds__(W == 1 ? 256 : 64 * W, 4) FinalProbabilities(int rows, int vocab, float *logits, int64_t ldLogits,
+    const float *bias, const int *target, float gradMult, bf16_t *grad, int64_t ldGrad)
+{
+    __shared__ float redM[W], redS[W];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int t = W == 1 ? blockIdx.x * 4 + wave : blockIdx.x, first = W == 1 ? lane : threadIdx.x;
+    if (t >= rows) { // (one wave per row: a whole wave, and no barrier below)
+        return;
+    }
+    float *row = (float *)((uint8_t *)logits + (int64_t)t * ldLogits);
+    bf16_t *grow = (bf16_t *)((uint8_t *)grad + (int64_t)t * ldGrad);
+    const int tg = target[t];
+    float4 x[NCH];
+    float m = -1e30f; // the row's largest logit with its bias
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+        const int k = (i * 64 * W + first) * 4;
+        x[i] = k < vocab ? *(const float4 *)(row + k) : make_float4(-1e30f, -1e30f, -1e30f, -1e30f);
+    }
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+        const int k = (i * 64 * W + first) * 4;
+        if (k < vocab) {
+            const float4 b = *(const float4 *)(bias + k);
+            x[i] = make_float4(x[i].x + b.x, x[i].y + b.y, x[i].z + b.z, x[i].w + b.w);
+        }
+        m = fmaxf(m, fmaxf(fmaxf(x[i].x, x[i].y), fmaxf(x[i].z, x[i].w)));
+    }
+    m = WaveMax(m);
+    if (W > 1) {
+        if (lane == 0) {
+            redM[wave] = m;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            m = fmaxf(m, redM[w]);
+        }
+    }
+    // weights in units of 2^-64: the hardware's exponential returns zero below 2^-126, which then is 2^-190 of the largest weight
+    m -= 64;
+    float sum = 0;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) { // (chunks beyond the vocabulary hold -1e30: weight zero)
+        x[i] = make_float4(__builtin_amdgcn_exp2f(x[i].x - m), __builtin_amdgcn_exp2f(x[i].y - m), __builtin_amdgcn_exp2f(x[i].z - m),
+            __builtin_amdgcn_exp2f(x[i].w - m));
+        sum += (x[i].x + x[i].y) + (x[i].z + x[i].w);
+    }
+    sum = WaveSum(sum);
+    if (W > 1) {
+        if (lane == 0) {
+            redS[wave] = sum;
+        }
+        __syncthreads();
+        sum = 0;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            sum += redS[w];
+        }
+    }
+    const float scale = 1 / sum, neg = tg < 0 ? 0.f : -gradMult;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+        const int k = (i * 64 * W + first) * 4;
+        if (k < vocab) {
+            const float p[4] = {x[i].x * scale, x[i].y * scale, x[i].z * scale, x[i].w * scale};
+            *(float4 *)(row + k) = make_float4(p[0], p[1], p[2], p[3]);
+            float g[4] = {p[0] * neg, p[1] * neg, p[2] * neg, p[3] * neg};
+            if ((unsigned)(tg - k) < 4u) { // the target's chunk (no chunk of a row without one)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    g[e] = e == tg - k ? (1 - p[e]) * gradMult : g[e];
+                }
+            }
+            *(uint2 *)(grow + k) = make_uint2(PackBf16x2(g[0], g[1]), PackBf16x2(g[2], g[3]));
+        }
+    }
+}
+
+// The same for vocabularies that do not fit the registers of sixteen waves: one workgroup per row, two passes with 16-byte accesses; the
+// first finds the maximum and the sum together (the sum is rescaled whenever a lane's maximum grows), the second, served by the caches,
+// writes.
+__global__ void __launch_bounds__(256) FinalProbabilitiesTwoPass(int vocab, float *logits, int64_t ldLogits, const float *bias, const int *target,
+    float gradMult, bf16_t *grad, int64_t ldGrad)
 {
     __shared__ float redM[4], redS[4];
     int t = blockIdx.x;
@@ -58,9 +144,6 @@ __global__ void __launch_bounds__(256) FinalSoftmaxGrad(int vocab, float *logits
     if (tg < 0) {
         for (int k = tid * 4; k < vocab; k += 1024) {
             *(uint2 *)(grow + k) = make_uint2(0, 0);
-        }
-        if (!keepProb) {
-            return;
         }
     }
     // lane-local running maximum m (of the logits without bias, never below 0) and sum of 2^(x + bias - m)
@@ -115,17 +198,12 @@ __global__ void __launch_bounds__(256) FinalSoftmaxGrad(int vocab, float *logits
             }
             float p[4] = {exp2f(x[i].x + bv[i].x - mx) * scale, exp2f(x[i].y + bv[i].y - mx) * scale, exp2f(x[i].z + bv[i].z - mx) * scale,
                 exp2f(x[i].w + bv[i].w - mx) * scale};
-            if (keepProb) {
-                *(float4 *)(row + k) = make_float4(p[0], p[1], p[2], p[3]);
-            }
+            *(float4 *)(row + k) = make_float4(p[0], p[1], p[2], p[3]);
             if (tg >= 0) {
                 float g[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     g[e] = ((k + e == tg ? 1.f : 0.f) - p[e]) * gradMult;
-                    if (k + e == tg && lossSum) {
-                        atomicAdd(lossSum, logf(p[e]));
-                    }
                 }
                 *(uint2 *)(grow + k) = make_uint2(PackBf16x2(g[0], g[1]), PackBf16x2(g[2], g[3]));
             }
@@ -615,11 +693,34 @@ int Ts2FinalSoftmaxGradHalf(int rows, int vocab, const ts2_mat *logits, const fl
     return TS2_OK;
 }
 
-int Ts2FinalSoftmaxGrad(int rows, int vocab, const ts2_mat *logits, const float *bias, const int *target, float gradMult, const ts2_mat *grad,
-    float *lossSum, int keepProb, void *stream)
+int Ts2FinalProbabilities(int rows, int vocab, const ts2_mat *logits, const float *bias, const int *target, float gradMult, const ts2_mat *grad,
+    void *stream)
 {
-    hipLaunchKernelGGL(FinalSoftmaxGrad, dim3(rows), dim3(256), 0, STREAM, vocab, (float *)logits->ptr, logits->strideBytes, bias, target, gradMult,
-        (bf16_t *)grad->ptr, grad->strideBytes, lossSum, keepProb);
+#define LAUNCH_P(W, N)                                                                                                                     \
+    hipLaunchKernelGGL((FinalProbabilities<W, N>), dim3(W == 1 ? (rows + 3) / 4 : rows), dim3(W == 1 ? 256 : 64 * W), 0, STREAM, rows, vocab, \
+        (float *)logits->ptr, logits->strideBytes, bias, target, gradMult, (bf16_t *)grad->ptr, grad->strideBytes)
+    const int chunks = (vocab + 255) / 256; // of 256 logits: one float4 per lane of a wave
+    if (chunks <= 2) {
+        LAUNCH_P(1, 2);
+    } else if (chunks <= 4) {
+        LAUNCH_P(1, 4);
+    } else if (chunks <= 8) {
+        LAUNCH_P(1, 8);
+    } else if (chunks <= 16) {
+        LAUNCH_P(4, 4);
+    } else if (chunks <= 32) {
+        LAUNCH_P(4, 8);
+    } else if (chunks <= 64) {
+        LAUNCH_P(8, 8);
+    } else if (chunks <= 104) {
+        LAUNCH_P(8, 13);
+    } else if (chunks <= 208) {
+        LAUNCH_P(16, 13);
+    } else {
+        hipLaunchKernelGGL(FinalProbabilitiesTwoPass, dim3(rows), dim3(256), 0, STREAM, vocab, (float *)logits->ptr, logits->strideBytes, bias, target,
+            gradMult, (bf16_t *)grad->ptr, grad->strideBytes);
+    }
+#undef LAUNCH_P
     TS2_CHECK_LAUNCH();
     return TS2_OK;
 }
