@@ -5,24 +5,46 @@
 
 namespace
 {
-// state0[t] = sum over labels of +-E[label] * scale (ComputeEmbedding, src/gpt/compute/cpu_transformer.cpp:76-100); one workgroup per row
-template <class TEmb>
-__global__ void __launch_bounds__(256) EmbedForward(int len, int dim, const int *labelPtr, const uint32_t *labels, const uint8_t *embed,
+// state0[t] = sum over labels of +-E[label] * scale (ComputeEmbedding, src/gpt/compute/cpu_transformer.cpp:76-100).  A row is a chain of
+// three loads (its labels' range, a label, the label's matrix row) before it is written, so a workgroup takes ROWS rows and has the first
+// label of all of them under way together: 65536 x 1024 of e4m3 99 -> 71 us (336 MB: 54 at the rate of a copy), 16384 x 512 12.2 -> 11.3.
+template <class TEmb, int ROWS>
+__global__ void __launch_bounds__(256) EmbedForward(int len, int lenRound, int dim, const int *labelPtr, const uint32_t *labels, const uint8_t *embed,
     int64_t ldEmb, float mult, const float *scalePtr, float *state, int64_t ldState)
 {
-    int t = blockIdx.x;
-    float s = mult * (scalePtr ? *scalePtr : 1.f);
+    const int t0 = blockIdx.x * ROWS;
+    const float s = mult * (scalePtr ? *scalePtr : 1.f);
+    int from[ROWS], to[ROWS];
+    uint32_t one[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+        const bool live = t0 + r < len;
+        from[r] = live ? labelPtr[t0 + r] : 0;
+        to[r] = live ? labelPtr[t0 + r + 1] : 0;
+    }
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+        one[r] = from[r] < to[r] ? labels[from[r]] : 0;
+    }
     for (int col = threadIdx.x * 4; col < dim; col += 1024) {
-        F4 acc = ZeroF4();
-        if (t < len) {
-            for (int k = labelPtr[t]; k < labelPtr[t + 1]; ++k) {
-                uint32_t label = labels[k];
-                float w = (label & 0x80000000u) ? -s : s;
-                label &= 0x7fffffffu;
-                acc = acc + Load4<TEmb>(embed + (int64_t)label * ldEmb + col * TEmb::SIZE) * w;
+        F4 acc[ROWS];
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            acc[r] = from[r] < to[r] ? Load4<TEmb>(embed + (int64_t)(one[r] & 0x7fffffffu) * ldEmb + col * TEmb::SIZE) : ZeroF4();
+        }
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            if (from[r] < to[r]) {
+                acc[r] = ZeroF4() + acc[r] * ((one[r] & 0x80000000u) ? -s : s);
+            }
+            for (int k = from[r] + 1; k < to[r]; ++k) {
+                const uint32_t label = labels[k];
+                acc[r] = acc[r] + Load4<TEmb>(embed + (int64_t)(label & 0x7fffffffu) * ldEmb + col * TEmb::SIZE) * ((label & 0x80000000u) ? -s : s);
+            }
+            if (t0 + r < lenRound) {
+                Store4<TF32>((uint8_t *)state + (int64_t)(t0 + r) * ldState + col * 4, acc[r]);
             }
         }
-        Store4<TF32>((uint8_t *)state + (int64_t)t * ldState + col * 4, acc);
     }
 }
 
@@ -637,12 +659,24 @@ __global__ void __launch_bounds__(256) FinalSoftmaxGradHalfWave(int rows, int vo
 int Ts2EmbedForward(int len, int lenRound, int dim, const int *labelPtr, const uint32_t *labels, const ts2_mat *embed, int embType, float mult,
     const float *scalePtr, const ts2_mat *state, void *stream)
 {
+    // (4096 x 512 with four rows to a workgroup 7.3 us, with one 6.8)
+    const int per = lenRound >= 8192 ? 4 : 1;
+#define LAUNCH_E(T, N)                                                                                                                     \
+    hipLaunchKernelGGL((EmbedForward<T, N>), dim3((lenRound + N - 1) / N), dim3(256), 0, STREAM, len, lenRound, dim, labelPtr, labels,      \
+        (const uint8_t *)embed->ptr, embed->strideBytes, mult, scalePtr, (float *)state->ptr, state->strideBytes)
     if (embType == TS2_I8) {
-        hipLaunchKernelGGL((EmbedForward<TI8>), dim3(lenRound), dim3(256), 0, STREAM, len, dim, labelPtr, labels, (const uint8_t *)embed->ptr,
-            embed->strideBytes, mult, scalePtr, (float *)state->ptr, state->strideBytes);
+        if (per == 4) {
+            LAUNCH_E(TI8, 4);
+        } else {
+            LAUNCH_E(TI8, 1);
+        }
     } else if (embType == TS2_E4M3) {
-        hipLaunchKernelGGL((EmbedForward<TE4M3>), dim3(lenRound), dim3(256), 0, STREAM, len, dim, labelPtr, labels, (const uint8_t *)embed->ptr,
-            embed->strideBytes, mult, scalePtr, (float *)state->ptr, state->strideBytes);
+        if (per == 4) {
+            LAUNCH_E(TE4M3, 4);
+        } else {
+            LAUNCH_E(TE4M3, 1);
+        }
+#undef LAUNCH_E
     } else {
         return TS2_ERR_UNSUPPORTED;
     }
