@@ -2525,7 +2525,7 @@ extern "C" int ts2_att_backward(const ts2_att_grad_args *a, void *stream)
         p.out2 = (uint8_t *)a->dQ.ptr;
         p.ldo2 = a->dQ.strideBytes;
         const int nKv = (a->which & 2) ? a->lenRound / 64 : 0, nQ = (a->which & 1) && !viaDs ? a->lenRound / BROWS : 0;
-        if (nKv + nQ > 0) {
+        if (a->which & 3) {
             auto kernel = f32 ? (alibi ? AttGradSmall<true, true, false> : AttGradSmall<true, false, false>)
                               : (alibi ? AttGradSmall<false, true, false> : AttGradSmall<false, false, false>);
             if (viaDs) {
