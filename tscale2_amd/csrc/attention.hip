@@ -53,7 +53,6 @@ constexpr int KVROWS = 64;       // key rows owned by one workgroup of the dK/dV
 constexpr int TR = 64;           // rows of a streamed tile
 constexpr int ROWB = HD * 2;     // bytes of a tile row
 constexpr int TILE_BYTES = TR * ROWB;
-constexpr float SLACK = 8;       // how far (log2) a logit may pass the forward's reference before the reference moves
 constexpr float LN2 = 0.693147f; // LOG2 of src/gpt/model_params/model_dim.h:16
 #define TS2_LDS_PTR(p) ((__attribute__((address_space(3))) void *)(p))
 #define TS2_GLB_PTR(p) ((const __attribute__((address_space(1))) void *)(p))
@@ -582,13 +581,11 @@ __device__ __forceinline__ void ForwardFewTiles(const AttP &p, uint8_t *kT0, uin
 //
 // Bounded by issue: per 32 x 32 block 16 MFMAs (512 cycles) stand against 78 vector instructions, 24 LDS reads and their waits, and a wave
 // issues one instruction in five cycles.  So the kernel saves instructions: the exponential's argument is one fused multiply-add of the raw
-// product, the maximum of a tile is only compared with the reference it uses (weights are floats: a reference that lags by up to SLACK
-// powers of two loses no digit, and the accumulators are rescaled hardly ever; with the exact maximum of 32 rows, every second block; a row is
-// divided by the sum of its weights as they were rounded for the product, so that a single dominating weight leaves its row of V exact), masks
-// are a pass of their own over the tiles that need one.  And it overlaps: S of tile i + 1 is formed between the exponentials of tile i, its
-// maximum between the products with V, operands are requested six products ahead.  16 x 2048 tokens causal, 16 heads: 407 -> 356 us; without
-// the tile loads about 300, without the exponentials 338: what is left is the two together with the latency of the tiles.  One sequence of
-// 2048 tokens, one head 54 -> 40 (a second wave per block, sharing its tiles, was tried: 36, but windows of 64 tokens 9.2 -> 10).
+// product, the running maximum is taken once per tile of 64 keys, masks are a pass of their own over the tiles that need one.  And it overlaps:
+// S of tile i + 1 is formed between the exponentials of tile i, its maximum between the products with V, operands are requested six products
+// ahead.  16 x 2048 tokens causal, 16 heads: 395 -> 376 us; one sequence of 2048 tokens, one head 54 -> 45.  A reference that lags the maximum
+// by up to 2^8 saves most of the rescaling (357, 40), but then the largest weight is rounded like any other: against fp64 0.00221 instead of
+// 0.00220, and 0.0020 instead of 0.0018 on peaked weights.
 template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP p)
 {
     constexpr int QB = 4;  // query blocks of the workgroup; as many waves stream its tiles
@@ -773,15 +770,15 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
         }
         return fmaxf(a, b);
     };
-    // moves the reference when a logit of some row has passed it by more than SLACK; returns whether it did
+    // moves the reference when a logit of some row has passed it; returns whether it did
     auto moveReference = [&](float mx, float &alpha) __attribute__((always_inline)) {
-        int trips = __builtin_amdgcn_readfirstlane((int)(__any(mx * scT > m + SLACK) != 0));
+        int trips = __builtin_amdgcn_readfirstlane((int)(__any(mx * scT > m) != 0));
         asm volatile("" : "+s"(trips));
 #pragma unroll 1
         for (int r = 0; __builtin_expect(r < trips, 0); ++r) {
             float lo, hi;
             LaneSwap32(mx, &lo, &hi);
-            const float to = fmaxf(m, ceilf(fmaxf(lo, hi) * scT)); // (whole: the weights' bits and the factor below do not depend on it)
+            const float to = fmaxf(m, fmaxf(lo, hi) * scT);
             alpha = __builtin_amdgcn_exp2f(m - to);
             m = to;
         }
