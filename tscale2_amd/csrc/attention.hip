@@ -91,14 +91,6 @@ __device__ __forceinline__ v8bf PackB(const float *x, int s)
     return __builtin_bit_cast(v8bf, r);
 }
 
-// acc + the two bf16 values of a word, in fp32
-__device__ __forceinline__ float AddBf16x2(float acc, int word)
-{
-    typedef __bf16 v2bf_t __attribute__((ext_vector_type(2)));
-    const v2bf_t one = {(__bf16)1.f, (__bf16)1.f};
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2bf_t, word), one, acc, false);
-}
-
 // row index inside a 32x32 MFMA result block held in register e by a lane of the given half
 __device__ __forceinline__ int BlkRow(int e, int half)
 {
@@ -583,7 +575,7 @@ __device__ __forceinline__ void ForwardFewTiles(const AttP &p, uint8_t *kT0, uin
 // issues one instruction in five cycles.  So the kernel saves instructions: the exponential's argument is one fused multiply-add of the raw
 // product, the running maximum is taken once per tile of 64 keys, masks are a pass of their own over the tiles that need one.  And it overlaps:
 // S of tile i + 1 is formed between the exponentials of tile i, its maximum between the products with V, operands are requested six products
-// ahead.  16 x 2048 tokens causal, 16 heads: 395 -> 376 us; one sequence of 2048 tokens, one head 54 -> 45.  A reference that lags the maximum
+// ahead.  16 x 2048 tokens causal, 16 heads: 395 -> 371 us; one sequence of 2048 tokens, one head 54 -> 43.  A reference that lags the maximum
 // by up to 2^8 saves most of the rescaling (357, 40), but then the largest weight is rounded like any other: against fp64 0.00221 instead of
 // 0.00220, and 0.0020 instead of 0.0018 on peaked weights.
 template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP p)
@@ -668,7 +660,7 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
     }
     v4i pb[4] = {};
     // the sink: a zero vector with weight 2^-m.  `sum` is the half's own part (the two halves of a row see different keys)
-    float m = 0, sum = half == 0 ? 1.f : 0.f, norm = sum, scT = sc; // norm: the sum of the weights as the products take them, rounded
+    float m = 0, sum = half == 0 ? 1.f : 0.f, scT = sc;
     auto seenAt = [&](int i) {
         const int t = tileKey(i);
         return i < nTiles && !(t > sp.waveMaxFinish || t + TR - 1 < sp.waveMinStart);
@@ -678,7 +670,7 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
     // AHEAD slots on and an eighth of the arithmetic that goes with it.
 #define SCHED_FENCE() __builtin_amdgcn_sched_barrier(0)
     // weights of two keys of a block: 2^(logit - m), rounded into word j of the operand, and their sum
-    float wa = 0, wb = 0, wr = 0;
+    float wa = 0, wb = 0;
     auto weights2 = [&](const v16f &s, v4i *pq, int j) __attribute__((always_inline)) {
         float x0 = s[2 * j], x1 = s[2 * j + 1];
         asm volatile("" : "+v"(x0), "+v"(x1)); // (arithmetic alone is not held by a fence: it stays between these two)
@@ -686,8 +678,7 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
         wa += w0;
         wb += w1;
         int word = (int)PackBf16x2(w0, w1);
-        wr = AddBf16x2(wr, word);
-        asm volatile("" : "+v"(wa), "+v"(wb), "+v"(wr), "+v"(word));
+        asm volatile("" : "+v"(wa), "+v"(wb), "+v"(word));
         pq[j >> 2][j & 3] = word;
     };
     // O^T += V^T P^T of a block of 32 keys (rows from vt on); the caller has requested the first AHEAD operands; `arith` is called in every
@@ -811,7 +802,7 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
 #pragma unroll 1
         for (int r = 0; __builtin_expect(r < hot, 1); ++r) {
             v8bf ft[AHEAD + 1], fu[AHEAD + 1];
-            wa = wb = wr = 0;
+            wa = wb = 0;
             const v16f old = s1;
             product1(
                 kt,
@@ -822,7 +813,6 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
                 },
                 [&](int i) __attribute__((always_inline)) { ft[i] = FragTr(vt, i >> 2, i & 3, fl); });
             sum += wa + wb;
-            norm += wr;
             maskTile(t0);
             float ma = -INFINITY, mb = -INFINITY;
             product2(
@@ -837,13 +827,12 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
                 [&](int i) __attribute__((always_inline)) { fu[i] = FragTr(vt + 32 * ROWB, i >> 2, i & 3, fl); });
             float alpha = 1;
             int moved = moveReference(fmaxf(ma, mb), alpha);
-            wa = wb = wr = 0;
+            wa = wb = 0;
             product2(vt + 32 * ROWB, fu, pb + 2, [&](int i) __attribute__((always_inline)) { weights2(s0, pb, i); }, [](int) {});
             asm volatile("" : "+s"(moved));
 #pragma unroll 1
             for (int q = 0; __builtin_expect(q < moved, 0); ++q) {
                 sum *= alpha;
-                norm *= alpha;
 #pragma unroll
                 for (int db = 0; db < 4; ++db) {
 #pragma unroll
@@ -853,7 +842,6 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
                 }
             }
             sum += wa + wb;
-            norm += wr;
         }
 #pragma unroll 1
         for (int r = 0; __builtin_expect(r < first, 0); ++r) { // the wave's first tile: nothing accumulated yet but the sink
@@ -861,18 +849,17 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
             maskTile(t0);
             float alpha = 1;
             moveReference(tileMax(), alpha);
-            wa = wb = wr = 0;
+            wa = wb = 0;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 weights2(s0, pb, j);
             }
             sum = sum * alpha + (wa + wb);
-            norm = norm * alpha + wr;
         }
 #pragma unroll 1
         for (int r = 0; __builtin_expect(r < last, 0); ++r) { // one round after its last tile
             v8bf ft[AHEAD + 1], fu[AHEAD + 1];
-            wa = wb = wr = 0;
+            wa = wb = 0;
 #pragma unroll
             for (int i = 0; i < AHEAD; ++i) {
                 ft[i] = FragTr(vt, i >> 2, i & 3, fl);
@@ -881,7 +868,6 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
                 vt, ft, pb, [&](int i) __attribute__((always_inline)) { weights2(s1, pb + 2, i); },
                 [&](int i) __attribute__((always_inline)) { fu[i] = FragTr(vt + 32 * ROWB, i >> 2, i & 3, fl); });
             sum += wa + wb;
-            norm += wr;
             product2(vt + 32 * ROWB, fu, pb + 2, [](int) {}, [](int) {});
         }
         seenPrev = seen;
@@ -900,10 +886,8 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
         float lo, hi;
         LaneSwap32(sum, &lo, &hi);
         sum = lo + hi;
-        LaneSwap32(norm, &lo, &hi);
-        norm = lo + hi;
     }
-    StoreOwnRows<false>(p.out0 + (int64_t)(myRow - l32) * p.ldo0, p.ldo0, head * HD, oacc, 1 / norm, l32, half);
+    StoreOwnRows<false>(p.out0 + (int64_t)(myRow - l32) * p.ldo0, p.ldo0, head * HD, oacc, 1 / sum, l32, half);
     if (half == 0) {
         p.sumWeightLog[(int64_t)head * p.ldStat + myRow] = m + log2f(sum);
     }
