@@ -428,7 +428,8 @@ int ts2_att_build_rev(int32_t len, int32_t lenRound, const int32_t *spanStart, c
  * the reference, whose two kernels each evaluate the scores): a block exists for every (32-query block, 32-key block) pair such that
  * the key block lies between the earliest span start and the latest span finish of the query block's rows.  dsBase[q] = number of
  * the first block of q's query block, dsBase[lenRound] = blocks per head; device arrays, spans of lenRound rows (empty: finish <
- * start).  ts2_att_ds_blocks counts the blocks per head on the host from host copies of the same spans (to size the array). */
+ * start).  ts2_att_ds_blocks counts the blocks per head on the host from host copies of the same spans (to size the array).  A block that
+ * no single row of its query block sees (spans of neighbouring rows may leave a gap) has a number, but need not be written and is not read. */
 int ts2_att_build_ds_index(int32_t lenRound, const int32_t *spanStart, const int32_t *spanFinish, int32_t *dsBase, void *stream);
 int64_t ts2_att_ds_blocks(int32_t lenRound, const int32_t *spanStartHost, const int32_t *spanFinishHost);
 

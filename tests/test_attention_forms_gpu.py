@@ -142,3 +142,44 @@ def test_zero_scale_and_masked_rows(L, heads):
     want = (v[np.maximum(finish[:n], -1) + 1] - v[np.where(count > 0, start[:n], finish[:n] + 1)]) / (1 + count)[:, None]
     got = out[0].float().cpu().numpy()[:n]
     assert np.abs(got - want).max() <= 2.0 ** -8 * np.abs(want).max() + 1e-3
+
+
+def spans_with_gaps(n):
+    """one key range per row, with 32-key blocks between the ranges of neighbouring rows that none of them sees: the rest of a 64-key tile, and
+    whole 128-key blocks that no query reaches at all (256..383); rows without a span"""
+    start, finish, t = np.zeros(n, np.int32), np.full(n, -1, np.int32), np.arange(n) % 64
+    for lo, hi, a, b in ((0, 16, 0, 10), (16, 28, 64, 95), (32, 50, 3, 40), (50, 60, 400, 450), (60, 64, 130, 131)):
+        start[(t >= lo) & (t < hi)], finish[(t >= lo) & (t < hi)] = a, b
+    return start, finish
+
+
+@pytest.mark.parametrize("heads", [1, 32])
+@pytest.mark.parametrize("f32", [False, True])
+def test_handed_over_score_gradients_of_spans_with_gaps(L, heads, f32):
+    """one launch (1 head) and two (32): a block of score gradients that no row sees is not written, and must not be read.  dK and dV are the
+    very same values with and without the hand-over; dQ is formed from dS rounded to bf16 in either case (2^-9 of every term, of which few
+    dozen are added: far below 4e-3 of the largest)"""
+    print("case att gaps", heads, f32, flush=True)
+    n = 512
+    start, finish = spans_with_gaps(n)
+    i16 = torch.int16
+    q, k, v, dval = [torch.from_numpy(x).cuda().bfloat16().view(i16) for x in inputs(n, heads, seed=3)]
+    ts, tf = torch.from_numpy(start).cuda(), torch.from_numpy(finish).cuda()
+    val, swl = torch.zeros((n, heads * 128), dtype=i16, device="cuda"), torch.zeros((heads, n), device="cuda")
+    L.att_forward(n, heads, q, k, v, ts, tf, SCALE, 0.0, val, swl)
+    lo = torch.zeros(n // 128, dtype=torch.int32, device="cuda")
+    hi = torch.zeros_like(lo)
+    L.call("ts2_att_build_rev", n, n, ts, tf, lo, hi)
+    ds = torch.from_numpy(np.random.default_rng(4).standard_normal((heads, n)).astype(np.float32) * 0.1).cuda()
+    handed = L.att_ds_scratch(n, heads, ts, tf)
+    handed[1].fill_(0x7f)  # NaN patterns where nothing is written
+    out = []
+    for pair in (None, handed):
+        o = [torch.full((n, heads * 128), 3.0, dtype=torch.float32 if f32 else torch.bfloat16, device="cuda") for _ in range(3)]
+        L.att_backward(n, heads, q, k, v, dval, ts, tf, lo, hi, SCALE, 0.0, swl, ds, *[t if f32 else t.view(i16) for t in o], L.F32 if f32 else L.BF16,
+                       ds=pair)
+        out.append(o)
+    torch.cuda.synchronize()
+    assert torch.equal(out[0][1], out[1][1]) and torch.equal(out[0][2], out[1][2])
+    a, b = out[0][0].float(), out[1][0].float()
+    assert (a - b).abs().max() <= 4e-3 * a.abs().max()

@@ -2267,7 +2267,8 @@ template <bool F32> __global__ void __launch_bounds__(256, 3) AttGradQFromDs(Att
         for (int kb = 0; kb < TR / 32; ++kb) {
             const int k0 = t0 + kb * 32;
             const uint8_t *kt2 = kt + kb * 32 * ROWB;
-            int trips = __builtin_amdgcn_readfirstlane((int)!(k0 > sp.waveMaxFinish || k0 + 31 < sp.waveMinStart)); // (see AttGradQ)
+            // a block that no row of the wave sees need not have been written, also where it lies between their spans
+            int trips = __builtin_amdgcn_readfirstlane((int)(__any(finish >= k0 && sp.start <= k0 + 31) != 0)); // (see AttGradQ)
             asm volatile("" : "+s"(trips));
 #pragma unroll 1
             for (int trip = 0; trip < trips; ++trip) {
