@@ -7,7 +7,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
-from model_harness import E4M3, Harness  # noqa: E402
+from model_harness import E4M3, I8, Harness  # noqa: E402
 from test_model_batches_gpu import batch, load  # noqa: E402
 
 
@@ -41,3 +41,28 @@ def test_probabilities_follow_the_bias(vocab):
     grad[rows, tokens[rows + 1]] += 1
     grad[~has] = 0
     assert (np.abs(g - grad) <= 2.0 ** -8 * np.abs(grad) + 1e-30).all()
+
+
+@pytest.mark.parametrize("vocab", [128, 53248, 53376])
+@pytest.mark.parametrize("big", [60.0, 70.0, 300.0, 1e5])
+def test_large_bias(vocab, big):
+    """two entries whose bias stands far above the logits (all below 1 in size) share the probability as 2 to 1.  In fp32 a sum of
+    about 1e5 is rounded by up to 2^-8 (of about 300 by 2^-16): two of them, ln 2 / 3 of which reaches the probability, are 1.8e-3 < 2^-9"""
+    print("case large bias", vocab, big, flush=True)
+    h = Harness(I8, dim=256, heads=1, ffn_tiles=1, depth=2, vocab=vocab, frag_count=2, frag_len=64, wide_window=64, seed=7)
+    bias = np.zeros(vocab, np.float32)
+    bias[5], bias[vocab - 1] = big, big - 1
+    m = load(h, 67)
+    try:
+        n = batch(m, h, np.random.default_rng(vocab).integers(0, vocab, 67), 50)
+        p = []
+        for b in (np.zeros(vocab, np.float32), bias):
+            m.set_bias(b)
+            m.forward()
+            torch.cuda.synchronize()
+            p.append(m.array("prediction")[:n, :vocab].double().cpu().numpy())
+    finally:
+        m.close()
+    a, b = p[0][:, 5] * 2, p[0][:, vocab - 1]
+    np.testing.assert_allclose(p[1][:, 5], a / (a + b), rtol=2 ** -9 if big > 1e4 else 2 ** -15)
+    np.testing.assert_allclose(p[1].sum(1), 1, rtol=1e-6)

@@ -168,7 +168,8 @@ __global__ void __launch_bounds__(256) FinalProbabilitiesTwoPass(int vocab, floa
             *(uint2 *)(grow + k) = make_uint2(0, 0);
         }
     }
-    // lane-local running maximum m (of the logits without bias, never below 0) and sum of 2^(x + bias - m)
+    // lane-local reference m (the running maximum of the logits with their bias where it exceeds 64, which leaves room for the sum, else 0) and
+    // sum of 2^(x + bias - m)
     float m = 0, sum = 0;
     for (int k0 = tid * 4; k0 < vocab; k0 += 4096) {
         float4 x[4], bv[4];
@@ -182,13 +183,16 @@ __global__ void __launch_bounds__(256) FinalProbabilitiesTwoPass(int vocab, floa
         float mNew = m;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
+            x[i] = make_float4(x[i].x + bv[i].x, x[i].y + bv[i].y, x[i].z + bv[i].z, x[i].w + bv[i].w);
             mNew = fmaxf(mNew, fmaxf(fmaxf(x[i].x, x[i].y), fmaxf(x[i].z, x[i].w)));
         }
-        sum *= exp2f(m - mNew);
-        m = mNew;
+        if (mNew > 64) {
+            sum *= exp2f(m - mNew);
+            m = mNew;
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            sum += (exp2f(x[i].x + bv[i].x - m) + exp2f(x[i].y + bv[i].y - m)) + (exp2f(x[i].z + bv[i].z - m) + exp2f(x[i].w + bv[i].w - m));
+            sum += (exp2f(x[i].x - m) + exp2f(x[i].y - m)) + (exp2f(x[i].z - m) + exp2f(x[i].w - m));
         }
     }
     float mx = WaveMax(m);
