@@ -64,18 +64,18 @@ __global__ void __launch_bounds__(256) EmbedBackward(int len, int dim, const int
     }
 }
 
-// SoftMax base 2 with running max starting at 0 and the (onehot - p) gradient (src/gpt/compute/cpu_transformer.cpp:12-37,146-159).
+// SoftMax base 2 and its (onehot - p) gradient (src/gpt/compute/cpu_transformer.cpp:12-37,146-159).
 // logits fp32 [row][vocab] are overwritten by probabilities, grad is bf16, zero in rows without a target; vocab is a multiple of 4.
 //
 // Bounded by HBM: a row is read once and held in registers, NCH chunks of four per lane, by W waves (one wave and no barrier for small
-// vocabularies, up to sixteen for large ones); one exponential and six other instructions per logit.  Against two passes by a workgroup of
-// four waves: 4096 x 1024 14.3 -> 9.2 us, x 8192 67 -> 54, x 16384 169 -> 113 (671 MB: 108 at the rate of a copy), 777 x 50304 133 -> 107
-// (three rounds of one workgroup per CU; twice the registers per lane and two workgroups to a CU spilled: 145).
+// vocabularies, up to sixteen for large ones); one exponential and seven other instructions per logit.  Against two passes by a workgroup
+// of four waves, repeated on one batch: 4096 x 1024 12.2 -> 7.3 us, x 8192 67 -> 51, x 16384 165 -> 140, 777 x 50304 91 -> 81 (one
+// workgroup per CU: four rounds, the last of nine rows; twice the registers per lane and two workgroups to a CU spilled).
 template <int W, int NCH>
 __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W, 4) FinalProbabilities(int rows, int vocab, float *logits, int64_t ldLogits,
     const float *bias, const int *target, float gradMult, bf16_t *grad, int64_t ldGrad)
 {
-    __shared__ float redM[W], redS[W];
+    __shared__ float redM[W], redL[W], redS[W];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int t = W == 1 ? blockIdx.x * 4 + wave : blockIdx.x, first = W == 1 ? lane : threadIdx.x;
     if (t >= rows) { // (one wave per row: a whole wave, and no barrier below)
@@ -85,7 +85,7 @@ __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W, 4) FinalProbabilities(i
     bf16_t *grow = (bf16_t *)((uint8_t *)grad + (int64_t)t * ldGrad);
     const int tg = target[t];
     float4 x[NCH];
-    float m = -1e30f; // the row's largest logit with its bias
+    float m = -1e30f, least = 1e30f; // the row's largest and smallest logit with their bias
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
         const int k = (i * 64 * W + first) * 4;
@@ -97,28 +97,48 @@ __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W, 4) FinalProbabilities(i
         if (k < vocab) {
             const float4 b = *(const float4 *)(bias + k);
             x[i] = make_float4(x[i].x + b.x, x[i].y + b.y, x[i].z + b.z, x[i].w + b.w);
+            least = fminf(least, fminf(fminf(x[i].x, x[i].y), fminf(x[i].z, x[i].w)));
         }
         m = fmaxf(m, fmaxf(fmaxf(x[i].x, x[i].y), fmaxf(x[i].z, x[i].w)));
     }
     m = WaveMax(m);
+    least = -WaveMax(-least);
     if (W > 1) {
         if (lane == 0) {
             redM[wave] = m;
+            redL[wave] = least;
         }
         __syncthreads();
 #pragma unroll
         for (int w = 0; w < W; ++w) {
             m = fmaxf(m, redM[w]);
+            least = fminf(least, redL[w]);
         }
     }
-    // weights in units of 2^-64: the hardware's exponential returns zero below 2^-126, which then is 2^-190 of the largest weight
-    m -= 64;
+    // A logit is the exponential's argument as it is while the largest leaves room for the sum, and relative to the largest otherwise: a
+    // subtraction rounds (relative to 64 below the largest, rms error of a probability 7.6e-7 instead of 6e-8).  The hardware's exponential
+    // returns zero below 2^-126; a row that reaches there takes exp2f, which goes on to 2^-149 at five instructions more.
+    m = fabsf(m) <= 64 ? 0.f : m;
     float sum = 0;
+    int plain = __builtin_amdgcn_readfirstlane((int)(least - m >= -125)), wide = plain ^ 1;
+    // loops of one trip or none, not branches: a join would cost registers
+    asm volatile("" : "+s"(plain), "+s"(wide));
+#pragma unroll 1
+    for (int r = 0; r < plain; ++r) {
 #pragma unroll
-    for (int i = 0; i < NCH; ++i) { // (chunks beyond the vocabulary hold -1e30: weight zero)
-        x[i] = make_float4(__builtin_amdgcn_exp2f(x[i].x - m), __builtin_amdgcn_exp2f(x[i].y - m), __builtin_amdgcn_exp2f(x[i].z - m),
-            __builtin_amdgcn_exp2f(x[i].w - m));
-        sum += (x[i].x + x[i].y) + (x[i].z + x[i].w);
+        for (int i = 0; i < NCH; ++i) { // (chunks beyond the vocabulary hold -1e30: weight zero)
+            x[i] = make_float4(__builtin_amdgcn_exp2f(x[i].x - m), __builtin_amdgcn_exp2f(x[i].y - m), __builtin_amdgcn_exp2f(x[i].z - m),
+                __builtin_amdgcn_exp2f(x[i].w - m));
+            sum += (x[i].x + x[i].y) + (x[i].z + x[i].w);
+        }
+    }
+#pragma unroll 1
+    for (int r = 0; __builtin_expect(r < wide, 0); ++r) {
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) {
+            x[i] = make_float4(exp2f(x[i].x - m), exp2f(x[i].y - m), exp2f(x[i].z - m), exp2f(x[i].w - m));
+            sum += (x[i].x + x[i].y) + (x[i].z + x[i].w);
+        }
     }
     sum = WaveSum(sum);
     if (W > 1) {
