@@ -106,3 +106,25 @@ def test_probabilities_against_float64(vocab, spread):
     print("  rms", np.sqrt((rel ** 2).mean()) / u, "u, max", rel.max() / u, "u, of the bound", np.sqrt(((rel / (4 * u + unit[some])) ** 2).mean()), flush=True)
     assert np.sqrt(((rel / (4 * u + unit[some])) ** 2).mean()) <= 1
     assert (rel <= 44 * u + unit[some]).all()
+
+
+@pytest.mark.parametrize("vocab", [128, 2048, 8192, 53248, 53376])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_rows_without_a_target_have_no_gradient(vocab, bad):
+    """one logit that is not finite makes its rows' probabilities NaN; the gradient of a row without a target is zero all the same"""
+    print("case rows without a target", vocab, bad, flush=True)
+    h = Harness(I8, dim=256, heads=1, ffn_tiles=1, depth=2, vocab=vocab, frag_count=2, frag_len=64, wide_window=64, seed=7)
+    bias = np.zeros(vocab, np.float32)
+    bias[5] = bad
+    m = load(h, 67)
+    try:
+        n = batch(m, h, np.random.default_rng(vocab).integers(0, vocab, 67), 50)
+        m.set_bias(bias)
+        m.forward()
+        torch.cuda.synchronize()
+        p = m.array("prediction")[:n, :vocab].float().cpu().numpy()
+        g = m.array("finalGrad")[:n, :vocab].float().cpu().numpy()
+    finally:
+        m.close()
+    none = np.array([t % 50 == 49 or t == n - 1 for t in range(n)])
+    assert (g[none] == 0).all() and np.isnan(p).all() and np.isnan(g[~none]).all()

@@ -152,7 +152,8 @@ __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W, 4) FinalProbabilities(i
             sum += redS[w];
         }
     }
-    const float scale = 1 / sum, neg = tg < 0 ? 0.f : -gradMult;
+    const float scale = 1 / sum, neg = -gradMult;
+    const uint32_t live = tg < 0 ? 0u : ~0u; // (zero in a row without a target, whatever its probabilities are)
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
         const int k = (i * 64 * W + first) * 4;
@@ -166,7 +167,7 @@ __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W, 4) FinalProbabilities(i
                     g[e] = e == tg - k ? (1 - p[e]) * gradMult : g[e];
                 }
             }
-            *(uint2 *)(grow + k) = make_uint2(PackBf16x2(g[0], g[1]), PackBf16x2(g[2], g[3]));
+            *(uint2 *)(grow + k) = make_uint2(PackBf16x2(g[0], g[1]) & live, PackBf16x2(g[2], g[3]) & live);
         }
     }
 }
