@@ -144,6 +144,30 @@ def test_zero_scale_and_masked_rows(L, heads):
     assert np.abs(got - want).max() <= 2.0 ** -8 * np.abs(want).max() + 1e-3
 
 
+@pytest.mark.parametrize("docs,window,heads", [([608, 1000], 4096, 2), ([608, 1000], 500, 1), ([1600], 333, 1), ([1600], 40, 1)])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_values_that_no_row_of_a_wave_sees_need_not_be_finite(L, docs, window, heads, bad):
+    """a value row that is not finite reaches the 32-row blocks some row of which has a key range over its block of 32 keys, and no others:
+    those have the very bits they have without it.  Key ranges over and under five tiles of 64 keys, documents that start inside a tile"""
+    print("case att values not finite", docs, window, bad, flush=True)
+    sp, spans = ragged_spans(docs, window)
+    n = sp.size - 1
+    n_round = (n + 127) // 128 * 128
+    start, finish = spans_to_ranges(sp, spans, n, n_round)
+    a = inputs(n, heads, seed=11)
+    clean, _ = device_pass(L, n, heads, a, start, finish, 0.0)
+    lo = np.where(finish >= start, start, 1 << 30).reshape(-1, 32).min(1)
+    hi = np.where(finish >= start, finish, -1).reshape(-1, 32).max(1)
+    for row in (100, 544, 575, 576, 607, 608, 640, 1200, 1300, n - 1):
+        b = [x.copy() for x in a]
+        b[2][row] = bad
+        got, _ = device_pass(L, n, heads, b, start, finish, 0.0)
+        k = row // 32 * 32
+        good = torch.from_numpy(np.repeat((lo > k + 31) | (hi < k), 32)).cuda()
+        assert good.any() and not good.all()
+        assert torch.equal(got[0][good], clean[0][good]), row
+
+
 def spans_with_gaps(n):
     """one key range per row, with 32-key blocks between the ranges of neighbouring rows that none of them sees: the rest of a 64-key tile, and
     whole 128-key blocks that no query reaches at all (256..383); rows without a span"""

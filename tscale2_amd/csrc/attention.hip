@@ -775,7 +775,7 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
         }
         return trips;
     };
-    bool seenPrev = false;
+    bool seenPrev = false, allPrev = false; // does the wave see tile i - 1, and both of its halves
     // round i: S of tile i, O += P V of tile i - 1.  K of tile i lies in buffer PAR = i % 2, V of tile i - 1 in the other one
     auto round = [&](auto parTag, int i) __attribute__((always_inline)) {
         constexpr int PAR = decltype(parTag)::value;
@@ -795,10 +795,11 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
             requestV(i, PAR);
         }
         const int t0 = tileKey(i);
+        // A half of a tile that no row of the wave sees (only its first and its last tile have one) stays out of the product with V: its
+        // weights are zero, but what V holds there need not be finite.  Tile i - 1 is then finished by itself, before tile i.
         const bool seen = seenAt(i);
-        int hot = __builtin_amdgcn_readfirstlane((int)(seen && seenPrev)), first = __builtin_amdgcn_readfirstlane((int)(seen && !seenPrev)),
-            last = __builtin_amdgcn_readfirstlane((int)(!seen && seenPrev));
-        asm volatile("" : "+s"(hot), "+s"(first), "+s"(last));
+        int hot = __builtin_amdgcn_readfirstlane((int)(seen && allPrev)), edge = __builtin_amdgcn_readfirstlane((int)((seen || seenPrev) && !(seen && allPrev)));
+        asm volatile("" : "+s"(hot), "+s"(edge));
 #pragma unroll 1
         for (int r = 0; __builtin_expect(r < hot, 1); ++r) {
             v8bf ft[AHEAD + 1], fu[AHEAD + 1];
@@ -844,32 +845,68 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
             sum += wa + wb;
         }
 #pragma unroll 1
-        for (int r = 0; __builtin_expect(r < first, 0); ++r) { // the wave's first tile: nothing accumulated yet but the sink
-            product1(kt, [](int) {}, [](int) {});
-            maskTile(t0);
-            float alpha = 1;
-            moveReference(tileMax(), alpha);
-            wa = wb = 0;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                weights2(s0, pb, j);
-            }
-            sum = sum * alpha + (wa + wb);
-        }
+        for (int r = 0; __builtin_expect(r < edge, 0); ++r) {
+            const int tp = t0 - TR;
+            const bool lo = seenPrev && tp + 31 >= sp.waveMinStart, hi = seenPrev && tp + 32 <= sp.waveMaxFinish;
+            int first = __builtin_amdgcn_readfirstlane((int)seen), lastLo = __builtin_amdgcn_readfirstlane((int)lo),
+                lastHi = __builtin_amdgcn_readfirstlane((int)hi), onlyHi = __builtin_amdgcn_readfirstlane((int)(hi && !lo));
+            asm volatile("" : "+s"(first), "+s"(lastLo), "+s"(lastHi), "+s"(onlyHi));
 #pragma unroll 1
-        for (int r = 0; __builtin_expect(r < last, 0); ++r) { // one round after its last tile
-            v8bf ft[AHEAD + 1], fu[AHEAD + 1];
-            wa = wb = 0;
+            for (int r = 0; __builtin_expect(r < lastLo, 0); ++r) { // tile i - 1 by itself: its first 32 keys and the weights of the others
+                v8bf ft[AHEAD + 1];
+                wa = wb = 0;
 #pragma unroll
-            for (int i = 0; i < AHEAD; ++i) {
-                ft[i] = FragTr(vt, i >> 2, i & 3, fl);
+                for (int i = 0; i < AHEAD; ++i) {
+                    ft[i] = FragTr(vt, i >> 2, i & 3, fl);
+                }
+                product2(vt, ft, pb, [&](int i) __attribute__((always_inline)) { weights2(s1, pb + 2, i); }, [](int) {});
+                sum += wa + wb;
             }
-            product2(
-                vt, ft, pb, [&](int i) __attribute__((always_inline)) { weights2(s1, pb + 2, i); },
-                [&](int i) __attribute__((always_inline)) { fu[i] = FragTr(vt + 32 * ROWB, i >> 2, i & 3, fl); });
-            sum += wa + wb;
-            product2(vt + 32 * ROWB, fu, pb + 2, [](int) {}, [](int) {});
+#pragma unroll 1
+            for (int r = 0; __builtin_expect(r < onlyHi, 0); ++r) {
+                wa = wb = 0;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    weights2(s1, pb + 2, j);
+                }
+                sum += wa + wb;
+            }
+#pragma unroll 1
+            for (int r = 0; __builtin_expect(r < lastHi, 0); ++r) { // ... and the product with the others
+                v8bf ft[AHEAD + 1];
+#pragma unroll
+                for (int i = 0; i < AHEAD; ++i) {
+                    ft[i] = FragTr(vt + 32 * ROWB, i >> 2, i & 3, fl);
+                }
+                product2(vt + 32 * ROWB, ft, pb + 2, [](int) {}, [](int) {});
+            }
+#pragma unroll 1
+            for (int r = 0; __builtin_expect(r < first, 0); ++r) { // the wave's first tile, or the one after a tile that was finished by itself
+                product1(kt, [](int) {}, [](int) {});
+                maskTile(t0);
+                float alpha = 1;
+                int moved = moveReference(tileMax(), alpha);
+                asm volatile("" : "+s"(moved));
+#pragma unroll 1
+                for (int q = 0; __builtin_expect(q < moved, 0); ++q) {
+                    sum *= alpha;
+#pragma unroll
+                    for (int db = 0; db < 4; ++db) {
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) {
+                            oacc[db][e] *= alpha;
+                        }
+                    }
+                }
+                wa = wb = 0;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    weights2(s0, pb, j);
+                }
+                sum += wa + wb;
+            }
         }
+        allPrev = seen && t0 + 31 >= sp.waveMinStart && t0 + 32 <= sp.waveMaxFinish;
         seenPrev = seen;
     };
     for (int i = 0;;) {
