@@ -148,7 +148,7 @@ def test_zero_scale_and_masked_rows(L, heads):
 @pytest.mark.parametrize("bad", [np.inf, np.nan])
 def test_values_that_no_row_of_a_wave_sees_need_not_be_finite(L, docs, window, heads, bad):
     """a value row that is not finite reaches the 32-row blocks some row of which has a key range over its block of 32 keys, and no others:
-    those have the very bits they have without it.  Key ranges over and under five tiles of 64 keys, documents that start inside a tile"""
+    those have the very bits they have without it.  Key ranges over and under seven tiles of 64 keys, documents that start inside a tile"""
     print("case att values not finite", docs, window, bad, flush=True)
     sp, spans = ragged_spans(docs, window)
     n = sp.size - 1

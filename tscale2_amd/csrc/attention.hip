@@ -412,7 +412,9 @@ __device__ __forceinline__ void WaveKeyRange(const int *spanStart, const int *sp
 
 // A workgroup whose keys fit a few tiles (narrow windows): one 32-key block after the other, skipped where the wave sees none of it, with the
 // exact running maximum.  The pipelined form below needs a barrier more and works on 64 keys at a time: 22.5 against 25 us for 16800 tokens,
-// 4 heads, 64-token windows over documents of unequal length.
+// 4 heads, 64-token windows over documents of unequal length.  Up to seven tiles (FEW below): 16 documents of 512 tokens, 7 heads, 200-token
+// windows 21.8 against 23.3 us; the rows of a 512-token sequence that see eight are faster the other way (8 sequences, 4 heads: 15.6, 17.3).
+// The key range is found by every wave for itself, without LDS and a barrier: 64-token windows 22.9 -> 22.1.
 template <bool ALIBI>
 __device__ __forceinline__ void ForwardFewTiles(const AttP &p, uint8_t *kT0, uint8_t *kT1, uint8_t *vT0, uint8_t *vT1, const uint8_t *gk, const uint8_t *gv,
     int tFirst, int kHi, int wave, int myRow, int l32, int half, int lane, int64_t hoff, int start, int finish, v16f (&oacc)[4], float &m, float &sum)
@@ -581,10 +583,9 @@ __device__ __forceinline__ void ForwardFewTiles(const AttP &p, uint8_t *kT0, uin
 template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP p)
 {
     constexpr int QB = 4;  // query blocks of the workgroup; as many waves stream its tiles
-    constexpr int FEW = 5; // key tiles up to which ForwardFewTiles is the faster one
+    constexpr int FEW = 7; // key tiles up to which ForwardFewTiles is the faster one
     // K and V of the even tiles, of the odd ones
     __shared__ __attribute__((aligned(1024))) uint8_t kT0[TILE_BYTES], kT1[TILE_BYTES], vT0[TILE_BYTES], vT1[TILE_BYTES];
-    __shared__ int red[8];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, half = lane >> 5;
     int blk, head;
     MapAttBlock(&blk, &head);
@@ -593,9 +594,7 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
     const int64_t hoff = (int64_t)head * HD * 2;
     const int start = p.spanStart[myRow], finish = p.spanFinish[myRow];
     int kLo, kHi;
-    BlockKeyRange(start, finish, tid, &kLo, &kHi, red);
-    kLo = __builtin_amdgcn_readfirstlane(kLo);
-    kHi = __builtin_amdgcn_readfirstlane(kHi);
+    WaveKeyRange<BROWS>(p.spanStart, p.spanFinish, row0, lane, &kLo, &kHi);
     const int tile0 = kHi >= kLo ? kLo / TR : 0, nTiles = kHi >= kLo ? kHi / TR - tile0 + 1 : 0;
     const uint8_t *gk = p.k + hoff, *gv = p.v + hoff;
     v16f oacc[4];
