@@ -2396,10 +2396,12 @@ bool ActOk(const ts2_mat *m, int rows, int cols)
 
 // The backward as one launch (AttGradSmall) while all of its workgroups are on the chip at once: dK/dV workgroups of 64 keys and dQ
 // workgroups of 128 queries, one to a CU.  2048 tokens, one head 118 -> 45 us; 512-token documents x 4, 4 heads (192 workgroups) 38.0 -> 20.0,
-// with 64-token windows 19.5 -> 13.7; beyond 256 workgroups (that with 6 heads, 288) 39.4 against 34.0 but 20.8 against 23.6 in narrow windows.
-bool OneLaunch(int lenRound, int heads)
+// with 64-token windows 19.4 -> 13.7; beyond 256 workgroups (that with 6 heads, 288) 39.4 against 34.0 but 20.8 against 23.6 in narrow windows:
+// the spans are not known here.  A call for one of the two keeps the kernels below, which are shorter in narrow windows (dQ alone 9.6 us,
+// not 13.0; dK/dV alone 7.7, not 8.9, on 128 tokens).
+bool OneLaunch(int which, int lenRound, int heads)
 {
-    return (int64_t)(lenRound / KVROWS + lenRound / BROWS) * heads <= 256;
+    return which == 3 && (int64_t)(lenRound / KVROWS + lenRound / BROWS) * heads <= 256;
 }
 
 } // namespace
@@ -2535,24 +2537,22 @@ extern "C" int ts2_att_backward(const ts2_att_grad_args *a, void *stream)
         p.ds = (uint8_t *)a->dsScratch;
         p.dsCap = a->dsCapacityBlocks;
     }
-    if (OneLaunch(a->lenRound, a->heads)) {
+    if (OneLaunch(a->which, a->lenRound, a->heads)) {
         p.out0 = (uint8_t *)a->dK.ptr;
         p.ldo0 = a->dK.strideBytes;
         p.out1 = (uint8_t *)a->dV.ptr;
         p.ldo1 = a->dV.strideBytes;
         p.out2 = (uint8_t *)a->dQ.ptr;
         p.ldo2 = a->dQ.strideBytes;
-        const int nKv = (a->which & 2) ? a->lenRound / 64 : 0, nQ = (a->which & 1) && !viaDs ? a->lenRound / BROWS : 0;
-        if (a->which & 3) {
-            auto kernel = f32 ? (alibi ? AttGradSmall<true, true, false> : AttGradSmall<true, false, false>)
-                              : (alibi ? AttGradSmall<false, true, false> : AttGradSmall<false, false, false>);
-            if (viaDs) {
-                kernel = f32 ? (alibi ? AttGradSmall<true, true, true> : AttGradSmall<true, false, true>)
-                             : (alibi ? AttGradSmall<false, true, true> : AttGradSmall<false, false, true>);
-            }
-            hipLaunchKernelGGL(kernel, dim3((nKv + nQ) * a->heads), dim3(512), 0, (hipStream_t)stream, p, nKv, nQ, a->heads);
-            TS2_CHECK_LAUNCH();
+        const int nKv = a->lenRound / KVROWS, nQ = viaDs ? 0 : a->lenRound / BROWS;
+        auto kernel = f32 ? (alibi ? AttGradSmall<true, true, false> : AttGradSmall<true, false, false>)
+                          : (alibi ? AttGradSmall<false, true, false> : AttGradSmall<false, false, false>);
+        if (viaDs) {
+            kernel = f32 ? (alibi ? AttGradSmall<true, true, true> : AttGradSmall<true, false, true>)
+                         : (alibi ? AttGradSmall<false, true, true> : AttGradSmall<false, false, true>);
         }
+        hipLaunchKernelGGL(kernel, dim3((nKv + nQ) * a->heads), dim3(512), 0, (hipStream_t)stream, p, nKv, nQ, a->heads);
+        TS2_CHECK_LAUNCH();
     } else {
         if ((a->which & 1) && !viaDs) {
             p.out0 = (uint8_t *)a->dQ.ptr;
