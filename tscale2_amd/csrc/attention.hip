@@ -1860,7 +1860,7 @@ constexpr int KV_GROUP = KV_STAT + BSTAT_SLOTS * BSTAT_BYTES;             // LDS
 constexpr int KV_P = 2 * KV_GROUP, KV_P_SLOT = 4096;                      // [pair of waves][slot][quarter][lane][4 values]
 constexpr int KV_LDS = KV_P + 4 * 2 * KV_P_SLOT;
 
-template <bool F32, bool ALIBI, bool DS, int ROLE> __device__ __forceinline__ void GradKVSplit(const AttP &p, uint8_t *lds, int blk, int head)
+template <bool F32, bool ALIBI, int ROLE> __device__ __forceinline__ void GradKVSplit(const AttP &p, uint8_t *lds, int blk, int head)
 {
     constexpr int KS = 2, NST = KV_STAGES, KB = 4 / KS, GW = 2 * KB; // key blocks of the workgroup; waves that share a group's tiles
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, half = lane >> 5;
@@ -2102,46 +2102,6 @@ template <bool F32, bool ALIBI, bool DS, int ROLE> __device__ __forceinline__ vo
                 asm volatile("" : "+v"(word));
                 b[j >> 2][j & 3] = word;
             };
-            // The block of dS goes to the dQ kernel, transposed on the way.  Here a lane is a key and its registers walk over the queries; the
-            // dQ kernel's lanes are queries.  The operand pair the wave is about to multiply with, taken as the A operand of two more MFMAs
-            // against the matching slices of the identity, comes back as dS^T with lane = query, registers = keys in the order of the other
-            // kernel's operand fetches (exact: every sum has one term, and the values are bf16 already).  Block number first(query block) +
-            // (this key block - first key block the query block sees); a lane's two operands of 16 bytes sit at lane * 16 and
-            // 1024 + lane * 16: a wave writes, and the dQ kernel's wave reads, 1 KB contiguous per instruction.
-            auto giveDs = [&]() __attribute__((always_inline)) {
-                if constexpr (DS) {
-                    const int s = *(const __attribute__((address_space(3))) int *)(statB + (i & (BSTAT_SLOTS - 1)) * BSTAT_BYTES + 2 * BT * 4 + l32 * 4);
-                    const int f = *(const __attribute__((address_space(3))) int *)(statB + (i & (BSTAT_SLOTS - 1)) * BSTAT_BYTES + 3 * BT * 4 + l32 * 4);
-                    const int startMin = __builtin_amdgcn_readfirstlane(WaveMinInt(f >= s ? s : 0x7fffffff));
-                    const int64_t id = (int64_t)head * p.dsBase[p.lenRound] + p.dsBase[query0 + i * (KS * BT)] + ((key0 >> 5) - (startMin >> 5));
-                    v16f tr;
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        tr[e] = 0;
-                    }
-#pragma unroll
-                    for (int sl = 0; sl < 2; ++sl) {
-                        v4i r;
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            // slot j of operand sl in a lane of half h stands for query 16 sl + (j >> 2) * 8 + 4 h + (j & 3)
-                            const int qa = 16 * sl + ((2 * q) >> 2) * 8 + 4 * half + ((2 * q) & 3), qb2 = qa + 1;
-                            r[q] = (qa == l32 ? 0x3f80 : 0) | (qb2 == l32 ? 0x3f800000 : 0);
-                        }
-                        tr = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, b[sl]), __builtin_bit_cast(v8bf, r), tr, 0, 0, 0);
-                    }
-                    float tv[16];
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        tv[e] = tr[e];
-                    }
-                    if (id >= 0 && id < p.dsCap) {
-                        uint8_t *dst16 = p.ds + id * DS_BLOCK_BYTES + lane * 16;
-                        *(v8bf *)dst16 = PackB(tv, 0);
-                        *(v8bf *)(dst16 + 1024) = PackB(tv, 1);
-                    }
-                }
-            };
 #pragma unroll 1
             for (int r = 0; __builtin_expect(r < hot, 1); ++r) {
                 TOperands fa, fc;
@@ -2156,7 +2116,6 @@ template <bool F32, bool ALIBI, bool DS, int ROLE> __device__ __forceinline__ vo
                 RowProduct(n, rows, fa, own, fl, [&](int j) __attribute__((always_inline)) { gradient2(j); },
                     [&](int k) __attribute__((always_inline)) { fc[k] = FragTr(cols, k >> 2, k & 3, fl); });
                 nxt = n;
-                giveDs();
                 TransposedProduct(acc, cols, fc, b, fl, [&](int j) __attribute__((always_inline)) { if (j == 4) { stats(i + 1, 1, st); } }, none);
             }
 #pragma unroll 1
@@ -2181,7 +2140,6 @@ template <bool F32, bool ALIBI, bool DS, int ROLE> __device__ __forceinline__ vo
                 for (int j = 0; j < 8; ++j) {
                     gradient2(j);
                 }
-                giveDs();
                 TransposedProduct(acc, cols, fc, b, fl, none, none);
             }
         }
@@ -2214,15 +2172,15 @@ template <bool F32, bool ALIBI, bool DS, int ROLE> __device__ __forceinline__ vo
 }
 
 // The backward of a launch that cannot fill the chip: dK/dV workgroups (64 keys) and dQ workgroups (128 queries) side by side in one grid
-template <bool F32, bool ALIBI, bool DS> __global__ void __launch_bounds__(512, 2) AttGradSmall(AttP p, int nKv, int nQ, int heads)
+template <bool F32, bool ALIBI> __global__ void __launch_bounds__(512, 2) AttGradSmall(AttP p, int nKv, int nQ, int heads)
 {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[KV_LDS > 2 * BSTAGES * BSTAGE ? KV_LDS : 2 * BSTAGES * BSTAGE];
     int id = blockIdx.x;
     if (id < nKv * heads) {
         if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 8)) { // waves 4..7, one beside each dV wave on its SIMD
-            GradKVSplit<F32, ALIBI, DS, 1>(p, lds, id % nKv, id / nKv);
+            GradKVSplit<F32, ALIBI, 1>(p, lds, id % nKv, id / nKv);
         } else {
-            GradKVSplit<F32, ALIBI, DS, 0>(p, lds, id % nKv, id / nKv);
+            GradKVSplit<F32, ALIBI, 0>(p, lds, id % nKv, id / nKv);
         }
     } else {
         id -= nKv * heads;
@@ -2527,7 +2485,9 @@ extern "C" int ts2_att_backward(const ts2_att_grad_args *a, void *stream)
     p.ldStat = a->sumWeightLog.strideBytes / 4;
     p.lenRound = a->lenRound;
     const bool alibi = a->alibiSlope != 0; // the kernels without a slope leave the position term out of every logit
-    // with a dS array the dK/dV kernel leaves its score gradients behind and dQ is one product over them (both must run: which == 3)
+    // with a dS array the dK/dV kernel leaves its score gradients behind and dQ is one product over them (both must run: which == 3).  One
+    // launch for both leaves the array alone: it is faster than writing and reading it (2048 tokens, one head 45 us, 71 with a dS array handed
+    // over; 128 tokens 11.4, 15.2)
     const bool viaDs = a->which == 3 && a->dsBase && a->dsScratch && a->dsCapacityBlocks > 0;
     if (viaDs) {
         if (((uintptr_t)a->dsScratch & 15) != 0) {
@@ -2544,37 +2504,32 @@ extern "C" int ts2_att_backward(const ts2_att_grad_args *a, void *stream)
         p.ldo1 = a->dV.strideBytes;
         p.out2 = (uint8_t *)a->dQ.ptr;
         p.ldo2 = a->dQ.strideBytes;
-        const int nKv = a->lenRound / KVROWS, nQ = viaDs ? 0 : a->lenRound / BROWS;
-        auto kernel = f32 ? (alibi ? AttGradSmall<true, true, false> : AttGradSmall<true, false, false>)
-                          : (alibi ? AttGradSmall<false, true, false> : AttGradSmall<false, false, false>);
-        if (viaDs) {
-            kernel = f32 ? (alibi ? AttGradSmall<true, true, true> : AttGradSmall<true, false, true>)
-                         : (alibi ? AttGradSmall<false, true, true> : AttGradSmall<false, false, true>);
-        }
+        const int nKv = a->lenRound / KVROWS, nQ = a->lenRound / BROWS;
+        auto kernel = f32 ? (alibi ? AttGradSmall<true, true> : AttGradSmall<true, false>) : (alibi ? AttGradSmall<false, true> : AttGradSmall<false, false>);
         hipLaunchKernelGGL(kernel, dim3((nKv + nQ) * a->heads), dim3(512), 0, (hipStream_t)stream, p, nKv, nQ, a->heads);
         TS2_CHECK_LAUNCH();
-    } else {
-        if ((a->which & 1) && !viaDs) {
-            p.out0 = (uint8_t *)a->dQ.ptr;
-            p.ldo0 = a->dQ.strideBytes;
-            auto kernel = f32 ? (alibi ? AttGradQ<true, true> : AttGradQ<true, false>) : (alibi ? AttGradQ<false, true> : AttGradQ<false, false>);
-            hipLaunchKernelGGL(kernel, dim3(a->lenRound / BROWS, a->heads), dim3(256), 0, (hipStream_t)stream, p);
-            TS2_CHECK_LAUNCH();
+        return TS2_OK;
+    }
+    if ((a->which & 1) && !viaDs) {
+        p.out0 = (uint8_t *)a->dQ.ptr;
+        p.ldo0 = a->dQ.strideBytes;
+        auto kernel = f32 ? (alibi ? AttGradQ<true, true> : AttGradQ<true, false>) : (alibi ? AttGradQ<false, true> : AttGradQ<false, false>);
+        hipLaunchKernelGGL(kernel, dim3(a->lenRound / BROWS, a->heads), dim3(256), 0, (hipStream_t)stream, p);
+        TS2_CHECK_LAUNCH();
+    }
+    if (a->which & 2) {
+        p.out0 = (uint8_t *)a->dK.ptr;
+        p.ldo0 = a->dK.strideBytes;
+        p.out1 = (uint8_t *)a->dV.ptr;
+        p.ldo1 = a->dV.strideBytes;
+        auto kernel = f32 ? (alibi ? AttGradKV<true, true, false> : AttGradKV<true, false, false>)
+                          : (alibi ? AttGradKV<false, true, false> : AttGradKV<false, false, false>);
+        if (viaDs) {
+            kernel = f32 ? (alibi ? AttGradKV<true, true, true> : AttGradKV<true, false, true>)
+                         : (alibi ? AttGradKV<false, true, true> : AttGradKV<false, false, true>);
         }
-        if (a->which & 2) {
-            p.out0 = (uint8_t *)a->dK.ptr;
-            p.ldo0 = a->dK.strideBytes;
-            p.out1 = (uint8_t *)a->dV.ptr;
-            p.ldo1 = a->dV.strideBytes;
-            auto kernel = f32 ? (alibi ? AttGradKV<true, true, false> : AttGradKV<true, false, false>)
-                              : (alibi ? AttGradKV<false, true, false> : AttGradKV<false, false, false>);
-            if (viaDs) {
-                kernel = f32 ? (alibi ? AttGradKV<true, true, true> : AttGradKV<true, false, true>)
-                             : (alibi ? AttGradKV<false, true, true> : AttGradKV<false, false, true>);
-            }
-            hipLaunchKernelGGL(kernel, dim3(a->lenRound / KVROWS, a->heads), dim3(256), 0, (hipStream_t)stream, p);
-            TS2_CHECK_LAUNCH();
-        }
+        hipLaunchKernelGGL(kernel, dim3(a->lenRound / KVROWS, a->heads), dim3(256), 0, (hipStream_t)stream, p);
+        TS2_CHECK_LAUNCH();
     }
     if (viaDs) {
         p.out0 = (uint8_t *)a->dQ.ptr;
