@@ -209,3 +209,49 @@ def test_handed_over_score_gradients_of_spans_with_gaps(L, heads, f32):
         assert torch.equal(out[0][0], out[1][0]) and (handed[1] == 0x7f).all()
     a, b = out[0][0].float(), out[1][0].float()
     assert (a - b).abs().max() <= 4e-3 * a.abs().max()
+
+
+@pytest.mark.parametrize("docs,window", [([300, 1, 299, 500], 40), ([1100], 4096)])
+def test_gradients_in_place_of_keys_and_values(L, docs, window):
+    """dK over K and dV over V: a workgroup reads the rows it writes, and dQ, which reads them all, is done before.  The very bits of the calls
+    for one gradient each, which run the same kernels.  Column ranges of one wide matrix are no such case: the same bits as separate
+    matrices, and as the call with both bits in one launch"""
+    print("case att in place", docs, window, flush=True)
+    sp, spans = ragged_spans(docs, window)
+    n, n_round, heads, w, i16 = sp.size - 1, (sp.size + 126) // 128 * 128, 2, 256, torch.int16
+    start, finish = spans_to_ranges(sp, spans, n, n_round)
+    ts, tf = torch.from_numpy(start).cuda(), torch.from_numpy(finish).cuda()
+
+    def padded(a):
+        t = torch.zeros((n_round, w), dtype=torch.bfloat16, device="cuda")
+        t[:n] = torch.from_numpy(a).cuda().bfloat16()
+        return t.view(i16)
+    q, k, v, dval = [padded(a) for a in inputs(n, heads, seed=13)]
+    val, swl = torch.zeros_like(q), torch.zeros((heads, n_round), device="cuda")
+    L.att_forward(n, heads, q, k, v, ts, tf, SCALE, 0.0, val, swl)
+    lo = torch.zeros(n_round // 128, dtype=torch.int32, device="cuda")
+    hi = torch.zeros_like(lo)
+    L.call("ts2_att_build_rev", n, n_round, ts, tf, lo, hi)
+    ds = torch.from_numpy(np.random.default_rng(4).standard_normal((heads, n_round)).astype(np.float32) * 0.1).cuda()
+
+    def back(k, v, out, which):
+        L.att_backward(n, heads, q, k, v, dval, ts, tf, lo, hi, SCALE, 0.0, swl, ds, *out, L.BF16, which=which)
+    apart, both = [[torch.full_like(q, 7) for _ in range(3)] for _ in range(2)]
+    back(k, v, apart, 1)
+    back(k, v, apart, 2)
+    back(k, v, both, 3)
+    wide = torch.full((n_round, 5 * w), 7, dtype=i16, device="cuda")
+    parts = [wide[:, i * w:(i + 1) * w] for i in range(5)]  # dQ, K, dK, V, dV side by side
+    parts[1].copy_(k)
+    parts[3].copy_(v)
+    back(parts[1], parts[3], [parts[0], parts[2], parts[4]], 3)
+    k2, v2, dq = k.clone(), v.clone(), torch.full_like(q, 7)
+    back(k2, v2, [dq, k2, v2], 3)
+    torch.cuda.synchronize()
+    for name, a, b in zip(("dq", "dk", "dv"), apart, (dq, k2, v2)):
+        assert torch.equal(a, b), name
+    for name, a, b, c in zip(("dq", "dk", "dv"), both, (parts[0], parts[2], parts[4]), apart):
+        assert torch.equal(a, b), name
+        # one launch adds a gradient in two halves: fp32 sums of at most 1100 terms in another order, then one bf16 step
+        x, y = a.view(torch.bfloat16).float(), c.view(torch.bfloat16).float()
+        assert ((x - y).abs() <= 2.0 ** -7 * y.abs() + 2.0 ** -14 * y.abs().max()).all(), name

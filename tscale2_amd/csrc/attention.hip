@@ -2362,6 +2362,21 @@ bool OneLaunch(int which, int lenRound, int heads)
     return which == 3 && (int64_t)(lenRound / KVROWS + lenRound / BROWS) * heads <= 256;
 }
 
+// may a row of a [rows][cols * ea bytes] share memory with one of b?  (column ranges of one wide matrix lie between each other and do not)
+bool Overlap(const ts2_mat &a, int ea, const ts2_mat &b, int eb, int rows, int cols)
+{
+    const uintptr_t a0 = (uintptr_t)a.ptr, b0 = (uintptr_t)b.ptr;
+    const int64_t la = a.strideBytes, lb = b.strideBytes, wa = (int64_t)cols * ea, wb = (int64_t)cols * eb;
+    if (a0 + (rows - 1) * la + wa <= b0 || b0 + (rows - 1) * lb + wb <= a0) {
+        return false;
+    }
+    if (la == lb) {
+        const int64_t d = b0 >= a0 ? (int64_t)((b0 - a0) % la) : (la - (int64_t)((a0 - b0) % la)) % la; // b's columns behind a's, around the row
+        return d < wa || la - d < wb;
+    }
+    return true;
+}
+
 } // namespace
 
 extern "C" int ts2_att_build_rev(int32_t len, int32_t lenRound, const int32_t *spanStart, const int32_t *spanFinish, int32_t *revLo, int32_t *revHi,
@@ -2497,7 +2512,11 @@ extern "C" int ts2_att_backward(const ts2_att_grad_args *a, void *stream)
         p.ds = (uint8_t *)a->dsScratch;
         p.dsCap = a->dsCapacityBlocks;
     }
-    if (OneLaunch(a->which, a->lenRound, a->heads)) {
+    // dK and dV may take the place of K and V, whose rows dQ workgroups read: then dQ is a launch of its own, before
+    const int es = f32 ? 4 : 2;
+    const bool inPlace = Overlap(a->dK, es, a->k, 2, a->lenRound, cols) || Overlap(a->dK, es, a->v, 2, a->lenRound, cols) ||
+        Overlap(a->dV, es, a->k, 2, a->lenRound, cols) || Overlap(a->dV, es, a->v, 2, a->lenRound, cols);
+    if (OneLaunch(a->which, a->lenRound, a->heads) && !inPlace) {
         p.out0 = (uint8_t *)a->dK.ptr;
         p.ldo0 = a->dK.strideBytes;
         p.out1 = (uint8_t *)a->dV.ptr;
