@@ -1,4 +1,4 @@
-"""The state a batch starts from, at the lengths where a workgroup of the embedding pass takes one row and four: rows without a label, with
+"""The state a batch starts from, at the lengths where a workgroup of the embedding pass takes one row, two and four: rows without a label, with
 one, with several, labels that are subtracted.  Sums of a few 8-bit values times one scale in fp32, in the order of the labels: each of up to
 four terms rounds once in the product and once in the sum, 8 * 2^-24 of the largest partial sum."""
 import numpy as np
@@ -12,7 +12,7 @@ from tscale2_amd import lib as L  # noqa: E402
 
 
 @pytest.mark.parametrize("mode", [I8, E4M3])
-@pytest.mark.parametrize("n", [1, 130, 8191, 8193])
+@pytest.mark.parametrize("n", [1, 130, 8191, 8193, 12161, 12291, 32641, 32771])
 def test_embedded_state(mode, n):
     print("case embedding", mode, n, flush=True)
     h = Harness(mode, dim=256, heads=1, ffn_tiles=1, depth=2, vocab=256, frag_count=2, frag_len=64, wide_window=64, seed=9)

@@ -6,21 +6,26 @@
 namespace
 {
 // state0[t] = sum over labels of +-E[label] * scale (ComputeEmbedding, src/gpt/compute/cpu_transformer.cpp:76-100).  A row is a chain of
-// three loads (its labels' range, a label, the label's matrix row) before it is written, so a workgroup takes ROWS rows and has the first
-// label of all of them under way together: 65536 x 1024 of e4m3 99 -> 71 us (336 MB: 54 at the rate of a copy), 16384 x 512 12.2 -> 11.3.
+// three loads (its labels' range, a label, the label's matrix row) before it is written, and two more for every further label, so a workgroup
+// takes ROWS rows and has the same label of all of them under way together: 65536 x 1024 of e4m3 99 -> 71 us inside a step (336 MB: 54 at the
+// rate of a copy), 16384 x 512 of int8 10.9 -> 9.6, with four labels per row 20.7 -> 18.6.
 template <class TEmb, int ROWS>
 __global__ void __launch_bounds__(256) EmbedForward(int len, int lenRound, int dim, const int *labelPtr, const uint32_t *labels, const uint8_t *embed,
     int64_t ldEmb, float mult, const float *scalePtr, float *state, int64_t ldState)
 {
+    if ((int)threadIdx.x * 4 >= dim) { // (waves beyond a narrow row do not wait for its labels)
+        return;
+    }
     const int t0 = blockIdx.x * ROWS;
     const float s = mult * (scalePtr ? *scalePtr : 1.f);
-    int from[ROWS], to[ROWS];
+    int from[ROWS], to[ROWS], most = 0;
     uint32_t one[ROWS];
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
         const bool live = t0 + r < len;
         from[r] = live ? labelPtr[t0 + r] : 0;
         to[r] = live ? labelPtr[t0 + r + 1] : 0;
+        most = max(most, to[r] - from[r]);
     }
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
@@ -37,10 +42,28 @@ __global__ void __launch_bounds__(256) EmbedForward(int len, int lenRound, int d
             if (from[r] < to[r]) {
                 acc[r] = ZeroF4() + acc[r] * ((one[r] & 0x80000000u) ? -s : s);
             }
-            for (int k = from[r] + 1; k < to[r]; ++k) {
-                const uint32_t label = labels[k];
-                acc[r] = acc[r] + Load4<TEmb>(embed + (int64_t)(label & 0x7fffffffu) * ldEmb + col * TEmb::SIZE) * ((label & 0x80000000u) ? -s : s);
+        }
+        for (int j = 1; j < most; ++j) {
+            auto has = [&](int r) { return ROWS == 1 || from[r] + j < to[r]; };
+            uint32_t label[ROWS];
+            F4 v[ROWS];
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) {
+                label[r] = has(r) ? labels[from[r] + j] : 0;
             }
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) {
+                v[r] = has(r) ? Load4<TEmb>(embed + (int64_t)(label[r] & 0x7fffffffu) * ldEmb + col * TEmb::SIZE) : ZeroF4();
+            }
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) {
+                if (has(r)) {
+                    acc[r] = acc[r] + v[r] * ((label[r] & 0x80000000u) ? -s : s);
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
             if (t0 + r < lenRound) {
                 Store4<TF32>((uint8_t *)state + (int64_t)(t0 + r) * ldState + col * 4, acc[r]);
             }
@@ -684,23 +707,25 @@ __global__ void __launch_bounds__(256) FinalSoftmaxGradHalfWave(int rows, int vo
 int Ts2EmbedForward(int len, int lenRound, int dim, const int *labelPtr, const uint32_t *labels, const ts2_mat *embed, int embType, float mult,
     const float *scalePtr, const ts2_mat *state, void *stream)
 {
-    // (4096 x 512 with four rows to a workgroup 7.3 us, with one 6.8)
-    const int per = lenRound >= 8192 ? 4 : 1;
+    // more rows than keep every CU's waves busy anyway, and then the more rows the better while the rows are short: 8192 x 512 with one, two and
+    // four rows to a workgroup 6.0, 6.1, 6.5 us, 16384 x 512 10.4, 9.6, 10.2, 65536 x 256 25.4, 20.7, 18.4 (four labels: 52.4, 43.8, 39.5)
+    const int per = lenRound >= 32768 ? 4 : lenRound >= 12288 ? 2 : 1;
 #define LAUNCH_E(T, N)                                                                                                                     \
     hipLaunchKernelGGL((EmbedForward<T, N>), dim3((lenRound + N - 1) / N), dim3(256), 0, STREAM, len, lenRound, dim, labelPtr, labels,      \
         (const uint8_t *)embed->ptr, embed->strideBytes, mult, scalePtr, (float *)state->ptr, state->strideBytes)
+#define LAUNCH_ROWS(T)                                                                                                                     \
+    if (per == 4) {                                                                                                                        \
+        LAUNCH_E(T, 4);                                                                                                                    \
+    } else if (per == 2) {                                                                                                                 \
+        LAUNCH_E(T, 2);                                                                                                                    \
+    } else {                                                                                                                               \
+        LAUNCH_E(T, 1);                                                                                                                    \
+    }
     if (embType == TS2_I8) {
-        if (per == 4) {
-            LAUNCH_E(TI8, 4);
-        } else {
-            LAUNCH_E(TI8, 1);
-        }
+        LAUNCH_ROWS(TI8)
     } else if (embType == TS2_E4M3) {
-        if (per == 4) {
-            LAUNCH_E(TE4M3, 4);
-        } else {
-            LAUNCH_E(TE4M3, 1);
-        }
+        LAUNCH_ROWS(TE4M3)
+#undef LAUNCH_ROWS
 #undef LAUNCH_E
     } else {
         return TS2_ERR_UNSUPPORTED;
