@@ -1435,10 +1435,9 @@ __global__ void __launch_bounds__(256) BackpropRowTileNormalizeRope8(int len, in
 // sum of `splits` fp32 partial products (slabs of [rows][cols]) -> packed delta: per row and 128-column tile scale = maxabs/127,
 // bytes = sat_i8(rne(v/scale)), TileScale[tile][row] = scale: the arithmetic of the GEMM's ROW_TILE_MAXNORM epilogue applied to the sum.
 //
-// Bounded by latency: one slice after the other is one trip to memory each.  So RU rows times SU slices are requested together, eight loads
-// per lane (the sum keeps the order of the slices, and its bits).  A small matrix of many slices gets one row per group of lanes and all of
-// eight slices at once, which also gives four times the groups: 512 x 512 of 8 slices 5.8 -> 2.8 us (10.8 -> 4 inside a step, from HBM),
-// 1024 x 512 of 32 32.9 -> 12.0, 1024 x 1024 of 8 7.2 -> 4.0, 256 x 256 of one 3.1 -> 2.9; 8192 x 2048 of 2 28.5 -> 23.8.
+// Bounded by latency: one slice after the other is one trip to memory each.  So RU rows times SU slices are requested together (the sum keeps
+// the order of the slices, and its bits).  Against four rows of one slice at a time: 512 x 512 of 8 slices 6.0 -> 3.2 us, 1024 x 512 of 32
+// 30.6 -> 12.0, 1024 x 1024 of 8 7.5 -> 4.3, 256 x 256 of one 3.5 -> 2.8; 8192 x 2048 of 2 28.8 -> 23.9.
 template <int RU, int SU>
 __global__ void __launch_bounds__(256) PackDelta(int rows, int tiles, int splits, const uint8_t *partial, int64_t ldPartial, int64_t slab, float alpha,
     const float *alphaPtr, Mat delta, Mat tileScale)
@@ -2141,11 +2140,13 @@ extern "C" int ts2_pack_delta(const ts2_mat *partial, int32_t splits, int64_t sl
         return TS2_ERR_SHAPE;
     }
     int tiles = cols / TILE;
-    // one row per group of lanes up to 16384 groups (eight waves on each SIMD of the chip; 1024 x 1024 of 8 slices takes 4.0 us so), and for
-    // more than two slices (of two, both forms have all in flight)
-    const bool small = splits > 2 && (int64_t)rows * tiles <= 16384;
-    const long units = (long)(small ? rows : (rows + 3) / 4) * tiles;
-    auto kernel = small ? PackDelta<1, 8> : PackDelta<4, 2>;
+    // While more than two slices together fit the L2s (32 MB), a row and eight slices at a time: 512 x 512 of 8 slices 3.2 us (3.7 with two
+    // rows and two slices), 2048 x 1024 of 4 4.7 (5.2); beyond them two rows and two slices: 2048 x 1024 of 8 12.3 (14.1 with one and eight),
+    // 8192 x 2048 of one 15.9.  Many slices from beyond the memory-side cache (256 MB) come one at a time: 2048 x 2048 of 32 89 (94)
+    const int64_t bytes = (int64_t)splits * rows * cols * 4;
+    const int form = splits > 2 && bytes <= 32 << 20 ? 1 : splits >= 8 && bytes > 256 << 20 ? 4 : 2; // rows of a group of lanes
+    const long units = (long)((rows + form - 1) / form) * tiles;
+    auto kernel = form == 1 ? PackDelta<1, 8> : form == 2 ? PackDelta<2, 2> : PackDelta<4, 1>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)((units * 32 + 255) / 256)), dim3(256), 0, STREAM, rows, tiles, splits, (const uint8_t *)partial->ptr,
         partial->strideBytes, slabBytes, alpha, alphaPtr, M(*delta), M(*deltaTileScale));
     TS2_CHECK_LAUNCH();
