@@ -98,7 +98,7 @@ template <int W, int NCH>
 __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W, 4) FinalProbabilities(int rows, int vocab, float *logits, int64_t ldLogits,
     const float *bias, const int *target, float gradMult, bf16_t *grad, int64_t ldGrad)
 {
-    __shared__ float redM[W], redL[W], redS[W];
+    __shared__ float redM[W], redS[W];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int t = W == 1 ? blockIdx.x * 4 + wave : blockIdx.x, first = W == 1 ? lane : threadIdx.x;
     if (t >= rows) { // (one wave per row: a whole wave, and no barrier below)
@@ -108,7 +108,7 @@ __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W, 4) FinalProbabilities(i
     bf16_t *grow = (bf16_t *)((uint8_t *)grad + (int64_t)t * ldGrad);
     const int tg = target[t];
     float4 x[NCH];
-    float m = -1e30f, least = 1e30f; // the row's largest and smallest logit with their bias
+    float m = -1e30f, least = 1e30f; // the row's largest logit with its bias, the lane's smallest
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
         const int k = (i * 64 * W + first) * 4;
@@ -125,25 +125,22 @@ __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W, 4) FinalProbabilities(i
         m = fmaxf(m, fmaxf(fmaxf(x[i].x, x[i].y), fmaxf(x[i].z, x[i].w)));
     }
     m = WaveMax(m);
-    least = -WaveMax(-least);
     if (W > 1) {
         if (lane == 0) {
             redM[wave] = m;
-            redL[wave] = least;
         }
         __syncthreads();
 #pragma unroll
         for (int w = 0; w < W; ++w) {
             m = fmaxf(m, redM[w]);
-            least = fminf(least, redL[w]);
         }
     }
     // A logit is the exponential's argument as it is while the largest leaves room for the sum, and relative to the largest otherwise: a
     // subtraction rounds (relative to 64 below the largest, rms error of a probability 7.6e-7 instead of 6e-8).  The hardware's exponential
-    // returns zero below 2^-126; a row that reaches there takes exp2f, which goes on to 2^-149 at five instructions more.
+    // returns zero below 2^-126; a wave that reaches there takes exp2f, which goes on to 2^-149 at five instructions more.
     m = fabsf(m) <= 64 ? 0.f : m;
     float sum = 0;
-    int plain = __builtin_amdgcn_readfirstlane((int)(least - m >= -125)), wide = plain ^ 1;
+    int plain = __builtin_amdgcn_readfirstlane((int)__all(least - m >= -125)), wide = plain ^ 1;
     // loops of one trip or none, not branches: a join would cost registers
     asm volatile("" : "+s"(plain), "+s"(wide));
 #pragma unroll 1
@@ -783,13 +780,14 @@ int Ts2FinalProbabilities(int rows, int vocab, const ts2_mat *logits, const floa
 #define LAUNCH_P(W, N)                                                                                                                     \
     hipLaunchKernelGGL((FinalProbabilities<W, N>), dim3(W == 1 ? (rows + 3) / 4 : rows), dim3(W == 1 ? 256 : 64 * W), 0, STREAM, rows, vocab, \
         (float *)logits->ptr, logits->strideBytes, bias, target, gradMult, (bf16_t *)grad->ptr, grad->strideBytes)
-    const int chunks = (vocab + 255) / 256; // of 256 logits: one float4 per lane of a wave
+    // of 256 logits: one float4 per lane of a wave.  (2048 logits in four waves, not one: 64 rows 4.4 -> 3.1 us, 4096 rows 15.9 -> 14.4)
+    const int chunks = (vocab + 255) / 256;
     if (chunks <= 2) {
         LAUNCH_P(1, 2);
     } else if (chunks <= 4) {
         LAUNCH_P(1, 4);
     } else if (chunks <= 8) {
-        LAUNCH_P(1, 8);
+        LAUNCH_P(4, 2);
     } else if (chunks <= 16) {
         LAUNCH_P(4, 4);
     } else if (chunks <= 32) {
