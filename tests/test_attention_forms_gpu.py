@@ -1,6 +1,7 @@
 """The forms of the attention kernels, which a rule on the number of workgroups (and on the key range of a workgroup) chooses between:
 a pipelined forward for long key ranges and a plain one for narrow windows; the backward as one launch with two waves (or pairs of waves)
-per row block where there are few workgroups, as two launches where there are many.  The repetition of two heads of data fills a launch of any size, and the oracle computes those two only.
+per row block where few workgroups are asked for both its halves, as one launch for dQ and one for dK and dV otherwise, with the score gradients
+handed from one to the other or formed twice.  The repetition of two heads of data fills a launch of any size, and the oracle computes those two only.
 Inputs are bf16-representable; the device rounds probabilities and score gradients to bf16 before a product, hence the same tolerance as in
 test_attention_gpu.py: max |err| <= 1e-2 * max |ref| per tensor."""
 import numpy as np
@@ -88,6 +89,60 @@ def test_forms_against_the_oracle(L, orc, docs, window, heads, slope):
         for h in range(rep):
             got = g[:n, h * base * 128:(h + 1) * base * 128]
             assert np.abs(got - ref[name]).max() <= 1e-2 * max(np.abs(ref[name]).max(), 1e-30), (name, h)
+
+
+@pytest.mark.parametrize("docs,window,heads,slope", [([300, 1, 299, 500], 40, 10, 0.25), ([1100], 4096, 10, 0.0), ([64, 65, 63, 128, 129, 651], 300, 16, 0.125),
+                                                      ([64, 65, 63, 128, 129, 651], 300, 16, 0.0), ([300, 1, 299, 500], 40, 2, 0.0), ([1100], 4096, 2, 0.01)])
+@pytest.mark.parametrize("f32", [False, True])
+def test_backward_in_every_way_it_can_be_asked_for(L, orc, docs, window, heads, slope, f32):
+    """gradients in fp32 and bf16; both bits, one bit at a time, both with the score gradients handed over (over NaN patterns).  With 10 and 16 heads
+    the two kernels run one after the other whatever is asked for: the bits of dK and dV are the same in every way, those of dQ but for the
+    hand-over.  With 2 heads both bits are one launch, which adds a gradient in two halves.  Row blocks that straddle document starts are seen
+    partly by one key block of a workgroup and completely by the other, so the dK/dV waves take their two-block and one-block paths in turn"""
+    print("case att ways", docs, window, heads, slope, f32, flush=True)
+    sp, spans = ragged_spans(docs, window)
+    n, i16, rep = sp.size - 1, torch.int16, heads // 2
+    n_round = (n + 127) // 128 * 128
+    start, finish = spans_to_ranges(sp, spans, n, n_round)
+    a = inputs(n, 2, seed=n + heads)
+    ref = orc.attention(2, 128, 128, slope, sp, spans, *a)
+
+    def padded(x):
+        t = torch.zeros((n_round, heads * 128), dtype=torch.bfloat16, device="cuda")
+        t[:n] = torch.from_numpy(np.tile(x, (1, rep))).cuda().bfloat16()
+        return t.view(i16)
+    q, k, v, dval = [padded(x) for x in a]
+    ts, tf = torch.from_numpy(start).cuda(), torch.from_numpy(finish).cuda()
+    val, swl = torch.zeros_like(q), torch.zeros((heads, n_round), device="cuda")
+    L.att_forward(n, heads, q, k, v, ts, tf, SCALE, slope, val, swl)
+    lo = torch.zeros(n_round // 128, dtype=torch.int32, device="cuda")
+    hi = torch.zeros_like(lo)
+    L.call("ts2_att_build_rev", n, n_round, ts, tf, lo, hi)
+    ds = torch.zeros((heads, n_round), device="cuda")
+    ds[:, :n] = torch.from_numpy(np.tile(ref["dscale"], (rep, 1))).cuda()
+    handed = L.att_ds_scratch(n_round, heads, ts, tf)
+    handed[1].fill_(0x7f)
+
+    def back(which, pair=None):
+        o = [torch.full((n_round, heads * 128), 7.0, dtype=torch.float32 if f32 else torch.bfloat16, device="cuda") for _ in range(3)]
+        L.att_backward(n, heads, q, k, v, dval, ts, tf, lo, hi, SCALE, slope, swl, ds, *[t if f32 else t.view(i16) for t in o], L.F32 if f32 else L.BF16,
+                       which=which, ds=pair)
+        torch.cuda.synchronize()
+        return o
+    both, dq_only, dkv_only, via = back(3), back(1), back(2), back(3, handed)
+    assert (dq_only[1] == 7).all() and (dq_only[2] == 7).all() and (dkv_only[0] == 7).all()
+    apart = [dq_only[0], dkv_only[1], dkv_only[2]]
+    for ways in (both, apart, via):
+        for name, t in zip(("dq", "dk", "dv"), ways):
+            g = t.float().cpu().numpy()
+            assert np.all(g[n:] == 0), name
+            for h in range(rep):
+                assert np.abs(g[:n, h * 256:(h + 1) * 256] - ref[name]).max() <= 1e-2 * np.abs(ref[name]).max(), (name, h)
+    if heads > 2:
+        assert all(torch.equal(x, y) for x, y in zip(both, apart))
+        assert torch.equal(via[1], both[1]) and torch.equal(via[2], both[2]) and not (handed[1] == 0x7f).all()
+    else:
+        assert all(torch.equal(x, y) for x, y in zip(both, via)) and (handed[1] == 0x7f).all()
 
 
 @pytest.mark.parametrize("heads", [2, 16])

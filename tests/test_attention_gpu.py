@@ -108,8 +108,8 @@ def run_case(L, orc, frag_count, frag_len, window, heads, slope, seed, grad_type
         print(name, "rel err", err)
         assert err <= 1e-2, name
         assert np.all(g[n:] == 0), name
-    # the same with the score gradients handed from the dK/dV kernel to the dQ kernel (5 products instead of 7): dK and dV are the very
-    # same values, dQ is formed from dS rounded to bf16 where the other kernel rounds its own evaluation of it: equal to bf16 noise
+    # the same with an array for the score gradients (5 products instead of 7): dK and dV are the very same values, and dQ is too where both
+    # run as one launch (as at these sizes), or is formed from dS rounded to bf16 where the other kernel rounds its own evaluation of it
     print("  ... dQ from the dK/dV kernel's score gradients", flush=True)
     ds_pair = L.att_ds_scratch(n_round, heads, ts, tf)
     ds_pair[1].fill_(0x7f)  # NaN patterns where nothing is written
@@ -150,8 +150,8 @@ def test_attention_remapped_block_order(L, orc):
 @pytest.mark.parametrize("window,slope,seed", [(96, 0.125, 31), (1000, 0.0, 32), (40, 0.0, 33)])
 def test_attention_ragged_documents(L, orc, window, slope, seed):
     """documents of random lengths between 1 and 400 tokens: rows without a span (first tokens), 32-row blocks that straddle document
-    starts (seen partly by one key block of a workgroup and completely by the other, so the dK/dV waves take their two-block and
-    their one-block paths in turn and the hand-over counters run through both), windows that end inside a tile"""
+    starts (seen partly by one key block of a workgroup and completely by the other), windows that end inside a tile.  (Launches of this
+    size run dQ, dK and dV as one kernel, which leaves a dS array alone; test_attention_forms_gpu.py has the two kernels of larger ones)"""
     print("case att ragged documents", window, slope, flush=True)
     r = np.random.default_rng(seed)
     lens = []
