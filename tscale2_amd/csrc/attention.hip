@@ -320,36 +320,28 @@ __device__ __forceinline__ v4i TileRsrc(const uint8_t *g, int bytes)
     return v4i{__builtin_amdgcn_readfirstlane((int)(uint32_t)u), __builtin_amdgcn_readfirstlane((int)(u >> 32)), bytes, 0x00020000};
 }
 
-// The waves w = 0 .. WPG - 1 (WPG = 2 or 4) fetch a tile of ROWS rows together, one row group (4 rows, 1 KB) per load: groups with the same
-// number modulo 4, which share one swizzle per lane (two of them where two waves fetch a tile).  What a lane adds is held in registers, what
-// a row group adds in scalar ones; a request is a handful of scalar instructions.
-template <int WPG, int ROWS> struct TTileLoader {
-    static constexpr int SWZ = WPG == 2 ? 2 : 1, PER = ROWS / 4 / WPG / SWZ; // swizzles of a wave, loads with each
-    int laneOff[SWZ];
+// Four waves w = 0 .. 3 fetch a tile of ROWS rows together, one row group (4 rows, 1 KB) per load: the groups of a wave have the same number
+// modulo 4, which share one swizzle per lane.  What a lane adds is held in a register, what a row group adds in scalar ones; a request is a
+// handful of scalar instructions.
+template <int ROWS> struct TTileLoader {
+    static constexpr int LOADS = ROWS / 16; // of a wave, per tile
+    int laneOff;
     int ld, dst; // bytes of a row; LDS offset of the wave's first row group
     __device__ __forceinline__ TTileLoader(int64_t ld64, int w, int lane) : ld((int)ld64), dst(w * 1024)
     {
         const int lrow = lane >> 4;
-#pragma unroll
-        for (int c = 0; c < SWZ; ++c) {
-            const int u = w + 2 * c;
-            laneOff[c] = (lrow + 4 * u) * ld + (((lane & 15) ^ ((lrow << 2) | (u & 3))) << 4);
-            asm volatile("" : "+v"(laneOff[c]));
-        }
+        laneOff = (lrow + 4 * w) * ld + (((lane & 15) ^ ((lrow << 2) | w)) << 4);
+        asm volatile("" : "+v"(laneOff));
     }
     __device__ __forceinline__ void Request(unsigned ldsTile, const uint8_t *g) const
     {
         const v4i rsrc = TileRsrc(g, ROWS * ld);
         const unsigned m0 = ldsTile + dst;
 #pragma unroll
-        for (int c = 0; c < SWZ; ++c) {
-#pragma unroll
-            for (int i = 0; i < PER; ++i) {
-                const int u = WPG * SWZ * i;
-                asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(m0), "v"(laneOff[c]), "s"(rsrc),
-                             "s"(4 * u * ld), "n"(u * 1024 + c * 2048)
-                             : "memory", "scc");
-            }
+        for (int i = 0; i < LOADS; ++i) {
+            asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(m0), "v"(laneOff), "s"(rsrc),
+                         "s"(16 * i * ld), "n"(i * 4096)
+                         : "memory", "scc");
         }
     }
 };
@@ -577,12 +569,11 @@ __device__ __forceinline__ void ForwardFewTiles(const AttP &p, uint8_t *kT0, uin
 // issues one instruction in five cycles.  So the kernel saves instructions: the exponential's argument is one fused multiply-add of the raw
 // product, the running maximum is taken once per tile of 64 keys, masks are a pass of their own over the tiles that need one.  And it overlaps:
 // S of tile i + 1 is formed between the exponentials of tile i, its maximum between the products with V, operands are requested six products
-// ahead.  16 x 2048 tokens causal, 16 heads: 395 -> 371 us; one sequence of 2048 tokens, one head 54 -> 43.  A reference that lags the maximum
-// by up to 2^8 saves most of the rescaling (357, 40), but then the largest weight is rounded like any other: against fp64 0.00221 instead of
-// 0.00220, and 0.0020 instead of 0.0018 on peaked weights.
+// ahead.  16 x 2048 tokens causal, 16 heads: 396 -> 361 us; one sequence of 2048 tokens, one head 54.1 -> 43.7.  A reference that lags the
+// maximum by up to 2^8 saves most of the rescaling (another 4 and 7 %), but then the largest weight is rounded like any other: against fp64
+// 0.00221 instead of 0.00220, and 0.0020 instead of 0.0018 on peaked weights.
 template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP p)
 {
-    constexpr int QB = 4;  // query blocks of the workgroup; as many waves stream its tiles
     constexpr int FEW = 7; // key tiles up to which ForwardFewTiles is the faster one
     // K and V of the even tiles, of the odd ones
     __shared__ __attribute__((aligned(1024))) uint8_t kT0[TILE_BYTES], kT1[TILE_BYTES], vT0[TILE_BYTES], vT1[TILE_BYTES];
@@ -630,7 +621,7 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
     }
     const unsigned ldsK0 = (unsigned)(uintptr_t)TS2_LDS_PTR(kT0), ldsK1 = (unsigned)(uintptr_t)TS2_LDS_PTR(kT1);
     const unsigned ldsV0 = (unsigned)(uintptr_t)TS2_LDS_PTR(vT0), ldsV1 = (unsigned)(uintptr_t)TS2_LDS_PTR(vT1);
-    const TTileLoader<QB, TR> loadK(p.ldk, wave, lane), loadV(p.ldv, wave, lane);
+    const TTileLoader<TR> loadK(p.ldk, wave, lane), loadV(p.ldv, wave, lane);
     auto tileKey = [&](int i) { return (tile0 + i) * TR; }; // first key of tile i
     auto requestK = [&](int i, int buf) {
         if (i < nTiles) {
@@ -780,12 +771,10 @@ template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP 
         constexpr int PAR = decltype(parTag)::value;
         const uint8_t *kt = PAR ? kT1 : kT0, *vt = PAR ? vT0 : vT1;
         if (i == 0) {
-            // K of the first tile has landed (loads complete in order; V and the second K may still be under way)
-            if (nTiles > 1) {
-                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * 16 / QB) : "memory");
-            } else {
-                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(16 / QB) : "memory");
-            }
+            // K of the first tile has landed (loads complete in order; V and the second K, which there is beyond FEW tiles, may still be
+            // under way)
+            static_assert(FEW >= 1);
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * TTileLoader<TR>::LOADS) : "memory");
             __syncthreads();
         } else {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // K of tile i and V of tile i - 1 have landed
@@ -1661,7 +1650,7 @@ template <bool F32, bool ALIBI> __device__ __forceinline__ void GradQSplit(const
     const int nIter = (nTiles + KS - 1) / KS, nMine = (nTiles - grp + KS - 1) / KS;
     const uint8_t *gk = p.k + hoff, *gv = p.v + hoff;
     const unsigned ldsGrp = (unsigned)(uintptr_t)TS2_LDS_PTR(lds) + grp * (BSTAGES * BSTAGE);
-    const TTileLoader<QB, BT> loadK(p.ldk, qb, lane), loadV(p.ldv, qb, lane);
+    const TTileLoader<BT> loadK(p.ldk, qb, lane), loadV(p.ldv, qb, lane);
     auto tileKey = [&](int i) { return (tile0 + i * KS + grp) * BT; };
     auto request = [&](int i, int stage) __attribute__((always_inline)) {
         if (i < nMine) {
@@ -1879,7 +1868,7 @@ template <bool F32, bool ALIBI, int ROLE> __device__ __forceinline__ void GradKV
     const int nIter = (nTiles + KS - 1) / KS, nMine = (nTiles - grp + KS - 1) / KS;
     const unsigned ldsGrp = (unsigned)(uintptr_t)TS2_LDS_PTR(lds) + grp * KV_GROUP;
     const int query0 = (tile0 + grp) * BT; // first query of the group's first tile
-    const TTileLoader<GW, BT> loadQ(p.ldq, loader, lane), loadO(p.lddo, loader, lane);
+    const TTileLoader<BT> loadQ(p.ldq, loader, lane), loadO(p.lddo, loader, lane);
     const uint8_t *gq = p.q + hoff + (int64_t)query0 * p.ldq, *go = p.dO + hoff + (int64_t)query0 * p.lddo; // next tile to request
     const int64_t stepQ = (int64_t)(KS * BT) * p.ldq, stepO = (int64_t)(KS * BT) * p.lddo;
     auto requestRows = [&](int i, int stage) __attribute__((always_inline)) {
