@@ -408,9 +408,10 @@ typedef struct ts2_att_grad_args {
     int32_t which; /* bit 0: dQ (Fp16AttGradQ), bit 1: dK and dV (Fp16AttGradKV) */
     /* optional, all three or none, used when which == 3: the score gradients dS leave the dK/dV kernel as 32 x 32 bf16 blocks (2 KB
      * each) in dsScratch and dQ is a single product over them instead of a second evaluation of S and dP (5 products per backward
-     * instead of 7); where few workgroups run both kernels in one launch, the array is left alone.  dsBase: [lenRound + 1] from ts2_att_build_ds_index on the same spans; dsScratch: 16-byte aligned,
-     * dsCapacityBlocks blocks of 2048 bytes, at least heads * ts2_att_ds_blocks(spans) (blocks beyond the capacity are dropped:
-     * wrong gradients for those rows, no access outside the array).  Without them the kernels of the two bits run independently. */
+     * instead of 7); where few workgroups run both kernels in one launch, the array is left alone.  dsBase: [lenRound + 1] from
+     * ts2_att_build_ds_index on the same spans; dsScratch: 16-byte aligned, dsCapacityBlocks blocks of 2048 bytes, at least
+     * heads * ts2_att_ds_blocks(spans) (blocks beyond the capacity are dropped: wrong gradients for those rows, no access outside the
+     * array).  Without them the kernels of the two bits run independently. */
     const int32_t *dsBase;
     void *dsScratch;
     int64_t dsCapacityBlocks;

@@ -310,3 +310,41 @@ def test_gradients_in_place_of_keys_and_values(L, docs, window):
         # one launch adds a gradient in two halves: fp32 sums of at most 1100 terms in another order, then one bf16 step
         x, y = a.view(torch.bfloat16).float(), c.view(torch.bfloat16).float()
         assert ((x - y).abs() <= 2.0 ** -7 * y.abs() + 2.0 ** -14 * y.abs().max()).all(), name
+
+
+@pytest.mark.parametrize("docs,window", [([300, 1, 299, 500], 40), ([1100], 4096)])
+@pytest.mark.parametrize("place", ["q", "v", "dval"])
+def test_dq_in_place_with_handed_over_score_gradients(L, docs, window, place):
+    """dQ formed from the handed-over score gradients reads K and them alone, so it may take the place of Q, V or the incoming gradient, which
+    the launch before it has read.  dK and dV are the very bits of a call for them alone; dQ is formed from dS rounded to bf16 either way (2^-9 of
+    every term, with signs either way: far below 4e-3 of the largest)"""
+    print("case att dq in place", docs, window, place, flush=True)
+    sp, spans = ragged_spans(docs, window)
+    n, n_round, heads, w, i16 = sp.size - 1, (sp.size + 126) // 128 * 128, 2, 256, torch.int16
+    start, finish = spans_to_ranges(sp, spans, n, n_round)
+    ts, tf = torch.from_numpy(start).cuda(), torch.from_numpy(finish).cuda()
+
+    def padded(a):
+        t = torch.zeros((n_round, w), dtype=torch.bfloat16, device="cuda")
+        t[:n] = torch.from_numpy(a).cuda().bfloat16()
+        return t.view(i16)
+    t = dict(zip(("q", "k", "v", "dval"), [padded(a) for a in inputs(n, heads, seed=17)]))
+    val, swl = torch.zeros_like(t["q"]), torch.zeros((heads, n_round), device="cuda")
+    L.att_forward(n, heads, t["q"], t["k"], t["v"], ts, tf, SCALE, 0.0, val, swl)
+    lo = torch.zeros(n_round // 128, dtype=torch.int32, device="cuda")
+    hi = torch.zeros_like(lo)
+    L.call("ts2_att_build_rev", n, n_round, ts, tf, lo, hi)
+    ds = torch.from_numpy(np.random.default_rng(4).standard_normal((heads, n_round)).astype(np.float32) * 0.1).cuda()
+
+    def back(t, out, which, pair=None):
+        L.att_backward(n, heads, t["q"], t["k"], t["v"], t["dval"], ts, tf, lo, hi, SCALE, 0.0, swl, ds, *out, L.BF16, which=which, ds=pair)
+    apart = [torch.full_like(val, 7) for _ in range(3)]
+    back(t, apart, 1)
+    back(t, apart, 2)
+    copy = {k: x.clone() for k, x in t.items()}
+    out = [copy[place], torch.full_like(val, 7), torch.full_like(val, 7)]
+    back(copy, out, 3, L.att_ds_scratch(n_round, heads, ts, tf))
+    torch.cuda.synchronize()
+    assert torch.equal(out[1], apart[1]) and torch.equal(out[2], apart[2])
+    x, y = out[0].view(torch.bfloat16).float(), apart[0].view(torch.bfloat16).float()
+    assert (x - y).abs().max() <= 4e-3 * y.abs().max()

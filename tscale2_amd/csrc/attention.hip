@@ -2501,10 +2501,15 @@ extern "C" int ts2_att_backward(const ts2_att_grad_args *a, void *stream)
         p.ds = (uint8_t *)a->dsScratch;
         p.dsCap = a->dsCapacityBlocks;
     }
-    // dK and dV may take the place of K and V, whose rows dQ workgroups read: then dQ is a launch of its own, before
+    // a gradient may take the place of an input that no later launch reads: dK and dV that of K and V (dQ comes first), with a dS array dQ
+    // that of Q, V or dValLookup (dQ comes last).  One launch has no such order
     const int es = f32 ? 4 : 2;
-    const bool inPlace = Overlap(a->dK, es, a->k, 2, a->lenRound, cols) || Overlap(a->dK, es, a->v, 2, a->lenRound, cols) ||
-        Overlap(a->dV, es, a->k, 2, a->lenRound, cols) || Overlap(a->dV, es, a->v, 2, a->lenRound, cols);
+    bool inPlace = false;
+    for (const ts2_mat *out : {&a->dQ, &a->dK, &a->dV}) {
+        for (const ts2_mat *in : {&a->q, &a->k, &a->v, &a->dValLookup}) {
+            inPlace = inPlace || Overlap(*out, es, *in, 2, a->lenRound, cols);
+        }
+    }
     if (OneLaunch(a->which, a->lenRound, a->heads) && !inPlace) {
         p.out0 = (uint8_t *)a->dK.ptr;
         p.ldo0 = a->dK.strideBytes;
