@@ -60,7 +60,7 @@ def inputs(n, heads, seed, q_mul=1.0):
 
 
 # documents, window, heads of the launch, slope.  1100 tokens are nine 128-row blocks: with 2 heads the backward is one launch of 54 workgroups,
-# with 10 and 16 it is two.  Windows of 40 keep a workgroup's keys within five tiles, whole documents go beyond; 64 and 65 tokens end a document
+# with 10 and 16 it is two.  Windows of 40 keep a workgroup's keys within seven tiles, whole documents go beyond; 64 and 65 tokens end a document
 # on a tile and one past it
 CASES = [
     ([300, 1, 299, 500], 40, 2, 0.0), ([300, 1, 299, 500], 40, 16, 0.0), ([300, 1, 299, 500], 40, 16, 0.25),

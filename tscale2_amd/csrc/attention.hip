@@ -406,6 +406,8 @@ __device__ __forceinline__ void WaveKeyRange(const int *spanStart, const int *sp
 // exact running maximum.  The pipelined form below needs a barrier more and works on 64 keys at a time: 22.5 against 25 us for 16800 tokens,
 // 4 heads, 64-token windows over documents of unequal length.  Up to seven tiles (FEW below): 16 documents of 512 tokens, 7 heads, 200-token
 // windows 21.8 against 23.3 us; the rows of a 512-token sequence that see eight are faster the other way (8 sequences, 4 heads: 15.6, 17.3).
+// (The line is a compromise: documents of 435 to 500 tokens that start inside a tile lose up to 3 % beyond it, windows of 320 tokens in launches
+// that leave CUs idle 4 % below it.  Rows of zeros in LDS in place of the unseen half, instead of finishing a tile by itself: 2 % slower.)
 // The key range is found by every wave for itself, without LDS and a barrier: 64-token windows 22.9 -> 22.1.
 template <bool ALIBI>
 __device__ __forceinline__ void ForwardFewTiles(const AttP &p, uint8_t *kT0, uint8_t *kT1, uint8_t *vT0, uint8_t *vT1, const uint8_t *gk, const uint8_t *gv,
@@ -569,9 +571,9 @@ __device__ __forceinline__ void ForwardFewTiles(const AttP &p, uint8_t *kT0, uin
 // issues one instruction in five cycles.  So the kernel saves instructions: the exponential's argument is one fused multiply-add of the raw
 // product, the running maximum is taken once per tile of 64 keys, masks are a pass of their own over the tiles that need one.  And it overlaps:
 // S of tile i + 1 is formed between the exponentials of tile i, its maximum between the products with V, operands are requested six products
-// ahead.  16 x 2048 tokens causal, 16 heads: 396 -> 361 us; one sequence of 2048 tokens, one head 54.1 -> 43.7.  A reference that lags the
-// maximum by up to 2^8 saves most of the rescaling (another 4 and 7 %), but then the largest weight is rounded like any other: against fp64
-// 0.00221 instead of 0.00220, and 0.0020 instead of 0.0018 on peaked weights.
+// ahead.  16 x 2048 tokens causal, 16 heads: 396 -> 361 us (404 -> 376 on another card); one sequence of 2048 tokens, one head 54.1 -> 43.7.
+// A reference that lags the maximum by up to 2^8 saves most of the rescaling (another 4 and 7 %), but then the largest weight is rounded like
+// any other: against fp64 0.00221 instead of 0.00220, and 0.0020 instead of 0.0018 on peaked weights.
 template <bool ALIBI> __global__ void __launch_bounds__(256, 2) AttForward(AttP p)
 {
     constexpr int FEW = 7; // key tiles up to which ForwardFewTiles is the faster one

@@ -451,7 +451,8 @@ extern "C" int ts2_matmul_forward_norm_rope(int32_t mode, int32_t len, int32_t l
 // Time of a delta product in microseconds.  Both kernels walk their contraction at the rate one CU can fill its LDS from the caches, so a
 // launch is (rounds of 256 workgroups) x (start and epilogue + steps): 0.7 us per 256-byte step on 64x128 for the kernel for few tiles, 1.17 us
 // per 128-byte step on 256x256 for the ring kernel (2048 x 2048 over 8192 rows: 61 us / 75 us measured, 53 / 81 by this).  Slices add a
-// write and a read of fp32 per slice (4 TB/s from the caches) and the packing launch.
+// write and a read of fp32 per slice (4 TB/s from the caches) and the packing launch: fitted to a packing kernel that asked for one slice after
+// the other (512 x 512 of 8 slices: 7.7 us by this, of which packing took 6.0 and now takes 3.2), so the counts are on the low side.
 static double DeltaCost(bool ring, int64_t tiles, int64_t rowBytes, int splits, double outElems)
 {
     const double rounds = (double)((tiles * splits + 255) / 256);
