@@ -8,6 +8,7 @@
 // coalesced 512-byte (fp32) runs.  The reference launches one 32-thread block per (tile, row) (src/lib/cuda/cuda_graph.cuh:359-365).
 #include "vec.h"
 #include "internal.h"
+#include <algorithm>
 
 namespace
 {
@@ -947,18 +948,20 @@ __global__ void __launch_bounds__(256) NormalizeRowsWave(int len, int lenRound, 
 // operands contraction-major).  A workgroup takes QT_ROWS rows, which lie in one k-tile; rows in [len, lenRound) are cleared.  blockIdx.y =
 // source; tileScale: [sources][lenRound / kTile].  Rows per workgroup 32 -> 8: 512 x 1024, two gradients 13.1 -> 5.3 us; 16384 x 512 9.6 -> 7.9
 constexpr int QT_ROWS = 8;
-struct TileQuantJobs {
-    Mat src[4], dst[4];
-    const float *rowAbsMax[4];
-    uint32_t seed[4];
+constexpr int QT_JOBS = 48; // most sources of a launch (56 bytes of its arguments each)
+template <int COUNT> struct TileQuantJobs {
+    TileQuantJob job[COUNT];
 };
 
-__global__ void __launch_bounds__(256) QuantTileRows(int len, int lenRound, int dim, int kTile, TileQuantJobs jobs, const float *rowMult, float *tileScale)
+template <int COUNT>
+__global__ void __launch_bounds__(256) QuantTileRows(int len, int lenRound, int kTile, TileQuantJobs<COUNT> jobs, const float *rowMult)
 {
     __shared__ float red[4];
-    const Mat src = jobs.src[blockIdx.y], dst = jobs.dst[blockIdx.y];
-    const float *rowAbsMax = jobs.rowAbsMax[blockIdx.y];
-    const uint32_t seed = jobs.seed[blockIdx.y];
+    const TileQuantJob &job = jobs.job[blockIdx.y];
+    const Mat src = {(uint8_t *)job.src, job.srcStride}, dst = {job.dst, job.dstStride};
+    const float *rowAbsMax = job.rowAbsMax;
+    const uint32_t seed = job.seed;
+    const int dim = job.dim;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int t0 = blockIdx.x * QT_ROWS, k0 = t0 / kTile * kTile;
     float mx = 0;
@@ -977,7 +980,7 @@ __global__ void __launch_bounds__(256) QuantTileRows(int len, int lenRound, int 
     const float tm = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
     const float mult = tm > 0 ? 1 / (tm / 127) : 0.f;
     if (tid == 0 && t0 == k0) {
-        tileScale[blockIdx.y * (lenRound / kTile) + t0 / kTile] = tm > 0 ? tm / 127 : 1.f;
+        job.tileScale[t0 / kTile] = tm > 0 ? tm / 127 : 1.f;
     }
     // units of 8 elements, walked by the whole workgroup: four 16-byte loads in flight per lane
     const int perRow = dim / 8, units = QT_ROWS * perRow;
@@ -1857,29 +1860,53 @@ int Ts2QuantRowsBatch(int count, int len, int lenRound, const ts2_mat *src, cons
     return LaunchRowQuant(count, len, lenRound, dst[0].x, jobs, nullptr, stream);
 }
 
-// The row-major k-tile quantiser over `count` bf16 gradients of one shape; tileScale [count][lenRound / kTile]
+// The row-major k-tile quantiser over any number of bf16 gradients with the same rows
+int Ts2QuantTileRowsJobs(int count, int len, int lenRound, int kTile, const TileQuantJob *jobs, const float *rowMult, void *stream)
+{
+    if (count < 1 || lenRound < len || kTile <= 0 || kTile % 128 || lenRound % kTile) {
+        return TS2_ERR_SHAPE;
+    }
+    for (int i = 0; i < count; ++i) {
+        if (((uintptr_t)jobs[i].src | (uintptr_t)jobs[i].srcStride) & 15 || ((uintptr_t)jobs[i].dst | (uintptr_t)jobs[i].dstStride) & 7) {
+            return TS2_ERR_ALIGN;
+        }
+        if (jobs[i].dim <= 0 || jobs[i].dim % 8 || jobs[i].srcStride < jobs[i].dim * 2 || jobs[i].dstStride < jobs[i].dim) {
+            return TS2_ERR_SHAPE;
+        }
+    }
+    for (int done = 0; done < count; done += QT_JOBS) {
+        const int n = count - done < QT_JOBS ? count - done : QT_JOBS;
+        const dim3 grid(lenRound / QT_ROWS, n);
+        if (n <= 4) {
+            TileQuantJobs<4> part = {};
+            std::copy(jobs + done, jobs + done + n, part.job);
+            hipLaunchKernelGGL((QuantTileRows<4>), grid, dim3(256), 0, STREAM, len, lenRound, kTile, part, rowMult);
+        } else {
+            TileQuantJobs<QT_JOBS> part = {};
+            std::copy(jobs + done, jobs + done + n, part.job);
+            hipLaunchKernelGGL((QuantTileRows<QT_JOBS>), grid, dim3(256), 0, STREAM, len, lenRound, kTile, part, rowMult);
+        }
+        TS2_CHECK_LAUNCH();
+    }
+    return TS2_OK;
+}
+
+// ... over `count` gradients of one shape; tileScale [count][lenRound / kTile]
 int Ts2QuantTileRows(int count, int len, int lenRound, int kTile, const ts2_mat *src, const ts2_mat *dst, const float *const *rowAbsMax,
     const uint32_t *seed, const float *rowMult, float *tileScale, void *stream)
 {
     if (count < 1 || count > 4 || dst[0].x % 8 || lenRound < len || kTile <= 0 || kTile % 128 || lenRound % kTile) {
         return TS2_ERR_SHAPE;
     }
-    TileQuantJobs jobs = {};
+    TileQuantJob jobs[4];
     for (int i = 0; i < count; ++i) {
         if (dst[i].x != dst[0].x || !MatOk(&src[i], len, dst[0].x, 2) || !MatOk(&dst[i], lenRound, dst[0].x, 1)) {
             return TS2_ERR_SHAPE;
         }
-        if (!Aligned16(src[i].ptr, src[i].strideBytes) || (((uintptr_t)dst[i].ptr | dst[i].strideBytes) & 7)) {
-            return TS2_ERR_ALIGN;
-        }
-        jobs.src[i] = M(src[i]);
-        jobs.dst[i] = M(dst[i]);
-        jobs.rowAbsMax[i] = rowAbsMax[i];
-        jobs.seed[i] = seed[i];
+        jobs[i] = {(const uint8_t *)src[i].ptr, (uint8_t *)dst[i].ptr, src[i].strideBytes, dst[i].strideBytes, rowAbsMax[i],
+            tileScale + (int64_t)i * (lenRound / kTile), dst[0].x, seed[i]};
     }
-    hipLaunchKernelGGL(QuantTileRows, dim3(lenRound / QT_ROWS, count), dim3(256), 0, STREAM, len, lenRound, dst[0].x, kTile, jobs, rowMult, tileScale);
-    TS2_CHECK_LAUNCH();
-    return TS2_OK;
+    return Ts2QuantTileRowsJobs(count, len, lenRound, kTile, jobs, rowMult, stream);
 }
 
 extern "C" int ts2_normalize_vecs_row_max_dither(int32_t len, int32_t lenRound, const ts2_mat *src, int32_t srcType, const float *colScale,

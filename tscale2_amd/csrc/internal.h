@@ -26,12 +26,25 @@ int Ts2QuantRowsBatch(int count, int len, int lenRound, const ts2_mat *src, cons
 // tileScale [count][lenRound / kTile]
 int Ts2QuantTileRows(int count, int len, int lenRound, int kTile, const ts2_mat *src, const ts2_mat *dst, const float *const *rowAbsMax,
     const uint32_t *seed, const float *rowMult, float *tileScale, void *stream);
+// ... over any number of gradients with the same rows, each with a width and a place of its own
+struct TileQuantJob {
+    const uint8_t *src;
+    uint8_t *dst;
+    int64_t srcStride, dstStride; // bytes
+    const float *rowAbsMax;
+    float *tileScale; // [lenRound / kTile]
+    int dim;
+    uint32_t seed;
+};
+int Ts2QuantTileRowsJobs(int count, int len, int lenRound, int kTile, const TileQuantJob *jobs, const float *rowMult, void *stream);
 // packed delta [gradDim][srcDim] = alpha * *alphaPtr * sum over the rows of grad^T src, both operands row-major as they lie (rows len ..
 // lenRound of both hold zeros); mode TS2_I8 (with kTileScale [gradDim / kTileScaleRows][lenRound / kTile]; kTileScaleRows 0 = one set),
 // TS2_E4M3 or TS2_BF16.  Chooses kernel and token slices by cost; partial: fp32 scratch for the slices.  TS2_ERR_UNSUPPORTED: no kernel for it
 int Ts2DeltaRows(int mode, int len, int lenRound, int srcDim, int gradDim, const ts2_mat *src, const ts2_mat *grad, const float *kTileScale, int kTile,
     int kTileScaleRows, float alpha, const float *alphaPtr, float *partial, int64_t partialFloats, const ts2_mat *delta, const ts2_mat *tileScale,
     void *stream);
+// estimated microseconds of that (TS2_E4M3 or TS2_BF16)
+double Ts2DeltaCost(int mode, int lenRound, int srcDim, int gradDim, int64_t partialFloats);
 // int8: srcGrad (+)= sum_i alpha_i * *alphaPtr_i * rowScale_i[t] * (grad8_i W_i^T), count <= 4 products of one shape added in order
 int Ts2BackpropGroupI8(int count, int len, int lenRound, int srcDim, int gradDim, const ts2_mat *grad8, const float *const *rowScale,
     const ts2_mat *transformT, const float *alpha, const float *const *alphaPtr, const ts2_mat *srcGrad, int srcGradType, int add, void *stream);

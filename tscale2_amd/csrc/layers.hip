@@ -7,6 +7,7 @@
 // (matrix scales, 1/24 storage scales) because its optimiser normalises every delta, this driver keeps every factor of the CPU
 // path (src/gpt/compute/cpu_transformer.cpp, layer_*.cu CPU classes), so its deltas are directly comparable with the CPU oracle.
 #include "common.h"
+#include "gemm_deltas.h"
 #include "internal.h"
 #include <math.h>
 #include <string.h>
@@ -82,6 +83,12 @@ struct TLayer {
     // The packed deltas of the matrices that read the layer input (attention: Q, K, V, gate; FFN: expand, gate) are row blocks of one
     // array (and column blocks of one tile-scale array): one delta product over their gradients, which lie side by side, fills them all
     TMatrix stack;
+    // What the layer's deltas read, kept until all deltas of a backward pass run in one launch (TDeltaQueue); without storage the layer
+    // writes the shared scratch and its deltas run at once
+    Arr gradStack;          // fast-gradient type [R][stack.dstDim]: the gradients of the stacked matrices side by side
+    Arr quantStack, quantOut; // int8: quantised gradients of the stack and of the last matrix
+    float *rowAbsMax = 0;   // int8: [5][R], the last for the gradient of the last matrix
+    float *tileScale = 0;   // int8: [5][R / kTile]
 };
 
 enum { LT_ATT = 0, LT_FFN = 2, LT_MOE = 3 };
@@ -97,6 +104,15 @@ struct TActs {
     Arr val16;  // bf16 attention output (its storage is reused for dQ by the backward)
     Arr swl;    // fp32 [heads][R] softmax statistics
     bool valid = false;
+};
+
+// The packed deltas of attention and feed-forward layers are results of a backward pass that nothing in it reads.  While a model's
+// products have few tiles each, they wait for the end of the pass: one launch (per 32 matrices) of the kernel for few tiles then has tiles
+// enough for the whole chip, and int8 quantises all gradients in one launch before it
+struct TDeltaQueue {
+    bool open = false; // inside ModelBackprop of a model that keeps its gradients
+    std::vector<gemmk::DeltaJob> deltas;
+    std::vector<TileQuantJob> quants;
 };
 } // namespace
 
@@ -150,6 +166,9 @@ struct ts2_model {
     // linear backward scratch
     uint8_t *sGrad8 = 0, *sGradT = 0, *sSrcT = 0, *sWT = 0;
     int stackW = 0; // columns of the gradient scratch sGradT (and sGrad8): maxW, or the stacked gradients of a layer
+    std::vector<Arr> stepFast; // fast state gradient entering each step of the backward pass (own storage where deltas wait for its end)
+    Arr fast;                  // the one the layer backward reads
+    TDeltaQueue queue;
     Arr lastFast[4]; // where the layer backward that ran last left its fast-type gradients
     float *sPartial = 0;                     // fp32 slices of a delta product with few output tiles
     size_t sPartialFloats = 0;
@@ -270,8 +289,9 @@ int BackpropDX(ts2_model *M, TMatrix &W, const Arr &gradFast, float alpha, bool 
 
 // srcGrad (+)= sum_i alpha [* scale_i] * grad_i * W_i for the matrices of a layer that share their input: every weight is transposed
 // into its own part of the transpose scratch, then one grouped Backprop
+// (int8: the row maxima of gradient i go to rowAbsMax + i * RP, the shared scratch where it is null)
 int BackpropDXGroup(ts2_model *M, int count, TMatrix *const *W, const Arr *const *grad, float alpha, const bool *useScale, const Arr &srcGrad,
-    bool add, void *s)
+    bool add, float *rowAbsMax, void *s)
 {
     ts2_matmul_bwd_buffers b[4];
     const ts2_matmul_bwd_buffers *bp[4];
@@ -294,7 +314,7 @@ int BackpropDXGroup(ts2_model *M, int count, TMatrix *const *W, const Arr *const
             g16[i] = grad[i]->m;
             g8[i] = Flat(M->sGrad8 + (size_t)i * M->R * dstDim, M->R, dstDim, TS2_I8).m;
             rs[i] = M->sRowScale + (size_t)i * M->RP;
-            ram[i] = M->sRowAbsMax + (size_t)i * M->RP;
+            ram[i] = rowAbsMax ? rowAbsMax + (size_t)i * M->R : M->sRowAbsMax + (size_t)i * M->RP;
             seed[i] = NextDither(M);
             al[i] = alpha;
             ap[i] = useScale[i] ? W[i]->scale : nullptr;
@@ -344,16 +364,72 @@ Arr ColBlock(const Arr &a, int k, int cols)
 // fp8: `grad` holds the gradients side by side ([R][count * width]) and the product reads both operands as they lie.
 // int8: grads[i] are bf16; their row maxima were left in slot i by the dX product that precedes this call (BackpropDXGroup with the
 // same gradients), the k-tile quantiser writes them side by side.
-int BackpropDelta(ts2_model *M, TMatrix &W, const Arr &src8, const Arr &grad, float alpha, const float *gradScale, void *s)
+// A delta whose operands stay as they are until the end of the pass joins the queue (kept).
+bool QueueDelta(ts2_model *M, TMatrix &W, const Arr &src8, const Arr &grad, const float *kTileScale, int kTileScaleRows, float alpha,
+    const float *gradScale)
 {
+    gemmk::DeltaJob d = {};
+    d.grad = (const uint8_t *)grad.m.ptr;
+    d.src = (const uint8_t *)src8.m.ptr;
+    d.delta = (uint8_t *)W.delta.m.ptr;
+    d.tileScale = (float *)W.deltaTileScale.m.ptr;
+    d.alphaPtr = gradScale;
+    d.kTileScale = kTileScale;
+    d.alpha = alpha;
+    d.ldGrad = (int)grad.m.strideBytes;
+    d.ldSrc = (int)src8.m.strideBytes;
+    d.ldDelta = (int)W.delta.m.strideBytes;
+    d.ldTileScale = (int)(W.deltaTileScale.m.strideBytes / 4);
+    d.gradDim = W.dstDim;
+    d.srcDim = W.srcDim;
+    d.kTileScaleRows = kTileScaleRows;
+    if (!gemmk::DeltaBatchCanRun(d, M->mode == TS2_I8 ? gemmk::T_I8 : gemmk::T_FP8, M->R, M->len, M->kTile)) {
+        return false;
+    }
+    M->queue.deltas.push_back(d);
+    return true;
+}
+
+int RunQueue(ts2_model *M, void *s)
+{
+    TDeltaQueue &q = M->queue;
+    q.open = false;
+    if (!q.quants.empty()) {
+        CK(Ts2QuantTileRowsJobs((int)q.quants.size(), M->len, M->R, M->kTile, q.quants.data(), nullptr, s));
+    }
+    return gemmk::RunDeltaBatch(q.deltas.data(), (int)q.deltas.size(), M->mode == TS2_I8 ? gemmk::T_I8 : gemmk::T_FP8, M->R, M->len, M->kTile,
+        (hipStream_t)s);
+}
+
+int BackpropDelta(ts2_model *M, TMatrix &W, const Arr &src8, const Arr &grad, float alpha, const float *gradScale, bool kept, void *s)
+{
+    if (kept && QueueDelta(M, W, src8, grad, nullptr, 0, alpha, gradScale)) {
+        return 0;
+    }
     return Ts2DeltaRows(M->mode, M->len, M->R, W.srcDim, W.dstDim, src8.P(), grad.P(), nullptr, 0, 0, alpha, gradScale, M->sPartial,
         (int64_t)M->sPartialFloats, W.delta.P(), W.deltaTileScale.P(), s);
 }
 
+// keep: the layer whose kept gradients these are (null: none); slot: their first row maxima and scales in it
 int BackpropDeltaI8(ts2_model *M, int count, TMatrix &stack, TMatrix *const *W, const Arr &src8, const Arr *const *grads, float alpha,
-    const float *gradScale, void *s)
+    const float *gradScale, TLayer *keep, int slot, void *s)
 {
     const int width = W[0]->dstDim, all = count * width;
+    if (keep && width <= QUANT_ROW_MAX && all <= M->stackW) {
+        const int nTiles = M->R / M->kTile;
+        const Arr g = slot ? keep->quantOut : keep->quantStack;
+        float *const scales = keep->tileScale + (size_t)slot * nTiles;
+        if (QueueDelta(M, stack, src8, g, scales, width, alpha, gradScale)) {
+            for (int i = 0; i < count; ++i) {
+                const Arr q = ColBlock(g, i, width);
+                M->queue.quants.push_back({(const uint8_t *)grads[i]->m.ptr, (uint8_t *)q.m.ptr, grads[i]->m.strideBytes, q.m.strideBytes,
+                    keep->rowAbsMax + (size_t)(slot + i) * M->R, scales + (size_t)i * nTiles, width, NextDither(M)});
+            }
+            return 0;
+        }
+    }
+    float *const rowMax = keep ? keep->rowAbsMax + (size_t)slot * M->R : M->sRowAbsMax;
+    const size_t rowMaxStride = keep ? M->R : M->RP;
     if (width <= QUANT_ROW_MAX && all <= M->stackW) {
         const int nTiles = (M->R / M->kTile + 3) / 4;
         if (nTiles == 1 || (size_t)nTiles * all * W[0]->srcDim <= M->sPartialFloats) {
@@ -364,7 +440,7 @@ int BackpropDeltaI8(ts2_model *M, int count, TMatrix &stack, TMatrix *const *W, 
             for (int i = 0; i < count; ++i) {
                 g16[i] = grads[i]->m;
                 g8[i] = ColBlock(g, i, width).m;
-                ram[i] = M->sRowAbsMax + (size_t)i * M->RP;
+                ram[i] = rowMax + i * rowMaxStride;
                 seed[i] = NextDither(M);
             }
             CK(Ts2QuantTileRows(count, M->len, M->R, M->kTile, g16, g8, ram, seed, nullptr, M->sTileScale, s));
@@ -381,7 +457,7 @@ int BackpropDeltaI8(ts2_model *M, int count, TMatrix &stack, TMatrix *const *W, 
         ts2_matmul_bwd_buffers b = Scratch(M, M->R, W[i]->srcDim, W[i]->dstDim);
         b.srcTValid = i > 0;
         if (width <= QUANT_ROW_MAX && all <= M->stackW) {
-            b.gradRowAbsMax = M->sRowAbsMax + (size_t)i * M->RP;
+            b.gradRowAbsMax = rowMax + i * rowMaxStride;
             b.gradRowAbsMaxValid = 1;
         }
         CK(ts2_matmul_backprop_delta(M->mode, M->len, M->R, W[i]->srcDim, W[i]->dstDim, src8.P(), nullptr, grads[i]->P(), grads[i]->type, alpha,
@@ -437,8 +513,9 @@ int FfnBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
     // drg travels in bf16 (the reference uses half here): its consumer rounds to the 8-bit gradient type anyway
     Arr drg = View(M->g16[0], R, F), dwide = View(M->gf[0], R, F), dgate = View(M->gf[1], R, F);
     const bool i8 = M->mode == TS2_I8;
-    Arr gStack = Flat(M->sGradT, R, 2 * F, M->fastGradType);
-    if (!i8) { // the two gradients side by side
+    TLayer *const keep = M->queue.open && L.gradStack.m.ptr ? &L : nullptr;
+    Arr gStack = keep ? L.gradStack : Flat(M->sGradT, R, 2 * F, M->fastGradType);
+    if (!i8 || keep) { // the two gradients side by side
         dwide = ColBlock(gStack, 0, F);
         dgate = ColBlock(gStack, 1, F);
     }
@@ -448,16 +525,17 @@ int FfnBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
     }
     // contract backward: dX, then the delta (its source is stored in 1/24 units)
     TMatrix *const wc[1] = {&L.w[2]};
-    const Arr *const sg[1] = {&M->stateGradFast};
+    const Arr *const sg[1] = {&M->fast};
     const bool scaled[2] = {true, false};
-    CK(BackpropDXGroup(M, 1, wc, sg, DISCR * Dot(F), scaled, drg, false, s));
-    CK(i8 ? BackpropDeltaI8(M, 1, L.w[2], wc, rg8, sg, VEC, gradScale, s) : BackpropDelta(M, L.w[2], rg8, M->stateGradFast, VEC, gradScale, s));
+    CK(BackpropDXGroup(M, 1, wc, sg, DISCR * Dot(F), scaled, drg, false, keep ? L.rowAbsMax + (size_t)4 * R : nullptr, s));
+    CK(i8 ? BackpropDeltaI8(M, 1, L.w[2], wc, rg8, sg, VEC, gradScale, keep, 4, s) : BackpropDelta(M, L.w[2], rg8, M->fast, VEC, gradScale, keep != nullptr, s));
     CK(ts2_backprop_row_tile_normalize_lolu(len, R, gate16.P(), wide16.P(), VEC, wideScale.P(), drg.P(), TS2_BF16, dgate.P(), dwide.P(),
         M->fastGradType, s));
     TMatrix *const ws[2] = {&L.w[0], &L.w[1]};
     const Arr *const gs[2] = {&dwide, &dgate};
-    CK(BackpropDXGroup(M, 2, ws, gs, DISCR * Dot(D), scaled, M->dNormState, false, s));
-    return i8 ? BackpropDeltaI8(M, 2, L.stack, ws, norm8, gs, VEC, gradScale, s) : BackpropDelta(M, L.stack, norm8, gStack, VEC, gradScale, s);
+    CK(BackpropDXGroup(M, 2, ws, gs, DISCR * Dot(D), scaled, M->dNormState, false, keep ? L.rowAbsMax : nullptr, s));
+    return i8 ? BackpropDeltaI8(M, 2, L.stack, ws, norm8, gs, VEC, gradScale, keep, 0, s)
+              : BackpropDelta(M, L.stack, norm8, gStack, VEC, gradScale, keep != nullptr, s);
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
@@ -521,8 +599,9 @@ int AttBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
     Arr dQf = View(M->gf[0], R, Q), dGate = View(M->gf[1], R, Q), dKf = View(M->gf[2], R, Q), dVf = View(M->gf[3], R, Q);
     const bool i8 = M->mode == TS2_I8;
     // fp8: the gradients of the four matrices that read the layer input side by side, as column blocks of one [R][4Q] array
-    Arr gStack = Flat(M->sGradT, R, 4 * Q, M->fastGradType);
-    if (!i8) {
+    TLayer *const keep = M->queue.open && L.gradStack.m.ptr ? &L : nullptr;
+    Arr gStack = keep ? L.gradStack : Flat(M->sGradT, R, 4 * Q, M->fastGradType);
+    if (!i8 || keep) {
         dQf = ColBlock(gStack, 0, Q);
         dKf = ColBlock(gStack, 1, Q);
         dVf = ColBlock(gStack, 2, Q);
@@ -535,10 +614,11 @@ int AttBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
     A.valid = false; // the backward reuses val16's storage for dQ
     // combiner backward
     TMatrix *const wc[1] = {&L.w[4]};
-    const Arr *const sg[1] = {&M->stateGradFast};
+    const Arr *const sg[1] = {&M->fast};
     const bool useScale[4] = {true, true, true, false};
-    CK(BackpropDXGroup(M, 1, wc, sg, DISCR * Dot(Q), useScale, dvlg, false, s));
-    CK(i8 ? BackpropDeltaI8(M, 1, L.w[4], wc, vlg8, sg, VEC, gradScale, s) : BackpropDelta(M, L.w[4], vlg8, M->stateGradFast, VEC, gradScale, s));
+    CK(BackpropDXGroup(M, 1, wc, sg, DISCR * Dot(Q), useScale, dvlg, false, keep ? L.rowAbsMax + (size_t)4 * R : nullptr, s));
+    CK(i8 ? BackpropDeltaI8(M, 1, L.w[4], wc, vlg8, sg, VEC, gradScale, keep, 4, s)
+          : BackpropDelta(M, L.w[4], vlg8, M->fast, VEC, gradScale, keep != nullptr, s));
     // gate backward + dScale
     CK(ts2_backprop_lolu_dscale(len, R, gate16.P(), val16.P(), 1.f, dvlg.P(), TS2_BF16, dGate.P(), M->fastGradType, dVal16.P(), TS2_BF16,
         M->dScale.P(), s));
@@ -573,8 +653,9 @@ int AttBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
     CK(Ts2BackpropNormRopeGroup(3, len, R, nrGrad, TS2_BF16, 1.f, nrNorm, nrScale, nrRope, nrDst, M->fastGradType, s));
     TMatrix *const ws[4] = {&L.w[0], &L.w[1], &L.w[2], &L.w[3]};
     const Arr *const gs[4] = {&dQf, &dKf, &dVf, &dGate};
-    CK(BackpropDXGroup(M, 4, ws, gs, DISCR * Dot(D), useScale, M->dNormState, false, s));
-    return i8 ? BackpropDeltaI8(M, 4, L.stack, ws, norm8, gs, VEC, gradScale, s) : BackpropDelta(M, L.stack, norm8, gStack, VEC, gradScale, s);
+    CK(BackpropDXGroup(M, 4, ws, gs, DISCR * Dot(D), useScale, M->dNormState, false, keep ? L.rowAbsMax : nullptr, s));
+    return i8 ? BackpropDeltaI8(M, 4, L.stack, ws, norm8, gs, VEC, gradScale, keep, 0, s)
+              : BackpropDelta(M, L.stack, norm8, gStack, VEC, gradScale, keep != nullptr, s);
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
@@ -689,7 +770,7 @@ int MoeBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
     TActs &A = M->shared;
     Arr wide16 = View(A.a16[0], RM, X), gate16 = View(A.a16[1], RM, X), wideScale = View(A.tsc[0], X / 128, RM), rg8 = View(A.rg8, RM, X);
     // state gradient into expert order
-    CK(ts2_moe_group_samples(RM, 1, M->stateGradFast.P(), M->moe.xpSampleId, M->sgMoe.P(), s));
+    CK(ts2_moe_group_samples(RM, 1, M->fast.P(), M->moe.xpSampleId, M->sgMoe.P(), s));
     // contract backward: dRG[row][x] = sum_d sg[row][d] Wc_e[d][x]: needs Wc_e^T = [X][D] per expert
     // (the experts' transposed matrices are kept from one backward to the next like the dense layers', and redone when a matrix is set
     // or updated)
@@ -723,7 +804,7 @@ int MoeBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
     // select matrix: dNormState += dMoe * Wsel / sqrt(D) and its delta through the same 8-bit operator as every other matrix (the
     // reference uses its fp16 kernels here, MatmulSelect.BackpropFp16, layer_moe.cu:264); rows >= experts of the matrix are zero
     CK(BackpropDX(M, L.w[3], M->dMoeSel, DISCR * Dot(D), false, M->dNormState, true, s));
-    CK(BackpropDelta(M, L.w[3], norm8, M->dMoeSel, VEC, gradScale, s));
+    CK(BackpropDelta(M, L.w[3], norm8, M->dMoeSel, VEC, gradScale, false, s));
     // expert deltas
     CK(GroupedDelta(M, L.w[2], rg8, M->sgMoe, VEC, gradScale, s));
     CK(GroupedDelta(M, L.w[0], M->normMoe, dwide, VEC, gradScale, s));
@@ -871,7 +952,7 @@ int FinalBackward(ts2_model *M, void *s)
         CK(Ts2DeltaRows(TS2_BF16, M->len, R, D, VP, fn16.P(), M->gradV.P(), nullptr, 0, 0, VEC, nullptr, M->sPartial, (int64_t)M->sPartialFloats,
             M->finalW.delta.P(), M->finalW.deltaTileScale.P(), s));
         return ts2_backprop_final_normalize(M->len, R, M->normState[depth].P(), M->mode, M->stateScale[depth].P(), M->dNormState.P(),
-            M->stateGrad.P(), M->stateGradFast.P(), M->fastGradType, M->gradMaxNorm, s);
+            M->stateGrad.P(), M->fast.P(), M->fastGradType, M->gradMaxNorm, s);
     }
     ts2_gemm_args h = {};
     h.a = M->gradV.m;
@@ -923,7 +1004,7 @@ int FinalBackward(ts2_model *M, void *s)
         CK(ts2_gemm_nt(&h, s));
     }
     return ts2_backprop_final_normalize(M->len, R, M->normState[depth].P(), M->mode, M->stateScale[depth].P(), M->dNormState.P(), M->stateGrad.P(),
-        M->stateGradFast.P(), M->fastGradType, M->gradMaxNorm, s);
+        M->fast.P(), M->fastGradType, M->gradMaxNorm, s);
 }
 
 // the transposes of the attention and feed-forward matrices that changed since they were made
@@ -966,26 +1047,119 @@ int ModelBackprop(ts2_model *M, void *s)
     CK(ModelForward(M, s));
     CK(Ts2ZeroRows(Flat(M->gradMaxNorm, 1, depth + 2, TS2_F32).P(), 1, (depth + 2) * 4, s));
     CK(Ts2FillFloats(M->gradMult, 1, 1.f, s)); // the multiplier the final normalisation applies to the fast gradient
+    M->fast = M->stepFast[0];
     CK(FinalBackward(M, s));
     CK(TransposeWeights(M, s));
     M->useKept = M->keep;
     struct TReset {
         ts2_model *M;
-        ~TReset() { M->useKept = false; }
+        ~TReset()
+        {
+            M->useKept = false;
+            M->queue.open = false;
+        }
     } reset = {M};
+    M->queue.deltas.clear();
+    M->queue.quants.clear();
+    M->queue.open = M->stepFast[0].m.ptr != M->stateGradFast.m.ptr;
     int stepId = 0;
     for (int d = depth - 1; d >= 0; --d, ++stepId) {
         float *prevMax = M->gradMaxNorm + stepId, *nextMax = M->gradMaxNorm + stepId + 1;
         float *gradScale = M->gradScale + stepId + 1, *gradMult = M->gradMult + stepId + 1;
         // the fast gradient is rewritten only when its power-of-two multiplier differs from the one its producer applied (the final
         // normalisation: 1, kept in gradMult[0]; a layer's normalisation backward: that layer's multiplier)
-        CK(ts2_scale_grad(prevMax, M->gradMult + stepId, M->stateGrad.P(), M->stateGradFast.P(), M->fastGradType, M->len, gradScale, gradMult, s));
+        M->fast = M->stepFast[stepId];
+        CK(ts2_scale_grad(prevMax, M->gradMult + stepId, M->stateGrad.P(), M->fast.P(), M->fastGradType, M->len, gradScale, gradMult, s));
         CK(LayerBackward(M, d, gradScale, s));
         CK(ts2_backprop_layer_normalize(M->normState[d].P(), M->mode, M->stateScale[d].P(), M->dNormState.P(), nullptr, gradScale, gradMult,
-            M->stateGrad.P(), M->stateGradFast.P(), M->fastGradType, nextMax, M->len, s));
+            M->stateGrad.P(), M->stepFast[stepId + 1].P(), M->fastGradType, nextMax, M->len, s));
+    }
+    if (M->queue.open) {
+        CK(RunQueue(M, s));
     }
     return Ts2EmbedBackward(M->len, D, M->labelPtr, M->labels, M->stateGrad.P(), Flat(M->embed.delta.m.ptr, M->cfg.labelCount, D, TS2_F32).P(),
         M->cfg.labelCount, s);
+}
+} // namespace
+
+namespace
+{
+// Whether the deltas of a backward pass wait for its end.  int8: always (the launch at the end reads both operands as they lie, quantised in one
+// launch; one by one they were slices of four k-tiles, or transposed: steps of three layer pairs, 512 to 1024 wide, over 2048 to 16384
+// tokens take 0.78 to 0.86 of the time, 2048 x 8192 over 8192 tokens 0.90).  e4m3: unless the products are so large that the 256x256 kernel fills the
+// chip with each (the same sizes 0.86 to 0.91, 1024 x 4096 over 16384 tokens, where the estimates below are equal, 0.98; 2048 x 8192 over 8192,
+// 1.8 times the estimate one by one, 1.02)
+bool DeltasWait(const ts2_model *M)
+{
+    if (M->mode == TS2_I8) {
+        return true;
+    }
+    double separate = 0;
+    int64_t tiles = 0;
+    auto add = [&](const TMatrix &W) {
+        separate += Ts2DeltaCost(M->mode, M->R, W.srcDim, W.dstDim, (int64_t)M->sPartialFloats) + 3;
+        tiles += (int64_t)((W.dstDim + 255) / 256) * (W.srcDim / 128);
+    };
+    for (const TLayer &L : M->layers) {
+        if (L.type != LT_MOE) {
+            add(L.stack);
+            add(L.type == LT_ATT ? L.w[4] : L.w[2]);
+        }
+    }
+    // a tile's step of 128 rows takes 1.1 us with all CUs at work
+    return tiles > 0 && (double)((tiles + 255) / 256) * (5 + 1.1 * (M->R / 128)) < 1.3 * separate;
+}
+
+// ... and the storage for that: gradients of every layer and the fast state gradient of every step, in one allocation of at most 16 GiB
+bool InitDeltaQueue(ts2_model *M)
+{
+    const int depth = (int)M->layers.size(), D = M->cfg.dim, R = M->R, nTiles = R / M->kTile;
+    const bool i8 = M->mode == TS2_I8;
+    M->stepFast.assign(depth + 1, M->stateGradFast);
+    if (!M->keep || !DeltasWait(M)) {
+        return true;
+    }
+    size_t bytes = 0;
+    uint8_t *base = nullptr;
+    auto take = [&](size_t n) -> uint8_t * {
+        uint8_t *p = base ? base + bytes : nullptr;
+        bytes += (n + 255) / 256 * 256;
+        return p;
+    };
+    auto layout = [&]() {
+        for (int k = 0; k < depth; ++k) {
+            M->stepFast[k].m.ptr = take((size_t)R * M->stateGradFast.m.strideBytes);
+        }
+        for (TLayer &L : M->layers) {
+            if (L.type == LT_MOE) {
+                continue;
+            }
+            const int all = L.stack.dstDim;
+            L.gradStack = Flat(take((size_t)R * all * ElemSz(M->fastGradType)), R, all, M->fastGradType);
+            if (i8) {
+                L.quantStack = Flat(take((size_t)R * all), R, all, TS2_I8);
+                L.quantOut = Flat(take((size_t)R * D), R, D, TS2_I8);
+                L.rowAbsMax = (float *)take((size_t)5 * R * 4);
+                L.tileScale = (float *)take((size_t)5 * nTiles * 4);
+            }
+        }
+    };
+    layout(); // sizes
+    size_t freeB = 0, totalB = 0;
+    if (bytes > ((size_t)16 << 30) || hipMemGetInfo(&freeB, &totalB) != hipSuccess || bytes > freeB / 4) {
+        for (TLayer &L : M->layers) {
+            L.gradStack = Arr();
+        }
+        M->stepFast.assign(depth + 1, M->stateGradFast);
+        return true;
+    }
+    base = (uint8_t *)M->Dev(bytes);
+    if (!base) {
+        return false;
+    }
+    bytes = 0;
+    layout();
+    return true;
 }
 } // namespace
 
@@ -1172,6 +1346,7 @@ extern "C" ts2_model *ts2_model_create(const ts2_model_config *cfg)
     }
     ok &= M->Alloc(&M->logits, R, VP, TS2_F32) && M->Alloc(&M->logits16, R, VP, TS2_F16) && M->Alloc(&M->gradV, R, VP, TS2_BF16) &&
           M->Alloc(&M->fnT, D, R, TS2_BF16) && M->Alloc(&M->wfT, D, VP, TS2_BF16);
+    ok = ok && InitDeltaQueue(M);
     if (!ok || !M->sGrad8 || !M->sGradT || !M->sSrcT || !M->sWT || !M->sPartial) {
         delete M;
         return nullptr;
@@ -1432,8 +1607,12 @@ extern "C" int ts2_model_set_batch(ts2_model *M, int32_t len, const int32_t *lab
     if (stream && hipStreamSynchronize((hipStream_t)stream) != hipSuccess) {
         return TS2_ERR_LAUNCH;
     }
-    if (len < M->len && Ts2ZeroRows(M->stateGradFast.P(), M->R, M->cfg.dim * ElemSz(M->fastGradType), stream) != TS2_OK) {
-        return TS2_ERR_LAUNCH; // rows beyond the batch hold zeros: the delta products contract over whole tiles of rows
+    for (size_t i = 0; len < M->len && i < M->stepFast.size(); ++i) {
+        // rows beyond the batch hold zeros: the delta products contract over whole tiles of rows
+        if ((i + 1 == M->stepFast.size() || M->stepFast[i].m.ptr != M->stateGradFast.m.ptr) &&
+            Ts2ZeroRows(M->stepFast[i].P(), M->R, M->cfg.dim * ElemSz(M->fastGradType), stream) != TS2_OK) {
+            return TS2_ERR_LAUNCH;
+        }
     }
     M->len = len;
     int R = M->R;
@@ -1484,6 +1663,7 @@ extern "C" int ts2_layer_backward(ts2_model *M, int32_t layer, void *stream)
     if (!M || M->len <= 0 || layer < 0 || layer >= (int)M->layers.size()) {
         return TS2_ERR_NULL;
     }
+    M->fast = M->stateGradFast;
     // gradient scale bookkeeping of one step of the backward loop, fed from stateGrad as it stands
     CK(ts2_scale_grad(M->gradMaxNorm, nullptr, M->stateGrad.P(), M->stateGradFast.P(), M->fastGradType, M->len, M->gradScale, M->gradMult, stream));
     CK(LayerBackward(M, layer, M->gradScale, stream));

@@ -460,11 +460,46 @@ static double DeltaCost(bool ring, int64_t tiles, int64_t rowBytes, int splits, 
     return rounds * (ring ? 6 + 1.17 * steps : 4 + 0.7 * steps) + (splits > 1 ? 3.5 + splits * outElems * 8 / 4e6 : 0);
 }
 
+// the cheapest of the forms of a delta product: kernel and slices; `ringRuns`: the ring kernel takes its operands
+static double CheapestDelta(int mode, int lenRound, int srcDim, int gradDim, int64_t partialFloats, bool ringRuns, bool *ring, int *splits)
+{
+    const int64_t outElems = (int64_t)gradDim * srcDim, sliceTiles = (int64_t)(gradDim / 64) * (srcDim / 128);
+    const int64_t rowBytes = (int64_t)lenRound * (mode == TS2_BF16 ? 2 : 1);
+    double best = 1e30;
+    *ring = false;
+    *splits = 1;
+    for (int s = 1; s <= 32 && (s == 1 || s * outElems <= partialFloats); s *= 2) {
+        if (s > 1 && rowBytes / s < 512) {
+            break;
+        }
+        double c = DeltaCost(false, sliceTiles, rowBytes, s, (double)outElems);
+        if (c < best) {
+            best = c;
+            *ring = false;
+            *splits = s;
+        }
+        c = DeltaCost(true, sliceTiles / 8, rowBytes, s, (double)outElems);
+        if (ringRuns && c < best) {
+            best = c;
+            *ring = true;
+            *splits = s;
+        }
+    }
+    return best;
+}
+
+double Ts2DeltaCost(int mode, int lenRound, int srcDim, int gradDim, int64_t partialFloats)
+{
+    bool ring;
+    int splits;
+    return CheapestDelta(mode, lenRound, srcDim, gradDim, partialFloats, gradDim % 256 == 0 && srcDim % 256 == 0, &ring, &splits);
+}
+
 int Ts2DeltaRows(int mode, int len, int lenRound, int srcDim, int gradDim, const ts2_mat *src, const ts2_mat *grad, const float *kTileScale, int kTile,
     int kTileScaleRows, float alpha, const float *alphaPtr, float *partial, int64_t partialFloats, const ts2_mat *delta, const ts2_mat *tileScale,
     void *stream)
 {
-    const int64_t outElems = (int64_t)gradDim * srcDim, sliceTiles = (int64_t)(gradDim / 64) * (srcDim / 128);
+    const int64_t outElems = (int64_t)gradDim * srcDim;
     if (mode == TS2_I8) {
         // up to four k-tiles per workgroup
         const int splits = (lenRound / kTile + 3) / 4;
@@ -474,28 +509,10 @@ int Ts2DeltaRows(int mode, int len, int lenRound, int srcDim, int gradDim, const
         return DeltaSlice(mode, len, lenRound, srcDim, gradDim, src, grad, kTileScale, kTile, kTileScaleRows, alpha, alphaPtr, splits, partial, delta,
             tileScale, stream);
     }
-    const int64_t rowBytes = (int64_t)lenRound * (mode == TS2_BF16 ? 2 : 1);
-    const bool ringRuns = (gradDim % 256) == 0 && (srcDim % 256) == 0 && grad->y >= lenRound && src->y >= lenRound;
-    double best = 1e30;
-    bool ring = false;
-    int splits = 1;
-    for (int s = 1; s <= 32 && (s == 1 || s * outElems <= partialFloats); s *= 2) {
-        if (s > 1 && rowBytes / s < 512) {
-            break;
-        }
-        double c = DeltaCost(false, sliceTiles, rowBytes, s, (double)outElems);
-        if (c < best) {
-            best = c;
-            ring = false;
-            splits = s;
-        }
-        c = DeltaCost(true, sliceTiles / 8, rowBytes, s, (double)outElems);
-        if (ringRuns && c < best) {
-            best = c;
-            ring = true;
-            splits = s;
-        }
-    }
+    bool ring;
+    int splits;
+    CheapestDelta(mode, lenRound, srcDim, gradDim, partialFloats, (gradDim % 256) == 0 && (srcDim % 256) == 0 && grad->y >= lenRound && src->y >= lenRound,
+        &ring, &splits);
     if (!ring) {
         return DeltaSlice(mode, len, lenRound, srcDim, gradDim, src, grad, nullptr, 0, 0, alpha, alphaPtr, splits, partial, delta, tileScale, stream);
     }
