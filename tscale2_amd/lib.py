@@ -32,8 +32,10 @@ def mat(t):
     """2-D view of a torch tensor (row-major, last dim contiguous)."""
     if t is None:
         return Mat(None, 0, 0, 0)
-    assert t.dim() == 2 and t.stride(1) == 1, "ts2_mat needs a row-major 2-D tensor"
-    return Mat(t.data_ptr(), t.stride(0) * t.element_size(), t.shape[1], t.shape[0])
+    stride = t.stride()
+    assert len(stride) == 2 and stride[1] == 1, "ts2_mat needs a row-major 2-D tensor"
+    rows, cols = t.shape
+    return Mat(t.data_ptr(), stride[0] * t.element_size(), cols, rows)
 
 
 def ptr(t):
@@ -56,8 +58,11 @@ class Lib:
 
     @staticmethod
     def stream():
+        # torch.cuda.current_stream() without the stream object it makes (4 of the 12 us that a call of eight arguments took)
         import torch
-        return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+        if not torch.cuda.is_initialized():
+            torch.cuda.init()
+        return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
 
     def check(self, rc, what):
         if rc != 0:
@@ -104,27 +109,23 @@ _lib = None
 
 
 def load():
-    global _lib
+    global _lib, _tensor
     if _lib is None:
         _lib = Lib()
+        import torch
+        _tensor = torch.Tensor
     return _lib
 
 
-def _conv(a, keep):
-    """torch 2-D tensor -> ts2_mat*, 1-D/0-D tensor -> raw device pointer, float -> c_float, int -> c_int32, None -> NULL."""
-    import torch
-    if a is None:
-        return None
-    if isinstance(a, torch.Tensor):
-        if a.dim() == 2:
-            m = mat(a)
-            keep.append(m)
-            return C.byref(m)
-        return C.c_void_p(a.data_ptr())
-    if isinstance(a, bool):
-        return C.c_int32(int(a))
-    if isinstance(a, int):
-        return C.c_int32(a)
+_tensor = None
+
+
+def _conv(a):
+    """torch 2-D tensor -> ts2_mat*, 1-D/0-D tensor -> raw device pointer, float -> c_float; int (a C int) and None (NULL) as they are"""
+    if a is None or isinstance(a, int):
+        return a
+    if isinstance(a, _tensor):
+        return C.byref(mat(a)) if a.dim() == 2 else C.c_void_p(a.data_ptr())  # (the reference keeps its matrix)
     if isinstance(a, float):
         return C.c_float(a)
     return a
@@ -133,9 +134,7 @@ def _conv(a, keep):
 def call(name, *args, check=True):
     """Invoke an entry point of the C ABI on torch's current stream (appended as the last argument)."""
     lib = load()
-    keep = []
-    cargs = [_conv(a, keep) for a in args]
-    rc = getattr(lib.dll, name)(*cargs, lib.stream())
+    rc = getattr(lib.dll, name)(*[_conv(a) for a in args], lib.stream())
     if check and rc != 0:
         raise RuntimeError(f"{name} failed with code {rc}")
     return rc
