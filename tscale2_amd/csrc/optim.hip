@@ -182,7 +182,8 @@ __global__ void __launch_bounds__(256) AddGradient(int xSize, int ySize, DeltaSr
 
 // first half of ConvertMatrixKernel (agpu_cuda.cuh:65-101): sko = rms of the whole matrix from the row sums, mult = 32 / sko (0 for a zero
 // matrix).  The reference recomputes this in every workgroup of the conversion; here one small launch leaves both scalars on the device.
-__device__ __forceinline__ void MatrixSkoBlock(int totalXSize, int totalYSize, const float *sum2arr, float *resDiscrScale, float *convertMult, float *red)
+// (1024 threads; every thread gets the result)
+__device__ __forceinline__ float MatrixSkoOf(int totalXSize, int totalYSize, const float *sum2arr, float *red)
 {
     float sum2 = 0;
     for (int k = threadIdx.x; k < totalYSize; k += 1024) {
@@ -193,22 +194,26 @@ __device__ __forceinline__ void MatrixSkoBlock(int totalXSize, int totalYSize, c
         red[threadIdx.x >> 6] = sum2;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        float tot = 0;
-        for (int i = 0; i < 16; ++i) {
-            tot += red[i];
-        }
-        float sko = sqrtf(tot / ((float)totalXSize * (float)totalYSize));
-        float discrScale = sko * (1 / 32.f); // MODEL_DISCR_SCALE, src/gpt/model_params/model_dim.h:9
-        convertMult[0] = sko == 0 ? 0.f : 1 / discrScale;
-        resDiscrScale[0] = sko;
+    float tot = 0;
+    for (int i = 0; i < 16; ++i) {
+        tot += red[i];
     }
+    return sqrtf(tot / ((float)totalXSize * (float)totalYSize));
+}
+
+__device__ __forceinline__ float ConvertMultOf(float sko)
+{
+    return sko == 0 ? 0.f : 1 / (sko * (1 / 32.f)); // MODEL_DISCR_SCALE, src/gpt/model_params/model_dim.h:9
 }
 
 __global__ void __launch_bounds__(1024) MatrixSko(int totalXSize, int totalYSize, const float *sum2arr, float *resDiscrScale, float *convertMult)
 {
     __shared__ float red[16];
-    MatrixSkoBlock(totalXSize, totalYSize, sum2arr, resDiscrScale, convertMult, red);
+    const float sko = MatrixSkoOf(totalXSize, totalYSize, sum2arr, red);
+    if (threadIdx.x == 0) {
+        convertMult[0] = ConvertMultOf(sko);
+        resDiscrScale[0] = sko;
+    }
 }
 
 // second half: fast = cvt(weights * mult), rows ySize .. yBufSize cleared
@@ -236,9 +241,9 @@ __global__ void __launch_bounds__(256) ConvertMatrix(int xSize, int ySize, int y
     }
 }
 
-// ---- "one delta, apply now" with a dispersion estimate per row, over up to OPT_JOBS matrices in three launches: rows, matrix scale,
-// conversion.  Small matrices are bound by launches (a 512 x 512 one took five of 2 to 4 us each), large ones by the second read of the
-// delta and by the two single-workgroup launches.
+// ---- "one delta, apply now" with a dispersion estimate per row, over up to OPT_JOBS matrices in two launches: rows, then
+// matrix scale and conversion.  Small matrices are bound by launches (a 512 x 512 one took five of 2 to 4 us each), large ones by the second
+// read of the delta and by the two single-workgroup launches.
 constexpr int OPT_JOBS = 16; // jobs travel as kernel arguments
 constexpr int OPT_ROW_MAX = 4096;
 
@@ -255,7 +260,7 @@ struct OptJobs {
 
 // RowSum2, UpdateGlobalRowDisp (one row per estimate) and AddGradient of a row by one team - a wave, or the workgroup - that keeps the
 // packed row in registers between its sum and its use (NCH chunks of four elements per thread), all operands of the row in flight at
-// once.  sumWeight is only read here; OptScale, which follows, moves it on.  8192 x 2048, with the row sums and estimates it
+// once.  sumWeight is only read here; OptConvert, which follows, moves it on.  8192 x 2048, with the row sums and estimates it
 // replaces: 50.5 + 8.4 + 5.9 us in three launches -> 53.5 (a wave per row, eight chunks in two goes: 57.8)
 template <int NCH, bool WG> __global__ void __launch_bounds__(256) OptRows(OptJobs jobs, const ts2_add_gradient_params *pParams)
 {
@@ -324,51 +329,60 @@ template <int NCH, bool WG> __global__ void __launch_bounds__(256) OptRows(OptJo
     }
 }
 
-// MatrixSko per job, and the weight of the dispersion estimates that OptRows used
-__global__ void __launch_bounds__(1024) OptScale(OptJobs jobs, const ts2_add_gradient_params *pParams)
+constexpr int CONVERT_CHUNKS = 4; // of 256 columns that a wave has under way
+
+__device__ __forceinline__ void ConvertLoad(const OptJob &o, int y, int x0, F4 (&v)[CONVERT_CHUNKS])
 {
-    __shared__ float red[16];
-    const OptJob &o = jobs.j[blockIdx.x];
-    MatrixSkoBlock(o.xSize, o.ySize, o.weightsRowSum2, o.matrixScale, o.convertMult, red);
-    if (threadIdx.x == 0) {
-        o.sumWeight[0] = o.sumWeight[0] * pParams->dispDecay + 1;
+    const float *srow = (const float *)(o.weights.p + (int64_t)y * o.weights.ld);
+#pragma unroll
+    for (int k = 0; k < CONVERT_CHUNKS; ++k) {
+        const int x = x0 + k * 256;
+        v[k] = y < o.ySize && x < o.xSize ? Load4<TF32>(srow + x) : ZeroF4();
     }
 }
 
-template <class TDst> __device__ __forceinline__ void ConvertRow(const OptJob &o, int y, int lane, float mult)
+template <class TDst> __device__ __forceinline__ void ConvertStore(const OptJob &o, int y, int x0, const F4 (&v)[CONVERT_CHUNKS], float mult)
 {
     uint8_t *drow = o.fast.p + (int64_t)y * o.fast.ld;
-    const float *srow = (const float *)(o.weights.p + (int64_t)y * o.weights.ld);
-    const bool live = y < o.ySize;
-    for (int x0 = lane * 4; x0 < o.xSize; x0 += 1024) {
-        F4 v[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int x = x0 + k * 256;
-            v[k] = live && x < o.xSize ? Load4<TF32>(srow + x) : ZeroF4();
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int x = x0 + k * 256;
-            if (x < o.xSize) {
-                Store4<TDst>(drow + (int64_t)x * TDst::SIZE, live ? v[k] * mult : ZeroF4());
-            }
+    for (int k = 0; k < CONVERT_CHUNKS; ++k) {
+        const int x = x0 + k * 256;
+        if (x < o.xSize) {
+            Store4<TDst>(drow + (int64_t)x * TDst::SIZE, y < o.ySize ? v[k] * mult : ZeroF4());
         }
     }
 }
 
-// ConvertMatrix per job, a wave per row
-__global__ void __launch_bounds__(256) OptConvert(OptJobs jobs)
+// MatrixSko and ConvertMatrix per job, a wave per row: every workgroup forms the matrix scale from the row sums itself (32 KB from L2 for 8192
+// rows, with its first weights under way meanwhile), which saves a launch of one workgroup between the passes (5 of 207 us per 3 matrices each)
+__global__ void __launch_bounds__(1024) OptConvert(OptJobs jobs, const ts2_add_gradient_params *pParams)
 {
+    __shared__ float red[16];
     const OptJob &o = jobs.j[blockIdx.y];
-    const float mult = o.convertMult[0];
-    for (int y = blockIdx.x * 4 + (threadIdx.x >> 6); y < o.yBufSize; y += gridDim.x * 4) {
-        if (o.fastType == TS2_I8) {
-            ConvertRow<TI8>(o, y, threadIdx.x & 63, mult);
-        } else if (o.fastType == TS2_E4M3) {
-            ConvertRow<TE4M3>(o, y, threadIdx.x & 63, mult);
-        } else {
-            ConvertRow<TBF16>(o, y, threadIdx.x & 63, mult);
+    const int first = (threadIdx.x & 63) * 4;
+    int y = blockIdx.x * 16 + (threadIdx.x >> 6);
+    F4 v[CONVERT_CHUNKS];
+    ConvertLoad(o, y, first, v);
+    const float sko = MatrixSkoOf(o.xSize, o.ySize, o.weightsRowSum2, red), mult = ConvertMultOf(sko);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        o.convertMult[0] = mult;
+        o.matrixScale[0] = sko;
+        o.sumWeight[0] = o.sumWeight[0] * pParams->dispDecay + 1; // the weight of the dispersion estimates that OptRows used
+    }
+    for (; y < o.yBufSize; y += gridDim.x * 16) {
+        for (int x0 = first; x0 < o.xSize; x0 += CONVERT_CHUNKS * 256) {
+            if (o.fastType == TS2_I8) {
+                ConvertStore<TI8>(o, y, x0, v, mult);
+            } else if (o.fastType == TS2_E4M3) {
+                ConvertStore<TE4M3>(o, y, x0, v, mult);
+            } else {
+                ConvertStore<TBF16>(o, y, x0, v, mult);
+            }
+            const bool more = x0 + CONVERT_CHUNKS * 256 < o.xSize;
+            const int nextY = more ? y : y + (int)gridDim.x * 16, nextX = more ? x0 + CONVERT_CHUNKS * 256 : first;
+            if (nextY < o.yBufSize) {
+                ConvertLoad(o, nextY, nextX, v);
+            }
         }
     }
 }
@@ -577,9 +591,7 @@ int Ts2OptApplyBatch(int count, const ts2_opt_matrix *const *mats, const ts2_mat
             hipLaunchKernelGGL((OptRows<4, true>), dim3(RowGrid(maxRows), n), dim3(256), 0, STREAM, jobs, params);
         }
         TS2_CHECK_LAUNCH();
-        hipLaunchKernelGGL(OptScale, dim3(n), dim3(1024), 0, STREAM, jobs, params);
-        TS2_CHECK_LAUNCH();
-        hipLaunchKernelGGL(OptConvert, dim3(RowGrid((maxBuf + 3) / 4), n), dim3(256), 0, STREAM, jobs);
+        hipLaunchKernelGGL(OptConvert, dim3(RowGrid((maxBuf + 15) / 16), n), dim3(1024), 0, STREAM, jobs, params);
         TS2_CHECK_LAUNCH();
     }
     return TS2_OK;
