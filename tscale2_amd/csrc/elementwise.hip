@@ -276,7 +276,7 @@ __device__ __forceinline__ float ComputeGradMult(float gradMaxNorm)
 
 template <class TFast>
 __global__ void __launch_bounds__(256) ScaleGrad(int len, int tiles, const float *gradMaxNorm, const float *prevGradMult, Mat grad, Mat gradFast,
-    float *gradScaleOut, float *gradMultOut)
+    float *gradScaleOut, float *gradMultOut, float *rowScale, float *rowAbsMax)
 {
     int t0, tile, h;
     float gradMult = ComputeGradMult(*gradMaxNorm);
@@ -301,6 +301,12 @@ __global__ void __launch_bounds__(256) ScaleGrad(int len, int tiles, const float
             if (t0 + k < len) {
                 Store4<TFast>(At<TFast>(gradFast, t0 + k, col), v[k] * gradMult);
             }
+        }
+        // the rows' codes (int8) belong to values times the old power of two
+        if (rowScale && tile == 0 && h < U && t0 + h < len) {
+            const float ratio = gradMult / *prevGradMult;
+            rowScale[t0 + h] *= ratio;
+            rowAbsMax[t0 + h] *= ratio;
         }
     }
 }
@@ -834,6 +840,52 @@ struct RowQuantJobs {
     uint32_t seed[4];
 };
 
+// codes, scale and (where asked for) plain maximum of a row that a wave holds as NCH chunks of 8 elements per lane; mx, plain: maxima of the
+// lane's own elements, with and without column scales
+template <int NCH>
+__device__ __forceinline__ void StoreRowCodes(const F4 (&v)[NCH][2], const bool (&in)[NCH], int lane, int t, float mx, float plain, uint8_t *out,
+    float *rowScale, float *rowAbsMax, uint32_t seed)
+{
+    mx = WaveMax(mx);
+    plain = WaveMax(plain);
+    float discr = 0, mult = 0;
+    if (mx > 0) {
+        discr = mx / 127;
+        mult = 1 / discr;
+    }
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+        if (!in[i]) {
+            continue;
+        }
+        if (seed) {
+            const int col4 = (i * 64 + lane) * 2;
+            *(uint2 *)(out + (i * 64 + lane) * 8) =
+                make_uint2(QuantDither4(v[i][0].x, v[i][0].y, v[i][0].z, v[i][0].w, mult, DitherWord(seed, t, col4)),
+                    QuantDither4(v[i][1].x, v[i][1].y, v[i][1].z, v[i][1].w, mult, DitherWord(seed, t, col4 + 1)));
+            continue;
+        }
+        F4 a = v[i][0] * mult, b = v[i][1] * mult;
+        uint32_t lo = (uint32_t)(CvtToI8(a.x) & 0xff) | ((uint32_t)(CvtToI8(a.y) & 0xff) << 8) | ((uint32_t)(CvtToI8(a.z) & 0xff) << 16) |
+                      ((uint32_t)(CvtToI8(a.w) & 0xff) << 24);
+        uint32_t hi = (uint32_t)(CvtToI8(b.x) & 0xff) | ((uint32_t)(CvtToI8(b.y) & 0xff) << 8) | ((uint32_t)(CvtToI8(b.z) & 0xff) << 16) |
+                      ((uint32_t)(CvtToI8(b.w) & 0xff) << 24);
+        *(uint2 *)(out + (i * 64 + lane) * 8) = make_uint2(lo, hi);
+    }
+    if (lane == 0) {
+        rowScale[t] = discr;
+        if (rowAbsMax) {
+            rowAbsMax[t] = plain;
+        }
+    }
+}
+
+__device__ __forceinline__ void Unpack8(const uint4 &raw, F4 (&v)[2])
+{
+    v[0] = MakeF4(__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xffff0000u), __uint_as_float(raw.y << 16), __uint_as_float(raw.y & 0xffff0000u));
+    v[1] = MakeF4(__uint_as_float(raw.z << 16), __uint_as_float(raw.z & 0xffff0000u), __uint_as_float(raw.w << 16), __uint_as_float(raw.w & 0xffff0000u));
+}
+
 // FULL: rows of exactly NCH * 512 elements.
 template <int NCH, bool FULL>
 __device__ __forceinline__ void NormalizeRowsWaveOf(int len, int lenRound, int dim, const Mat &src, const float *colScale, const Mat &dst,
@@ -893,38 +945,7 @@ __device__ __forceinline__ void NormalizeRowsWaveOf(int len, int lenRound, int d
             }
             mx = fmaxf(mx, fmaxf(HMaxAbs(v[i][0]), HMaxAbs(v[i][1])));
         }
-        mx = WaveMax(mx);
-        plain = WaveMax(plain);
-        float discr = 0, mult = 0;
-        if (mx > 0) {
-            discr = mx / 127;
-            mult = 1 / discr;
-        }
-#pragma unroll
-        for (int i = 0; i < NCH; ++i) {
-            if (!in[i]) {
-                continue;
-            }
-            if (seed) {
-                const int col4 = (i * 64 + lane) * 2;
-                *(uint2 *)(out + (i * 64 + lane) * 8) =
-                    make_uint2(QuantDither4(v[i][0].x, v[i][0].y, v[i][0].z, v[i][0].w, mult, DitherWord(seed, t, col4)),
-                        QuantDither4(v[i][1].x, v[i][1].y, v[i][1].z, v[i][1].w, mult, DitherWord(seed, t, col4 + 1)));
-                continue;
-            }
-            F4 a = v[i][0] * mult, b = v[i][1] * mult;
-            uint32_t lo = (uint32_t)(CvtToI8(a.x) & 0xff) | ((uint32_t)(CvtToI8(a.y) & 0xff) << 8) | ((uint32_t)(CvtToI8(a.z) & 0xff) << 16) |
-                          ((uint32_t)(CvtToI8(a.w) & 0xff) << 24);
-            uint32_t hi = (uint32_t)(CvtToI8(b.x) & 0xff) | ((uint32_t)(CvtToI8(b.y) & 0xff) << 8) | ((uint32_t)(CvtToI8(b.z) & 0xff) << 16) |
-                          ((uint32_t)(CvtToI8(b.w) & 0xff) << 24);
-            *(uint2 *)(out + (i * 64 + lane) * 8) = make_uint2(lo, hi);
-        }
-        if (lane == 0) {
-            rowScale[t] = discr;
-            if (rowAbsMax) {
-                rowAbsMax[t] = plain;
-            }
-        }
+        StoreRowCodes<NCH>(v, in, lane, t, mx, plain, out, rowScale, rowAbsMax, seed);
     }
 }
 
@@ -941,6 +962,226 @@ __global__ void __launch_bounds__(256) NormalizeRowsWave(int len, int lenRound, 
     float *rowAbsMax, uint32_t seed)
 {
     NormalizeRowsWaveOf<NCH, FULL>(len, lenRound, FULL ? NCH * 512 : dim, src, colScale, dst, rowScale, rowAbsMax, seed);
+}
+
+// ---- int8: gradient passes that also quantise the rows they write, for the dX product that reads them next (the arithmetic of the passes and of
+// NormalizeRowsWave).  A wave owns a row, a lane NCH chunks of 8 elements of it, so that a 128-wide tile is 16 lanes (a lane adds its two groups of
+// four before the first step across lanes: the same tree of sums as on 32 lanes) and the row's maximum is a wave reduction over values that are
+// still in registers.  A quantiser of its own reads everything again and costs a launch: per layer of the 512-token int8 step 6.1 + 3.1, 7.4 +
+// 3.5, 5.7 + 3.7 us -> 4.5, 5.7, 4.3; 16384 x 512 (normalisation, gate) 27.3 + 7.6, 28.1 + 12.5 -> 28.7, 24.3; 16384 x 384 (gate; Q, K, V) 16 + 24.6 +
+// 24 -> 16.2, 26.3
+
+__device__ __forceinline__ F4 ApplyRope4(F4 v, F4 rope, float dir)
+{
+    float s0 = rope.y * dir, s1 = rope.w * dir;
+    return MakeF4(v.x * rope.x - v.y * s0, v.x * s0 + v.y * rope.x, v.z * rope.z - v.w * s1, v.z * s1 + v.w * rope.z);
+}
+
+__device__ __forceinline__ uint4 Pack8(const F4 &a, const F4 &b)
+{
+    return make_uint4(PackBf16x2(a.x, a.y), PackBf16x2(a.z, a.w), PackBf16x2(b.x, b.y), PackBf16x2(b.z, b.w));
+}
+
+// TileNormBackprop of a tile on 16 lanes
+__device__ __forceinline__ void TileNormBackprop8(const F4 (&src)[2], F4 (&g)[2])
+{
+    const float sum2 = Row16Sum(HSum(src[0] * src[0]) + HSum(src[1] * src[1]));
+    const float dp = Row16Sum(HSum(src[0] * g[0]) + HSum(src[1] * g[1]));
+    if (sum2 == 0) {
+        g[0] = g[1] = ZeroF4();
+        return;
+    }
+    const float inv = 1 / sum2;
+    const float sigma = dp * inv, scale = sqrtf(TILE * inv);
+    g[0] = (g[0] - src[0] * sigma) * scale;
+    g[1] = (g[1] - src[1] * sigma) * scale;
+}
+
+// a row of bf16 values that the wave kept (zeros beyond the live rows), quantised
+template <int NCH> __device__ __forceinline__ void QuantKeptRow(const uint4 (&kept)[NCH], const bool (&in)[NCH], int lane, int t, const RowQuantOut &q)
+{
+    F4 v[NCH][2];
+    float mx = 0;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+        Unpack8(kept[i], v[i]);
+        mx = fmaxf(mx, fmaxf(HMaxAbs(v[i][0]), HMaxAbs(v[i][1])));
+    }
+    StoreRowCodes<NCH>(v, in, lane, t, mx, mx, q.dst + (int64_t)t * q.dstStride, q.rowScale, q.rowAbsMax, q.seed);
+}
+
+// BackpropLoLU<TBF16, TBF16, TBF16, MODE> over whole rows; MODE 1 quantises the gate's gradient only
+template <int NCH, int MODE>
+__global__ void __launch_bounds__(256) BackpropLoLURows(int len, int lenRound, int dim, Mat gate, Mat vals, float valsScale, Mat valsSrcTileScale,
+    Mat gradArr, Mat gradGate, Mat gradVals, Mat dScale, RowQuantOut qGate, RowQuantOut qVals)
+{
+    const int lane = threadIdx.x & 63, t = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (t >= lenRound) {
+        return;
+    }
+    const bool live = t < len;
+    bool in[NCH];
+    uint4 g[NCH], v[NCH], grad[NCH];
+    float ts[NCH];
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+        const int col = (i * 64 + lane) * 8;
+        in[i] = col < dim;
+        const bool use = live && in[i];
+        g[i] = use ? *(const uint4 *)At<TBF16>(gate, t, col) : make_uint4(0, 0, 0, 0);
+        v[i] = use ? *(const uint4 *)At<TBF16>(vals, t, col) : make_uint4(0, 0, 0, 0);
+        grad[i] = use ? *(const uint4 *)At<TBF16>(gradArr, t, col) : make_uint4(0, 0, 0, 0);
+        ts[i] = use && MODE == 0 ? ScaleAt(valsSrcTileScale, col / TILE, t) : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+        const int col = (i * 64 + lane) * 8;
+        F4 gg[2], vv[2], gr[2], resGate[2], resVals[2];
+        Unpack8(g[i], gg);
+        Unpack8(v[i], vv);
+        Unpack8(grad[i], gr);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            vv[k] = vv[k] * valsScale;
+            const F4 mult = LoLU4(gg[k]);
+            resGate[k] = gr[k] * vv[k] * LoLUGrad4(mult);
+            resVals[k] = gr[k] * mult;
+        }
+        if (MODE == 0) {
+            const float unNorm = ts[i] / valsScale;
+            const F4 src[2] = {vv[0] * unNorm, vv[1] * unNorm};
+            TileNormBackprop8(src, resVals);
+        } else {
+            const float ds = Row16Sum(HSum(vv[0] * resVals[0]) + HSum(vv[1] * resVals[1]));
+            if (in[i] && (lane & 15) == 0) {
+                ScaleAt(dScale, col / TILE, t) = live ? ds : 0.f;
+            }
+        }
+        // (rows that are not live hold zeros)
+        g[i] = live ? Pack8(resGate[0], resGate[1]) : make_uint4(0, 0, 0, 0);
+        v[i] = live ? Pack8(resVals[0], resVals[1]) : make_uint4(0, 0, 0, 0);
+        if (in[i]) {
+            *(uint4 *)At<TBF16>(gradGate, t, col) = g[i];
+            *(uint4 *)At<TBF16>(gradVals, t, col) = v[i];
+        }
+    }
+    QuantKeptRow<NCH>(g, in, lane, t, qGate);
+    if (MODE == 0) {
+        QuantKeptRow<NCH>(v, in, lane, t, qVals);
+    }
+}
+
+// BackpropRowTileNormalizeRope<TBF16, TBF16> over whole rows, blockIdx.y = gradient
+struct NormRopeRowJobs {
+    Mat grad[3], srcNorm[3], srcTileScale[3], rope[3], dst[3];
+    RowQuantOut q[3];
+};
+template <int NCH> __global__ void __launch_bounds__(256) BackpropNormRopeRows(int len, int lenRound, int dim, float gradMult, NormRopeRowJobs jobs)
+{
+    const int j = blockIdx.y;
+    const Mat grad = jobs.grad[j], srcNorm = jobs.srcNorm[j], srcTileScale = jobs.srcTileScale[j], rope = jobs.rope[j], dst = jobs.dst[j];
+    const int lane = threadIdx.x & 63, t = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (t >= lenRound) {
+        return;
+    }
+    const bool live = t < len;
+    bool in[NCH];
+    uint4 g[NCH], sn[NCH];
+    float sc[NCH];
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+        const int col = (i * 64 + lane) * 8;
+        in[i] = col < dim;
+        const bool use = live && in[i];
+        g[i] = use ? *(const uint4 *)At<TBF16>(grad, t, col) : make_uint4(0, 0, 0, 0);
+        sn[i] = use && srcNorm.p ? *(const uint4 *)At<TBF16>(srcNorm, t, col) : make_uint4(0, 0, 0, 0);
+        sc[i] = use && srcNorm.p ? ScaleAt(srcTileScale, col / TILE, t) : 0.f;
+    }
+    F4 rp[2] = {ZeroF4(), ZeroF4()};
+    if (rope.p && live) {
+        rp[0] = Load4<TF32>(At<TF32>(rope, t, (lane & 15) * 8));
+        rp[1] = Load4<TF32>(At<TF32>(rope, t, (lane & 15) * 8 + 4));
+    }
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+        F4 x[2], s[2];
+        Unpack8(g[i], x);
+        x[0] = x[0] * gradMult;
+        x[1] = x[1] * gradMult;
+        if (srcNorm.p) {
+            Unpack8(sn[i], s);
+            const F4 src[2] = {s[0] * sc[i], s[1] * sc[i]};
+            TileNormBackprop8(src, x);
+        }
+        if (rope.p) {
+            x[0] = ApplyRope4(x[0], rp[0], -1.f);
+            x[1] = ApplyRope4(x[1], rp[1], -1.f);
+        }
+        g[i] = live ? Pack8(x[0], x[1]) : make_uint4(0, 0, 0, 0);
+        if (in[i]) {
+            *(uint4 *)At<TBF16>(dst, t, (i * 64 + lane) * 8) = g[i];
+        }
+    }
+    QuantKeptRow<NCH>(g, in, lane, t, jobs.q[j]);
+}
+
+// BackpropLayerNormalize<TI8, TBF16, FINAL> over whole rows.  Rows len .. lenRound: codes and scales are cleared, FINAL clears its results there too
+template <int NCH, bool FINAL, int NT>
+__global__ void __launch_bounds__(NT) BackpropLayerNormalizeRows(int len, int lenRound, int dim, Mat normState, Mat stateScale, Mat dNormState,
+    const float *gradScale, const float *gradMult, Mat stateGrad, Mat stateGradFast, float *nextMaxNorm, RowQuantOut q)
+{
+    __shared__ float red[NT / 64];
+    const int lane = threadIdx.x & 63;
+    const float s = !FINAL && gradScale ? *gradScale : 1.f, gm = !FINAL && gradMult ? *gradMult : 1.f;
+    float gmax = 0;
+    for (int t = blockIdx.x * (NT / 64) + (threadIdx.x >> 6); t < lenRound; t += gridDim.x * (NT / 64)) {
+        const bool live = t < len;
+        bool in[NCH];
+        uint2 nv[NCH];
+        F4 grad[NCH][2], prev[NCH][2];
+        float sc[NCH];
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) {
+            const int col = (i * 64 + lane) * 8;
+            in[i] = col < dim;
+            const bool use = live && in[i];
+            nv[i] = use ? *(const uint2 *)At<TI8>(normState, t, col) : make_uint2(0, 0);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                grad[i][k] = use ? Load4<TF32>(At<TF32>(dNormState, t, col + k * 4)) : ZeroF4();
+                prev[i][k] = use && !FINAL ? Load4<TF32>(At<TF32>(stateGrad, t, col + k * 4)) : ZeroF4();
+            }
+            sc[i] = use ? ScaleAt(stateScale, col / TILE, t) : 0.f;
+        }
+        uint4 kept[NCH];
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) {
+            const int col = (i * 64 + lane) * 8;
+            const F4 src[2] = {Load4<TI8>(&nv[i].x) * sc[i], Load4<TI8>(&nv[i].y) * sc[i]};
+            F4 g[2] = {grad[i][0], grad[i][1]};
+            if (!FINAL) {
+                g[0] = g[0] * s;
+                g[1] = g[1] * s;
+            }
+            TileNormBackprop8(src, g);
+            if (!FINAL) {
+                g[0] = g[0] + prev[i][0];
+                g[1] = g[1] + prev[i][1];
+            }
+            if (!live) {
+                g[0] = g[1] = ZeroF4();
+            }
+            gmax = fmaxf(gmax, fmaxf(HMaxAbs(g[0]), HMaxAbs(g[1])));
+            kept[i] = Pack8(g[0] * gm, g[1] * gm);
+            if (in[i] && (FINAL || live)) {
+                Store4<TF32>(At<TF32>(stateGrad, t, col), g[0]);
+                Store4<TF32>(At<TF32>(stateGrad, t, col + 4), g[1]);
+                *(uint4 *)At<TBF16>(stateGradFast, t, col) = kept[i];
+            }
+        }
+        QuantKeptRow<NCH>(kept, in, lane, t, q);
+    }
+    PublishBlockMax<NT>(gmax, red, nextMaxNorm);
 }
 
 // Row-major k-tile quantiser: dst[t][x] = sat_i8(rne(src[t][x] * rowMult[t] / scale)) with one scale per kTile rows, formed from the row maxima
@@ -1259,12 +1500,6 @@ __global__ void __launch_bounds__(256) TransposeBytes(int count, TransposeJobs j
 }
 
 // rope pairs are (cos, sin) interleaved: lane holds two pairs
-__device__ __forceinline__ F4 ApplyRope4(F4 v, F4 rope, float dir)
-{
-    float s0 = rope.y * dir, s1 = rope.w * dir;
-    return MakeF4(v.x * rope.x - v.y * s0, v.x * s0 + v.y * rope.x, v.z * rope.z - v.w * s1, v.z * s1 + v.w * rope.z);
-}
-
 template <class TSrc>
 __global__ void __launch_bounds__(256) RowTileNormalizeRope(int len, int lenRound, int tiles, Mat src, float srcMult, int normalize, float vecScale,
     Mat rope, Mat dst, Mat tileScale)
@@ -1643,10 +1878,10 @@ extern "C" int ts2_scale_grad(const float *gradMaxNorm, const float *prevGradMul
     float *scaleNow = later ? nullptr : gradScaleOut, *multNow = later ? nullptr : gradMultOut;
     if (fastType == TS2_BF16) {
         hipLaunchKernelGGL((ScaleGrad<TBF16>), GridFor(len, tiles), dim3(256), 0, STREAM, len, tiles, gradMaxNorm, prevGradMult, M(*grad),
-            M(*gradFast), scaleNow, multNow);
+            M(*gradFast), scaleNow, multNow, nullptr, nullptr);
     } else if (fastType == TS2_E4M3) {
         hipLaunchKernelGGL((ScaleGrad<TE4M3>), GridFor(len, tiles), dim3(256), 0, STREAM, len, tiles, gradMaxNorm, prevGradMult, M(*grad),
-            M(*gradFast), scaleNow, multNow);
+            M(*gradFast), scaleNow, multNow, nullptr, nullptr);
     } else {
         return TS2_ERR_UNSUPPORTED;
     }
@@ -1858,6 +2093,129 @@ int Ts2QuantRowsBatch(int count, int len, int lenRound, const ts2_mat *src, cons
         jobs.seed[i] = seed[i];
     }
     return LaunchRowQuant(count, len, lenRound, dst[0].x, jobs, nullptr, stream);
+}
+
+#define LAUNCH_ROW_CHUNKS(K, ...)                                                                                                          \
+    switch ((dim + 511) / 512) {                                                                                                           \
+    case 1: { constexpr int N = 1; hipLaunchKernelGGL(K, __VA_ARGS__); } break;                                                            \
+    case 2: { constexpr int N = 2; hipLaunchKernelGGL(K, __VA_ARGS__); } break;                                                            \
+    case 3: { constexpr int N = 3; hipLaunchKernelGGL(K, __VA_ARGS__); } break;                                                            \
+    case 4: { constexpr int N = 4; hipLaunchKernelGGL(K, __VA_ARGS__); } break;                                                            \
+    case 5: case 6: { constexpr int N = 6; hipLaunchKernelGGL(K, __VA_ARGS__); } break;                                                    \
+    default: { constexpr int N = 8; hipLaunchKernelGGL(K, __VA_ARGS__); } break;                                                           \
+    }
+
+static bool RowQuantOk(const RowQuantOut &q, int dim)
+{
+    return q.dst && q.rowScale && q.dstStride >= dim && (((uintptr_t)q.dst | (uintptr_t)q.dstStride) & 7) == 0;
+}
+
+int Ts2BackpropLoluRows(int mode, int len, int lenRound, const ts2_mat *gate, const ts2_mat *vals, float valsScale, const ts2_mat *valsSrcTileScale,
+    const ts2_mat *grad, const ts2_mat *gradGate, const ts2_mat *gradVals, const ts2_mat *dScale, const RowQuantOut &qGate, const RowQuantOut &qVals,
+    void *stream)
+{
+    const int dim = gradGate->x;
+    if (dim % TILE || dim > 4096 || lenRound <= 0 || lenRound < len || !MatOk(gate, len, dim, 2) || !MatOk(vals, len, dim, 2) || !MatOk(grad, len, dim, 2) ||
+        !MatOk(gradGate, lenRound, dim, 2) || !MatOk(gradVals, lenRound, dim, 2) || (mode == 0 && !MatOk(valsSrcTileScale, dim / TILE, len, 4)) ||
+        (mode == 1 && !MatOk(dScale, dim / TILE, lenRound, 4)) || !RowQuantOk(qGate, dim) || (mode == 0 && !RowQuantOk(qVals, dim))) {
+        return TS2_ERR_UNSUPPORTED;
+    }
+    if (!Aligned16(gate->ptr, gate->strideBytes) || !Aligned16(vals->ptr, vals->strideBytes) || !Aligned16(grad->ptr, grad->strideBytes) ||
+        !Aligned16(gradGate->ptr, gradGate->strideBytes) || !Aligned16(gradVals->ptr, gradVals->strideBytes)) {
+        return TS2_ERR_UNSUPPORTED;
+    }
+    const dim3 blocks((lenRound + 3) / 4);
+    if (mode == 0) {
+        LAUNCH_ROW_CHUNKS((BackpropLoLURows<N, 0>), blocks, dim3(256), 0, STREAM, len, lenRound, dim, M(*gate), M(*vals), valsScale, M(*valsSrcTileScale),
+            M(*grad), M(*gradGate), M(*gradVals), Mat{nullptr, 0}, qGate, qVals)
+    } else {
+        LAUNCH_ROW_CHUNKS((BackpropLoLURows<N, 1>), blocks, dim3(256), 0, STREAM, len, lenRound, dim, M(*gate), M(*vals), valsScale, Mat{nullptr, 0},
+            M(*grad), M(*gradGate), M(*gradVals), M(*dScale), qGate, qVals)
+    }
+    TS2_CHECK_LAUNCH();
+    return TS2_OK;
+}
+
+int Ts2BackpropNormRopeRows(int count, int len, int lenRound, const ts2_mat *const *grad, float gradMult, const ts2_mat *const *srcNorm,
+    const ts2_mat *const *srcTileScale, const ts2_mat *const *ropeBuf, const ts2_mat *const *dst, const RowQuantOut *q, void *stream)
+{
+    if (count < 1 || count > 3 || lenRound <= 0 || lenRound < len) {
+        return TS2_ERR_UNSUPPORTED;
+    }
+    const int dim = dst[0]->x;
+    NormRopeRowJobs jobs = {};
+    for (int i = 0; i < count; ++i) {
+        if (dim % TILE || dim > 4096 || dst[i]->x != dim || !MatOk(grad[i], len, dim, 2) || !MatOk(dst[i], lenRound, dim, 2) || !RowQuantOk(q[i], dim) ||
+            !Aligned16(grad[i]->ptr, grad[i]->strideBytes) || !Aligned16(dst[i]->ptr, dst[i]->strideBytes) ||
+            (srcNorm[i] && (!MatOk(srcNorm[i], len, dim, 2) || !Aligned16(srcNorm[i]->ptr, srcNorm[i]->strideBytes) ||
+                               !MatOk(srcTileScale[i], dim / TILE, len, 4))) ||
+            (ropeBuf[i] && (!MatOk(ropeBuf[i], len, TILE, 4) || !Aligned16(ropeBuf[i]->ptr, ropeBuf[i]->strideBytes)))) {
+            return TS2_ERR_UNSUPPORTED;
+        }
+        jobs.grad[i] = M(*grad[i]);
+        jobs.dst[i] = M(*dst[i]);
+        if (srcNorm[i]) {
+            jobs.srcNorm[i] = M(*srcNorm[i]);
+            jobs.srcTileScale[i] = M(*srcTileScale[i]);
+        }
+        if (ropeBuf[i]) {
+            jobs.rope[i] = M(*ropeBuf[i]);
+        }
+        jobs.q[i] = q[i];
+    }
+    LAUNCH_ROW_CHUNKS((BackpropNormRopeRows<N>), dim3((lenRound + 3) / 4, count), dim3(256), 0, STREAM, len, lenRound, dim, gradMult, jobs)
+    TS2_CHECK_LAUNCH();
+    return TS2_OK;
+}
+
+int Ts2BackpropLayerNormalizeRows(bool final, int len, int lenRound, const ts2_mat *normState, const ts2_mat *stateScale, const ts2_mat *dNormState,
+    const float *gradScale, const float *gradMult, const ts2_mat *stateGrad, const ts2_mat *stateGradFast, float *nextMaxNorm, const RowQuantOut &q,
+    void *stream)
+{
+    const int dim = dNormState->x;
+    if (dim % TILE || dim > 1536 || lenRound <= 0 || lenRound < len || !MatOk(normState, len, dim, 1) || !MatOk(stateScale, dim / TILE, len, 4) ||
+        !MatOk(dNormState, len, dim, 4) || !MatOk(stateGrad, final ? lenRound : len, dim, 4) || !MatOk(stateGradFast, final ? lenRound : len, dim, 2) ||
+        !RowQuantOk(q, dim) || (((uintptr_t)normState->ptr | normState->strideBytes) & 7) || !Aligned16(dNormState->ptr, dNormState->strideBytes) ||
+        !Aligned16(stateGrad->ptr, stateGrad->strideBytes) || !Aligned16(stateGradFast->ptr, stateGradFast->strideBytes)) {
+        return TS2_ERR_UNSUPPORTED;
+    }
+    // one update of the maximum per workgroup, 10 ns each on its one address: workgroups of 1024 threads beyond 256 small ones
+    const bool large = lenRound > 1024;
+    const dim3 blocks(large ? (lenRound / 16 < 512 ? lenRound / 16 : 512) : (lenRound + 3) / 4);
+#define BN_ROWS_OF(N, FINAL, NT)                                                                                                           \
+    hipLaunchKernelGGL((BackpropLayerNormalizeRows<N, FINAL, NT>), blocks, dim3(NT), 0, STREAM, len, lenRound, dim, M(*normState), M(*stateScale), \
+        M(*dNormState), gradScale, gradMult, M(*stateGrad), M(*stateGradFast), nextMaxNorm, q)
+#define BN_ROWS(FINAL, NT)                                                                                                                 \
+    if (dim <= 512) {                                                                                                                      \
+        BN_ROWS_OF(1, FINAL, NT);                                                                                                          \
+    } else if (dim <= 1024) {                                                                                                              \
+        BN_ROWS_OF(2, FINAL, NT);                                                                                                          \
+    } else {                                                                                                                               \
+        BN_ROWS_OF(3, FINAL, NT); /* (wider rows do not fit the registers of 16 waves) */                                                  \
+    }
+    if (final && large) {
+        BN_ROWS(true, 1024)
+    } else if (final) {
+        BN_ROWS(true, 256)
+    } else if (large) {
+        BN_ROWS(false, 1024)
+    } else {
+        BN_ROWS(false, 256)
+    }
+#undef BN_ROWS
+#undef BN_ROWS_OF
+    TS2_CHECK_LAUNCH();
+    return TS2_OK;
+}
+
+int Ts2ScaleGradRows(const float *gradMaxNorm, const float *prevGradMult, const ts2_mat *grad, const ts2_mat *gradFast, int len, float *gradScaleOut,
+    float *gradMultOut, float *rowScale, float *rowAbsMax, void *stream)
+{
+    const int tiles = grad->x / TILE;
+    hipLaunchKernelGGL((ScaleGrad<TBF16>), GridFor(len, tiles), dim3(256), 0, STREAM, len, tiles, gradMaxNorm, prevGradMult, M(*grad), M(*gradFast),
+        gradScaleOut, gradMultOut, rowScale, rowAbsMax);
+    TS2_CHECK_LAUNCH();
+    return TS2_OK;
 }
 
 // The row-major k-tile quantiser over any number of bf16 gradients with the same rows

@@ -22,6 +22,27 @@ int Ts2MoeRouteSetup();
 // the int8 row quantiser (ts2_normalize_vecs_row_max_dither) over `count` <= 4 bf16 gradients of one width <= 4096, one launch
 int Ts2QuantRowsBatch(int count, int len, int lenRound, const ts2_mat *src, const ts2_mat *dst, float *const *rowScale, float *const *rowAbsMax,
     const uint32_t *seed, void *stream);
+// where a gradient pass leaves the rows it writes quantised as well (the row quantiser's results); seed 0: no dither
+struct RowQuantOut {
+    uint8_t *dst;
+    int64_t dstStride; // bytes
+    float *rowScale, *rowAbsMax;
+    uint32_t seed;
+};
+// int8 forms, bf16 gradients, rows of up to 4096: ts2_backprop_row_tile_normalize_lolu (mode 0) / ts2_backprop_lolu_dscale (mode 1, quantises the
+// gate's gradient), ts2_backprop_row_tile_normalize_rope of up to three gradients, ts2_backprop_layer_normalize / ts2_backprop_final_normalize.
+// (rows of up to 1536).  TS2_ERR_UNSUPPORTED: nothing was launched
+int Ts2BackpropLoluRows(int mode, int len, int lenRound, const ts2_mat *gate, const ts2_mat *vals, float valsScale, const ts2_mat *valsSrcTileScale,
+    const ts2_mat *grad, const ts2_mat *gradGate, const ts2_mat *gradVals, const ts2_mat *dScale, const RowQuantOut &qGate, const RowQuantOut &qVals,
+    void *stream);
+int Ts2BackpropNormRopeRows(int count, int len, int lenRound, const ts2_mat *const *grad, float gradMult, const ts2_mat *const *srcNorm,
+    const ts2_mat *const *srcTileScale, const ts2_mat *const *ropeBuf, const ts2_mat *const *dst, const RowQuantOut *q, void *stream);
+int Ts2BackpropLayerNormalizeRows(bool final, int len, int lenRound, const ts2_mat *normState, const ts2_mat *stateScale, const ts2_mat *dNormState,
+    const float *gradScale, const float *gradMult, const ts2_mat *stateGrad, const ts2_mat *stateGradFast, float *nextMaxNorm, const RowQuantOut &q,
+    void *stream);
+// ts2_scale_grad (bf16) that moves the rows' scales and maxima along with the values when their power of two changes
+int Ts2ScaleGradRows(const float *gradMaxNorm, const float *prevGradMult, const ts2_mat *grad, const ts2_mat *gradFast, int len, float *gradScaleOut,
+    float *gradMultOut, float *rowScale, float *rowAbsMax, void *stream);
 // the k-tile quantiser without the transpose, over `count` <= 4 bf16 gradients of one width: dst[t][x] with one scale per kTile rows,
 // tileScale [count][lenRound / kTile]
 int Ts2QuantTileRows(int count, int len, int lenRound, int kTile, const ts2_mat *src, const ts2_mat *dst, const float *const *rowAbsMax,

@@ -168,6 +168,7 @@ struct ts2_model {
     int stackW = 0; // columns of the gradient scratch sGradT (and sGrad8): maxW, or the stacked gradients of a layer
     std::vector<Arr> stepFast; // fast state gradient entering each step of the backward pass (own storage where deltas wait for its end)
     Arr fast;                  // the one the layer backward reads
+    bool fastQuantised = false; // int8: ... and slot 0 of the row quantiser holds it already
     TDeltaQueue queue;
     Arr lastFast[4]; // where the layer backward that ran last left its fast-type gradients
     float *sPartial = 0;                     // fp32 slices of a delta product with few output tiles
@@ -289,9 +290,21 @@ int BackpropDX(ts2_model *M, TMatrix &W, const Arr &gradFast, float alpha, bool 
 
 // srcGrad (+)= sum_i alpha [* scale_i] * grad_i * W_i for the matrices of a layer that share their input: every weight is transposed
 // into its own part of the transpose scratch, then one grouped Backprop
-// (int8: the row maxima of gradient i go to rowAbsMax + i * RP, the shared scratch where it is null)
+// int8: where the row quantiser leaves gradient i of a layer: codes, scales and maxima of slot i of the scratch (maxima: of the layer's own, where
+// its deltas wait)
+float *RowMaxSlot(ts2_model *M, float *rowAbsMax, int i)
+{
+    return rowAbsMax ? rowAbsMax + (size_t)i * M->R : M->sRowAbsMax + (size_t)i * M->RP;
+}
+
+RowQuantOut RowSlot(ts2_model *M, float *rowAbsMax, int i, int width)
+{
+    return {M->sGrad8 + (size_t)i * M->R * width, width, M->sRowScale + (size_t)i * M->RP, RowMaxSlot(M, rowAbsMax, i), NextDither(M)};
+}
+
+// (int8: the row maxima of gradient i go to RowMaxSlot(rowAbsMax, i); quantised: the passes that wrote the gradients have filled the slots)
 int BackpropDXGroup(ts2_model *M, int count, TMatrix *const *W, const Arr *const *grad, float alpha, const bool *useScale, const Arr &srcGrad,
-    bool add, float *rowAbsMax, void *s)
+    bool add, float *rowAbsMax, bool quantised, void *s)
 {
     ts2_matmul_bwd_buffers b[4];
     const ts2_matmul_bwd_buffers *bp[4];
@@ -314,8 +327,8 @@ int BackpropDXGroup(ts2_model *M, int count, TMatrix *const *W, const Arr *const
             g16[i] = grad[i]->m;
             g8[i] = Flat(M->sGrad8 + (size_t)i * M->R * dstDim, M->R, dstDim, TS2_I8).m;
             rs[i] = M->sRowScale + (size_t)i * M->RP;
-            ram[i] = rowAbsMax ? rowAbsMax + (size_t)i * M->R : M->sRowAbsMax + (size_t)i * M->RP;
-            seed[i] = NextDither(M);
+            ram[i] = RowMaxSlot(M, rowAbsMax, i);
+            seed[i] = quantised ? 0 : NextDither(M);
             al[i] = alpha;
             ap[i] = useScale[i] ? W[i]->scale : nullptr;
             if (!W[i]->fastTValid) {
@@ -324,7 +337,9 @@ int BackpropDXGroup(ts2_model *M, int count, TMatrix *const *W, const Arr *const
             }
             wT[i] = W[i]->fastT.m;
         }
-        CK(Ts2QuantRowsBatch(count, M->len, M->R, g16, g8, rs, ram, seed, s));
+        if (!quantised) {
+            CK(Ts2QuantRowsBatch(count, M->len, M->R, g16, g8, rs, ram, seed, s));
+        }
         return Ts2BackpropGroupI8(count, M->len, M->R, srcDim, dstDim, g8, rs, wT, al, ap, srcGrad.P(), srcGrad.type, add, s);
     }
     for (int i = 0; i < count; ++i) {
@@ -527,13 +542,20 @@ int FfnBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
     TMatrix *const wc[1] = {&L.w[2]};
     const Arr *const sg[1] = {&M->fast};
     const bool scaled[2] = {true, false};
-    CK(BackpropDXGroup(M, 1, wc, sg, DISCR * Dot(F), scaled, drg, false, keep ? L.rowAbsMax + (size_t)4 * R : nullptr, s));
+    CK(BackpropDXGroup(M, 1, wc, sg, DISCR * Dot(F), scaled, drg, false, keep ? L.rowAbsMax + (size_t)4 * R : nullptr, M->fastQuantised, s));
     CK(i8 ? BackpropDeltaI8(M, 1, L.w[2], wc, rg8, sg, VEC, gradScale, keep, 4, s) : BackpropDelta(M, L.w[2], rg8, M->fast, VEC, gradScale, keep != nullptr, s));
-    CK(ts2_backprop_row_tile_normalize_lolu(len, R, gate16.P(), wide16.P(), VEC, wideScale.P(), drg.P(), TS2_BF16, dgate.P(), dwide.P(),
-        M->fastGradType, s));
+    float *const rowMax = keep ? L.rowAbsMax : nullptr;
+    bool quantised = i8 && F <= QUANT_ROW_MAX;
+    if (quantised) {
+        const RowQuantOut qWide = RowSlot(M, rowMax, 0, F), qGate = RowSlot(M, rowMax, 1, F);
+        CK(Ts2BackpropLoluRows(0, len, R, gate16.P(), wide16.P(), VEC, wideScale.P(), drg.P(), dgate.P(), dwide.P(), nullptr, qGate, qWide, s));
+    } else {
+        CK(ts2_backprop_row_tile_normalize_lolu(len, R, gate16.P(), wide16.P(), VEC, wideScale.P(), drg.P(), TS2_BF16, dgate.P(), dwide.P(),
+            M->fastGradType, s));
+    }
     TMatrix *const ws[2] = {&L.w[0], &L.w[1]};
     const Arr *const gs[2] = {&dwide, &dgate};
-    CK(BackpropDXGroup(M, 2, ws, gs, DISCR * Dot(D), scaled, M->dNormState, false, keep ? L.rowAbsMax : nullptr, s));
+    CK(BackpropDXGroup(M, 2, ws, gs, DISCR * Dot(D), scaled, M->dNormState, false, rowMax, quantised, s));
     return i8 ? BackpropDeltaI8(M, 2, L.stack, ws, norm8, gs, VEC, gradScale, keep, 0, s)
               : BackpropDelta(M, L.stack, norm8, gStack, VEC, gradScale, keep != nullptr, s);
 }
@@ -616,12 +638,22 @@ int AttBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
     TMatrix *const wc[1] = {&L.w[4]};
     const Arr *const sg[1] = {&M->fast};
     const bool useScale[4] = {true, true, true, false};
-    CK(BackpropDXGroup(M, 1, wc, sg, DISCR * Dot(Q), useScale, dvlg, false, keep ? L.rowAbsMax + (size_t)4 * R : nullptr, s));
+    CK(BackpropDXGroup(M, 1, wc, sg, DISCR * Dot(Q), useScale, dvlg, false, keep ? L.rowAbsMax + (size_t)4 * R : nullptr, M->fastQuantised, s));
     CK(i8 ? BackpropDeltaI8(M, 1, L.w[4], wc, vlg8, sg, VEC, gradScale, keep, 4, s)
           : BackpropDelta(M, L.w[4], vlg8, M->fast, VEC, gradScale, keep != nullptr, s));
     // gate backward + dScale
-    CK(ts2_backprop_lolu_dscale(len, R, gate16.P(), val16.P(), 1.f, dvlg.P(), TS2_BF16, dGate.P(), M->fastGradType, dVal16.P(), TS2_BF16,
-        M->dScale.P(), s));
+    float *const rowMax = keep ? L.rowAbsMax : nullptr;
+    const bool quantised = i8 && Q <= QUANT_ROW_MAX;
+    RowQuantOut slots[4] = {};
+    for (int i = 0; quantised && i < 4; ++i) {
+        slots[i] = RowSlot(M, rowMax, i, Q);
+    }
+    if (quantised) {
+        CK(Ts2BackpropLoluRows(1, len, R, gate16.P(), val16.P(), 1.f, nullptr, dvlg.P(), dGate.P(), dVal16.P(), M->dScale.P(), slots[3], slots[3], s));
+    } else {
+        CK(ts2_backprop_lolu_dscale(len, R, gate16.P(), val16.P(), 1.f, dvlg.P(), TS2_BF16, dGate.P(), M->fastGradType, dVal16.P(), TS2_BF16,
+            M->dScale.P(), s));
+    }
     // attention backward (dQ, dK, dV in bf16; val16's buffer is reused for dQ once dScale is known)
     Arr dQ = View(A.val16, R, Q), dK = View(M->g16[2], R, Q), dV = View(M->g16[3], R, Q);
     ts2_att_grad_args ag = {};
@@ -650,10 +682,14 @@ int AttBackward(ts2_model *M, TLayer &L, const Arr &norm8, const float *gradScal
     const ts2_mat *const nrGrad[3] = {dQ.P(), dK.P(), dV.P()}, *const nrNorm[3] = {q16.P(), nullptr, v16.P()};
     const ts2_mat *const nrScale[3] = {qScale.P(), nullptr, vScale.P()}, *const nrRope[3] = {M->rope.P(), M->rope.P(), nullptr};
     const ts2_mat *const nrDst[3] = {dQf.P(), dKf.P(), dVf.P()};
-    CK(Ts2BackpropNormRopeGroup(3, len, R, nrGrad, TS2_BF16, 1.f, nrNorm, nrScale, nrRope, nrDst, M->fastGradType, s));
+    if (quantised) {
+        CK(Ts2BackpropNormRopeRows(3, len, R, nrGrad, 1.f, nrNorm, nrScale, nrRope, nrDst, slots, s));
+    } else {
+        CK(Ts2BackpropNormRopeGroup(3, len, R, nrGrad, TS2_BF16, 1.f, nrNorm, nrScale, nrRope, nrDst, M->fastGradType, s));
+    }
     TMatrix *const ws[4] = {&L.w[0], &L.w[1], &L.w[2], &L.w[3]};
     const Arr *const gs[4] = {&dQf, &dKf, &dVf, &dGate};
-    CK(BackpropDXGroup(M, 4, ws, gs, DISCR * Dot(D), useScale, M->dNormState, false, keep ? L.rowAbsMax : nullptr, s));
+    CK(BackpropDXGroup(M, 4, ws, gs, DISCR * Dot(D), useScale, M->dNormState, false, rowMax, quantised, s));
     return i8 ? BackpropDeltaI8(M, 4, L.stack, ws, norm8, gs, VEC, gradScale, keep, 0, s)
               : BackpropDelta(M, L.stack, norm8, gStack, VEC, gradScale, keep != nullptr, s);
 }
@@ -916,7 +952,33 @@ int FinalLogits(ts2_model *M, const Arr &logits, void *s)
     return Forward(M, M->finalW, M->normState[depth], VEC * DISCR * Dot(D) / LN2F, true, logits, false, s);
 }
 
-int FinalBackward(ts2_model *M, void *s)
+// int8: where the row quantiser's results go for the gradient that layer d starts from, and whether the passes that write it can leave them there
+RowQuantOut EntrySlot(ts2_model *M, int d)
+{
+    TLayer &L = M->layers[d];
+    return RowSlot(M, M->stepFast[0].m.ptr != M->stateGradFast.m.ptr && L.gradStack.m.ptr ? L.rowAbsMax + (size_t)4 * M->R : nullptr, 0, M->cfg.dim);
+}
+
+bool QuantiseEntry(const ts2_model *M, int d)
+{
+    return M->mode == TS2_I8 && d >= 0 && M->layers[d].type != LT_MOE && M->cfg.dim <= 1536 && M->cfg.dim <= M->stackW;
+}
+
+int FinalNormalizeBackward(ts2_model *M, RowQuantOut *entry, void *s)
+{
+    const int depth = (int)M->layers.size();
+    const Arr &n8 = M->normState[depth], &scale = M->stateScale[depth];
+    M->fastQuantised = QuantiseEntry(M, depth - 1);
+    if (M->fastQuantised) {
+        *entry = EntrySlot(M, depth - 1);
+        return Ts2BackpropLayerNormalizeRows(true, M->len, M->R, n8.P(), scale.P(), M->dNormState.P(), nullptr, nullptr, M->stateGrad.P(), M->fast.P(),
+            M->gradMaxNorm, *entry, s);
+    }
+    return ts2_backprop_final_normalize(M->len, M->R, n8.P(), M->mode, scale.P(), M->dNormState.P(), M->stateGrad.P(), M->fast.P(), M->fastGradType,
+        M->gradMaxNorm, s);
+}
+
+int FinalBackward(ts2_model *M, RowQuantOut *entry, void *s)
 {
     int D = M->cfg.dim, V = M->cfg.vocab, VP = M->VP, depth = (int)M->layers.size(), R = M->R;
     // logits in IEEE half like the reference's logit window: a third of the traffic of fp32 logits written once and read twice
@@ -951,8 +1013,7 @@ int FinalBackward(ts2_model *M, void *s)
     if ((VP % 256) || (D % 256) || (VP / 256) * (D / 256) < 192) {
         CK(Ts2DeltaRows(TS2_BF16, M->len, R, D, VP, fn16.P(), M->gradV.P(), nullptr, 0, 0, VEC, nullptr, M->sPartial, (int64_t)M->sPartialFloats,
             M->finalW.delta.P(), M->finalW.deltaTileScale.P(), s));
-        return ts2_backprop_final_normalize(M->len, R, M->normState[depth].P(), M->mode, M->stateScale[depth].P(), M->dNormState.P(),
-            M->stateGrad.P(), M->fast.P(), M->fastGradType, M->gradMaxNorm, s);
+        return FinalNormalizeBackward(M, entry, s);
     }
     ts2_gemm_args h = {};
     h.a = M->gradV.m;
@@ -1003,8 +1064,7 @@ int FinalBackward(ts2_model *M, void *s)
     } else {
         CK(ts2_gemm_nt(&h, s));
     }
-    return ts2_backprop_final_normalize(M->len, R, M->normState[depth].P(), M->mode, M->stateScale[depth].P(), M->dNormState.P(), M->stateGrad.P(),
-        M->fast.P(), M->fastGradType, M->gradMaxNorm, s);
+    return FinalNormalizeBackward(M, entry, s);
 }
 
 // the transposes of the attention and feed-forward matrices that changed since they were made
@@ -1048,7 +1108,8 @@ int ModelBackprop(ts2_model *M, void *s)
     CK(Ts2ZeroRows(Flat(M->gradMaxNorm, 1, depth + 2, TS2_F32).P(), 1, (depth + 2) * 4, s));
     CK(Ts2FillFloats(M->gradMult, 1, 1.f, s)); // the multiplier the final normalisation applies to the fast gradient
     M->fast = M->stepFast[0];
-    CK(FinalBackward(M, s));
+    RowQuantOut entry = {}; // int8: of the layer that is next
+    CK(FinalBackward(M, &entry, s));
     CK(TransposeWeights(M, s));
     M->useKept = M->keep;
     struct TReset {
@@ -1057,6 +1118,7 @@ int ModelBackprop(ts2_model *M, void *s)
         {
             M->useKept = false;
             M->queue.open = false;
+            M->fastQuantised = false;
         }
     } reset = {M};
     M->queue.deltas.clear();
@@ -1069,10 +1131,22 @@ int ModelBackprop(ts2_model *M, void *s)
         // the fast gradient is rewritten only when its power-of-two multiplier differs from the one its producer applied (the final
         // normalisation: 1, kept in gradMult[0]; a layer's normalisation backward: that layer's multiplier)
         M->fast = M->stepFast[stepId];
-        CK(ts2_scale_grad(prevMax, M->gradMult + stepId, M->stateGrad.P(), M->fast.P(), M->fastGradType, M->len, gradScale, gradMult, s));
+        if (M->fastQuantised) {
+            CK(Ts2ScaleGradRows(prevMax, M->gradMult + stepId, M->stateGrad.P(), M->fast.P(), M->len, gradScale, gradMult, M->sRowScale,
+                entry.rowAbsMax, s));
+        } else {
+            CK(ts2_scale_grad(prevMax, M->gradMult + stepId, M->stateGrad.P(), M->fast.P(), M->fastGradType, M->len, gradScale, gradMult, s));
+        }
         CK(LayerBackward(M, d, gradScale, s));
-        CK(ts2_backprop_layer_normalize(M->normState[d].P(), M->mode, M->stateScale[d].P(), M->dNormState.P(), nullptr, gradScale, gradMult,
-            M->stateGrad.P(), M->stepFast[stepId + 1].P(), M->fastGradType, nextMax, M->len, s));
+        M->fastQuantised = QuantiseEntry(M, d - 1);
+        if (M->fastQuantised) {
+            entry = EntrySlot(M, d - 1);
+            CK(Ts2BackpropLayerNormalizeRows(false, M->len, M->R, M->normState[d].P(), M->stateScale[d].P(), M->dNormState.P(), gradScale, gradMult,
+                M->stateGrad.P(), M->stepFast[stepId + 1].P(), nextMax, entry, s));
+        } else {
+            CK(ts2_backprop_layer_normalize(M->normState[d].P(), M->mode, M->stateScale[d].P(), M->dNormState.P(), nullptr, gradScale, gradMult,
+                M->stateGrad.P(), M->stepFast[stepId + 1].P(), M->fastGradType, nextMax, M->len, s));
+        }
     }
     if (M->queue.open) {
         CK(RunQueue(M, s));
@@ -1664,6 +1738,7 @@ extern "C" int ts2_layer_backward(ts2_model *M, int32_t layer, void *stream)
         return TS2_ERR_NULL;
     }
     M->fast = M->stateGradFast;
+    M->fastQuantised = false;
     // gradient scale bookkeeping of one step of the backward loop, fed from stateGrad as it stands
     CK(ts2_scale_grad(M->gradMaxNorm, nullptr, M->stateGrad.P(), M->stateGradFast.P(), M->fastGradType, M->len, M->gradScale, M->gradMult, stream));
     CK(LayerBackward(M, layer, M->gradScale, stream));
