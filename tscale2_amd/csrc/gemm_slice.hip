@@ -340,7 +340,7 @@ template <int TYPE, bool TN, bool KT = false> __global__ void __launch_bounds__(
     // partial tiles of the four wave pairs -> LDS, sums of the thread's 16 columns back.  16-byte chunks of a 512-byte row are swizzled
     // by the row like the stages.
     float val[16]; // KT: the scaled sum over the k-tiles; otherwise set from the sum
-    auto reduce = [&](TAcc &sum) {
+    auto partials = [&]() {
         SLICE_BARRIER(); // every wave has read its last operands
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
@@ -360,6 +360,9 @@ template <int TYPE, bool TN, bool KT = false> __global__ void __launch_bounds__(
             }
         }
         __syncthreads();
+    };
+    auto reduce = [&](TAcc &sum) {
+        partials();
         if constexpr (KT) {
             const float *ts = p.kTileScale + (sp.kTileScaleRows ? (int64_t)(rowBase / sp.kTileScaleRows) * (p.kBytes / p.kTileBytes) : 0) + kt0;
 #pragma unroll
@@ -454,8 +457,97 @@ template <int TYPE, bool TN, bool KT = false> __global__ void __launch_bounds__(
     };
     TAcc sum;
     float sumScale = 1.f; // factor of `sum` in the epilogue
+    bool done = false;
+    if constexpr (TYPE == T_I8 && !TN && !KT) {
+        if ((p.nSeg == 2 || (p.nSeg == 4 && p.kBytes <= 1536)) && !p.tileGroup && !p.groupOffsets && p.splits <= 1) {
+            // Two or four products with row scales of their own: wave pair kg takes the kg-th product, or half of the (kg / 2)-th, so that all of
+            // them are one pipeline and one reduction; one after the other, each paid its start and its reduction.  Four of K = 256: 512x256 12.5 ->
+            // 7.8 us, 4096x512 15.5 -> 10.7, 8192x512 29.6 -> 19.4; two of 1024: 11.3 -> 9.8, 14.3 -> 12.7, 25.4 -> 23.5.  The operands of a load's four
+            // lane groups lie in different arrays, and four products fetch half lines: at K = 2048 that costs what the rest gains (8192x512 71.3 ->
+            // 73.9)
+            done = true;
+            const int share = p.nSeg == 2 ? 1 : 0, steps = (p.kBytes / 64) >> share; // (the halves are every other 64 bytes: whole lines)
+            const uint8_t *aPtr[2], *bPtr[4];
+            {
+                const int r = lane >> 4, slot = lane & 15;
+                auto at = [&](int rr, const uint8_t *q0, const uint8_t *q1, const uint8_t *q2, const uint8_t *q3, int64_t ld, int base) {
+                    const int ch = slot ^ (rr & 15), pair = ch >> 2, seg = pair >> share;
+                    const uint8_t *q = seg == 0 ? q0 : seg == 1 ? q1 : seg == 2 ? q2 : q3;
+                    return q + (base + rr) * ld + (pair & ((1 << share) - 1)) * 64 + (ch & 3) * 16;
+                };
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    aPtr[i] = at((wave + 8 * i) * 4 + r, p.a, p.segA[0], p.segA[1], p.segA[2], p.lda, rowBase);
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    bPtr[i] = at((wave + 8 * i) * 4 + r, p.b, p.segB[0], p.segB[1], p.segB[2], p.ldb, colBase);
+                }
+            }
+            auto load = [&](int stage) {
+                const unsigned st = ldsBase + stage * STAGE;
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(st + (wave + 8 * i) * 1024), "v"(aPtr[i]) : "memory");
+                    aPtr[i] += 64 << share;
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(st + SA + (wave + 8 * i) * 1024), "v"(bPtr[i]) : "memory");
+                    bPtr[i] += 64 << share;
+                }
+            };
+            float rs[4]; // (on their way before the operands)
+#pragma unroll
+            for (int seg = 0; seg < 4; ++seg) {
+                const float *rsp = seg == 0 ? p.rowScale : seg == 1 ? p.segRowScale[0] : seg == 2 ? p.segRowScale[1] : p.segRowScale[2];
+                rs[seg] = seg < p.nSeg && rsp ? rsp[row] : 1.f;
+            }
+            zeroAcc();
+            load(0);
+            if (steps > 1) {
+                load(1);
+            }
+            int stage = 0;
+            for (int t = 0; t < steps; ++t) {
+                if (t + 1 < steps) {
+                    asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+                } else {
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                }
+                SLICE_BARRIER();
+                if (t + 2 < steps) {
+                    load(stage == 0 ? NSTAGE - 1 : stage - 1);
+                }
+                multiply(-1, stage);
+                stage = stage == NSTAGE - 1 ? 0 : stage + 1;
+            }
+            const float f[4] = {factorOf(0) * rs[0], factorOf(1) * rs[1], p.nSeg > 2 ? factorOf(2) * rs[2] : 0.f, p.nSeg > 2 ? factorOf(3) * rs[3] : 0.f};
+            partials();
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const uint8_t *q = lds + er * 512 + ((chunkOf(c) ^ (er & 15)) << 4);
+                const v4i q0 = *(const v4i *)q, q1 = *(const v4i *)(q + SBM * SBN * 4), q2 = *(const v4i *)(q + 2 * (SBM * SBN * 4)),
+                          q3 = *(const v4i *)(q + 3 * (SBM * SBN * 4));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int k = c * 4 + e;
+                    if (share) {
+                        out[k] = out[k] + (float)(q0[e] + q1[e]) * f[0];
+                        sum[k] = q2[e] + q3[e];
+                    } else {
+                        out[k] = out[k] + (float)q0[e] * f[0];
+                        out[k] = out[k] + (float)q1[e] * f[1];
+                        out[k] = out[k] + (float)q2[e] * f[2];
+                        sum[k] = q3[e];
+                    }
+                }
+            }
+            sumScale = share ? f[1] : f[3];
+        }
+    }
     if constexpr (TYPE == T_I8) {
-        for (int seg = 0; seg < p.nSeg; ++seg) {
+        for (int seg = 0; seg < p.nSeg && !done; ++seg) {
             zeroAcc();
             float f = factorOf(seg);
             const float *rsp = seg == 0 ? p.rowScale : seg == 1 ? p.segRowScale[0] : seg == 2 ? p.segRowScale[1] : p.segRowScale[2];
