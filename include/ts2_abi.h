@@ -109,7 +109,8 @@ typedef struct ts2_gemm_args {
      * k >= 512 bytes, c and its stride are multiples of 16 bytes and (m/128)*(n/256) >= 512 - or when bit 12 asks for it;
      * results are bit-identical to the 128x128 kernels'.  Results with few tiles go to a kernel whose workgroups cut the contraction
      * between their waves (64x128 tiles; 16-byte aligned rows of C): bit 16 (65536) asks for it (TS2_ERR_UNSUPPORTED for calls it cannot
-     * run), bit 17 (131072) keeps the other kernels. */
+     * run), bit 17 (131072) keeps the other kernels.  Short contractions of more tiles go to a 256x128 kernel (TS2_I8, TS2_E4M3; m a
+     * multiple of 256): bit 18 (262144) asks for it (TS2_ERR_UNSUPPORTED for calls it cannot run). */
     int32_t tileConfig;
     /* Expert-grouped products (TMoeMatMulKernelCall / TMoeDeltaMatMulKernelCall, src/gpt/compute/moe_matmul.cuh:47-215):
      * tileGroup [m/128] (device): rows of A and C are grouped by expert in 128-row tiles; tile i multiplies the B slab

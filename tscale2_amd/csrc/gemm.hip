@@ -19,6 +19,7 @@
 //     can be cut into stored slices (deterministic split-K) or expert groups (MoE), and several products can be added into one
 //     result in one launch.
 #include "gemm_slice.h"
+#include "gemm_tall.h"
 #include <stdlib.h>
 
 using namespace gemmk;
@@ -1316,6 +1317,14 @@ extern "C" int ts2_gemm_nt(const ts2_gemm_args *a, void *streamPtr)
                        : a->cType == TS2_I32                     ? C_I32
                                                                  : -1;
         const int epi = a->epilogue == TS2_EPI_ADD ? TS2_EPI_ADD : TS2_EPI_STORE;
+        // the 256x128 tile for products of medium size: bit 18 asks for it (TS2_ERR_UNSUPPORTED if it cannot run the call)
+        if (ct >= 0 && (a->tileConfig & 262144)) {
+            return splitK <= 1 ? RunTall(p, type, ct, epi, stream) : TS2_ERR_UNSUPPORTED;
+        }
+        if (ct >= 0 && splitK <= 1 && !(a->tileConfig & (3 | 8 | 16 | 128 | 2048 | 4096 | 32768 | 65536 | 131072)) && PreferTall(p, type, ct, epi) &&
+            TallCanRun(p, type, ct, epi)) {
+            return RunTall(p, type, ct, epi, stream);
+        }
         // the kernel for results with few tiles: bit 16 asks for it, bit 17 keeps the others (comparison)
         const bool askSlice = a->tileConfig & 65536;
         if (ct >= 0 && splitK <= 1 && (askSlice || (!(a->tileConfig & (3 | 8 | 16 | 128 | 2048 | 4096 | 32768 | 131072)) && PreferSlice(p, type, ct, epi)))) {

@@ -2,6 +2,7 @@
 // over the kernels of this library.  Host code only; every step is enqueued on the caller's stream.
 #include "common.h"
 #include "gemm_slice.h"
+#include "gemm_tall.h"
 #include "internal.h"
 
 namespace
@@ -404,10 +405,17 @@ extern "C" int ts2_matmul_forward_norm_rope(int32_t mode, int32_t len, int32_t l
     // the 128x128 tile, whose normalising store rounds like the stand-alone pass (the large ones use the hardware's square root and
     // reciprocal), reads the rotation table in pairs; the pass takes it at any fp32 address and stride
     const bool small = mode == TS2_E4M3 && (!ropeBuf || (((uintptr_t)ropeBuf->ptr | ropeBuf->strideBytes) & 7) == 0);
+    // int8: the 256x128 tile
+    gemmk::GemmP shape = {};
+    shape.m = lenRound;
+    shape.n = dstDim;
+    shape.kBytes = srcDim;
+    const bool tall = mode == TS2_I8 && lenRound % 256 == 0 && gemmk::PreferTall(shape, gemmk::T_I8, gemmk::C_BF16NORM, TS2_EPI_STORE) &&
+                      Aligned16(res->ptr, res->strideBytes) && (!ropeBuf || Aligned16(ropeBuf->ptr, ropeBuf->strideBytes));
     // (the scratch of the two-launch sequence is part of the call, whichever kernel runs; an empty batch: the product's live length of 0
     // would mean all rows, the stand-alone pass clears them)
     const bool scratch = raw && raw->ptr && raw->x >= dstDim && raw->y >= lenRound;
-    if (large || (len > 0 && scratch && (few || small))) {
+    if (large || (len > 0 && scratch && (few || small || tall))) {
         g.c = *res;
         g.cType = TS2_BF16;
         g.epilogue = TS2_EPI_ROW_TILE_NORM;
@@ -419,7 +427,7 @@ extern "C" int ts2_matmul_forward_norm_rope(int32_t mode, int32_t len, int32_t l
         if (normalize) {
             g.tileScale = *tileScale;
         }
-        g.tileConfig = large || few ? 0 : 2;
+        g.tileConfig = large || few || tall ? 0 : 2;
         const int rc = ts2_gemm_nt(&g, stream);
         // rows off 16 bytes and the like: a product and the stand-alone pass take them
         if (large || (rc != TS2_ERR_UNSUPPORTED && rc != TS2_ERR_ALIGN)) {
@@ -585,11 +593,12 @@ int Ts2BackpropGroupI8(int count, int len, int lenRound, int srcDim, int gradDim
     if (count < 1 || count > 4) {
         return TS2_ERR_SHAPE;
     }
-    // one launch: the kernel for few tiles, or up to the size where 256x256 tiles fill the chip the 128x128 one (16384 x 512 x 512 inside the
-    // e512 step: a sum of four and a sum of two products 111 us together as six launches, 72 as two)
+    // one launch: the kernel for few tiles, the 256x128 one (PreferTall), or, for rows off its grid, up to the size where 256x256 tiles fill the chip
+    // the 128x128 one (16384 x 512 x 512 inside the e512 step: a sum of four and a sum of two products 111 us together as six launches, 72 as two)
     const bool few = (int64_t)(lenRound / 64) * (srcDim / 128) <= 640;
-    const bool sum = srcGradType == TS2_F32 && !add && (int64_t)lenRound * srcDim < (int64_t)192 * 65536;
-    bool one = count > 1 && (srcGradType == TS2_F32 || srcGradType == TS2_BF16) && (few || sum);
+    const bool tall = srcGradType == TS2_F32 && !add;
+    const bool sum = tall && (int64_t)lenRound * srcDim < (int64_t)192 * 65536;
+    bool one = count > 1 && (srcGradType == TS2_F32 || srcGradType == TS2_BF16) && (few || tall);
     for (int i = 1; i < count && one; ++i) {
         one = grad8[i].strideBytes == grad8[0].strideBytes && transformT[i].strideBytes == transformT[0].strideBytes;
     }
@@ -620,6 +629,9 @@ int Ts2BackpropGroupI8(int count, int len, int lenRound, int srcDim, int gradDim
         }
         sp.ct = srcGradType == TS2_F32 ? gemmk::C_F32 : gemmk::C_BF16;
         sp.epi = add ? TS2_EPI_ADD : TS2_EPI_STORE;
+        if (tall && gemmk::PreferTall(g, gemmk::T_I8, gemmk::C_F32, TS2_EPI_STORE) && gemmk::TallCanRun(g, gemmk::T_I8, gemmk::C_F32, TS2_EPI_STORE)) {
+            return gemmk::RunTall(g, gemmk::T_I8, gemmk::C_F32, TS2_EPI_STORE, (hipStream_t)stream);
+        }
         if (few && gemmk::SliceCanRun(sp, gemmk::T_I8, false)) {
             return gemmk::RunSlice(sp, gemmk::T_I8, false, (hipStream_t)stream);
         }
