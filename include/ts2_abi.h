@@ -110,7 +110,8 @@ typedef struct ts2_gemm_args {
      * results are bit-identical to the 128x128 kernels'.  Results with few tiles go to a kernel whose workgroups cut the contraction
      * between their waves (64x128 tiles; 16-byte aligned rows of C): bit 16 (65536) asks for it (TS2_ERR_UNSUPPORTED for calls it cannot
      * run), bit 17 (131072) keeps the other kernels.  Short contractions of more tiles go to a 256x128 kernel (TS2_I8, TS2_E4M3; m a
-     * multiple of 256): bit 18 (262144) asks for it (TS2_ERR_UNSUPPORTED for calls it cannot run). */
+     * multiple of 256): bit 18 (262144) asks for it (TS2_ERR_UNSUPPORTED for calls it cannot run).  Stored and accumulated fp32 and bf16
+     * results of at most 256 tiles of 64x64 go to a kernel of that tile (TS2_I8, TS2_E4M3): bit 19 (524288) asks for it likewise. */
     int32_t tileConfig;
     /* Expert-grouped products (TMoeMatMulKernelCall / TMoeDeltaMatMulKernelCall, src/gpt/compute/moe_matmul.cuh:47-215):
      * tileGroup [m/128] (device): rows of A and C are grouped by expert in 128-row tiles; tile i multiplies the B slab

@@ -19,6 +19,7 @@
 //     can be cut into stored slices (deterministic split-K) or expert groups (MoE), and several products can be added into one
 //     result in one launch.
 #include "gemm_slice.h"
+#include "gemm_square.h"
 #include "gemm_tall.h"
 #include <stdlib.h>
 
@@ -1380,3 +1381,11 @@ extern "C" int ts2_gemm_nt(const ts2_gemm_args *a, void *streamPtr)
         return DispatchTile<T_BF16>(a, p, stream);
     }
 }
+        // the 64x64 tile for results with fewer tiles still: bit 19 asks for it (TS2_ERR_UNSUPPORTED if it cannot run the call)
+        if (ct >= 0 && (a->tileConfig & 524288)) {
+            return splitK <= 1 ? RunSquare(p, type, ct, epi, stream) : TS2_ERR_UNSUPPORTED;
+        }
+        if (ct >= 0 && splitK <= 1 && !(a->tileConfig & (3 | 8 | 16 | 128 | 2048 | 4096 | 32768 | 65536 | 131072)) && PreferSquare(p) &&
+            SquareCanRun(p, type, ct, epi)) {
+            return RunSquare(p, type, ct, epi, stream);
+        }
