@@ -4,8 +4,9 @@
 
 int Ts2EmbedForward(int len, int lenRound, int dim, const int *labelPtr, const uint32_t *labels, const ts2_mat *embed, int embType, float mult,
     const float *scalePtr, const ts2_mat *state, void *stream);
+// mark: scratch of labelCount ints, or null
 int Ts2EmbedBackward(int len, int dim, const int *labelPtr, const uint32_t *labels, const ts2_mat *grad, const ts2_mat *delta, int labelCount,
-    void *stream);
+    int *mark, void *stream);
 int Ts2FinalProbabilities(int rows, int vocab, const ts2_mat *logits, const float *bias, const int *target, float gradMult, const ts2_mat *grad,
     void *stream);
 int Ts2FinalSoftmaxGradHalf(int rows, int vocab, const ts2_mat *logits, const float *bias, const int *target, float gradMult, const ts2_mat *grad,

@@ -135,6 +135,7 @@ struct ts2_model {
     ts2_add_gradient_params *optParams = 0; // device copy of the optimiser step parameters
     // batch
     int *labelPtr = 0;
+    int *labelMark = 0; // scratch of the embedding's backward, per label
     uint32_t *labels = 0;
     int labelCap = 0;
     int *target = 0;
@@ -1152,7 +1153,7 @@ int ModelBackprop(ts2_model *M, void *s)
         CK(RunQueue(M, s));
     }
     return Ts2EmbedBackward(M->len, D, M->labelPtr, M->labels, M->stateGrad.P(), Flat(M->embed.delta.m.ptr, M->cfg.labelCount, D, TS2_F32).P(),
-        M->cfg.labelCount, s);
+        M->cfg.labelCount, M->labelMark, s);
 }
 } // namespace
 
@@ -1312,6 +1313,7 @@ extern "C" ts2_model *ts2_model_create(const ts2_model_config *cfg)
     M->labelCap = R * 4;
     M->labelPtr = (int *)M->Dev((size_t)(R + 1) * 4);
     M->labels = (uint32_t *)M->Dev((size_t)M->labelCap * 4);
+    M->labelMark = (int *)M->Dev((size_t)cfg->labelCount * 4);
     M->target = (int *)M->Dev((size_t)R * 4);
     for (int a = 0; a < cfg->attTypeCount; ++a) {
         M->spanStart.push_back((int *)M->Dev((size_t)R * 4));
