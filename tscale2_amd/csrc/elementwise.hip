@@ -1205,6 +1205,23 @@ __global__ void __launch_bounds__(256) QuantTileRows(int len, int lenRound, int 
     const int dim = job.dim;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int t0 = blockIdx.x * QT_ROWS, k0 = t0 / kTile * kTile;
+    // units of 8 elements, walked by the whole workgroup: four 16-byte loads in flight per lane, the first four before the maxima
+    const int perRow = dim / 8, units = QT_ROWS * perRow;
+    const unsigned magic = (0x400000u + perRow - 1) / perRow; // u / perRow = u * magic >> 22 for u < units, perRow in 1 .. 512 (a division took half of the pass)
+    uint4 raw[4];
+    float rm[4];
+    int r[4], c[4];
+    auto fetch = [&](int u0) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int u = u0 + k * 256, row = (int)((unsigned)u * magic >> 22);
+            r[k] = u < units ? t0 + row : lenRound;
+            c[k] = (u - row * perRow) * 8;
+            raw[k] = r[k] < len ? *(const uint4 *)At<TBF16>(src, r[k], c[k]) : make_uint4(0, 0, 0, 0);
+            rm[k] = (rowMult && r[k] < len) ? rowMult[r[k]] : 1.f;
+        }
+    };
+    fetch(tid);
     float mx = 0;
     for (int t = k0 + tid; t < k0 + kTile && t < len; t += 256) {
         float m = rowAbsMax[t];
@@ -1223,19 +1240,9 @@ __global__ void __launch_bounds__(256) QuantTileRows(int len, int lenRound, int 
     if (tid == 0 && t0 == k0) {
         job.tileScale[t0 / kTile] = tm > 0 ? tm / 127 : 1.f;
     }
-    // units of 8 elements, walked by the whole workgroup: four 16-byte loads in flight per lane
-    const int perRow = dim / 8, units = QT_ROWS * perRow;
     for (int u0 = tid; u0 < units; u0 += 1024) {
-        uint4 raw[4];
-        float rm[4];
-        int r[4], c[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int u = u0 + k * 256;
-            r[k] = u < units ? t0 + u / perRow : lenRound;
-            c[k] = (u % perRow) * 8;
-            raw[k] = r[k] < len ? *(const uint4 *)At<TBF16>(src, r[k], c[k]) : make_uint4(0, 0, 0, 0);
-            rm[k] = (rowMult && r[k] < len) ? rowMult[r[k]] : 1.f;
+        if (u0 != tid) {
+            fetch(u0);
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -2228,7 +2235,7 @@ int Ts2QuantTileRowsJobs(int count, int len, int lenRound, int kTile, const Tile
         if (((uintptr_t)jobs[i].src | (uintptr_t)jobs[i].srcStride) & 15 || ((uintptr_t)jobs[i].dst | (uintptr_t)jobs[i].dstStride) & 7) {
             return TS2_ERR_ALIGN;
         }
-        if (jobs[i].dim <= 0 || jobs[i].dim % 8 || jobs[i].srcStride < jobs[i].dim * 2 || jobs[i].dstStride < jobs[i].dim) {
+        if (jobs[i].dim <= 0 || jobs[i].dim > 4096 || jobs[i].dim % 8 || jobs[i].srcStride < jobs[i].dim * 2 || jobs[i].dstStride < jobs[i].dim) {
             return TS2_ERR_SHAPE;
         }
     }
