@@ -37,9 +37,13 @@ namespace
 // SEG: two products into the same accumulators (C = alpha0 A0 B0^T + alpha1 A1 B1^T with the same k), the second operand pair and its
 // factors in segA[0], segB[0], segAlpha[0], segAlphaPtr[0]; with tileGroup both B operands take the tile's slab.  i8 (with KT: the second
 // accumulator set): p.nSeg products, each with row scales of its own, added in fp32 in their order.
-template <int TYPE, int WTM, int WTN, int CT, int EPI, bool KT, int WM = 2, int WN = 2, bool SEG = false>
+// JOBS: blockIdx.z picks one of several products (GemmP).
+template <int TYPE, int WTM, int WTN, int CT, int EPI, bool KT, int WM = 2, int WN = 2, bool SEG = false, bool JOBS = false>
 __global__ void __launch_bounds__(64 * WM * WN, (WM * WN) / 4) GemmNTDirect(GemmP p)
 {
+    if constexpr (JOBS) {
+        PickJob(p);
+    }
     typedef typename AccT<TYPE>::type TAcc;
     constexpr int NW = WM * WN; // waves per workgroup
     constexpr int BM = 32 * WTM * WM;
@@ -332,8 +336,12 @@ __global__ void __launch_bounds__(64 * WM * WN, (WM * WN) / 4) GemmNTDirect(Gemm
 // WT = 2 is the same pipeline on a 128x128 tile (wave tile 64x64): the stages are 16 KB, the ring 80 KB, and two workgroups share a
 // CU, so that one's start-up and stores fall into the other's main loop - for products whose workgroups are short (a contraction of
 // 512 .. 2048 bytes: the expert-grouped products, whose 128-row tiles each take their expert's slab of B, tileGroup).  e4m3 only.
-template <int TYPE, int CT, int EPI, bool TN = false, int WT = 4> __global__ void __launch_bounds__(256, WT == 4 ? 1 : 2) GemmNTRing(GemmP p)
+template <int TYPE, int CT, int EPI, bool TN = false, int WT = 4, bool JOBS = false>
+__global__ void __launch_bounds__(256, WT == 4 ? 1 : 2) GemmNTRing(GemmP p)
 {
+    if constexpr (JOBS) {
+        PickJob(p);
+    }
     typedef typename AccT<TYPE>::type TAcc;
     constexpr int WTM = WT, WTN = WT, WN = 2, NW = 4, BM = 64 * WT, BN = 64 * WT;
     static_assert(WT == 4 || (WT == 2 && TYPE == T_FP8 && !TN), "the 128x128 ring takes e4m3 operands with the contraction along the rows");
@@ -1138,6 +1146,60 @@ bool PreferSlice(const GemmP &p, int type, int ct, int epi)
 }
 } // namespace
 
+// Products that share A as one launch of the kernels for more tiles.  By the 128x128 tiles T of one product and the bytes K of the contraction, measured
+// in a graph of 40 launches against the launch of gemm_slice.hip (us, four products; with 256 workgroups of that kernel in all it is better, 5.5
+// to 11.5 against 6.9 to 12.7, with 512 it is not, and up to one and a half rounds the results are those of single calls bit by bit):
+//   T = 64   e4m3 1024x1024 K 512 12.4 -> 9.4, K 1024 15.2 -> 10.7, K 2048 21.5 -> 15.0; i8 equal
+//   T = 128  4096x512 e4m3 K 512 22.4 -> 10.9 (two products 12.0 -> 7.7), K 1024 28.6 -> 15.7; i8 22.8 -> 13.7 (12.1 -> 9.3), 28.7 -> 18.0
+// and beyond its range against one launch per product:
+//   T 192 .. 384  e4m3 0.37-0.56 of the time; i8 K <= 2048 0.51-0.87 (two products 0.60-0.99)
+//   T 512 and more  e4m3 K 256, 512 0.79-0.96, K 1024, 2048 0.91-1.27; i8 K 256 0.72-0.92, K 512 0.83-0.98 (two products 0.85-1.14 at T = 512), K 1024 up 1.00-1.25
+bool gemmk::PreferJobs(const GemmP &p, int type)
+{
+    const int64_t T = (int64_t)(p.m / 128) * (p.n / 128);
+    const int K = p.kBytes;
+    if (2 * T * p.jobs <= 384) {
+        return false;
+    }
+    if (type == T_FP8) {
+        return T < 512 || K <= 512;
+    }
+    return type == T_I8 && (T < 512 ? K <= 2048 : K <= 256 || (K <= 512 && (p.jobs > 2 || T >= 1024)));
+}
+
+int gemmk::RunJobs(const GemmP &p, int type, hipStream_t stream)
+{
+    if (p.jobs < 2 || p.jobs > 4 || (p.m % 128) || (p.n % 128) || (p.kBytes % BKB) || p.kBytes <= 0 || p.splits > 1 || p.nSeg > 1 || p.tileGroup ||
+        p.groupOffsets || (((uintptr_t)p.a | (uintptr_t)p.lda | (uintptr_t)p.ldb | (uintptr_t)p.ldc) & 15) || 128 * p.lda >= ((int64_t)1 << 31) ||
+        128 * p.ldb >= ((int64_t)1 << 31) || 128 * p.ldc >= ((int64_t)1 << 31) || (p.jobRope && (!p.rope || ((uintptr_t)p.rope & 15) || (p.ldRope & 3)))) {
+        return TS2_ERR_UNSUPPORTED;
+    }
+    for (int i = 0; i < p.jobs; ++i) {
+        if ((((uintptr_t)p.jobB[i] | (uintptr_t)p.jobC[i]) & 15) || (((p.jobNormalize >> i) & 1) && !p.jobTileScale[i])) {
+            return TS2_ERR_UNSUPPORTED;
+        }
+    }
+    if (type == T_I8) {
+        return RunTall(p, T_I8, C_BF16NORM, TS2_EPI_STORE, stream);
+    }
+    if (type != T_FP8) {
+        return TS2_ERR_UNSUPPORTED;
+    }
+    GemmP q = p;
+    q.tilesM = p.m / 128;
+    q.tilesN = p.n / 128;
+    const int nb = q.tilesM * q.tilesN, chunk = (nb % 8) == 0 ? nb / 8 : nb;
+    q.mapGroup = chunk >= 64 ? 8 : chunk >= 8 ? 4 : 2; // (as for one product)
+    const dim3 grid(nb, 1, p.jobs);
+    if (p.kBytes >= 8 * BKB) { // (where one product takes the ring)
+        hipLaunchKernelGGL((GemmNTRing<T_FP8, C_BF16NORM, TS2_EPI_STORE, false, 2, true>), grid, dim3(256), 0, stream, q);
+    } else {
+        hipLaunchKernelGGL((GemmNTDirect<T_FP8, 2, 2, C_BF16NORM, TS2_EPI_STORE, false, 2, 2, false, true>), grid, dim3(256), 0, stream, q);
+    }
+    TS2_CHECK_LAUNCH();
+    return TS2_OK;
+}
+
 int gemmk::RunSumI8(const GemmP &p, hipStream_t stream)
 {
     if (p.nSeg < 2 || p.nSeg > 4 || (p.m % 128) || (p.n % 128) || (p.kBytes % BKB) || p.splits > 1 ||
@@ -1210,7 +1272,7 @@ extern "C" int ts2_gemm_nt(const ts2_gemm_args *a, void *streamPtr)
     if (a->epilogue == TS2_EPI_ROW_TILE_MAXNORM && (!a->tileScale.ptr || a->tileScale.y < a->n / 128 || a->tileScale.x < a->m)) {
         return TS2_ERR_SHAPE;
     }
-    GemmP p;
+    GemmP p = {};
     p.a = (const uint8_t *)a->a.ptr;
     p.b = (const uint8_t *)a->b.ptr;
     p.c = (uint8_t *)a->c.ptr;
@@ -1326,6 +1388,14 @@ extern "C" int ts2_gemm_nt(const ts2_gemm_args *a, void *streamPtr)
             TallCanRun(p, type, ct, epi)) {
             return RunTall(p, type, ct, epi, stream);
         }
+        // the 64x64 tile for results with fewer tiles still: bit 19 asks for it (TS2_ERR_UNSUPPORTED if it cannot run the call)
+        if (ct >= 0 && (a->tileConfig & 524288)) {
+            return splitK <= 1 ? RunSquare(p, type, ct, epi, stream) : TS2_ERR_UNSUPPORTED;
+        }
+        if (ct >= 0 && splitK <= 1 && !(a->tileConfig & (3 | 8 | 16 | 128 | 2048 | 4096 | 32768 | 65536 | 131072)) && PreferSquare(p) &&
+            SquareCanRun(p, type, ct, epi)) {
+            return RunSquare(p, type, ct, epi, stream);
+        }
         // the kernel for results with few tiles: bit 16 asks for it, bit 17 keeps the others (comparison)
         const bool askSlice = a->tileConfig & 65536;
         if (ct >= 0 && splitK <= 1 && (askSlice || (!(a->tileConfig & (3 | 8 | 16 | 128 | 2048 | 4096 | 32768 | 131072)) && PreferSlice(p, type, ct, epi)))) {
@@ -1381,11 +1451,3 @@ extern "C" int ts2_gemm_nt(const ts2_gemm_args *a, void *streamPtr)
         return DispatchTile<T_BF16>(a, p, stream);
     }
 }
-        // the 64x64 tile for results with fewer tiles still: bit 19 asks for it (TS2_ERR_UNSUPPORTED if it cannot run the call)
-        if (ct >= 0 && (a->tileConfig & 524288)) {
-            return splitK <= 1 ? RunSquare(p, type, ct, epi, stream) : TS2_ERR_UNSUPPORTED;
-        }
-        if (ct >= 0 && splitK <= 1 && !(a->tileConfig & (3 | 8 | 16 | 128 | 2048 | 4096 | 32768 | 65536 | 131072)) && PreferSquare(p) &&
-            SquareCanRun(p, type, ct, epi)) {
-            return RunSquare(p, type, ct, epi, stream);
-        }

@@ -51,7 +51,26 @@ struct GemmP {
     const float *segAlphaPtr[3];
     const float *segRowScale[3]; // i8: row scales of the further products
     int rowsF16; // persistent kernel, row-owning epilogue: the 16-bit rows are IEEE half instead of bf16
+    // > 1: blockIdx.z picks one of several products of one shape that share A and are stored separately (C_BF16NORM; of p, b, c, tileScale,
+    // alphaPtr, normalize and rope's use are each product's own)
+    int jobs, jobNormalize, jobRope; // the latter two: bit per product
+    const uint8_t *jobB[4];
+    uint8_t *jobC[4];
+    float *jobTileScale[4];
+    const float *jobAlphaPtr[4];
 };
+
+__device__ __forceinline__ void PickJob(GemmP &p)
+{
+    const int j = blockIdx.z;
+    auto pick = [&](auto *const(&v)[4]) { return j == 0 ? v[0] : j == 1 ? v[1] : j == 2 ? v[2] : v[3]; };
+    p.b = pick(p.jobB);
+    p.c = pick(p.jobC);
+    p.tileScale = pick(p.jobTileScale);
+    p.alphaPtr = pick(p.jobAlphaPtr);
+    p.normalize = (p.jobNormalize >> j) & 1;
+    p.rope = ((p.jobRope >> j) & 1) ? p.rope : nullptr;
+}
 
 enum { T_I8 = 0, T_FP8 = 1, T_BF16 = 2 };
 enum { C_F32 = 0, C_BF16 = 1, C_I32 = 2, C_I8PACK = 3, C_BF16NORM = 4, C_F16 = 5 };

@@ -64,14 +64,14 @@ template <int TYPE, bool TN, bool KT = false> __global__ void __launch_bounds__(
     const uint8_t *bBase = p.b;
     const float *alphaPtr = p.alphaPtr;
     bool normalize = p.normalize, rotate = p.rope != nullptr;
-    if (sp.jobs > 1) {
+    if (p.jobs > 1) {
         const int j = blockIdx.z;
-        bBase = sp.jobB[j];
-        cBase = sp.jobC[j];
-        tileScale = sp.jobTileScale[j];
-        alphaPtr = sp.jobAlphaPtr[j];
-        normalize = (sp.jobNormalize >> j) & 1;
-        rotate = (sp.jobRope >> j) & 1;
+        bBase = p.jobB[j];
+        cBase = p.jobC[j];
+        tileScale = p.jobTileScale[j];
+        alphaPtr = p.jobAlphaPtr[j];
+        normalize = (p.jobNormalize >> j) & 1;
+        rotate = (p.jobRope >> j) & 1;
     }
     int64_t bSlab = 0;
     if (p.tileGroup) {
@@ -734,13 +734,13 @@ bool SliceCanRun(const SliceP &sp, int type, bool tn)
     if (sp.ct == C_I8PACK && p.nSeg > 1) {
         return false;
     }
-    if (sp.jobs > 1) {
-        if (sp.jobs > 4 || sp.ct != C_BF16NORM || sp.epi != TS2_EPI_STORE || tn || p.splits > 1 || p.groupOffsets || p.tileGroup || p.nSeg > 1 ||
-            p.kTileScale || (sp.jobRope && !p.rope)) {
+    if (p.jobs > 1) {
+        if (p.jobs > 4 || sp.ct != C_BF16NORM || sp.epi != TS2_EPI_STORE || tn || p.splits > 1 || p.groupOffsets || p.tileGroup || p.nSeg > 1 ||
+            p.kTileScale || (p.jobRope && !p.rope)) {
             return false;
         }
-        for (int i = 0; i < sp.jobs; ++i) {
-            if (((uintptr_t)sp.jobB[i] | (uintptr_t)sp.jobC[i]) & 15 || (((sp.jobNormalize >> i) & 1) && !sp.jobTileScale[i])) {
+        for (int i = 0; i < p.jobs; ++i) {
+            if (((uintptr_t)p.jobB[i] | (uintptr_t)p.jobC[i]) & 15 || (((p.jobNormalize >> i) & 1) && !p.jobTileScale[i])) {
                 return false;
             }
         }
@@ -769,7 +769,7 @@ int RunSlice(const SliceP &in, int type, bool tn, hipStream_t stream)
     sp.g.tilesM = sp.g.m / SBM;
     sp.g.tilesN = sp.g.n / SBN;
     const dim3 grid(sp.g.tilesM * sp.g.tilesN, sp.g.groupOffsets ? sp.g.splitK_groups : sp.g.splits > 1 ? sp.g.splits : 1,
-        sp.jobs > 1 ? sp.jobs : 1);
+        sp.g.jobs > 1 ? sp.g.jobs : 1);
     if (type == T_I8 && sp.g.kTileScale) {
         if (tn) {
             hipLaunchKernelGGL((GemmSlice<T_I8, true, true>), grid, dim3(512), 0, stream, sp);

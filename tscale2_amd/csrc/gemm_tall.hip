@@ -31,8 +31,12 @@ __device__ __forceinline__ v4i TallRsrc(const uint8_t *base)
 }
 
 // SEG (i8, fp32 result): p.nSeg products, each with row scales of its own, added in fp32 in their order
-template <int TYPE, int CT, int EPI, bool SEG> __global__ void __launch_bounds__(512, 2) GemmTall(GemmP p)
+// JOBS: blockIdx.z picks one of several products (GemmP)
+template <int TYPE, int CT, int EPI, bool SEG, bool JOBS = false> __global__ void __launch_bounds__(512, 2) GemmTall(GemmP p)
 {
+    if constexpr (JOBS) {
+        PickJob(p);
+    }
     typedef typename AccT<TYPE>::type TAcc;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[TSTAGES * TSTAGE];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -261,6 +265,10 @@ template <int TYPE> int Launch(const GemmP &p, int ct, int epi, hipStream_t stre
         } else {
             TALL(C_F32, TS2_EPI_STORE, false);
         }
+    } else if (ct == C_BF16NORM && p.jobs > 1) {
+        if constexpr (TYPE == T_I8) {
+            hipLaunchKernelGGL((GemmTall<TYPE, C_BF16NORM, TS2_EPI_STORE, false, true>), dim3(grid.x, 1, p.jobs), dim3(512), 0, stream, p);
+        }
     } else if (ct == C_BF16NORM) {
         TALL(C_BF16NORM, TS2_EPI_STORE, false);
     } else {
@@ -328,6 +336,9 @@ bool TallCanRun(const GemmP &p, int type, int ct, int epi)
         }
     }
     if (((uintptr_t)p.a | (uintptr_t)p.lda | (uintptr_t)p.b | (uintptr_t)p.ldb | (uintptr_t)p.c | (uintptr_t)p.ldc) & 15) {
+        return false;
+    }
+    if (p.jobs > 1 && (type != T_I8 || ct != C_BF16NORM)) {
         return false;
     }
     if (ct == C_BF16NORM && ((p.normalize && !p.tileScale) || (p.rope && (((uintptr_t)p.rope & 15) || (p.ldRope & 3))))) {

@@ -70,9 +70,9 @@ double Ts2DeltaCost(int mode, int lenRound, int srcDim, int gradDim, int64_t par
 // int8: srcGrad (+)= sum_i alpha_i * *alphaPtr_i * rowScale_i[t] * (grad8_i W_i^T), count <= 4 products of one shape added in order
 int Ts2BackpropGroupI8(int count, int len, int lenRound, int srcDim, int gradDim, const ts2_mat *grad8, const float *const *rowScale,
     const ts2_mat *transformT, const float *alpha, const float *const *alphaPtr, const ts2_mat *srcGrad, int srcGradType, int add, void *stream);
-// forward products of up to four matrices of one shape that read the same source, in one launch of the kernel for few tiles: res_i =
-// rope(normalise(alpha * *alphaPtr_i * src * W_i^T)) as bf16, normalisation and rotation each where asked for.  TS2_ERR_UNSUPPORTED: not
-// by this kernel, or not worth it; nothing was launched then
+// forward products of up to four matrices of one shape that read the same source, in one launch: res_i = rope(normalise(alpha *
+// *alphaPtr_i * src * W_i^T)) as bf16, normalisation and rotation each where asked for.  TS2_ERR_UNSUPPORTED: not possible, or not worth it;
+// nothing was launched then
 int Ts2ForwardGroup(int mode, int count, int len, int lenRound, int srcDim, int dstDim, const ts2_mat *src, const ts2_mat *const *w, float alpha,
     const float *const *alphaPtr, int normalizeBits, float vecScale, int rotateBits, const ts2_mat *rope, const ts2_mat *res,
     const ts2_mat *const *tileScale, void *stream);

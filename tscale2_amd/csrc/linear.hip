@@ -666,13 +666,13 @@ int Ts2BackpropGroupI8(int count, int len, int lenRound, int srcDim, int gradDim
 
 // While one product alone fits the chip (256 workgroups, one per CU), a launch is a chain of latencies and four of them cost four.  Whole passes,
 // separate -> one launch: 512-token int8 step 1133 -> 1016 us, 777-token prompt 1007 -> 874, 3885-token
-// 8-expert step 1632 -> 1538.  Beyond, the large-tile kernels are as good one by one
+// 8-expert step 1632 -> 1538.  Where all of them are more than a round of the kernel for few tiles, PreferJobs (gemm.hip) decides
 int Ts2ForwardGroup(int mode, int count, int len, int lenRound, int srcDim, int dstDim, const ts2_mat *src, const ts2_mat *const *w, float alpha,
     const float *const *alphaPtr, int normalizeBits, float vecScale, int rotateBits, const ts2_mat *rope, const ts2_mat *res,
     const ts2_mat *const *tileScale, void *stream)
 {
     const int64_t wgs = (int64_t)(lenRound / 64) * (dstDim / 128);
-    if (count < 2 || count > 4 || !Is8(mode) || wgs > 256 || lenRound % 128 || dstDim % 128 || srcDim % 128 || src->x < srcDim || src->y < lenRound) {
+    if (count < 2 || count > 4 || !Is8(mode) || lenRound % 128 || dstDim % 128 || srcDim % 128 || src->x < srcDim || src->y < lenRound) {
         return TS2_ERR_UNSUPPORTED;
     }
     gemmk::SliceP sp = {};
@@ -698,24 +698,31 @@ int Ts2ForwardGroup(int mode, int count, int len, int lenRound, int srcDim, int 
     }
     sp.ct = gemmk::C_BF16NORM;
     sp.epi = TS2_EPI_STORE;
-    sp.jobs = count;
-    sp.jobNormalize = normalizeBits;
-    sp.jobRope = rotateBits;
+    g.jobs = count;
+    g.jobNormalize = normalizeBits;
+    g.jobRope = rotateBits;
     for (int i = 0; i < count; ++i) {
         if (w[i]->strideBytes != g.ldb || res[i].strideBytes != g.ldc || w[i]->x < srcDim || w[i]->y < dstDim || res[i].x < dstDim || res[i].y < lenRound) {
             return TS2_ERR_UNSUPPORTED;
         }
-        sp.jobB[i] = (const uint8_t *)w[i]->ptr;
-        sp.jobC[i] = (uint8_t *)res[i].ptr;
-        sp.jobAlphaPtr[i] = alphaPtr[i];
+        g.jobB[i] = (const uint8_t *)w[i]->ptr;
+        g.jobC[i] = (uint8_t *)res[i].ptr;
+        g.jobAlphaPtr[i] = alphaPtr[i];
         if ((normalizeBits >> i) & 1) {
             const int64_t ld = tileScale[i]->strideBytes / 4;
             if (tileScale[i]->x < lenRound || tileScale[i]->y < dstDim / TILE || (g.ldTileScale && g.ldTileScale != ld)) {
                 return TS2_ERR_UNSUPPORTED;
             }
             g.ldTileScale = ld;
-            sp.jobTileScale[i] = (float *)tileScale[i]->ptr;
+            g.jobTileScale[i] = (float *)tileScale[i]->ptr;
         }
     }
-    return gemmk::RunSlice(sp, SliceType(mode), false, (hipStream_t)stream);
+    const int type = SliceType(mode);
+    if (gemmk::PreferJobs(g, type)) {
+        const int rc = gemmk::RunJobs(g, type, (hipStream_t)stream);
+        if (rc != TS2_ERR_UNSUPPORTED) {
+            return rc;
+        }
+    }
+    return wgs <= 256 ? gemmk::RunSlice(sp, type, false, (hipStream_t)stream) : TS2_ERR_UNSUPPORTED;
 }
