@@ -274,9 +274,60 @@ __device__ __forceinline__ float ComputeGradMult(float gradMaxNorm)
     return __uint_as_float(__float_as_uint(128.f / gradMaxNorm) & 0xff800000u);
 }
 
-template <class TFast>
+// 32 lanes move the codes of rows t0 .. t0 + U to another power of two of the gradients.  The codes stay and scale and maximum move along, exactly,
+// while bf16 holds the row at both powers: rows whose maximum leaves 2^-100 .. 2^100 (bf16 rounds their smaller elements to fewer bits, and from 2^-121
+// on the reciprocal of the scale overflows) or that bf16 has rounded to zero (scale 1) are quantised again from the fp32 gradients.
+__device__ __forceinline__ void MoveRowCodes(int t0, int len, int dim, const Mat &grad, float gradMult, float ratio, int h, const RowQuantOut &q)
+{
+    auto held = [](float x) { return x >= 0x1p-100f && x <= 0x1p100f; };
+    bool again = false;
+    if (h < U && t0 + h < len) {
+        const float top = q.rowAbsMax[t0 + h], scale = q.rowScale[t0 + h];
+        again = q.dst && (top == 0 ? scale != 0 : !held(top) || !held(top * ratio));
+        if (!again) {
+            q.rowScale[t0 + h] = scale * ratio;
+            q.rowAbsMax[t0 + h] = top * ratio;
+        }
+    }
+    const unsigned rows = (unsigned)(__ballot(again) >> (threadIdx.x & 32)); // (of these 32 lanes: the others may be elsewhere)
+    for (int k = 0; k < U; ++k) {
+        if (!((rows >> k) & 1)) {
+            continue;
+        }
+        const int t = t0 + k;
+        auto load = [&](int col) {
+            const F4 v = Load4<TF32>(At<TF32>(grad, t, col)) * gradMult;
+            const uint32_t lo = PackBf16x2(v.x, v.y), hi = PackBf16x2(v.z, v.w);
+            return MakeF4(__uint_as_float(lo << 16), __uint_as_float(lo & 0xffff0000u), __uint_as_float(hi << 16), __uint_as_float(hi & 0xffff0000u));
+        };
+        float mx = 0;
+        for (int col = h * 4; col < dim; col += 128) {
+            mx = fmaxf(mx, HMaxAbs(load(col)));
+        }
+        for (int d = 16; d > 0; d >>= 1) {
+            mx = fmaxf(mx, __shfl_xor(mx, d));
+        }
+        const float discr = mx > 0 ? mx / 127 : 0.f, mult = mx > 0 ? 1 / discr : 0.f;
+        for (int col = h * 4; col < dim; col += 128) {
+            const F4 v = load(col);
+            uint8_t *const dst = q.dst + (int64_t)t * q.dstStride + col;
+            if (q.seed) {
+                *(uint32_t *)dst = QuantDither4(v.x, v.y, v.z, v.w, mult, DitherWord(q.seed, t, col >> 2));
+            } else {
+                Store4<TI8>(dst, v * mult);
+            }
+        }
+        if (h == 0) {
+            q.rowScale[t] = discr;
+            q.rowAbsMax[t] = mx;
+        }
+    }
+}
+
+// ROWS: the rows are quantised already (q)
+template <class TFast, bool ROWS>
 __global__ void __launch_bounds__(256) ScaleGrad(int len, int tiles, const float *gradMaxNorm, const float *prevGradMult, Mat grad, Mat gradFast,
-    float *gradScaleOut, float *gradMultOut, float *rowScale, float *rowAbsMax)
+    float *gradScaleOut, float *gradMultOut, RowQuantOut q)
 {
     int t0, tile, h;
     float gradMult = ComputeGradMult(*gradMaxNorm);
@@ -303,10 +354,8 @@ __global__ void __launch_bounds__(256) ScaleGrad(int len, int tiles, const float
             }
         }
         // the rows' codes (int8) belong to values times the old power of two
-        if (rowScale && tile == 0 && h < U && t0 + h < len) {
-            const float ratio = gradMult / *prevGradMult;
-            rowScale[t0 + h] *= ratio;
-            rowAbsMax[t0 + h] *= ratio;
+        if (ROWS && tile == 0) {
+            MoveRowCodes(t0, len, tiles * TILE, grad, gradMult, gradMult / *prevGradMult, h, q);
         }
     }
 }
@@ -841,9 +890,9 @@ struct RowQuantJobs {
 };
 
 // codes, scale and (where asked for) plain maximum of a row that a wave holds as NCH chunks of 8 elements per lane; mx, plain: maxima of the
-// lane's own elements, with and without column scales
+// lane's own elements, with and without column scales.  Returns the row's maximum with them
 template <int NCH>
-__device__ __forceinline__ void StoreRowCodes(const F4 (&v)[NCH][2], const bool (&in)[NCH], int lane, int t, float mx, float plain, uint8_t *out,
+__device__ __forceinline__ float StoreRowCodes(const F4 (&v)[NCH][2], const bool (&in)[NCH], int lane, int t, float mx, float plain, uint8_t *out,
     float *rowScale, float *rowAbsMax, uint32_t seed)
 {
     mx = WaveMax(mx);
@@ -878,6 +927,7 @@ __device__ __forceinline__ void StoreRowCodes(const F4 (&v)[NCH][2], const bool 
             rowAbsMax[t] = plain;
         }
     }
+    return mx;
 }
 
 __device__ __forceinline__ void Unpack8(const uint4 &raw, F4 (&v)[2])
@@ -997,8 +1047,8 @@ __device__ __forceinline__ void TileNormBackprop8(const F4 (&src)[2], F4 (&g)[2]
     g[1] = (g[1] - src[1] * sigma) * scale;
 }
 
-// a row of bf16 values that the wave kept (zeros beyond the live rows), quantised
-template <int NCH> __device__ __forceinline__ void QuantKeptRow(const uint4 (&kept)[NCH], const bool (&in)[NCH], int lane, int t, const RowQuantOut &q)
+// a row of bf16 values that the wave kept (zeros beyond the live rows), quantised; returns its maximum
+template <int NCH> __device__ __forceinline__ float QuantKeptRow(const uint4 (&kept)[NCH], const bool (&in)[NCH], int lane, int t, const RowQuantOut &q)
 {
     F4 v[NCH][2];
     float mx = 0;
@@ -1007,7 +1057,7 @@ template <int NCH> __device__ __forceinline__ void QuantKeptRow(const uint4 (&ke
         Unpack8(kept[i], v[i]);
         mx = fmaxf(mx, fmaxf(HMaxAbs(v[i][0]), HMaxAbs(v[i][1])));
     }
-    StoreRowCodes<NCH>(v, in, lane, t, mx, mx, q.dst + (int64_t)t * q.dstStride, q.rowScale, q.rowAbsMax, q.seed);
+    return StoreRowCodes<NCH>(v, in, lane, t, mx, mx, q.dst + (int64_t)t * q.dstStride, q.rowScale, q.rowAbsMax, q.seed);
 }
 
 // BackpropLoLU<TBF16, TBF16, TBF16, MODE> over whole rows; MODE 1 quantises the gate's gradient only
@@ -1125,7 +1175,8 @@ template <int NCH> __global__ void __launch_bounds__(256) BackpropNormRopeRows(i
     QuantKeptRow<NCH>(g, in, lane, t, jobs.q[j]);
 }
 
-// BackpropLayerNormalize<TI8, TBF16, FINAL> over whole rows.  Rows len .. lenRound: codes and scales are cleared, FINAL clears its results there too
+// BackpropLayerNormalize<TI8, TBF16, FINAL> over whole rows; the codes belong to the multiplier known here and move to the next one in ScaleGrad.
+// Rows len .. lenRound: codes and scales are cleared, FINAL clears its results there too
 template <int NCH, bool FINAL, int NT>
 __global__ void __launch_bounds__(NT) BackpropLayerNormalizeRows(int len, int lenRound, int dim, Mat normState, Mat stateScale, Mat dNormState,
     const float *gradScale, const float *gradMult, Mat stateGrad, Mat stateGradFast, float *nextMaxNorm, RowQuantOut q)
@@ -1154,6 +1205,7 @@ __global__ void __launch_bounds__(NT) BackpropLayerNormalizeRows(int len, int le
             sc[i] = use ? ScaleAt(stateScale, col / TILE, t) : 0.f;
         }
         uint4 kept[NCH];
+        float top = 0;
 #pragma unroll
         for (int i = 0; i < NCH; ++i) {
             const int col = (i * 64 + lane) * 8;
@@ -1171,7 +1223,7 @@ __global__ void __launch_bounds__(NT) BackpropLayerNormalizeRows(int len, int le
             if (!live) {
                 g[0] = g[1] = ZeroF4();
             }
-            gmax = fmaxf(gmax, fmaxf(HMaxAbs(g[0]), HMaxAbs(g[1])));
+            top = fmaxf(top, fmaxf(HMaxAbs(g[0]), HMaxAbs(g[1])));
             kept[i] = Pack8(g[0] * gm, g[1] * gm);
             if (in[i] && (FINAL || live)) {
                 Store4<TF32>(At<TF32>(stateGrad, t, col), g[0]);
@@ -1179,7 +1231,10 @@ __global__ void __launch_bounds__(NT) BackpropLayerNormalizeRows(int len, int le
                 *(uint4 *)At<TBF16>(stateGradFast, t, col) = kept[i];
             }
         }
-        QuantKeptRow<NCH>(kept, in, lane, t, q);
+        gmax = fmaxf(gmax, top);
+        if (QuantKeptRow<NCH>(kept, in, lane, t, q) == 0 && __any(top != 0) && lane == 0) {
+            q.rowScale[t] = 1; // the codes are zeros, the gradients are not (MoveRowCodes)
+        }
     }
     PublishBlockMax<NT>(gmax, red, nextMaxNorm);
 }
@@ -1884,11 +1939,11 @@ extern "C" int ts2_scale_grad(const float *gradMaxNorm, const float *prevGradMul
     const bool later = reads(gradScaleOut) || reads(gradMultOut);
     float *scaleNow = later ? nullptr : gradScaleOut, *multNow = later ? nullptr : gradMultOut;
     if (fastType == TS2_BF16) {
-        hipLaunchKernelGGL((ScaleGrad<TBF16>), GridFor(len, tiles), dim3(256), 0, STREAM, len, tiles, gradMaxNorm, prevGradMult, M(*grad),
-            M(*gradFast), scaleNow, multNow, nullptr, nullptr);
+        hipLaunchKernelGGL((ScaleGrad<TBF16, false>), GridFor(len, tiles), dim3(256), 0, STREAM, len, tiles, gradMaxNorm, prevGradMult, M(*grad),
+            M(*gradFast), scaleNow, multNow, RowQuantOut{});
     } else if (fastType == TS2_E4M3) {
-        hipLaunchKernelGGL((ScaleGrad<TE4M3>), GridFor(len, tiles), dim3(256), 0, STREAM, len, tiles, gradMaxNorm, prevGradMult, M(*grad),
-            M(*gradFast), scaleNow, multNow, nullptr, nullptr);
+        hipLaunchKernelGGL((ScaleGrad<TE4M3, false>), GridFor(len, tiles), dim3(256), 0, STREAM, len, tiles, gradMaxNorm, prevGradMult, M(*grad),
+            M(*gradFast), scaleNow, multNow, RowQuantOut{});
     } else {
         return TS2_ERR_UNSUPPORTED;
     }
@@ -2216,13 +2271,19 @@ int Ts2BackpropLayerNormalizeRows(bool final, int len, int lenRound, const ts2_m
 }
 
 int Ts2ScaleGradRows(const float *gradMaxNorm, const float *prevGradMult, const ts2_mat *grad, const ts2_mat *gradFast, int len, float *gradScaleOut,
-    float *gradMultOut, float *rowScale, float *rowAbsMax, void *stream)
+    float *gradMultOut, const RowQuantOut &q, void *stream)
 {
     const int tiles = grad->x / TILE;
-    hipLaunchKernelGGL((ScaleGrad<TBF16>), GridFor(len, tiles), dim3(256), 0, STREAM, len, tiles, gradMaxNorm, prevGradMult, M(*grad), M(*gradFast),
-        gradScaleOut, gradMultOut, rowScale, rowAbsMax);
+    hipLaunchKernelGGL((ScaleGrad<TBF16, true>), GridFor(len, tiles), dim3(256), 0, STREAM, len, tiles, gradMaxNorm, prevGradMult, M(*grad), M(*gradFast),
+        gradScaleOut, gradMultOut, q);
     TS2_CHECK_LAUNCH();
     return TS2_OK;
+}
+
+int Ts2ScaleGradRows(const float *gradMaxNorm, const float *prevGradMult, const ts2_mat *grad, const ts2_mat *gradFast, int len, float *gradScaleOut,
+    float *gradMultOut, float *rowScale, float *rowAbsMax, void *stream)
+{
+    return Ts2ScaleGradRows(gradMaxNorm, prevGradMult, grad, gradFast, len, gradScaleOut, gradMultOut, RowQuantOut{nullptr, 0, rowScale, rowAbsMax, 0}, stream);
 }
 
 // The row-major k-tile quantiser over any number of bf16 gradients with the same rows

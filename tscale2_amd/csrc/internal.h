@@ -41,7 +41,10 @@ int Ts2BackpropNormRopeRows(int count, int len, int lenRound, const ts2_mat *con
 int Ts2BackpropLayerNormalizeRows(bool final, int len, int lenRound, const ts2_mat *normState, const ts2_mat *stateScale, const ts2_mat *dNormState,
     const float *gradScale, const float *gradMult, const ts2_mat *stateGrad, const ts2_mat *stateGradFast, float *nextMaxNorm, const RowQuantOut &q,
     void *stream);
-// ts2_scale_grad (bf16) that moves the rows' scales and maxima along with the values when their power of two changes
+// ts2_scale_grad (bf16) that moves the rows' codes, scales and maxima (q) along with the values when their power of two changes; the second
+// form leaves the codes, for rows whose maxima lie within 2^-100 .. 2^100 before and after
+int Ts2ScaleGradRows(const float *gradMaxNorm, const float *prevGradMult, const ts2_mat *grad, const ts2_mat *gradFast, int len, float *gradScaleOut,
+    float *gradMultOut, const RowQuantOut &q, void *stream);
 int Ts2ScaleGradRows(const float *gradMaxNorm, const float *prevGradMult, const ts2_mat *grad, const ts2_mat *gradFast, int len, float *gradScaleOut,
     float *gradMultOut, float *rowScale, float *rowAbsMax, void *stream);
 // the k-tile quantiser without the transpose, over `count` <= 4 bf16 gradients of one width: dst[t][x] with one scale per kTile rows,

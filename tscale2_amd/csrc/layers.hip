@@ -1133,8 +1133,7 @@ int ModelBackprop(ts2_model *M, void *s)
         // normalisation: 1, kept in gradMult[0]; a layer's normalisation backward: that layer's multiplier)
         M->fast = M->stepFast[stepId];
         if (M->fastQuantised) {
-            CK(Ts2ScaleGradRows(prevMax, M->gradMult + stepId, M->stateGrad.P(), M->fast.P(), M->len, gradScale, gradMult, M->sRowScale,
-                entry.rowAbsMax, s));
+            CK(Ts2ScaleGradRows(prevMax, M->gradMult + stepId, M->stateGrad.P(), M->fast.P(), M->len, gradScale, gradMult, entry, s));
         } else {
             CK(ts2_scale_grad(prevMax, M->gradMult + stepId, M->stateGrad.P(), M->fast.P(), M->fastGradType, M->len, gradScale, gradMult, s));
         }
