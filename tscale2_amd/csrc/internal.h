@@ -79,7 +79,7 @@ int Ts2BackpropGroupI8(int count, int len, int lenRound, int srcDim, int gradDim
 int Ts2ForwardGroup(int mode, int count, int len, int lenRound, int srcDim, int dstDim, const ts2_mat *src, const ts2_mat *const *w, float alpha,
     const float *const *alphaPtr, int normalizeBits, float vecScale, int rotateBits, const ts2_mat *rope, const ts2_mat *res,
     const ts2_mat *const *tileScale, void *stream);
-// ts2_opt_add_delta(.., TS2_BM_GRAD_APPLY) of several matrices in two launches (per 16 of them).  Ts2OptBatchable: one dispersion
+// ts2_opt_add_delta(.., TS2_BM_GRAD_APPLY) of several matrices in two or three launches (per 16 of them).  Ts2OptBatchable: one dispersion
 // estimate per row, rows of at most 4096 elements
 bool Ts2OptBatchable(const ts2_opt_matrix *m);
 int Ts2OptApplyBatch(int count, const ts2_opt_matrix *const *mats, const ts2_mat *const *delta, const ts2_mat *const *tileScale,

@@ -182,16 +182,23 @@ __global__ void __launch_bounds__(256) AddGradient(int xSize, int ySize, DeltaSr
 
 // first half of ConvertMatrixKernel (agpu_cuda.cuh:65-101): sko = rms of the whole matrix from the row sums, mult = 32 / sko (0 for a zero
 // matrix).  The reference recomputes this in every workgroup of the conversion; here one small launch leaves both scalars on the device.
-// (1024 threads; every thread gets the result)
-__device__ __forceinline__ float MatrixSkoOf(int totalXSize, int totalYSize, const float *sum2arr, float *red)
+// (NT threads, which add in the order of 1024; every thread gets the result)
+template <int NT> __device__ __forceinline__ float MatrixSkoOf(int totalXSize, int totalYSize, const float *sum2arr, float *red)
 {
-    float sum2 = 0;
+    constexpr int SETS = 1024 / NT; // of the 16 waves of 64 whose sums are added at the end
+    float sum2[SETS] = {};
     for (int k = threadIdx.x; k < totalYSize; k += 1024) {
-        sum2 += sum2arr[k];
+#pragma unroll
+        for (int i = 0; i < SETS; ++i) {
+            sum2[i] += i == 0 || k + i * NT < totalYSize ? sum2arr[k + i * NT] : 0.f;
+        }
     }
-    sum2 = WaveSum(sum2);
-    if ((threadIdx.x & 63) == 0) {
-        red[threadIdx.x >> 6] = sum2;
+#pragma unroll
+    for (int i = 0; i < SETS; ++i) {
+        const float s = WaveSum(sum2[i]);
+        if ((threadIdx.x & 63) == 0) {
+            red[i * (NT / 64) + (threadIdx.x >> 6)] = s;
+        }
     }
     __syncthreads();
     float tot = 0;
@@ -209,7 +216,7 @@ __device__ __forceinline__ float ConvertMultOf(float sko)
 __global__ void __launch_bounds__(1024) MatrixSko(int totalXSize, int totalYSize, const float *sum2arr, float *resDiscrScale, float *convertMult)
 {
     __shared__ float red[16];
-    const float sko = MatrixSkoOf(totalXSize, totalYSize, sum2arr, red);
+    const float sko = MatrixSkoOf<1024>(totalXSize, totalYSize, sum2arr, red);
     if (threadIdx.x == 0) {
         convertMult[0] = ConvertMultOf(sko);
         resDiscrScale[0] = sko;
@@ -241,8 +248,8 @@ __global__ void __launch_bounds__(256) ConvertMatrix(int xSize, int ySize, int y
     }
 }
 
-// ---- "one delta, apply now" with a dispersion estimate per row, over up to OPT_JOBS matrices in two launches: rows, then
-// matrix scale and conversion.  Small matrices are bound by launches (a 512 x 512 one took five of 2 to 4 us each), large ones by the second
+// ---- "one delta, apply now" with a dispersion estimate per row, over up to OPT_JOBS matrices in two or three launches: rows,
+// matrix scale, conversion.  Small matrices are bound by launches (a 512 x 512 one took five of 2 to 4 us each), large ones by the second
 // read of the delta and by the two single-workgroup launches.
 constexpr int OPT_JOBS = 16; // jobs travel as kernel arguments
 constexpr int OPT_ROW_MAX = 4096;
@@ -260,7 +267,7 @@ struct OptJobs {
 
 // RowSum2, UpdateGlobalRowDisp (one row per estimate) and AddGradient of a row by one team - a wave, or the workgroup - that keeps the
 // packed row in registers between its sum and its use (NCH chunks of four elements per thread), all operands of the row in flight at
-// once.  sumWeight is only read here; OptConvert, which follows, moves it on.  8192 x 2048, with the row sums and estimates it
+// once.  sumWeight is only read here; PublishScale, in a launch that follows, moves it on.  8192 x 2048, with the row sums and estimates it
 // replaces: 50.5 + 8.4 + 5.9 us in three launches -> 53.5 (a wave per row, eight chunks in two goes: 57.8)
 template <int NCH, bool WG> __global__ void __launch_bounds__(256) OptRows(OptJobs jobs, const ts2_add_gradient_params *pParams)
 {
@@ -353,23 +360,48 @@ template <class TDst> __device__ __forceinline__ void ConvertStore(const OptJob 
     }
 }
 
-// MatrixSko and ConvertMatrix per job, a wave per row: every workgroup forms the matrix scale from the row sums itself (32 KB from L2 for 8192
-// rows, with its first weights under way meanwhile), which saves a launch of one workgroup between the passes (5 of 207 us per 3 matrices each)
-__global__ void __launch_bounds__(1024) OptConvert(OptJobs jobs, const ts2_add_gradient_params *pParams)
+// the scale of a job's matrix, and the weight of the dispersion estimates that OptRows used
+__device__ __forceinline__ void PublishScale(const OptJob &o, float sko, const ts2_add_gradient_params *pParams)
+{
+    o.convertMult[0] = ConvertMultOf(sko);
+    o.matrixScale[0] = sko;
+    o.sumWeight[0] = o.sumWeight[0] * pParams->dispDecay + 1;
+}
+
+__global__ void __launch_bounds__(1024) OptScale(OptJobs jobs, const ts2_add_gradient_params *pParams)
+{
+    __shared__ float red[16];
+    const OptJob &o = jobs.j[blockIdx.x];
+    const float sko = MatrixSkoOf<1024>(o.xSize, o.ySize, o.weightsRowSum2, red);
+    if (threadIdx.x == 0) {
+        PublishScale(o, sko, pParams);
+    }
+}
+
+// ConvertMatrix per job, a wave per row, four rows to a workgroup.  OWN: every workgroup forms the matrix scale from the row sums itself, with its
+// first weights under way meanwhile, and OptScale falls away (OwnScale)
+template <bool OWN> __global__ void __launch_bounds__(256) OptConvert(OptJobs jobs, const ts2_add_gradient_params *pParams)
 {
     __shared__ float red[16];
     const OptJob &o = jobs.j[blockIdx.y];
+    if ((int)blockIdx.x * 4 >= o.yBufSize) {
+        return; // (the grid is the tallest matrix's)
+    }
     const int first = (threadIdx.x & 63) * 4;
-    int y = blockIdx.x * 16 + (threadIdx.x >> 6);
+    int y = blockIdx.x * 4 + (threadIdx.x >> 6);
     F4 v[CONVERT_CHUNKS];
     ConvertLoad(o, y, first, v);
-    const float sko = MatrixSkoOf(o.xSize, o.ySize, o.weightsRowSum2, red), mult = ConvertMultOf(sko);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        o.convertMult[0] = mult;
-        o.matrixScale[0] = sko;
-        o.sumWeight[0] = o.sumWeight[0] * pParams->dispDecay + 1; // the weight of the dispersion estimates that OptRows used
+    float mult;
+    if constexpr (OWN) {
+        const float sko = MatrixSkoOf<256>(o.xSize, o.ySize, o.weightsRowSum2, red);
+        mult = ConvertMultOf(sko);
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            PublishScale(o, sko, pParams);
+        }
+    } else {
+        mult = o.convertMult[0];
     }
-    for (; y < o.yBufSize; y += gridDim.x * 16) {
+    for (; y < o.yBufSize; y += gridDim.x * 4) {
         for (int x0 = first; x0 < o.xSize; x0 += CONVERT_CHUNKS * 256) {
             if (o.fastType == TS2_I8) {
                 ConvertStore<TI8>(o, y, x0, v, mult);
@@ -379,7 +411,7 @@ __global__ void __launch_bounds__(1024) OptConvert(OptJobs jobs, const ts2_add_g
                 ConvertStore<TBF16>(o, y, x0, v, mult);
             }
             const bool more = x0 + CONVERT_CHUNKS * 256 < o.xSize;
-            const int nextY = more ? y : y + (int)gridDim.x * 16, nextX = more ? x0 + CONVERT_CHUNKS * 256 : first;
+            const int nextY = more ? y : y + (int)gridDim.x * 4, nextX = more ? x0 + CONVERT_CHUNKS * 256 : first;
             if (nextY < o.yBufSize) {
                 ConvertLoad(o, nextY, nextX, v);
             }
@@ -390,6 +422,17 @@ __global__ void __launch_bounds__(1024) OptConvert(OptJobs jobs, const ts2_add_g
 int RowGrid(int rows)
 {
     return rows < 8192 ? rows : 8192;
+}
+
+// Whether the workgroups of the conversion form the scales: together they read the square of the rows from L2, a launch of its own reads the
+// rows once and costs 1.2 us (more outside a graph).  Own against separate launch, us in a graph, by the sum S of the squares:
+//   S <= 2^24   300x512 7.0, 8.1; 2048x1024 12.2, 13.4; 4096x512 12.9, 13.3; 4096x1024 18.3, 19.1; 16 of 1024x1024 60.0, 61.2
+//   S <= 2^26   2048 columns and more 8192x2048 60.6, 61.4; 8192x4096 116.9, 119.6; 8 of 2048x2048 113.2, 115.9; fewer 8192x512 21.1, 20.9; 16 of
+//               2048x512 64.0, 61.6; 8 of 4096x1024 119.4, 116.4 (2^27)
+//   beyond      12288x1024 53.2, 49.9; 32768x256 71.5, 43.0; 50304x2048 beside 15 of 8192x2048 1532, 1511, beside 15 of 2048x2048 747, 726
+bool OwnScale(double squares, int minX)
+{
+    return squares <= (minX >= 2048 ? 1 << 26 : 1 << 24);
 }
 
 bool F32Ok(const ts2_mat *m, int x, int y)
@@ -553,7 +596,8 @@ int Ts2OptApplyBatch(int count, const ts2_opt_matrix *const *mats, const ts2_mat
     for (int first = 0; first < count; first += OPT_JOBS) {
         OptJobs jobs = {};
         const int n = count - first < OPT_JOBS ? count - first : OPT_JOBS;
-        int maxX = 0, maxRows = 0, maxBuf = 0;
+        int maxX = 0, minX = OPT_ROW_MAX, maxRows = 0, maxBuf = 0;
+        double squares = 0;
         for (int i = 0; i < n; ++i) {
             const ts2_opt_matrix *m = mats[first + i];
             const ts2_mat *d = delta[first + i], *ts = tileScale[first + i];
@@ -578,6 +622,8 @@ int Ts2OptApplyBatch(int count, const ts2_opt_matrix *const *mats, const ts2_mat
             jobs.j[i] = {M(*d), M(*ts), M(m->avgGrad), M(m->weights), M(m->fast), m->gradRowSum2, m->weightsRowSum2, m->rowScale, m->rowDisp,
                 m->sumWeight, m->matrixScale, m->convertMult, m->sparsity, m->xSize, m->ySize, m->yBufSize, m->fastType};
             maxX = maxX > m->xSize ? maxX : m->xSize;
+            minX = minX < m->xSize ? minX : m->xSize;
+            squares += (double)m->ySize * m->ySize;
             maxRows = maxRows > m->ySize ? maxRows : m->ySize;
             maxBuf = maxBuf > m->yBufSize ? maxBuf : m->yBufSize;
         }
@@ -591,7 +637,14 @@ int Ts2OptApplyBatch(int count, const ts2_opt_matrix *const *mats, const ts2_mat
             hipLaunchKernelGGL((OptRows<4, true>), dim3(RowGrid(maxRows), n), dim3(256), 0, STREAM, jobs, params);
         }
         TS2_CHECK_LAUNCH();
-        hipLaunchKernelGGL(OptConvert, dim3(RowGrid((maxBuf + 15) / 16), n), dim3(1024), 0, STREAM, jobs, params);
+        const dim3 grid(RowGrid((maxBuf + 3) / 4), n);
+        if (OwnScale(squares, minX)) {
+            hipLaunchKernelGGL(OptConvert<true>, grid, dim3(256), 0, STREAM, jobs, params);
+        } else {
+            hipLaunchKernelGGL(OptScale, dim3(n), dim3(1024), 0, STREAM, jobs, params);
+            TS2_CHECK_LAUNCH();
+            hipLaunchKernelGGL(OptConvert<false>, grid, dim3(256), 0, STREAM, jobs, params);
+        }
         TS2_CHECK_LAUNCH();
     }
     return TS2_OK;
