@@ -54,3 +54,19 @@ def test_sums(half_steps, factors):
                          tile_config=config)
     assert torch.equal(got, few)
     assert bool(((got.double() - want).abs() <= len(factors) * 2e-4 * want.abs().max()).all())
+
+
+# sizes that the 256x128 kernel takes by itself: asked for, it is this kernel (e4m3 sums in the order of the kernel for few tiles, which the other's is not)
+@pytest.mark.parametrize("ct,epi", [(L.F32, L.EPI_STORE), (L.F32, L.EPI_ADD)])
+def test_asked_for_beyond_its_range(ct, epi):
+    print("case square asked for", ct, epi, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    m, n, k = 2048, 1152, 512
+    # (magnitudes of 2^-9 to 2^8: sums that fp32 does not hold exactly)
+    a, b = [(torch.randn((r, k), device="cuda", generator=gen) * torch.exp2(torch.randint(-7, 7, (r, k), device="cuda", generator=gen).float())).to(
+        torch.float8_e4m3fn).view(torch.uint8) for r in (m, n)]
+    c0 = torch.randn((m, n), device="cuda", generator=gen)
+    got, few, tall, free = [c0.clone() for _ in range(4)]
+    for c, config in ((got, SQUARE), (few, SLICE), (tall, 262144), (free, 0)):
+        L.load().gemm_nt(a, b, c, L.E4M3, ct, alpha=0.25, epilogue=epi, tile_config=config)
+    assert torch.equal(got, few) and torch.equal(free, tall) and not torch.equal(got, tall)

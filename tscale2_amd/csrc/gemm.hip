@@ -1380,18 +1380,18 @@ extern "C" int ts2_gemm_nt(const ts2_gemm_args *a, void *streamPtr)
                        : a->cType == TS2_I32                     ? C_I32
                                                                  : -1;
         const int epi = a->epilogue == TS2_EPI_ADD ? TS2_EPI_ADD : TS2_EPI_STORE;
-        // the 256x128 tile for products of medium size: bit 18 asks for it (TS2_ERR_UNSUPPORTED if it cannot run the call)
+        // the 256x128 tile for products of medium size: bit 18 asks for it, bit 19 for the 64x64 one (TS2_ERR_UNSUPPORTED if it cannot run the call)
         if (ct >= 0 && (a->tileConfig & 262144)) {
             return splitK <= 1 ? RunTall(p, type, ct, epi, stream) : TS2_ERR_UNSUPPORTED;
+        }
+        if (ct >= 0 && (a->tileConfig & 524288)) {
+            return splitK <= 1 ? RunSquare(p, type, ct, epi, stream) : TS2_ERR_UNSUPPORTED;
         }
         if (ct >= 0 && splitK <= 1 && !(a->tileConfig & (3 | 8 | 16 | 128 | 2048 | 4096 | 32768 | 65536 | 131072)) && PreferTall(p, type, ct, epi) &&
             TallCanRun(p, type, ct, epi)) {
             return RunTall(p, type, ct, epi, stream);
         }
-        // the 64x64 tile for results with fewer tiles still: bit 19 asks for it (TS2_ERR_UNSUPPORTED if it cannot run the call)
-        if (ct >= 0 && (a->tileConfig & 524288)) {
-            return splitK <= 1 ? RunSquare(p, type, ct, epi, stream) : TS2_ERR_UNSUPPORTED;
-        }
+        // the 64x64 tile for results with fewer tiles still
         if (ct >= 0 && splitK <= 1 && !(a->tileConfig & (3 | 8 | 16 | 128 | 2048 | 4096 | 32768 | 65536 | 131072)) && PreferSquare(p) &&
             SquareCanRun(p, type, ct, epi)) {
             return RunSquare(p, type, ct, epi, stream);
