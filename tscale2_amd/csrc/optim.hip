@@ -390,9 +390,10 @@ template <bool OWN> __global__ void __launch_bounds__(256) OptConvert(OptJobs jo
     const int first = (threadIdx.x & 63) * 4;
     int y = blockIdx.x * 4 + (threadIdx.x >> 6);
     F4 v[CONVERT_CHUNKS];
-    ConvertLoad(o, y, first, v);
     float mult;
+    bool loaded = OWN;
     if constexpr (OWN) {
+        ConvertLoad(o, y, first, v);
         const float sko = MatrixSkoOf<256>(o.xSize, o.ySize, o.weightsRowSum2, red);
         mult = ConvertMultOf(sko);
         if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -403,17 +404,16 @@ template <bool OWN> __global__ void __launch_bounds__(256) OptConvert(OptJobs jo
     }
     for (; y < o.yBufSize; y += gridDim.x * 4) {
         for (int x0 = first; x0 < o.xSize; x0 += CONVERT_CHUNKS * 256) {
+            if (!loaded) {
+                ConvertLoad(o, y, x0, v);
+            }
+            loaded = false;
             if (o.fastType == TS2_I8) {
                 ConvertStore<TI8>(o, y, x0, v, mult);
             } else if (o.fastType == TS2_E4M3) {
                 ConvertStore<TE4M3>(o, y, x0, v, mult);
             } else {
                 ConvertStore<TBF16>(o, y, x0, v, mult);
-            }
-            const bool more = x0 + CONVERT_CHUNKS * 256 < o.xSize;
-            const int nextY = more ? y : y + (int)gridDim.x * 4, nextX = more ? x0 + CONVERT_CHUNKS * 256 : first;
-            if (nextY < o.yBufSize) {
-                ConvertLoad(o, nextY, nextX, v);
             }
         }
     }
@@ -426,8 +426,8 @@ int RowGrid(int rows)
 
 // Whether the workgroups of the conversion form the scales: together they read the square of the rows from L2, a launch of its own reads the
 // rows once and costs 1.2 us (more outside a graph).  Own against separate launch, us in a graph, by the sum S of the squares:
-//   S <= 2^24   300x512 7.0, 8.1; 2048x1024 12.2, 13.4; 4096x512 12.9, 13.3; 4096x1024 18.3, 19.1; 16 of 1024x1024 60.0, 61.2
-//   S <= 2^26   2048 columns and more 8192x2048 60.6, 61.4; 8192x4096 116.9, 119.6; 8 of 2048x2048 113.2, 115.9; fewer 8192x512 21.1, 20.9; 16 of
+//   S <= 2^24   300x512 7.0, 8.1; 2048x1024 11.2, 12.2; 4096x512 12.0, 12.4; 4096x1024 18.0, 18.7; 16 of 1024x1024 60.2, 61.2
+//   S <= 2^26   2048 columns and more 8192x2048 60.7, 61.3; 8192x4096 117.1, 119.1; 8 of 2048x2048 114.5, 116.5; fewer 8192x512 21.1, 20.9; 16 of
 //               2048x512 64.0, 61.6; 8 of 4096x1024 119.4, 116.4 (2^27)
 //   beyond      12288x1024 53.2, 49.9; 32768x256 71.5, 43.0; 50304x2048 beside 15 of 8192x2048 1532, 1511, beside 15 of 2048x2048 747, 726
 bool OwnScale(double squares, int minX)
