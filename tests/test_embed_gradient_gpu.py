@@ -13,7 +13,7 @@ from tscale2_amd import lib as L  # noqa: E402
 EMBED_BACKWARD = "_Z16Ts2EmbedBackwardiiPKiPKjPK7ts2_matS5_iPiPv"
 
 
-@pytest.mark.parametrize("labels,dim", [(65536, 1024), (174763, 384), (300, 256)])  # from 2^26 elements on the labels are marked, if a quarter as many rows are there
+@pytest.mark.parametrize("labels,dim", [(65536, 1024), (174763, 384), (300, 256)])  # (the labels of the first are marked from 30720 rows on)
 @pytest.mark.parametrize("n", [257, 43690, 50001])
 def test_embed_gradient(labels, dim, n):
     print("case embed gradient", labels, dim, n, flush=True)
@@ -47,3 +47,33 @@ def test_embed_gradient(labels, dim, n):
         want, mag, named = np.zeros((labels, dim)), np.zeros((labels, dim)), np.bincount(ids[:k], minlength=labels)
         np.add.at(want, ids[:k], term[:k])
         np.add.at(mag, ids[:k], np.abs(term[:k]))
+
+
+# both sides of every line of the choice: elements, rows, labels, rows to labels (few, many).  The marked form stores where one term names a label, the
+# other adds to a cleared row, and both are sums in fp32 of any order; the marks tell which ran
+@pytest.mark.parametrize("labels,dim,n,marked", [
+    (57344, 1024, 57345, True), (57343, 1024, 57345, False), (65536, 896, 30720, True), (65536, 896, 30719, False), (45056, 1408, 40000, True), (45055, 1408, 40000, False),
+    (81920, 768, 35840, True), (81920, 768, 35839, False), (58720, 1024, 88080, True), (58720, 1024, 88081, False)])
+def test_choice_of_the_embed_gradient(labels, dim, n, marked):
+    print("case embed gradient choice", labels, dim, n, marked, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    ids = (torch.rand(n, device="cuda", generator=gen) ** 2 * labels).long().clamp(0, labels - 1)
+    minus = torch.rand(n, device="cuda", generator=gen) < 0.3
+    raw = torch.where(minus, ids - 2 ** 31, ids).to(torch.int32)  # (the sign bit subtracts)
+    ptr = torch.arange(n + 1, dtype=torch.int32, device="cuda")
+    grad = torch.randn((n, dim), device="cuda", generator=gen)
+    mark = torch.full((labels,), 5, dtype=torch.int32, device="cuda")
+    out = torch.full((labels, dim), float("nan"), device="cuda")
+    lib = L.load()
+    assert raw.numel() == n and int(ids.min()) >= 0 and int(ids.max()) < labels
+    rc = getattr(lib.dll, EMBED_BACKWARD)(n, dim, C.c_void_p(ptr.data_ptr()), C.c_void_p(raw.data_ptr()), C.byref(L.mat(grad)), C.byref(L.mat(out)), labels,
+                                          C.c_void_p(mark.data_ptr()), lib.stream())
+    assert rc == 0
+    assert bool((mark == 5).all()) != marked
+    named = torch.bincount(ids, minlength=labels)
+    for c in range(0, dim, 128):
+        term = grad[:, c:c + 128].double() * torch.where(minus, -1.0, 1.0).double()[:, None]
+        want = torch.zeros((labels, 128), device="cuda", dtype=torch.float64).index_add_(0, ids, term)
+        size = torch.zeros((labels, 128), device="cuda", dtype=torch.float64).index_add_(0, ids, term.abs())
+        got = out[:, c:c + 128].double()
+        assert bool((got[named <= 1] == want[named <= 1]).all()) and bool(((got - want).abs() <= named[:, None] * 2.0 ** -24 * size).all())

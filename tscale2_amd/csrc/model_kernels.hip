@@ -807,12 +807,25 @@ int Ts2EmbedForward(int len, int lenRound, int dim, const int *labelPtr, const u
     return TS2_OK;
 }
 
+// Where the marks pay: five launches instead of two, and waves instead of workgroups on the rows that share a label.  Measured over 16385 to 131073
+// labels, 256 to 4096 columns and a quarter to four times as many rows as labels, with labels drawn evenly (e), by Zipf's law (z) and as the sixth power
+// of an even number (p, 16 % of the rows name one label); time with marks over time without, e z p:
+//   elements   65537 x 512 (2^25), 65536 rows 0.75 0.94 1.01; 50305 x 1024 (2^25.6), 32768 rows 0.72 0.97 1.03, 50000 rows 0.74 0.95 1.02; 65537 x 1024 (2^26),
+//              32768 rows 0.74 0.97 1.00, 65536 rows 0.72 0.92 0.98; 131073 x 2048, 131072 rows 0.70 0.88 0.88
+//   rows       65537 x 1024, 16385 rows 0.84 1.04 1.12, 28672 rows 0.76 0.98 1.03; 50305 x 1536, 25000 rows 0.75 0.96 1.04, 32768 rows 0.70 0.93 0.99
+//   labels     40961 x 1536, 32768 rows 0.71 0.92 1.02, 50305 as above; 32769 x 2048, 32768 rows 0.73 1.00 1.02; 16385 x 4096, 16384 rows 0.74 1.07 1.11
+//   rows to labels  98305 x 768, a third 0.80 0.94 1.02, half 0.73 0.92 0.99; 131073 x 512, a quarter 0.79 1.01 1.04, half 0.67 0.94 0.98; 65537 x 1024, 1.4 0.80 0.92
+//              0.98, twice 0.89 0.93 0.98 but 1.03 where each is named twice
+static bool MarkLabels(int len, int dim, int labelCount)
+{
+    return (int64_t)labelCount * dim >= (int64_t)7 << 23 && len >= 30720 && labelCount >= 45056 && (int64_t)len * 16 >= (int64_t)labelCount * 7 &&
+           (int64_t)len * 2 <= (int64_t)labelCount * 3;
+}
+
 int Ts2EmbedBackward(int len, int dim, const int *labelPtr, const uint32_t *labels, const ts2_mat *grad, const ts2_mat *delta, int labelCount,
     int *mark, void *stream)
 {
-    // Five launches instead of two, for large deltas whose labels are about as many as the rows.  16385 x 1024 gain 64 -> 54 us where every label is as
-    // likely and lose 132 -> 173 where few are in most rows (50305 x 2048 of such labels: 355 -> 348); 1024 rows of 50305 labels 33 -> 42
-    if (mark && labelCount >= len && labelCount / 4 <= len && (int64_t)labelCount * dim >= ((int64_t)1 << 26)) {
+    if (mark && MarkLabels(len, dim, labelCount)) {
         const dim3 terms((len + 255) / 256);
         hipLaunchKernelGGL(LabelsNone, dim3((labelCount + 255) / 256), dim3(256), 0, STREAM, labelCount, mark);
         hipLaunchKernelGGL(LabelsNamed, terms, dim3(256), 0, STREAM, len, labelPtr, labels, mark);
