@@ -70,6 +70,8 @@ int Ts2DeltaRows(int mode, int len, int lenRound, int srcDim, int gradDim, const
     void *stream);
 // estimated microseconds of that (TS2_E4M3 or TS2_BF16)
 double Ts2DeltaCost(int mode, int lenRound, int srcDim, int gradDim, int64_t partialFloats);
+// how many deltas of the model's last backward pass waited for its end (a layer's stacked matrices count as one)
+int Ts2ModelWaitingDeltas(const ts2_model *M);
 // int8: srcGrad (+)= sum_i alpha_i * *alphaPtr_i * rowScale_i[t] * (grad8_i W_i^T), count <= 4 products of one shape added in order
 int Ts2BackpropGroupI8(int count, int len, int lenRound, int srcDim, int gradDim, const ts2_mat *grad8, const float *const *rowScale,
     const ts2_mat *transformT, const float *alpha, const float *const *alphaPtr, const ts2_mat *srcGrad, int srcGradType, int add, void *stream);

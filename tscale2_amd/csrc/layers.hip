@@ -1156,6 +1156,11 @@ int ModelBackprop(ts2_model *M, void *s)
 }
 } // namespace
 
+int Ts2ModelWaitingDeltas(const ts2_model *M)
+{
+    return (int)M->queue.deltas.size();
+}
+
 namespace
 {
 // Whether the deltas of a backward pass wait for its end.  int8: always (the launch at the end reads both operands as they lie, quantised in one
