@@ -1,6 +1,6 @@
 """The packed deltas that wait for the end of a backward pass (one launch for all of them) against the same model in recompute mode, where every
-layer's deltas run at once on the kernels for single products.  The operands are the same bits.  int8 sums are exact per k-tile, and up to
-four k-tiles are added in the same order: same bits.  Otherwise fp32 sums are added in another order, which moves a value by far less than
+layer's deltas run at once on the kernels for single products.  The operands are the same bits.  int8 sums are exact per k-tile, and the k-tiles
+are added in the same groups: same bits (held to here up to four k-tiles, for more in a test of its own).  e4m3: fp32 sums are added in another order, which moves a value by far less than
 the step of its tile (largest / 127) and can turn one rounding: one step, and the scale's own 1e-5."""
 import numpy as np
 import pytest
@@ -55,6 +55,15 @@ def test_deltas_at_the_end_of_a_pass_equal_deltas_layer_by_layer(mode, dim, head
         top = np.abs(b).reshape(b.shape[0], -1, 128).max(2).repeat(128, 1)
         assert (np.abs(a - b) <= top * (1.0 / 127 + 2e-5)).all()
         assert (a != b).mean() < 0.02 or (np.abs(a - b) <= 2e-5 * np.abs(b)).mean() > 0.98
+
+
+# the groups of k-tiles: three and two, four each and three, one each beyond a register of scales
+@pytest.mark.parametrize("dim,heads,ffn,depth,k_tile,n", [(256, 2, 384, 1, 128, 600), (384, 1, 640, 1, 128, 1400), (128, 1, 256, 2, 256, 5000), (256, 3, 384, 1, 128, 8300)])
+def test_k_tiles_are_summed_as_layer_by_layer(dim, heads, ffn, depth, k_tile, n):
+    print("case k-tile groups", dim, heads, ffn, depth, k_tile, n, flush=True)
+    args = (L.I8, dim, heads, ffn, depth, k_tile, n, 500)
+    for a, b in zip(deltas(*args, False), deltas(*args, True)):
+        assert b.any() and np.array_equal(a, b)
 
 
 WAITING = "_Z21Ts2ModelWaitingDeltasPK9ts2_model"

@@ -19,7 +19,7 @@ struct DeltaJob {
 constexpr int DELTA_JOBS = 32;
 struct DeltaBatchP {
     DeltaJob job[DELTA_JOBS];
-    int count, kBytes, kLive, kTileBytes;
+    int count, kBytes, kLive, kTileBytes, kGroup; // kGroup (i8): k-tiles that are summed apart
 };
 // any number of deltas over the same rows, 32 to a launch (T_I8 with k-tile scales, T_FP8)
 bool DeltaBatchCanRun(const DeltaJob &d, int type, int kBytes, int kLive, int kTileBytes);

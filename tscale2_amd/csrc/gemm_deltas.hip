@@ -9,7 +9,8 @@
 // packing's row maxima need one exchange between the two waves of a row; the bytes leave through LDS as whole 128-byte rows.
 // Measured (MI355X): 16 products of the e512 d8 int8 step (16384 rows, 464 GOP) 902 us + 180 of packing their slices -> 321; those of a step of 512 x
 // 2048 over 4096 tokens in e4m3 (146 GFLOP) 286 + 23 -> 100; of 256 x 1024 over 512 tokens in int8 184 -> 14.  The same batch on 64x128 tiles: 708, 162, 26.
-// i8: one scale per kTile rows; the exact int32 sum of a k-tile is added, scaled, to fp32 accumulators in tile order.
+// i8: one scale per kTile rows; the exact int32 sums of up to four k-tiles are added, scaled, in fp32, and these sums to each other, both in tile order: the
+// sums of the delta products one by one, bit by bit.  (One chain over all k-tiles had 1.6 times their error from 64 bits at 32 k-tiles.)
 #include "gemm_deltas.h"
 
 using namespace gemmk;
@@ -160,7 +161,7 @@ template <int TYPE> __global__ void __launch_bounds__(512, 2) GemmDeltas(DeltaBa
     // ---- k-tiles (i8)
     const int kTiles = KT ? bp.kBytes / bp.kTileBytes : 0, perTile = KT ? bp.kTileBytes / DK : 0;
     const float *scales = KT ? d.kTileScale + (d.kTileScaleRows ? (int64_t)min((rowBase + wm * 64) / d.kTileScaleRows, (d.gradDim - 1) / d.kTileScaleRows) * kTiles : 0) : nullptr;
-    float total[2][2][16];
+    float total[2][2][16], part[KT ? 2 : 1][2][16];
     float kScale = 0; // lane i: scale of k-tile i of the current 64
     if constexpr (KT) {
 #pragma unroll
@@ -170,22 +171,39 @@ template <int TYPE> __global__ void __launch_bounds__(512, 2) GemmDeltas(DeltaBa
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
                     total[i][n][e] = 0;
+                    part[i][n][e] = 0;
                 }
             }
         }
     }
+    int left = bp.kGroup;
     auto endOfTile = [&](int kt) {
         if ((kt & 63) == 0) {
             kScale = kt + lane < kTiles ? scales[kt + lane] : 0.f;
         }
         const float sc = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(kScale), kt & 63));
+        const bool last = --left == 0 || kt + 1 == kTiles;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
 #pragma unroll
             for (int n = 0; n < 2; ++n) {
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
-                    total[i][n][e] = __builtin_fmaf(sc, (float)acc[i][n][e], total[i][n][e]);
+                    part[i][n][e] = __builtin_fmaf(sc, (float)acc[i][n][e], part[i][n][e]);
+                }
+            }
+        }
+        if (last) {
+            left = bp.kGroup;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+#pragma unroll
+                for (int n = 0; n < 2; ++n) {
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        total[i][n][e] += part[i][n][e];
+                        part[i][n][e] = 0;
+                    }
                 }
             }
         }
@@ -306,11 +324,14 @@ bool DeltaBatchCanRun(const DeltaJob &d, int type, int kBytes, int kLive, int kT
 
 int RunDeltaBatch(const DeltaJob *jobs, int count, int type, int kBytes, int kLive, int kTileBytes, hipStream_t stream)
 {
+    // (the groups of Ts2DeltaRows: as few as hold four k-tiles each at most, of equal size)
+    const int kTiles = type == T_I8 && kTileBytes > 0 && kBytes > kTileBytes ? kBytes / kTileBytes : 1, groups = (kTiles + 3) / 4, kGroup = (kTiles + groups - 1) / groups;
     for (int done = 0; done < count;) {
         DeltaBatchP bp = {};
         bp.kBytes = kBytes;
         bp.kLive = kLive;
         bp.kTileBytes = kTileBytes;
+        bp.kGroup = kGroup;
         int blocks = 0;
         for (; done < count && bp.count < DELTA_JOBS; ++done) {
             if (!DeltaBatchCanRun(jobs[done], type, kBytes, kLive, kTileBytes)) {
