@@ -86,3 +86,20 @@ def test_sums(count, rows, cols, k):
         want, size = want + part, size + part.abs()
     # exact int32 sums; a conversion, a product of two factors and an addition each
     assert bool(((c.double() - want).abs() <= 5 * 2.0 ** -24 * count * size)[:live].all()) and not bool(c[live:].any())
+
+
+# operands whose sums are exact: what is left is a fused multiply-add per element, the same in every kernel
+@pytest.mark.parametrize("t", [L.I8, L.E4M3])
+@pytest.mark.parametrize("row_scale", [True, False])
+def test_accumulates_with_one_rounding(t, row_scale):
+    print("case tall one rounding", t, row_scale, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    m, n, k = 512, 384, 640
+    a, b = operand(t, m, k, gen), operand(t, n, k, gen)
+    rs = torch.rand(m, device="cuda", generator=gen) + 0.5 if row_scale else None
+    factor = torch.full((1,), 0.37, device="cuda")
+    c0 = torch.randn((m, n), device="cuda", generator=gen) * 100
+    got, few = c0.clone(), c0.clone()
+    for c, config in ((got, TALL), (few, 65536)):
+        L.load().gemm_nt(a, b, c, t, L.F32, row_scale=rs, alpha=0.3, alpha_ptr=factor, epilogue=L.EPI_ADD, tile_config=config, m_live=m - 9)
+    assert torch.equal(got, few)

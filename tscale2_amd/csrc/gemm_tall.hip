@@ -209,15 +209,22 @@ template <int TYPE, int CT, int EPI, bool SEG, bool JOBS = false> __global__ voi
     TALL_BARRIER(); // every wave has read its last operands
 
     if constexpr (CT == C_F32) {
+        // ADD: the sums are scaled where the lane holds what they are added to, in one fused operation like in the other kernels (scaled before, the
+        // product was rounded once more: 2.64e-8 from 64 bits instead of 2.50e-8)
+        constexpr bool ADD = EPI == TS2_EPI_ADD;
         uint8_t *const mine = lds + wave * 16384;
+        float *const rowFactor = (float *)(lds + 8 * 16384) + wave * 64;
         float scale = p.alpha;
         if (!SEG && p.alphaPtr) {
             scale *= *p.alphaPtr;
         }
+        if constexpr (ADD) {
+            rowFactor[lane] = p.rowScale ? scale * p.rowScale[firstRow + lane] : scale;
+        }
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int r = i * 32 + l32;
-            const float rs = SEG ? 1.f : p.rowScale ? scale * p.rowScale[firstRow + r] : scale;
+            const float rs = SEG || ADD ? 1.f : p.rowScale ? scale * p.rowScale[firstRow + r] : scale;
 #pragma unroll
             for (int n = 0; n < 2; ++n) {
 #pragma unroll
@@ -225,7 +232,7 @@ template <int TYPE, int CT, int EPI, bool SEG, bool JOBS = false> __global__ voi
                     float v[4];
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        v[e] = SEG ? facc[i][n][q * 4 + e] : (float)acc[i][n][q * 4 + e] * rs;
+                        v[e] = SEG ? facc[i][n][q * 4 + e] : ADD ? (float)acc[i][n][q * 4 + e] : (float)acc[i][n][q * 4 + e] * rs;
                     }
                     *(float4 *)(mine + r * 256 + (((n * 8 + q * 2 + half) ^ (r & 15)) << 4)) = make_float4(v[0], v[1], v[2], v[3]);
                 }
@@ -238,9 +245,11 @@ template <int TYPE, int CT, int EPI, bool SEG, bool JOBS = false> __global__ voi
             float4 v = *(const float4 *)(mine + r * 256 + ((cc ^ (r & 15)) << 4));
             const bool live = firstRow + r < mLive;
             uint8_t *q = cWave + (int64_t)r * p.ldc + cc * 16;
-            if constexpr (EPI == TS2_EPI_ADD) {
+            if constexpr (ADD) {
+                const float f = rowFactor[r];
                 if (live) {
-                    *(float4 *)q = make_float4(old[it].x + v.x, old[it].y + v.y, old[it].z + v.z, old[it].w + v.w);
+                    *(float4 *)q = make_float4(__builtin_fmaf(v.x, f, old[it].x), __builtin_fmaf(v.y, f, old[it].y), __builtin_fmaf(v.z, f, old[it].z),
+                        __builtin_fmaf(v.w, f, old[it].w));
                 }
             } else {
                 *(float4 *)q = live ? v : make_float4(0, 0, 0, 0);
