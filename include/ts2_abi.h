@@ -370,8 +370,9 @@ int ts2_matmul_forward(int32_t mode, int32_t len, int32_t lenRound, int32_t srcD
  * src/lib/cuda/cuda_matmul.cuh:495-525 and src/gpt/compute/gpu_rope.cuh:25-60): res (TS2_BF16) = rope(normalise(alpha * (*alphaPtr) *
  * src * W^T)), tileScale fp32 [dstDim/128][lenRound] when normalize.  Fused into the product's epilogue where the 256x256-tile kernel
  * applies (lenRound, dstDim multiples of 256, at least 192 tiles).  Otherwise `raw` (fp32 [lenRound][dstDim] scratch) is required: the
- * product goes there and ts2_row_tile_normalize_rope finishes it, unless the kernel for few tiles or, for TS2_E4M3, the 128x128 tile
- * takes the call and leaves raw as it is; the result has the same bits either way but for the contraction of a rotation's products. */
+ * product goes there and ts2_row_tile_normalize_rope finishes it, unless the kernel for few tiles, for TS2_I8 the 256x128 tile or for
+ * TS2_E4M3 the 128x128 tile takes the call and leaves raw as it is.  The result has the same bits either way but for the contraction of a
+ * rotation's products and, on the 128x128 tile, the order in which a row's squares are added (a unit of fp32 in the scale). */
 int ts2_matmul_forward_norm_rope(int32_t mode, int32_t len, int32_t lenRound, int32_t srcDim, int32_t dstDim, const ts2_mat *src,
     const ts2_mat *transformFast, float alpha, const float *alphaPtr, int32_t normalize, float vecScale, const ts2_mat *ropeBuf,
     const ts2_mat *res, const ts2_mat *tileScale, const ts2_mat *raw, void *stream);

@@ -103,3 +103,30 @@ def test_accumulates_with_one_rounding(t, row_scale):
     for c, config in ((got, TALL), (few, 65536)):
         L.load().gemm_nt(a, b, c, t, L.F32, row_scale=rs, alpha=0.3, alpha_ptr=factor, epilogue=L.EPI_ADD, tile_config=config, m_live=m - 9)
     assert torch.equal(got, few)
+
+
+# int8 sums are exact, so that the rows have the bits of a stored product that the stand-alone pass normalises; of a rotation's two products either may
+# be fused with their sum: an fp32 unit of the larger, a bf16 unit of the result at most
+@pytest.mark.parametrize("normalize,rotate", [(True, True), (True, False), (False, True)])
+def test_normalised_rows_are_the_passes(normalize, rotate):
+    print("case tall norm bits", normalize, rotate, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    m, n, k, live = 768, 640, 512, 700
+    a, b = operand(L.I8, m, k, gen), operand(L.I8, n, k, gen)
+    rope = torch.randn((m, 128), device="cuda", generator=gen) if rotate else None
+    lib = L.load()
+    raw = torch.zeros((m, n), device="cuda")
+    lib.gemm_nt(a, b, raw, L.I8, L.F32, alpha=0.3, m_live=live)
+    got, want = [torch.zeros((m, n), dtype=torch.int16, device="cuda") for _ in range(2)]
+    gs, ws = [torch.zeros((n // 128, m), device="cuda") for _ in range(2)]
+    lib.gemm_nt(a, b, got, L.I8, L.BF16, alpha=0.3, epilogue=L.EPI_ROW_TILE_NORM, normalize=normalize, vec_scale=1 / 24, tile_scale=gs, rope=rope, tile_config=TALL,
+                m_live=live)
+    L.call("ts2_row_tile_normalize_rope", live, m, raw, L.F32, 1.0, int(normalize), 1 / 24, rope, want, ws if normalize else None)
+    torch.cuda.synchronize()
+    assert torch.equal(gs, ws)
+    if not rotate:
+        assert torch.equal(got, want)
+        return
+    x, y = got.view(torch.bfloat16).double(), want.view(torch.bfloat16).double()
+    pair = y.view(m, -1, 2).norm(dim=-1, keepdim=True).expand(-1, -1, 2).reshape(m, n)
+    assert bool(((x - y).abs() <= 2.0 ** -7 * y.abs() + 2.0 ** -22 * pair).all()) and float((got != want).double().mean()) < 1e-3

@@ -671,7 +671,7 @@ __device__ __forceinline__ void NormRowValues(const GemmP &p, TAcc (&accRow)[WT]
 // NORM false: the plain 16-bit store (TStoreScaled) through the same staging; F16: IEEE half instead of bf16.
 // WT = 2: the same for the 64x64 wave tile of the 128x128 kernels: rows of 128 bytes, 8 KB of the wave's stage array, eight lanes per
 // row on the way out.  A 128-column tile spans the two waves of a row there: each leaves its 64-column sums of squares in xchg (LDS,
-// 4 x 64 floats outside the staged rows) and adds its neighbour's after one workgroup barrier.
+// 64 floats per wave outside the staged rows) and adds its neighbour's after one workgroup barrier.
 // BLOCKWISE: one block row (32 rows) is staged and stored at a time, so a wave needs 32 x RB bytes of LDS instead of its whole tile.
 template <int TYPE, bool NORM, bool F16, int WTM, int WTN, bool BLOCKWISE = false, class TAcc>
 __device__ __forceinline__ void NormEpilogueRows(const GemmP &p, TAcc (&acc)[WTM][WTN], uint8_t *waveLds, float *xchg, int rowBase, int colBase,
@@ -702,18 +702,38 @@ __device__ __forceinline__ void NormEpilogueRows(const GemmP &p, TAcc (&acc)[WTM
                 if (p.rowScale) {
                     rs *= p.rowScale[firstRow + i * 32 + l32];
                 }
-                float own = 0;
+                auto at = [&](int j, int e) { return live ? (float)acc[i][j][e] * rs : 0.f; };
+                if constexpr (TYPE == T_I8) {
+                    // the association of the stand-alone pass (sums of four columns, then a butterfly over the 32 of them): the products are
+                    // exact, so that the rows do not depend on which of them normalised
+                    float col[WT];
 #pragma unroll
-                for (int j = 0; j < WT; ++j) {
+                    for (int j = 0; j < WT; ++j) {
+                        float four[4];
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        const float x = live ? (float)acc[i][j][e] * rs : 0.f;
-                        own += x * x;
+                        for (int q = 0; q < 4; ++q) {
+                            const float x0 = at(j, q * 4), x1 = at(j, q * 4 + 1), x2 = at(j, q * 4 + 2), x3 = at(j, q * 4 + 3);
+                            float a, b;
+                            LaneSwap32((x0 * x0 + x1 * x1) + (x2 * x2 + x3 * x3), &a, &b);
+                            four[q] = a + b;
+                        }
+                        col[j] = (four[0] + four[1]) + (four[2] + four[3]);
                     }
+                    tileSum2[i] = col[0] + col[1];
+                } else {
+                    float own = 0;
+#pragma unroll
+                    for (int j = 0; j < WT; ++j) {
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) {
+                            const float x = at(j, e);
+                            own += x * x;
+                        }
+                    }
+                    float a, b;
+                    LaneSwap32(own, &a, &b);
+                    tileSum2[i] = a + b;
                 }
-                float a, b;
-                LaneSwap32(own, &a, &b);
-                tileSum2[i] = a + b;
                 if (half == 0) {
                     xchg[wave * 64 + i * 32 + l32] = tileSum2[i];
                 }
