@@ -43,3 +43,30 @@ def test_codes_follow_the_multiplier(final, seed, n, rows, dim, power):
     if power == 7:  # (nothing moved; a row that bf16 rounds to zero keeps the scale 1 that says so)
         slot.scale[(slot.top == 0) & (slot.scale == 1)] = 0
     assert slot.equals_quantiser_of(fast, n)
+
+
+# every width of registers, a workgroup per four rows and walked rows
+@pytest.mark.parametrize("final", [False, True])
+@pytest.mark.parametrize("n,rows,dim", [(999, 1024, 384), (1000, 1024, 896), (333, 384, 1536), (8211, 8320, 512), (1999, 2048, 1024), (1500, 1536, 1408)])
+def test_layer_norm_backward_has_the_bits_of_the_pass(final, n, rows, dim):
+    print("case layer norm backward bits", final, n, rows, dim, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(dim)
+    norm = torch.randint(-127, 128, (rows, dim), device="cuda", generator=gen).to(torch.int8)
+    scale = torch.rand((dim // 128, rows), device="cuda", generator=gen) * 0.01
+    dn, state = [torch.randn((rows, dim), device="cuda", generator=gen) for _ in range(2)]
+    gs, gm = torch.full((1,), 0.25, device="cuda"), torch.full((1,), 4.0, device="cuda")
+    out = []
+    for rows_form in (True, False):
+        st, fast, top = state.clone(), empty(rows, dim), torch.zeros(1, device="cuda")
+        if rows_form:
+            slot, a = Slot(rows, dim, 0), [L.mat(t) for t in (norm, scale, dn, st, fast)]
+            call(LAYER_NORM, C.c_bool(final), n, rows, C.byref(a[0]), C.byref(a[1]), C.byref(a[2]), None if final else p(gs), None if final else p(gm),
+                 C.byref(a[3]), C.byref(a[4]), p(top), C.byref(slot.c))
+        elif final:
+            L.call("ts2_backprop_final_normalize", n, rows, norm, L.I8, scale, dn, st, fast, L.BF16, top)
+        else:
+            L.call("ts2_backprop_layer_normalize", norm, L.I8, scale, dn, None, gs, gm, st, fast, L.BF16, top, n)
+        torch.cuda.synchronize()
+        out.append((st, fast, top))
+    for a, b in zip(*out):
+        assert torch.equal(a, b)

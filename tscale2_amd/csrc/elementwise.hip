@@ -1032,11 +1032,10 @@ __device__ __forceinline__ uint4 Pack8(const F4 &a, const F4 &b)
     return make_uint4(PackBf16x2(a.x, a.y), PackBf16x2(a.z, a.w), PackBf16x2(b.x, b.y), PackBf16x2(b.z, b.w));
 }
 
-// TileNormBackprop of a tile on 16 lanes
-__device__ __forceinline__ void TileNormBackprop8(const F4 (&src)[2], F4 (&g)[2])
+// TileNormBackprop of a tile on 16 lanes; ownSum2, ownDp: the lane's parts of sum(src * src) and sum(src * g)
+__device__ __forceinline__ void TileNormBackprop8(const F4 (&src)[2], F4 (&g)[2], float ownSum2, float ownDp)
 {
-    const float sum2 = Row16Sum(HSum(src[0] * src[0]) + HSum(src[1] * src[1]));
-    const float dp = Row16Sum(HSum(src[0] * g[0]) + HSum(src[1] * g[1]));
+    const float sum2 = Row16Sum(ownSum2), dp = Row16Sum(ownDp);
     if (sum2 == 0) {
         g[0] = g[1] = ZeroF4();
         return;
@@ -1045,6 +1044,11 @@ __device__ __forceinline__ void TileNormBackprop8(const F4 (&src)[2], F4 (&g)[2]
     const float sigma = dp * inv, scale = sqrtf(TILE * inv);
     g[0] = (g[0] - src[0] * sigma) * scale;
     g[1] = (g[1] - src[1] * sigma) * scale;
+}
+
+__device__ __forceinline__ void TileNormBackprop8(const F4 (&src)[2], F4 (&g)[2])
+{
+    TileNormBackprop8(src, g, HSum(src[0] * src[0]) + HSum(src[1] * src[1]), HSum(src[0] * g[0]) + HSum(src[1] * g[1]));
 }
 
 // a row of bf16 values that the wave kept (zeros beyond the live rows), quantised; returns its maximum
@@ -1215,7 +1219,10 @@ __global__ void __launch_bounds__(NT) BackpropLayerNormalizeRows(int len, int le
                 g[0] = g[0] * s;
                 g[1] = g[1] * s;
             }
-            TileNormBackprop8(src, g);
+            // (the products that the compiler fuses in BackpropLayerNormalize, so that the gradients are its bits)
+            auto squares = [](const F4 &a) { return __builtin_fmaf(a.x, a.x, a.y * a.y) + __builtin_fmaf(a.z, a.z, a.w * a.w); };
+            auto dot = [](const F4 &a, const F4 &b) { return __builtin_fmaf(a.y, b.y, a.x * b.x) + __builtin_fmaf(a.w, b.w, a.z * b.z); };
+            TileNormBackprop8(src, g, squares(src[0]) + squares(src[1]), dot(src[0], g[0]) + dot(src[1], g[1]));
             if (!FINAL) {
                 g[0] = g[0] + prev[i][0];
                 g[1] = g[1] + prev[i][1];
