@@ -1267,23 +1267,6 @@ __global__ void __launch_bounds__(256) QuantTileRows(int len, int lenRound, int 
     const int dim = job.dim;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int t0 = blockIdx.x * QT_ROWS, k0 = t0 / kTile * kTile;
-    // units of 8 elements, walked by the whole workgroup: four 16-byte loads in flight per lane, the first four before the maxima
-    const int perRow = dim / 8, units = QT_ROWS * perRow;
-    const unsigned magic = (0x400000u + perRow - 1) / perRow; // u / perRow = u * magic >> 22 for u < units, perRow in 1 .. 512 (a division took half of the pass)
-    uint4 raw[4];
-    float rm[4];
-    int r[4], c[4];
-    auto fetch = [&](int u0) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int u = u0 + k * 256, row = (int)((unsigned)u * magic >> 22);
-            r[k] = u < units ? t0 + row : lenRound;
-            c[k] = (u - row * perRow) * 8;
-            raw[k] = r[k] < len ? *(const uint4 *)At<TBF16>(src, r[k], c[k]) : make_uint4(0, 0, 0, 0);
-            rm[k] = (rowMult && r[k] < len) ? rowMult[r[k]] : 1.f;
-        }
-    };
-    fetch(tid);
     float mx = 0;
     for (int t = k0 + tid; t < k0 + kTile && t < len; t += 256) {
         float m = rowAbsMax[t];
@@ -1302,9 +1285,22 @@ __global__ void __launch_bounds__(256) QuantTileRows(int len, int lenRound, int 
     if (tid == 0 && t0 == k0) {
         job.tileScale[t0 / kTile] = tm > 0 ? tm / 127 : 1.f;
     }
+    // units of 8 elements, walked by the whole workgroup: four 16-byte loads in flight per lane.  (Asked for before the maxima, the first four of them cost
+    // launches of few gradients and of 1024 columns 4-5 %: 16384 x 512, two gradients 14.3 -> 15.1, 8192 x 1024, 24 of them 113 -> 120; 40 of 16384 x 384
+    // and 512 gained 202 -> 188.)
+    const int perRow = dim / 8, units = QT_ROWS * perRow;
+    const unsigned magic = (0x400000u + perRow - 1) / perRow; // u / perRow = u * magic >> 22 for u < units, perRow in 1 .. 512
     for (int u0 = tid; u0 < units; u0 += 1024) {
-        if (u0 != tid) {
-            fetch(u0);
+        uint4 raw[4];
+        float rm[4];
+        int r[4], c[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int u = u0 + k * 256, row = (int)((unsigned)u * magic >> 22);
+            r[k] = u < units ? t0 + row : lenRound;
+            c[k] = (u - row * perRow) * 8;
+            raw[k] = r[k] < len ? *(const uint4 *)At<TBF16>(src, r[k], c[k]) : make_uint4(0, 0, 0, 0);
+            rm[k] = (rowMult && r[k] < len) ? rowMult[r[k]] : 1.f;
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
