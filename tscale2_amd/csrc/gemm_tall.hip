@@ -296,8 +296,9 @@ namespace gemmk
 // 30 to 70 shapes of 1024 to 32768 rows and 256 to 2048 columns in each interval.  Up to 64 tiles the kernel for few tiles is better (0.6 to 0.9
 // of this one's time).
 //   accumulating  4096x1024 (T = 128) K 512 i8 13.7 -> 11.9, e4m3 13.2 -> 12.0; 16384x512 (256) K 256 18.6 -> 14.2, 18.3 -> 14.0, K 2048 31.6 -> 26.2, 30.2 ->
-//                 26.1; T 65 .. 128 i8 0.81-0.96 to K 4096, e4m3 0.83-0.95 to K 1024 (2048 1.01, 4096 1.20); 129 .. 256 0.71-0.93, e4m3 K 4096 0.94-1.05; 257 ..
-//                 448 0.72-0.99 to K 2048 (e4m3 3072 1.08); 449 .. 512 0.72-0.95 to K 1024 (4096 1.16); 513 .. 640 i8 0.61-0.87 to K 2048, e4m3 0.79-0.90 to K 512
+//                 26.1; T 65 .. 128 i8 0.81-0.97 to K 4096 (8192x512 K 1024 1.05), e4m3 K 256 0.87-0.97, 384 0.90-0.98, 512 0.93-1.03, 640 0.94-1.06, 768
+//                 0.97-1.09, 1024 0.96-1.11; 129 .. 256 0.71-0.93, e4m3 K 4096 0.94-1.05; 257 .. 448 0.72-0.99 to K 2048 (e4m3 3072 1.08); 449 .. 512
+//                 0.72-0.95 to K 1024 (4096 1.16); 513 .. 640 i8 0.61-0.87 to K 2048, e4m3 0.79-0.90 to K 512
 //   sums (i8)     two products 16384x512 K 512 25.9 -> 16.9, 16384x1024 53.2 -> 29.9 (two launches before), 8192x512 (128) K 1024 21.6 -> 22.0, 2048 31.8 -> 35.7;
 //                 four 16384x512 K 384 35.2 -> 22.4, 16384x1024 (512) K 512 124.8 -> 48.9 (four launches), 32768x2048 (2048) K 2048 808 -> 632, 4096 1190 -> 1255
 //   normalised    i8: 4096x1024 (128) K 512 13.4 -> 12.6, 16384x384 (192) 19.1 -> 13, 16384x512 (256), product and pass before, 27 -> 13.9; T 65 .. 128 0.89-1.00,
@@ -316,7 +317,7 @@ bool PreferTall(const GemmP &p, int type, int ct, int epi)
         return (p.nSeg > 2 || T > 128 || K <= 1024) && (K <= 2048 || (T > 128 && T <= 256));
     }
     if (epi == TS2_EPI_ADD) {
-        return K <= (T <= 128 ? (i8 ? 4096 : 1024) : T <= 256 ? (i8 ? 4096 : 3072) : T <= 448 ? 2048 : T <= 512 ? 1024 : T <= 640 ? (i8 ? 2048 : 512) : 0);
+        return K <= (T <= 128 ? (i8 ? 4096 : 512) : T <= 256 ? (i8 ? 4096 : 3072) : T <= 448 ? 2048 : T <= 512 ? 1024 : T <= 640 ? (i8 ? 2048 : 512) : 0);
     }
     if (ct == C_BF16NORM) {
         return i8 && K <= (T <= 320 ? 2048 : T <= 448 ? 1024 : T <= 768 ? 512 : 0);
