@@ -1,5 +1,6 @@
 """Calls that the operators refuse before anything is launched.  The arrays are host memory: nothing here may reach a kernel, so the file
 does not run where a GPU is present."""
+import builtins
 import ctypes as C
 
 import pytest
@@ -93,3 +94,24 @@ def test_normalised_forward_wants_its_scratch_below_the_large_tile(mode, rows, c
     m = [L.mat(t) for t in (x, w, res, scale, raw)]
     assert L.load().dll.ts2_matmul_forward_norm_rope(mode, 200, 256, 128, 384, C.byref(m[0]), C.byref(m[1]), C.c_float(1), None, 1, C.c_float(1), None,
                                                      C.byref(m[2]), C.byref(m[3]), C.byref(m[4]) if rows else None, None) == code
+
+
+def test_a_thread_that_finds_the_library_loaded_can_convert_its_arguments(monkeypatch):
+    """load() publishes the library last: a thread that meets another's load half done either loads for itself or has all that a call needs"""
+    seen = []
+
+    lib = L.load()
+    importer = builtins.__import__
+
+    def spy(name, *args, **kw):
+        if name == "torch":
+            seen.append(L._lib is not None)
+            if seen[-1]:
+                L._conv(u8(2, 2))
+        return importer(name, *args, **kw)
+    monkeypatch.setattr(L, "_lib", None)
+    monkeypatch.setattr(L, "_tensor", None)
+    monkeypatch.setattr(L, "Lib", lambda: lib)
+    monkeypatch.setattr(builtins, "__import__", spy)
+    assert L.load() is lib and seen == [False]
+    L._conv(u8(2, 2))

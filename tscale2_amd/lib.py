@@ -111,9 +111,9 @@ _lib = None
 def load():
     global _lib, _tensor
     if _lib is None:
-        _lib = Lib()
         import torch
-        _tensor = torch.Tensor
+        _tensor = torch.Tensor  # (first: another thread that finds the library set goes on to _conv)
+        _lib = Lib()
     return _lib
 
 
