@@ -606,7 +606,9 @@ typedef struct ts2_model_config {
     int32_t vocab, labelCount, maxLen;
     int32_t kTile; /* rows sharing one scale in the int8 delta GEMM (0 = 512) */
     /* 0: every FFN and attention layer keeps what its forward pass computed for its backward pass when that fits into half of the
-     * free device memory; 1: the backward recomputes it, as the reference's AddBackward does (layer_ffn.cu:83-113, layer_att.cu:160-226) */
+     * free device memory; 1: the backward recomputes it, as the reference's AddBackward does (layer_ffn.cu:83-113, layer_att.cu:160-226).
+     * With 0, models of small products also keep every layer's gradients (at most 16 GiB and a quarter of the free memory) and form all
+     * deltas at the end of ts2_model_backprop; e4m3 deltas then have another order of their fp32 sums than without that storage */
     int32_t recompute;
     /* != 0 (TS2_I8 models): the int8 quantisers of every linear backward dither (ts2_matmul_bwd_buffers.ditherSeed), each call under a
      * seed of its own derived from this one and a call counter; 0: round to nearest */

@@ -152,7 +152,8 @@ def test_delta_from_rows_stops_at_the_last_live_one(mode, n, rows):
 @pytest.mark.parametrize("count", [1, 2, 3, 4])
 @pytest.mark.parametrize("c_type,add", [(L.F32, 0), (L.F32, 1), (L.BF16, 0), (L.BF16, 1)])
 def test_sum_of_int8_products(rows, src, count, c_type, add):
-    """up to 640 workgroups of the kernel for few tiles, beyond it the 128x128 tile's sum (fp32, stored) or one product after the other"""
+    """fp32, stored: beyond 64 tiles of 256x128 that tile; else up to 640 workgroups of the kernel for few tiles, beyond it (2176 rows, off the tile's grid) the
+    128x128 tile's sum.  bf16 or added: the kernel for few tiles, beyond it one product after the other"""
     print("case int8 sum", rows, src, count, c_type, add, flush=True)
     gen = generator(rows + src + count)
     grad, n = 384, rows - 29

@@ -1021,6 +1021,7 @@ __global__ void __launch_bounds__(256) NormalizeRowsWave(int len, int lenRound, 
 // 3.5, 5.7 + 3.7 us -> 4.5, 5.7, 4.3; 16384 x 512 (normalisation, gate) 27.3 + 7.6, 28.1 + 12.5 -> 28.7, 24.3; 16384 x 384 (gate; Q, K, V) 16 + 24.6 +
 // 24 -> 16.2, 26.3
 
+// rope pairs are (cos, sin) interleaved: a lane holds two of them
 __device__ __forceinline__ F4 ApplyRope4(F4 v, F4 rope, float dir)
 {
     float s0 = rope.y * dir, s1 = rope.w * dir;
@@ -1564,7 +1565,6 @@ __global__ void __launch_bounds__(256) TransposeBytes(int count, TransposeJobs j
     TransposeOut128<PITCH>(buf, jobs.dst[j], xBlock, tBlock, tid);
 }
 
-// rope pairs are (cos, sin) interleaved: lane holds two pairs
 template <class TSrc>
 __global__ void __launch_bounds__(256) RowTileNormalizeRope(int len, int lenRound, int tiles, Mat src, float srcMult, int normalize, float vecScale,
     Mat rope, Mat dst, Mat tileScale)

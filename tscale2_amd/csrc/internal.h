@@ -31,7 +31,7 @@ struct RowQuantOut {
     uint32_t seed;
 };
 // int8 forms, bf16 gradients, rows of up to 4096: ts2_backprop_row_tile_normalize_lolu (mode 0) / ts2_backprop_lolu_dscale (mode 1, quantises the
-// gate's gradient), ts2_backprop_row_tile_normalize_rope of up to three gradients, ts2_backprop_layer_normalize / ts2_backprop_final_normalize.
+// gate's gradient), ts2_backprop_row_tile_normalize_rope of up to three gradients, ts2_backprop_layer_normalize / ts2_backprop_final_normalize
 // (rows of up to 1536).  TS2_ERR_UNSUPPORTED: nothing was launched
 int Ts2BackpropLoluRows(int mode, int len, int lenRound, const ts2_mat *gate, const ts2_mat *vals, float valsScale, const ts2_mat *valsSrcTileScale,
     const ts2_mat *grad, const ts2_mat *gradGate, const ts2_mat *gradVals, const ts2_mat *dScale, const RowQuantOut &qGate, const RowQuantOut &qVals,

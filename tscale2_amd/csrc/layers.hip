@@ -107,8 +107,8 @@ struct TActs {
 };
 
 // The packed deltas of attention and feed-forward layers are results of a backward pass that nothing in it reads.  While a model's
-// products have few tiles each, they wait for the end of the pass: one launch (per 32 matrices) of the kernel for few tiles then has tiles
-// enough for the whole chip, and int8 quantises all gradients in one launch before it
+// products have few tiles each (DeltasWait), they wait for the end of the pass: one launch of GemmDeltas (per 32 matrices) then has tiles
+// enough for the whole chip, and int8 quantises all gradients in one launch (per 48) before it
 struct TDeltaQueue {
     bool open = false; // inside ModelBackprop of a model that keeps its gradients
     std::vector<gemmk::DeltaJob> deltas;
@@ -289,8 +289,6 @@ int BackpropDX(ts2_model *M, TMatrix &W, const Arr &gradFast, float alpha, bool 
         srcGrad.type, add, s);
 }
 
-// srcGrad (+)= sum_i alpha [* scale_i] * grad_i * W_i for the matrices of a layer that share their input: every weight is transposed
-// into its own part of the transpose scratch, then one grouped Backprop
 // int8: where the row quantiser leaves gradient i of a layer: codes, scales and maxima of slot i of the scratch (maxima: of the layer's own, where
 // its deltas wait)
 float *RowMaxSlot(ts2_model *M, float *rowAbsMax, int i)
@@ -303,6 +301,8 @@ RowQuantOut RowSlot(ts2_model *M, float *rowAbsMax, int i, int width)
     return {M->sGrad8 + (size_t)i * M->R * width, width, M->sRowScale + (size_t)i * M->RP, RowMaxSlot(M, rowAbsMax, i), NextDither(M)};
 }
 
+// srcGrad (+)= sum_i alpha [* scale_i] * grad_i * W_i for the matrices of a layer that share their input: one grouped Backprop over the weights'
+// kept transposes, or over those that it makes, each in its own part of the transpose scratch
 // (int8: the row maxima of gradient i go to RowMaxSlot(rowAbsMax, i); quantised: the passes that wrote the gradients have filled the slots)
 int BackpropDXGroup(ts2_model *M, int count, TMatrix *const *W, const Arr *const *grad, float alpha, const bool *useScale, const Arr &srcGrad,
     bool add, float *rowAbsMax, bool quantised, void *s)
@@ -375,11 +375,6 @@ Arr ColBlock(const Arr &a, int k, int cols)
     return r;
 }
 
-// Deltas alpha * gradScale * grad_i^T * src8 (TMatMulBuffers::BackpropDelta) of `count` matrices of one shape that read the same input, as
-// row blocks of W.delta; W is the layer's stack, or the one matrix.
-// fp8: `grad` holds the gradients side by side ([R][count * width]) and the product reads both operands as they lie.
-// int8: grads[i] are bf16; their row maxima were left in slot i by the dX product that precedes this call (BackpropDXGroup with the
-// same gradients), the k-tile quantiser writes them side by side.
 // A delta whose operands stay as they are until the end of the pass joins the queue (kept).
 bool QueueDelta(ts2_model *M, TMatrix &W, const Arr &src8, const Arr &grad, const float *kTileScale, int kTileScaleRows, float alpha,
     const float *gradScale)
@@ -417,6 +412,9 @@ int RunQueue(ts2_model *M, void *s)
         (hipStream_t)s);
 }
 
+// Deltas alpha * gradScale * grad_i^T * src8 (TMatMulBuffers::BackpropDelta) of matrices of one shape that read the same input, as row blocks of
+// W.delta; W is the layer's stack, or the one matrix.  kept: `src8` and `grad` stay until the end of the pass.
+// fp8: `grad` holds the gradients side by side ([R][count * width]) and the product reads both operands as they lie
 int BackpropDelta(ts2_model *M, TMatrix &W, const Arr &src8, const Arr &grad, float alpha, const float *gradScale, bool kept, void *s)
 {
     if (kept && QueueDelta(M, W, src8, grad, nullptr, 0, alpha, gradScale)) {
@@ -426,7 +424,9 @@ int BackpropDelta(ts2_model *M, TMatrix &W, const Arr &src8, const Arr &grad, fl
         (int64_t)M->sPartialFloats, W.delta.P(), W.deltaTileScale.P(), s);
 }
 
-// keep: the layer whose kept gradients these are (null: none); slot: their first row maxima and scales in it
+// int8: grads[i] are bf16; their row maxima were left in slot i by the dX product that precedes this call (BackpropDXGroup with the same gradients),
+// the k-tile quantiser writes them side by side.  keep: the layer whose kept gradients these are (null: none); slot: their first row maxima and
+// scales in it
 int BackpropDeltaI8(ts2_model *M, int count, TMatrix &stack, TMatrix *const *W, const Arr &src8, const Arr *const *grads, float alpha,
     const float *gradScale, TLayer *keep, int slot, void *s)
 {
