@@ -41,3 +41,24 @@ def test_products_that_share_their_input(mode, count, rows, n, dst, src):
         assert bool(((a - b).abs() <= 2.0 ** -7 * b.abs() + (off + 2.0 ** -18) * 1.5 * largest).all()) and not bool(a[n:].any())
         if norm:
             assert bool(((gs[i] - ws[i]).abs() <= (off + 2.0 ** -20) * ws[i].abs().amax()).all())
+
+
+# whole numbers, so that no order of a product's sum rounds: what single calls store (the kernel for few tiles), scales and rows bit by bit.  65 to 256
+# workgroups of that kernel, K below and above eight steps
+@pytest.mark.parametrize("count,rows,n,dst", [(4, 2048, 1790, 512), (4, 1152, 1152, 768), (2, 4096, 4000, 512), (3, 2304, 2049, 512)])
+@pytest.mark.parametrize("src", [128, 1152])
+def test_e4m3_squares_are_added_as_in_single_calls(count, rows, n, dst, src):
+    print("case forward jobs' squares", count, rows, n, dst, src, flush=True)
+    gen = generator(rows + src + 1)
+    x, *w = [torch.randint(-4, 5, (r, src), device="cuda", generator=gen).float().to(torch.float8_e4m3fn).view(torch.uint8) for r in (rows, *[dst] * count)]
+    new = lambda: ([torch.zeros((rows, dst), dtype=torch.int16, device="cuda") for _ in range(count)],  # noqa: E731
+                   [torch.zeros((dst // 128, rows), device="cuda") for _ in range(count)])
+    (got, gs), (want, ws) = new(), new()
+    pad = lambda a: a + [a[0]] * (4 - count)  # noqa: E731
+    wm, sm = [L.mat(t) for t in w], [L.mat(t) for t in gs]
+    run(FORWARD_GROUP, L.E4M3, count, n, rows, src, dst, x, mat_pointers(pad(wm)), 0.01, pointers([None] * 4), (1 << count) - 1, 1 / 24, 0,
+        torch.zeros((rows, 128), device="cuda"), mats(pad(got)), mat_pointers(pad(sm)))
+    raw = torch.empty((rows, dst), device="cuda")
+    for i in range(count):
+        L.call("ts2_matmul_forward_norm_rope", L.E4M3, n, rows, src, dst, x, w[i], 0.01, None, 1, 1 / 24, None, want[i], ws[i], raw)
+        assert want[i][:n].any() and torch.equal(got[i], want[i]) and torch.equal(gs[i], ws[i])

@@ -319,7 +319,7 @@ __global__ void __launch_bounds__(64 * WM * WN, (WM * WN) / 4) GemmNTDirect(Gemm
     __syncthreads();
     if constexpr (SWAPC) {
         uint8_t *waveLds = wave == 0 ? sA0 : wave == 1 ? sB0 : wave == 2 ? sA1 : sB1;
-        NormEpilogueRows<TYPE, CT == C_BF16NORM, CT == C_F16, 2, 2>(p, acc, waveLds, (float *)(sA0 + 8192), rowBase, colBase, wm, wn, lane);
+        NormEpilogueRows<TYPE, CT == C_BF16NORM, CT == C_F16, 2, 2, false, JOBS>(p, acc, waveLds, (float *)(sA0 + 8192), rowBase, colBase, wm, wn, lane);
     } else {
         Epilogue<TYPE, WTM, WTN, CT, EPI, KT>(p, acc, facc, sA0, rowBase, colBase, wm, wn, half, l32);
     }
@@ -687,7 +687,7 @@ __global__ void __launch_bounds__(256, WT == 4 ? 1 : 2) GemmNTRing(GemmP p)
         if constexpr (CT == C_I8PACK) {
             PackEpilogueRows(p, acc, waveLds, rowBase, colBase, wm, wn, lane);
         } else {
-            NormEpilogueRows<TYPE, CT == C_BF16NORM, CT == C_F16, WT, WT>(p, acc, waveLds, (float *)sB1, rowBase, colBase, wm, wn, lane);
+            NormEpilogueRows<TYPE, CT == C_BF16NORM, CT == C_F16, WT, WT, false, JOBS>(p, acc, waveLds, (float *)sB1, rowBase, colBase, wm, wn, lane);
         }
     } else {
         Epilogue<TYPE, WTM, WTN, CT, EPI, false>(p, acc, facc, sA0, rowBase, colBase, wm, wn, half, l32);

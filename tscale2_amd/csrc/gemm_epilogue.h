@@ -673,7 +673,8 @@ __device__ __forceinline__ void NormRowValues(const GemmP &p, TAcc (&accRow)[WT]
 // row on the way out.  A 128-column tile spans the two waves of a row there: each leaves its 64-column sums of squares in xchg (LDS,
 // 64 floats per wave outside the staged rows) and adds its neighbour's after one workgroup barrier.
 // BLOCKWISE: one block row (32 rows) is staged and stored at a time, so a wave needs 32 x RB bytes of LDS instead of its whole tile.
-template <int TYPE, bool NORM, bool F16, int WTM, int WTN, bool BLOCKWISE = false, class TAcc>
+// JOBS: products of at most a round of the kernel for few tiles, which one call of them runs on, add their squares in that kernel's order.
+template <int TYPE, bool NORM, bool F16, int WTM, int WTN, bool BLOCKWISE = false, bool JOBS = false, class TAcc>
 __device__ __forceinline__ void NormEpilogueRows(const GemmP &p, TAcc (&acc)[WTM][WTN], uint8_t *waveLds, float *xchg, int rowBase, int colBase,
     int wm, int wn, int lane)
 {
@@ -695,6 +696,7 @@ __device__ __forceinline__ void NormEpilogueRows(const GemmP &p, TAcc (&acc)[WTM
     if constexpr (NORM && WT == 2) {
         if (p.normalize) { // (uniform over the workgroup)
             const int wave = wm * 2 + wn;
+            const bool passOrder = TYPE == T_I8 || (JOBS && (int64_t)p.m * p.n <= 256 * 64 * 128);
 #pragma unroll
             for (int i = 0; i < WTM; ++i) {
                 const bool live = firstRow + i * 32 + l32 < mLive;
@@ -703,9 +705,9 @@ __device__ __forceinline__ void NormEpilogueRows(const GemmP &p, TAcc (&acc)[WTM
                     rs *= p.rowScale[firstRow + i * 32 + l32];
                 }
                 auto at = [&](int j, int e) { return live ? (float)acc[i][j][e] * rs : 0.f; };
-                if constexpr (TYPE == T_I8) {
-                    // the association of the stand-alone pass (sums of four columns, then a butterfly over the 32 of them): the products are
-                    // exact, so that the rows do not depend on which of them normalised
+                if (passOrder) {
+                    // the association of the stand-alone pass (sums of four columns, then a butterfly over the 32 of them): the rows do not depend
+                    // on which of them normalised
                     float col[WT];
 #pragma unroll
                     for (int j = 0; j < WT; ++j) {
