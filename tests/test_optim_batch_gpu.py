@@ -47,7 +47,7 @@ def apply(jobs):
 # scales formed by the conversion; by a launch of their own (a tall matrix first, last); alone on either side of both lines; more than one launch takes
 @pytest.mark.parametrize("shapes", [
     [(1, 128), (130, 512), (64, 256), (1000, 384)], [(4097, 256), (1, 512), (257, 384)], [(300, 384), (4096, 256)], [(8192, 2048), (8193, 2048), (127, 1536)],
-    [(64, 4096), (200, 2176)], [(128 + 3 * i, 128) for i in range(17)]])
+    [(64, 4096), (200, 2176)], [(128 + 3 * i, 128) for i in range(17)], [(5793, 256), (1, 512), (257, 384)], [(8193, 256), (64, 128)]])
 def test_matrices_of_unequal_height(shapes):
     print("case optimiser batch", shapes, flush=True)
     make = lambda: [Job(r, c, (L.I8, L.E4M3)[i & 1], i) for i, (r, c) in enumerate(shapes)]  # noqa: E731

@@ -425,14 +425,19 @@ int RowGrid(int rows)
 }
 
 // Whether the workgroups of the conversion form the scales: together they read the square of the rows from L2, a launch of its own reads the
-// rows once and costs 1.2 us (more outside a graph).  Own against separate launch, us in a graph, by the sum S of the squares:
-//   S <= 2^24   300x512 7.0, 8.1; 2048x1024 11.2, 12.2; 4096x512 12.0, 12.4; 4096x1024 18.0, 18.7; 16 of 1024x1024 60.2, 61.2
-//   S <= 2^26   2048 columns and more 8192x2048 60.7, 61.3; 8192x4096 117.1, 119.1; 8 of 2048x2048 114.5, 116.5; fewer 8192x512 21.1, 20.9; 16 of
-//               2048x512 64.0, 61.6; 8 of 4096x1024 119.4, 116.4 (2^27)
-//   beyond      12288x1024 53.2, 49.9; 32768x256 71.5, 43.0; 50304x2048 beside 15 of 8192x2048 1532, 1511, beside 15 of 2048x2048 747, 726
-bool OwnScale(double squares, int minX)
+// rows once and costs 1.2 us (3 to 4 where calls follow each other faster than the device).  Own against separate launch, us a launch sequence, by the
+// sum S of the squares:
+//   one matrix  4096x256 10.8, 11.7; 4410x256 11.4, 12.2; 8192x256 15.6, 15.7; 5000x1024 22.1, 23.3; 8192x1024 35.1, 35.2; 8192x2048 69.3, 71.3; 8192x512 21.2,
+//               21.0 (2^26); 12288x1024 53.2, 49.9; 32768x256 71.5, 43.0
+//   S = 2^24    16 of 1024x1024 60.2, 61.2
+//   S = 2^25    2 of 4096x512 17.6, 18.5; 4 of 3000x512 27.2, 27.1; 8 of 2048x512 34.4, 34.1; 16 of 1450x512 46.5, 45.9; 2 of 4096x1024 33.7, 34.3; 16 of
+//               1450x1024 81.7, 82.5
+//   S = 2^26    2 of 5800x512 27.7, 26.9; 4 of 4096x512 36.6, 34.7; 4 of 4096x1024 62.3, 61.0; 16 of 2048x512 64.0, 61.6; 16 of 2048x1024 115.9, 116.2
+//   2048 columns and more  8 of 2048x2048 (2^25) 114.5, 116.5; 8192x4096 (2^26) 117.1, 119.1; 50304x2048 beside 15 of 8192x2048 1532, 1511, beside 15 of
+//               2048x2048 747, 726
+bool OwnScale(int count, double squares, int minX)
 {
-    return squares <= (minX >= 2048 ? 1 << 26 : 1 << 24);
+    return squares <= (count == 1 || minX >= 2048 ? 1 << 26 : 1 << 25);
 }
 
 bool F32Ok(const ts2_mat *m, int x, int y)
@@ -638,7 +643,7 @@ int Ts2OptApplyBatch(int count, const ts2_opt_matrix *const *mats, const ts2_mat
         }
         TS2_CHECK_LAUNCH();
         const dim3 grid(RowGrid((maxBuf + 3) / 4), n);
-        if (OwnScale(squares, minX)) {
+        if (OwnScale(n, squares, minX)) {
             hipLaunchKernelGGL(OptConvert<true>, grid, dim3(256), 0, STREAM, jobs, params);
         } else {
             hipLaunchKernelGGL(OptScale, dim3(n), dim3(1024), 0, STREAM, jobs, params);
