@@ -24,17 +24,6 @@ constexpr int DGROUP = 4;        // tile rows that are walked together
 
 typedef __attribute__((address_space(3))) uint8_t *TLds3;
 
-__device__ __forceinline__ v4i DeltaRsrc(const uint8_t *base, int bytes)
-{
-    const uint64_t u = (uint64_t)(uintptr_t)base;
-    v4i r;
-    r[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)u);
-    r[1] = __builtin_amdgcn_readfirstlane((int)((u >> 32) & 0xffff));
-    r[2] = __builtin_amdgcn_readfirstlane(bytes);
-    r[3] = 0x00020000;
-    return r;
-}
-
 template <int TYPE> __global__ void __launch_bounds__(512, 2) GemmDeltas(DeltaBatchP bp)
 {
     typedef typename AccT<TYPE>::type TAcc;
@@ -80,22 +69,20 @@ template <int TYPE> __global__ void __launch_bounds__(512, 2) GemmDeltas(DeltaBa
             bOff[i] = rr * ldb + (((sb >> 1) ^ ((rr >> 1) & 3)) << 5) + (sb & 1) * 16;
         }
     }
-#define DELTA_LOAD(M0VAL, VOFF, RSRC)                                                                                                      \
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(M0VAL), "v"(VOFF), "s"(RSRC) : "memory")
     const int live = KT ? bp.kBytes : bp.kLive; // (i8: rows beyond the live ones hold zeros)
     const int steps = (live + DK - 1) / DK;
     auto loadStep = [&](int step, int stage) {
         const unsigned st = ldsBase + stage * DSTAGE;
         const int k0 = step * DK, rows = min(live - k0, DK); // later rows read as zeros: the descriptor ends there
-        const v4i ra = DeltaRsrc(d.grad + (int64_t)k0 * lda + rowBase, (rows - 1) * lda + rowsHere);
-        const v4i rb = DeltaRsrc(d.src + (int64_t)k0 * ldb + colBase, (rows - 1) * ldb + DBN);
+        const v4i ra = BufferRsrc(d.grad + (int64_t)k0 * lda + rowBase, (rows - 1) * lda + rowsHere);
+        const v4i rb = BufferRsrc(d.src + (int64_t)k0 * ldb + colBase, (rows - 1) * ldb + DBN);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            DELTA_LOAD(st + (wave + 8 * i) * 1024, aOff[i], ra);
+            TS2_LOAD_LDS16(st + (wave + 8 * i) * 1024, aOff[i], ra);
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            DELTA_LOAD(st + DA + (wave + 8 * i) * 1024, bOff[i], rb);
+            TS2_LOAD_LDS16(st + DA + (wave + 8 * i) * 1024, bOff[i], rb);
         }
     };
 

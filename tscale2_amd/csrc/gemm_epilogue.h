@@ -72,6 +72,22 @@ __device__ __forceinline__ void PickJob(GemmP &p)
     p.rope = ((p.jobRope >> j) & 1) ? p.rope : nullptr;
 }
 
+// descriptor of buffer loads (uniform over the wave): `bytes` bytes from `base` on, beyond them the loads read zeros
+__device__ __forceinline__ v4i BufferRsrc(const uint8_t *base, int bytes = 0x7fffffff)
+{
+    const uint64_t u = (uint64_t)(uintptr_t)base;
+    v4i r;
+    r[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)u);
+    r[1] = __builtin_amdgcn_readfirstlane((int)((u >> 32) & 0xffff));
+    r[2] = __builtin_amdgcn_readfirstlane(bytes);
+    r[3] = 0x00020000;
+    return r;
+}
+
+// 16 bytes of each lane, at VOFF of RSRC, to LDS address LDSADDR + lane * 16, without registers; counted by vmcnt
+#define TS2_LOAD_LDS16(LDSADDR, VOFF, RSRC)                                                                                                \
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(LDSADDR), "v"(VOFF), "s"(RSRC) : "memory")
+
 enum { T_I8 = 0, T_FP8 = 1, T_BF16 = 2 };
 enum { C_F32 = 0, C_BF16 = 1, C_I32 = 2, C_I8PACK = 3, C_BF16NORM = 4, C_F16 = 5 };
 

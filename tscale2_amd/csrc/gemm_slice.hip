@@ -29,17 +29,6 @@ constexpr int NSTAGE = 3;
 
 typedef __attribute__((address_space(3))) uint8_t *TLds3;
 
-__device__ __forceinline__ v4i SliceRsrc(const uint8_t *base, int bytes)
-{
-    const uint64_t u = (uint64_t)(uintptr_t)base;
-    v4i r;
-    r[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)u);
-    r[1] = __builtin_amdgcn_readfirstlane((int)((u >> 32) & 0xffff));
-    r[2] = __builtin_amdgcn_readfirstlane(bytes);
-    r[3] = 0x00020000;
-    return r;
-}
-
 template <int TYPE, bool TN, bool KT = false> __global__ void __launch_bounds__(512, 2) GemmSlice(SliceP sp)
 {
     typedef typename AccT<TYPE>::type TAcc;
@@ -185,8 +174,6 @@ template <int TYPE, bool TN, bool KT = false> __global__ void __launch_bounds__(
             bOff[i] = ((wave + 8 * i) * 4 + rb) * ldb + cb;
         }
     }
-#define SLICE_LOAD(M0VAL, VOFF, RSRC)                                                                                                      \
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(M0VAL), "v"(VOFF), "s"(RSRC) : "memory")
     const int kLive = sp.kLive;
     auto loadStep = [&](const uint8_t *a, const uint8_t *b, int step, int stage) {
         const unsigned st = ldsBase + stage * STAGE;
@@ -194,18 +181,18 @@ template <int TYPE, bool TN, bool KT = false> __global__ void __launch_bounds__(
         int cut = 0;
         if constexpr (KT) {
             const int64_t k0 = (int64_t)kt0 * p.kTileBytes + step * 64;
-            ra = SliceRsrc(TN ? a + k0 * p.lda + rowBase : a + (int64_t)rowBase * p.lda + k0, 0x7fffffff);
-            rb = SliceRsrc(TN ? b + k0 * p.ldb + colBase : b + (int64_t)colBase * p.ldb + k0, 0x7fffffff);
+            ra = BufferRsrc(TN ? a + k0 * p.lda + rowBase : a + (int64_t)rowBase * p.lda + k0);
+            rb = BufferRsrc(TN ? b + k0 * p.ldb + colBase : b + (int64_t)colBase * p.ldb + k0);
         } else if constexpr (TN) {
             const int k0 = kBeg * (BKB / ESZ) + step * KR;
             // rows of this step that belong to the slice and are live
             const int rows = min(min(kBeg * (BKB / ESZ) + kUnits * (BKB / ESZ), kLive) - k0, KR);
-            ra = SliceRsrc(a + (int64_t)k0 * p.lda + rowBase * ESZ, rows > 0 ? (rows - 1) * lda + SBM * ESZ : 0);
-            rb = SliceRsrc(b + (int64_t)k0 * p.ldb + colBase * ESZ, rows > 0 ? (rows - 1) * ldb + SBN * ESZ : 0);
+            ra = BufferRsrc(a + (int64_t)k0 * p.lda + rowBase * ESZ, rows > 0 ? (rows - 1) * lda + SBM * ESZ : 0);
+            rb = BufferRsrc(b + (int64_t)k0 * p.ldb + colBase * ESZ, rows > 0 ? (rows - 1) * ldb + SBN * ESZ : 0);
         } else {
             const int64_t k0 = (int64_t)kBeg * BKB + (int64_t)step * SK;
-            ra = SliceRsrc(a + (int64_t)rowBase * p.lda + k0, 0x7fffffff);
-            rb = SliceRsrc(b + (int64_t)colBase * p.ldb + k0, 0x7fffffff);
+            ra = BufferRsrc(a + (int64_t)rowBase * p.lda + k0);
+            rb = BufferRsrc(b + (int64_t)colBase * p.ldb + k0);
             // the upper half of a 128-byte last step is not multiplied: its lanes fetch the lower half again
             cut = (oddTail && step == nSteps - 1) ? 1 : 0;
         }
@@ -216,7 +203,7 @@ template <int TYPE, bool TN, bool KT = false> __global__ void __launch_bounds__(
                 const int rr = (wave + 8 * i) * 4 + (lane >> 4);
                 off -= ((((lane & 15) ^ (rr & 15)) >> 3) & 1) * 128;
             }
-            SLICE_LOAD(st + (wave + 8 * i) * 1024, off, ra);
+            TS2_LOAD_LDS16(st + (wave + 8 * i) * 1024, off, ra);
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -225,7 +212,7 @@ template <int TYPE, bool TN, bool KT = false> __global__ void __launch_bounds__(
                 const int rr = (wave + 8 * i) * 4 + (lane >> 4);
                 off -= ((((lane & 15) ^ (rr & 15)) >> 3) & 1) * 128;
             }
-            SLICE_LOAD(st + SA + (wave + 8 * i) * 1024, off, rb);
+            TS2_LOAD_LDS16(st + SA + (wave + 8 * i) * 1024, off, rb);
         }
     };
 

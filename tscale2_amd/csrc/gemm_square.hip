@@ -18,17 +18,6 @@ constexpr int QSTAGES = 4, QPART = QT * QT * 4;
 
 typedef __attribute__((address_space(3))) uint8_t *TLds3;
 
-__device__ __forceinline__ v4i SquareRsrc(const uint8_t *base)
-{
-    const uint64_t u = (uint64_t)(uintptr_t)base;
-    v4i r;
-    r[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)u);
-    r[1] = __builtin_amdgcn_readfirstlane((int)((u >> 32) & 0xffff));
-    r[2] = 0x7fffffff;
-    r[3] = 0x00020000;
-    return r;
-}
-
 // CT: C_F32 or C_BF16; ADD: accumulate; SEG (fp8): p.nSeg products in one set of accumulators, brought to the next product's factor at each seam
 template <int TYPE, int CT, bool ADD, bool SEG> __global__ void __launch_bounds__(512, 2) GemmSquare(GemmP p)
 {
@@ -85,8 +74,6 @@ template <int TYPE, int CT, bool ADD, bool SEG> __global__ void __launch_bounds_
         bOff[i] = rr * ldb + ch * 16;
         back[i] = (ch >> 3) * 128;
     }
-#define SQUARE_LOAD(M0VAL, VOFF, RSRC)                                                                                                     \
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(M0VAL), "v"(VOFF), "s"(RSRC) : "memory")
     auto aOf = [&](int seg) { return !SEG || seg == 0 ? p.a : seg == 1 ? p.segA[0] : seg == 2 ? p.segA[1] : p.segA[2]; };
     auto bOf = [&](int seg) { return !SEG || seg == 0 ? p.b : seg == 1 ? p.segB[0] : seg == 2 ? p.segB[1] : p.segB[2]; };
     auto factorOf = [&](int seg) -> float {
@@ -115,17 +102,17 @@ template <int TYPE, int CT, bool ADD, bool SEG> __global__ void __launch_bounds_
     auto loadNext = [&]() {
         const int seg = loadList & 3;
         const int64_t k0 = (int64_t)loadStepNo * QK;
-        const v4i ra = SquareRsrc(aOf(seg) + (int64_t)rowBase * p.lda + k0), rb = SquareRsrc(bOf(seg) + (int64_t)colBase * p.ldb + k0);
+        const v4i ra = BufferRsrc(aOf(seg) + (int64_t)rowBase * p.lda + k0), rb = BufferRsrc(bOf(seg) + (int64_t)colBase * p.ldb + k0);
         const unsigned st = ldsBase + loadStage * QSTAGE;
         // the upper half of a 128-byte last step is not multiplied: its lanes fetch the lower half again
         const bool cut = oddTail && loadStepNo == nSteps - 1;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            SQUARE_LOAD(st + (wave + 8 * i) * 1024, aOff[i] - (cut ? back[i] : 0), ra);
+            TS2_LOAD_LDS16(st + (wave + 8 * i) * 1024, aOff[i] - (cut ? back[i] : 0), ra);
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            SQUARE_LOAD(st + QA + (wave + 8 * i) * 1024, bOff[i] - (cut ? back[i] : 0), rb);
+            TS2_LOAD_LDS16(st + QA + (wave + 8 * i) * 1024, bOff[i] - (cut ? back[i] : 0), rb);
         }
         loadStage = loadStage == QSTAGES - 1 ? 0 : loadStage + 1;
         if (++loadStepNo == nSteps) {

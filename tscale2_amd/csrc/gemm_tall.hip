@@ -19,17 +19,6 @@ constexpr int TA = TBM * BKB, TSTAGE = (TBM + TBN) * BKB, TSTAGES = 3;
 
 typedef __attribute__((address_space(3))) uint8_t *TLds3;
 
-__device__ __forceinline__ v4i TallRsrc(const uint8_t *base)
-{
-    const uint64_t u = (uint64_t)(uintptr_t)base;
-    v4i r;
-    r[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)u);
-    r[1] = __builtin_amdgcn_readfirstlane((int)((u >> 32) & 0xffff));
-    r[2] = 0x7fffffff;
-    r[3] = 0x00020000;
-    return r;
-}
-
 // SEG (i8, fp32 result): p.nSeg products, each with row scales of its own, added in fp32 in their order
 // JOBS: blockIdx.z picks one of several products (GemmP)
 template <int TYPE, int CT, int EPI, bool SEG, bool JOBS = false> __global__ void __launch_bounds__(512, 2) GemmTall(GemmP p)
@@ -64,8 +53,6 @@ template <int TYPE, int CT, int EPI, bool SEG, bool JOBS = false> __global__ voi
         }
     }
     const int64_t aTile = (int64_t)rowBase * p.lda, bTile = (int64_t)colBase * p.ldb;
-#define TALL_LOAD(M0VAL, VOFF, RSRC)                                                                                                       \
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(M0VAL), "v"(VOFF), "s"(RSRC) : "memory")
     int loadStepNo = 0, loadSeg = 0, loadStage = 0, loaded = 0;
     auto loadNext = [&]() {
         const uint8_t *a = p.a, *b = p.b;
@@ -74,14 +61,14 @@ template <int TYPE, int CT, int EPI, bool SEG, bool JOBS = false> __global__ voi
             b = loadSeg == 0 ? p.b : loadSeg == 1 ? p.segB[0] : loadSeg == 2 ? p.segB[1] : p.segB[2];
         }
         const unsigned st = ldsBase + loadStage * TSTAGE;
-        const v4i ra = TallRsrc(a + aTile + (int64_t)loadStepNo * BKB), rb = TallRsrc(b + bTile + (int64_t)loadStepNo * BKB);
+        const v4i ra = BufferRsrc(a + aTile + (int64_t)loadStepNo * BKB), rb = BufferRsrc(b + bTile + (int64_t)loadStepNo * BKB);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            TALL_LOAD(st + (wave + 8 * i) * 1024, aOff[i], ra);
+            TS2_LOAD_LDS16(st + (wave + 8 * i) * 1024, aOff[i], ra);
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            TALL_LOAD(st + TA + (wave + 8 * i) * 1024, bOff[i], rb);
+            TS2_LOAD_LDS16(st + TA + (wave + 8 * i) * 1024, bOff[i], rb);
         }
         ++loaded;
         loadStage = loadStage == TSTAGES - 1 ? 0 : loadStage + 1;
