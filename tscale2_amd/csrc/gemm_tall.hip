@@ -283,13 +283,14 @@ namespace gemmk
 // 30 to 70 shapes of 1024 to 32768 rows and 256 to 2048 columns in each interval.  Up to 64 tiles the kernel for few tiles is better (0.6 to 0.9
 // of this one's time).
 //   accumulating  4096x1024 (T = 128) K 512 i8 13.7 -> 11.9, e4m3 13.2 -> 12.0; 16384x512 (256) K 256 18.6 -> 14.2, 18.3 -> 14.0, K 2048 31.6 -> 26.2, 30.2 ->
-//                 26.1; T 65 .. 128 i8 0.81-0.97 to K 4096 (8192x512 K 1024 1.05), e4m3 K 256 0.87-0.97, 384 0.90-0.98, 512 0.93-1.03, 640 0.94-1.06, 768
-//                 0.97-1.09, 1024 0.96-1.11; 129 .. 256 0.71-0.93, e4m3 K 4096 0.94-1.05; 257 .. 448 0.72-0.99 to K 2048 (e4m3 3072 1.08); 449 .. 512
+//                 26.1; T 65 .. 128 i8 K 256 0.83-0.90, 512 0.89-0.99, 1024 0.89-1.13, 1536 0.99-1.14, 2048 0.98-1.22 (4096x640 15.3 -> 18.7), 3072 to T = 96 0.93-1.09,
+//                 beyond 0.91-0.93, 4096 0.92-0.97, e4m3 K 256 0.85-0.97, 384 0.90-0.98, 512 0.91-1.03, 640 0.94-1.06, 768 0.97-1.09, 1024 0.96-1.11; 129 .. 256 0.71-0.93, e4m3 K 4096 0.94-1.05; 257 .. 448 0.72-0.99 to K 2048 (e4m3 3072 1.08); 449 .. 512
 //                 0.72-0.95 to K 1024 (4096 1.16); 513 .. 640 i8 0.61-0.87 to K 2048, e4m3 0.79-0.90 to K 512
 //   sums (i8)     two products 16384x512 K 512 25.9 -> 16.9, 16384x1024 53.2 -> 29.9 (two launches before), 8192x512 (128) K 1024 21.6 -> 22.0, 2048 31.8 -> 35.7;
 //                 four 16384x512 K 384 35.2 -> 22.4, 16384x1024 (512) K 512 124.8 -> 48.9 (four launches), 32768x2048 (2048) K 2048 808 -> 632, 4096 1190 -> 1255
 //   normalised    i8: 4096x1024 (128) K 512 13.4 -> 12.6, 16384x384 (192) 19.1 -> 13, 16384x512 (256), product and pass before, 27 -> 13.9; T 65 .. 128 0.89-1.00,
-//                 129 .. 320 0.47-0.83 to K 2048, 321 .. 448 0.61-0.95 to K 1024 (2048 1.03), 449 .. 768 0.59-0.89 to K 512 (1024 1.06)
+//                 129 .. 320 0.34-0.83 to K 2048, 321 .. 448 0.45-0.65 to K 1024 (2048 1.03), 449 .. 768 0.59-0.89 to K 512 (1024 1.06); where 256x256 tiles fill
+//                 the chip (T from 384 on, whole ones) 384 .. 448 K 256 0.94-0.97, 512 1.00-1.03, 768 1.05-1.08, 1024 1.05-1.10, 449 .. 768 K 256 0.82-0.96, 512 0.86-0.99
 //   stored fp32   T 65 .. 768 K 256, 512 i8 0.75-0.99, e4m3 0.84-1.02; K 1024 0.92-1.30, 0.99-1.40
 //   stored bf16   i8: T 129 .. 256 0.90-1.01 to K 2048; 449 .. 768 K 256, 512 0.71-1.01; e4m3 (and others) equal or worse
 bool PreferTall(const GemmP &p, int type, int ct, int epi)
@@ -304,10 +305,14 @@ bool PreferTall(const GemmP &p, int type, int ct, int epi)
         return (p.nSeg > 2 || T > 128 || K <= 1024) && (K <= 2048 || (T > 128 && T <= 256));
     }
     if (epi == TS2_EPI_ADD) {
-        return K <= (T <= 128 ? (i8 ? 4096 : 512) : T <= 256 ? (i8 ? 4096 : 3072) : T <= 448 ? 2048 : T <= 512 ? 1024 : T <= 640 ? (i8 ? 2048 : 512) : 0);
+        if (T <= 128) {
+            return K <= 512 || (i8 && K >= (T <= 96 ? 4096 : 3072) && K <= 4096);
+        }
+        return K <= (T <= 256 ? (i8 ? 4096 : 3072) : T <= 448 ? 2048 : T <= 512 ? 1024 : T <= 640 ? (i8 ? 2048 : 512) : 0);
     }
     if (ct == C_BF16NORM) {
-        return i8 && K <= (T <= 320 ? 2048 : T <= 448 ? 1024 : T <= 768 ? 512 : 0);
+        const bool large = T >= 384 && p.n % 256 == 0;
+        return i8 && K <= (T <= 320 ? 2048 : T <= 448 ? (large ? 256 : 1024) : T <= 768 ? 512 : 0);
     }
     if (ct == C_F32) {
         return T <= 768 && K <= 512;
