@@ -1148,9 +1148,10 @@ bool PreferSlice(const GemmP &p, int type, int ct, int epi)
 
 // Products that share A as one launch of the kernels for more tiles.  By the 128x128 tiles T of one product and the bytes K of the contraction, measured
 // in a graph of 40 launches against the launch of gemm_slice.hip (us, four products; with 256 workgroups of that kernel in all it is better, 5.5
-// to 11.5 against 6.9 to 12.7, with 512 it is not but for i8 at T = 64, and up to one and a half rounds the results are those of single calls bit by bit):
-//   T = 64   e4m3 1024x1024 K 512 12.4 -> 9.4, K 1024 15.2 -> 10.7, K 2048 21.5 -> 15.0; i8 0.98 at K 256, 1.01 at 512, 0.97-1.05 at 1024,
-//            1.01-1.04 at 2048
+// to 11.5 against 6.9 to 12.7, with 512 it is not but for i8 at T = 64 and K > 256, and up to one and a half rounds the results are those of single
+// calls bit by bit):
+//   T = 64   e4m3 1024x1024 K 512 12.4 -> 9.4, K 1024 15.2 -> 10.7, K 2048 21.5 -> 15.0; i8 0.98 at K 256 (1024x896 inside a step 14.2 -> 12.3),
+//            1.01 at 512, 0.97-1.05 at 1024, 1.01-1.04 at 2048
 //   T = 96   i8 4096x384 K 256 16.6 -> 12.0, K 2048 30.4 -> 23.4
 //   T = 128  4096x512 e4m3 K 512 22.4 -> 10.9 (two products 12.0 -> 7.7), K 1024 28.6 -> 15.7; i8 22.8 -> 13.7 (12.1 -> 9.3), 28.7 -> 18.0
 // and beyond its range against one launch per product:
@@ -1160,7 +1161,7 @@ bool gemmk::PreferJobs(const GemmP &p, int type)
 {
     const int64_t T = (int64_t)(p.m / 128) * (p.n / 128);
     const int K = p.kBytes;
-    if (2 * T * p.jobs <= 384 || (type == T_I8 && T <= 64)) {
+    if (2 * T * p.jobs <= 384 || (type == T_I8 && T <= 64 && K > 256)) {
         return false;
     }
     if (type == T_FP8) {
